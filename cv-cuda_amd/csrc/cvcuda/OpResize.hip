@@ -9,7 +9,7 @@
 // point on those indices and weights (bilinear: FixedPointBlend.hpp; bicubic: kFixedCubic; box filter:
 // kAreaFixed), at most 1 from the reference's goldens.
 //
-// Six kernel shapes, all with streaming stores, var-shape batches on a packed tile grid:
+// Seven kernel shapes, all with streaming stores, var-shape batches on a packed tile grid:
 //  * pixels of up to 8 bytes: wave patches (64 columns x 4 rows per wave; adjacent taps in one load,
 //    row terms computed once per wave, 4x4 lane transposes so that every lane stores whole dwords);
 //  * 8-bit bilinear at horizontal scales up to 2: a lane owns 2 columns x 4 rows (image batches x 2; 4 x 8 when
@@ -21,6 +21,8 @@
 //  * bicubic reductions >= 2x of 12/16-byte pixels: tap-major loads exchanged through LDS;
 //  * AREA of 8-bit pixels at reductions of up to 3: fixed-point row sums, a wave owns 64 columns x 16 rows and
 //    produces vertically adjacent rows in pairs from the source rows they share;
+//  * bilinear one-channel float tensors whose rows are not reduced, launches of 512 blocks and more: whole rows
+//    gathered in LDS and written out on 64-byte boundaries;
 //  * everything else (12/16-byte pixels, other AREA): one lane per output pixel, a 256-thread block covers
 //    64 columns x 4 rows, pixels moved as whole C-channel vectors.
 #include "DeviceUtils.hpp"
@@ -3088,6 +3090,133 @@ __global__ __launch_bounds__(256) void ResizeCubicStagedKernel(const ResizeArgs 
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Bilinear resize of one-channel float pixels where rows are not reduced (maps and masks brought to their frames'
+// size). Bound by the output's writes. Rows of such outputs rarely start at a multiple of 64 bytes (a dense row of 1917
+// floats), and then every store instruction of a wave ends in two partly written 64-byte sectors that its neighbours
+// complete in stores of their own: 3.78 M write requests where the output has 3.10 M sectors (24 x 513 x 289 ->
+// 1917 x 1079). So a block produces kRowsPerGroup whole rows (`groups` times, where one group does not give every wave a
+// piece of 256 columns), collects them in LDS at the place they have relative to a 64-byte boundary and writes them
+// out 16 bytes per lane on 16-byte boundaries: a dense output's rows as one run, whose two ends alone are partial. A
+// lane's columns are 64 apart (LDS writes without bank conflicts); the tap pairs of all source rows that 4 output
+// rows can need are requested before the first is used: 3, 4 or 5 by the scale. Against wave patches: 68.8 -> 44.1 us, 4.8 TB/s
+// (24 x 513 x 289 -> 1917 x 1079), 22.8 -> 15.4 us (16 x 320 x 180 -> 1280 x 720), 13.9 -> 12.1 us (3 x 1901 x 900 -> 1300 x
+// 1920). The first case by other forms, each 3 to 4 us longer for an event behind every launch: this one 48.2 us, with 8 rows
+// per group 61.6 us (61 KB of LDS leave two blocks per CU), streaming stores from the lanes that formed the values
+// 53.5 us, cached stores, which the L2 merges to 3.13 M requests, 79 us (they evict the source rows).
+constexpr int kRowsPerGroup = 4;
+
+// Source rows from the first on that kRowsPerGroup output rows span, 3 to 5; 0: more than 5 (rows reduced). A place is
+// a rounded product and a rounded difference, each off by at most 2^-11 below 8192: two of them by less than the margin.
+static inline int LinearRowsSources(const ResizeArgs &a)
+{
+    const float span = (kRowsPerGroup - 1) * a.scaleY + (a.srcH == a.dstH ? 0.f : 4e-3f);
+    return a.srcH > 8192 ? 0 : span <= 1.f ? 3 : span <= 2.f ? 4 : span <= 3.f ? 5 : 0;
+}
+
+template<int S>
+__global__ __launch_bounds__(256) void ResizeLinearRowsKernel(const ResizeArgs a, const int chunks, const int groups)
+{
+    extern __shared__ __attribute__((aligned(16))) float stage[];
+    const Plane p    = GetPlanes<false>(a, blockIdx.y);
+    const int   lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int R  = kRowsPerGroup;
+    const int   yBlock = blockIdx.x * groups * R, rowsBlock = min(groups * R, p.dstH - yBlock);
+    // Row i of the block is staged from float i * pitch + lead(i) on, where lead is the row's distance from the 64-byte
+    // boundary in front of it; dense rows follow one another in LDS as they do in memory (and keep the block's lead).
+    const bool  dense = p.dstRow == 4 * p.dstW;
+    const int   pitch = dense ? p.dstW : ((p.dstW + 15) & ~15) + 16;
+    auto        lead  = [&](int i)
+    {
+        return (int)(reinterpret_cast<uintptr_t>(p.dst + (int64_t)(yBlock + (dense ? 0 : i)) * p.dstRow) & 63) / 4;
+    };
+    for (int t = wave; t < chunks * groups; t += 4)
+    {
+        const int g = t / chunks, x0 = (t - g * chunks) * 256, y0 = yBlock + g * R;
+        const int rows = min(R, p.dstH - y0);
+        if (rows <= 0)
+        {
+            break;
+        }
+        float    wx1[4], wx0[4];
+        uint32_t off[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+        {
+            const float fx = (min(x0 + lane + 64 * k, p.dstW - 1) + .5f) * p.scaleX - .5f;
+            const int   sx = (int)floorf(fx);
+            wx1[k]         = sx < 0 ? 0.f : (sx > p.srcW - 2 ? 1.f : fx - sx);
+            wx0[k]         = 1.f - wx1[k];
+            off[k]         = (uint32_t)max(0, min(sx, p.srcW - 2)) * 4u;
+        }
+        const float fy = (min(y0 + min(lane, R - 1), p.dstH - 1) + .5f) * p.scaleY - .5f;
+        const int   sy = (int)floorf(fy);
+        const float wyLane = sy < 0 ? 0.f : (sy > p.srcH - 2 ? 1.f : fy - sy);
+        const int   syLane = max(0, min(sy, p.srcH - 2));
+        using Pair = Pixel<float, 2>;
+        Pair          src[S][4];
+        const int     first = __builtin_amdgcn_readlane(syLane, 0), last = __builtin_amdgcn_readlane(syLane, rows - 1) + 1;
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+        {
+            const uint8_t *row = p.src + (int64_t)min(first + i, last) * p.srcRow;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                src[i][k] = *reinterpret_cast<const Pair *>(row + off[k]);
+            }
+        }
+        int r = 0;
+#pragma unroll
+        for (int i = 0; i < S - 1; ++i)
+        {
+#pragma unroll 1
+            for (; r < rows && __builtin_amdgcn_readlane(syLane, r) == first + i; ++r)
+            {
+                const float wy1 = ReadLane(wyLane, r), wy0 = 1.f - wy1;
+                float      *to  = stage + (g * R + r) * pitch + lead(g * R + r) + x0 + lane;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                {
+                    const float w00 = wx0[k] * wy0, w01 = wx1[k] * wy0, w10 = wx0[k] * wy1, w11 = wx1[k] * wy1;
+                    const float v = src[i][k].v[0] * w00 + src[i][k].v[1] * w01 + src[i + 1][k].v[0] * w10 + src[i + 1][k].v[1] * w11;
+                    if (x0 + lane + 64 * k < p.dstW)
+                    {
+                        to[64 * k] = v;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int run = 0; run < (dense ? 1 : rowsBlock); ++run)
+    {
+        const int    first = lead(run), end = first + (dense ? rowsBlock * p.dstW : p.dstW);
+        const float *from = stage + run * pitch;
+        uint8_t     *to   = p.dst + (int64_t)(yBlock + run) * p.dstRow - 4 * first;
+        for (int i = threadIdx.x * 4; i < end; i += 1024)
+        {
+            uint32_t w[4];
+            __builtin_memcpy(w, __builtin_assume_aligned(from + i, 16), 16);
+            if (i >= first && i + 4 <= end)
+            {
+                StoreDwordsNT<4>(to + 4 * i, w);
+            }
+            else
+            {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                {
+                    if (i + k >= first && i + k < end)
+                    {
+                        *reinterpret_cast<uint32_t *>(to + 4 * (i + k)) = w[k];
+                    }
+                }
+            }
+        }
+    }
+}
+
 // Which (type, channels, interpolation) run as wave patches.
 template<class T, int C, int INTERP>
 constexpr bool kPatchForm = INTERP != NVCV_INTERP_AREA && sizeof(Pixel<T, C>) <= 8;
@@ -3168,6 +3297,23 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
                 hipLaunchKernelGGL((ResizeCubicStripU8Kernel<C, 8>), sgrid, dim3(256), 0, stream, a, (int)flat);
             }
             CheckLaunch("ResizeCubicStripU8Kernel");
+            return;
+        }
+    }
+    if constexpr (std::is_same_v<T, float> && C == 1 && INTERP == NVCV_INTERP_LINEAR)
+    {
+        const int sources = LinearRowsSources(a), chunks = DivUp(a.dstW, 256);
+        const int groups = chunks >= 3 ? 1 : chunks == 2 ? 2 : 4;
+        const int lds = (groups * kRowsPerGroup * (((a.dstW + 15) & ~15) + 16) + 16) * 4;
+        const dim3 rgrid(DivUp(a.dstH, groups * kRowsPerGroup), N);
+        // Two blocks and more per CU: below that the wave patches spread further (one 513 x 289 -> 1917 x 1079, 270 blocks:
+        // 5.3 us as patches, 6.3 as rows; 4 x 1280 x 720 -> 1281 x 722, 724 blocks: 8.9 and 8.5). Rows of up to 4000 floats:
+        // from there on the LDS holds one block per CU (4 x 1901 x 900 -> 3841 x 1922, two per CU: 45.6 and 43.2 us).
+        if (sources != 0 && a.srcW >= 2 && a.srcH >= 2 && lds <= 65536 && (int64_t)rgrid.x * N >= 512)
+        {
+            auto kernel = sources == 3 ? ResizeLinearRowsKernel<3> : sources == 4 ? ResizeLinearRowsKernel<4> : ResizeLinearRowsKernel<5>;
+            hipLaunchKernelGGL(kernel, rgrid, dim3(256), lds, stream, a, chunks, groups);
+            CheckLaunch("ResizeLinearRowsKernel");
             return;
         }
     }

@@ -426,6 +426,33 @@ def test_area_varshape(cv, K, orc, gpu, dt, c):
             assert bad.mean() <= (0.0 if (sw, sh, dw, dh) in sizes[:3] else 0.02), (sw, sh, dw, dh, bad.mean())
 
 
+# one-channel float maps whose rows are not reduced, in launches large enough for the whole-rows form: 1, 2 and 3 pieces
+# of 256 columns (4, 2 and 1 groups of 4 rows per block) with remainders, 3, 4 and 5 source rows per group, the smallest
+# source, equal heights; dense odd rows, the library's padded rows, and views whose rows start 4 bytes off
+@pytest.mark.parametrize("n,sw,sh,dw,dh", [(512, 2, 2, 5, 7), (300, 40, 9, 257, 21), (256, 30, 20, 256, 33), (130, 100, 13, 700, 61),
+                                           (50, 1301, 41, 1025, 41), (90, 5, 50, 513, 73), (520, 9, 5, 13, 6)])
+@pytest.mark.parametrize("kind", ["dense", "padded", "view"])
+def test_linear_float_maps_by_whole_rows(cv, orc, gpu, n, sw, sh, dw, dh, kind):
+    src = make_input(orc, (n, sh, sw, 1), np.float32, 0xF10A + sw + dw)
+    want = orc.resize(src, (dh, dw), LINEAR, variant=1, threads=8)
+    tin = cv.Tensor.from_torch(torch.from_numpy(src).cuda(), "NHWC")
+    if kind == "padded":
+        tout = cv.Tensor.alloc([n, dh, dw, 1], np.float32, "NHWC")
+        view, spare = tout.torch_view(), None
+    else:
+        lead, pitch = (0, dw) if kind == "dense" else (1, dw + 3)
+        spare = torch.full((n * dh * pitch + 8,), -7.0, device="cuda")
+        view = torch.as_strided(spare, (n, dh, dw, 1), (dh * pitch, pitch, 1, 1), lead)
+        tout = cv.Tensor.from_torch(view, "NHWC")
+    cv.Resize()(None, tin, tout, LINEAR)
+    torch.cuda.synchronize()
+    # four products of values below 1 and three sums, each rounded once or twice: under 12 roundings of 2^-24
+    assert np.abs(view.cpu().numpy() - want).max() <= 12 * 2.0 ** -24 * max(1.0, float(np.abs(src).max()))
+    if spare is not None:
+        view.fill_(-7.0)
+        assert bool((spare == -7.0).all()), "floats outside the rows written"
+
+
 # seeded random cases: 8-bit pixels of 1, 3 and 4 channels, every interpolation, scales of 0.42 to 2.4 per axis (now
 # and then equal, or exactly 1/2, 2/3, 1, 1.5, 2), small and 1080p-sized images, batches below and above the sizes
 # at which the strip kernels take over, as packed tensors, as views with odd leads and pitches (bytes outside the
