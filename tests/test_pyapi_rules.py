@@ -167,3 +167,45 @@ def test_submit_bookkeeping_under_parallel_readers(api, monkeypatch):
     api._submit(writer, [], [shared], lambda s: None)
     assert sorted(e.stream for e in writer.waited) == [100 + i for i in range(8)]
     assert shared._read == {} and shared._wrote[0] == 7
+
+
+def test_submit_orders_the_default_stream_by_events_recorded_when_needed(api, monkeypatch):
+    # the default stream's work leaves no event behind it; another stream that reads or overwrites its results waits
+    # for one recorded on the default stream then, and the default stream waits for the other stream's own events.
+    # No GPU: streams and events are stand-ins that only record what was asked of them.
+    class FakeStream:
+        def __init__(self, key):
+            self.cuda_stream, self.waited = key, []
+
+        def wait_event(self, event):
+            self.waited.append(event.stream)
+
+    made = []
+
+    class FakeEvent:
+        def __init__(self):
+            made.append(self)
+
+        def record(self, stream):
+            self.stream = stream.cuda_stream
+
+    class Box:
+        pass
+
+    default, side, other = FakeStream(0), FakeStream(7), FakeStream(9)
+    monkeypatch.setattr(api, "_torch_stream", lambda s: s)
+    monkeypatch.setattr(api, "_default_stream", lambda: default)
+    monkeypatch.setattr(api, "_new_event", FakeEvent)
+    a, b, c = Box(), Box(), Box()
+    handles = []
+    for _ in range(3):
+        api._submit(default, [a], [b], handles.append)
+    assert handles == [0, 0, 0] and not made and not default.waited  # one stream: no events, no waits
+    api._submit(side, [b], [c], lambda s: None)   # reads what the default stream wrote
+    assert side.waited == [0] and [e.stream for e in made] == [0, 7]
+    api._submit(other, [], [a], lambda s: None)   # overwrites what the default stream read
+    assert other.waited == [0]
+    api._submit(default, [c], [b], lambda s: None)  # reads what `side` wrote and overwrites what `side` read
+    assert default.waited == [7, 7]
+    api._submit(default, [b], [c], lambda s: None)  # its own result, and c, which only it has read since
+    assert default.waited == [7, 7, 7]  # c was written by `side`
