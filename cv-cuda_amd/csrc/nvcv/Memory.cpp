@@ -2,6 +2,7 @@
 // Requirements: src/nvcv/src/priv/Requirements.cpp:49-109. Default allocator:
 // src/nvcv/src/priv/DefaultAllocator.cpp:29-84, on the HIP runtime (hipMalloc / hipHostMalloc).
 // Handle pools: external behaviour of src/nvcv/src/priv/HandleManagerImpl.hpp:251-439.
+#include "BlockPool.hpp"
 #include "Priv.hpp"
 
 #include <hip/hip_runtime_api.h>
@@ -263,42 +264,122 @@ void DefaultFreeHost(void *, void *p, int64_t, int32_t)
     std::free(p);
 }
 
-void *DefaultAllocPinned(void *, int64_t size, int32_t)
+int CurrentDevice()
 {
-    void *p = nullptr;
-    if (hipHostMalloc(&p, (size_t)std::max<int64_t>(size, 1), hipHostMallocDefault) != hipSuccess)
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess)
     {
         (void)hipGetLastError();
-        return nullptr;
     }
-    return p;
+    return device;
+}
+
+bool SynchronizeDevice()
+{
+    // not possible while a stream of the device is being captured
+    if (hipDeviceSynchronize() != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+struct PinnedMemory
+{
+    static void *alloc(size_t size)
+    {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, size, hipHostMallocDefault) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        return p;
+    }
+
+    static void free(void *p)
+    {
+        (void)SynchronizeDevice(); // a copy may still read or write it
+        (void)hipHostFree(p);
+    }
+
+    static int device()
+    {
+        return CurrentDevice();
+    }
+
+    static bool synchronize()
+    {
+        return SynchronizeDevice();
+    }
+};
+
+struct DeviceMemory
+{
+    static void *alloc(size_t size)
+    {
+        // hipMalloc returns at least 256-byte aligned addresses; larger requests come back page aligned.
+        void *p = nullptr;
+        if (hipMalloc(&p, size) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        return p;
+    }
+
+    static void free(void *p)
+    {
+        (void)hipFree(p);
+    }
+
+    static int device()
+    {
+        return CurrentDevice();
+    }
+
+    static bool synchronize()
+    {
+        return SynchronizeDevice();
+    }
+};
+
+BlockPool<DeviceMemory> &DevicePool()
+{
+    static auto *pool = new BlockPool<DeviceMemory>(int64_t(1) << 30);
+    return *pool;
+}
+
+BlockPool<PinnedMemory> &PinnedPool()
+{
+    static auto *pool = new BlockPool<PinnedMemory>(int64_t(1) << 26);
+    return *pool;
+}
+
+void *DefaultAllocPinned(void *, int64_t size, int32_t)
+{
+    return PinnedPool().alloc(std::max<int64_t>(size, 1));
 }
 
 void DefaultFreePinned(void *, void *p, int64_t, int32_t)
 {
     if (p != nullptr)
     {
-        (void)hipHostFree(p);
+        PinnedPool().free(p);
     }
 }
 
 void *DefaultAllocDevice(void *, int64_t size, int32_t)
 {
-    // hipMalloc returns at least 256-byte aligned addresses; larger requests come back page aligned.
-    void *p = nullptr;
-    if (hipMalloc(&p, (size_t)std::max<int64_t>(size, 1)) != hipSuccess)
-    {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return p;
+    return DevicePool().alloc(std::max<int64_t>(size, 1));
 }
 
 void DefaultFreeDevice(void *, void *p, int64_t, int32_t)
 {
     if (p != nullptr)
     {
-        (void)hipFree(p);
+        DevicePool().free(p);
     }
 }
 

@@ -7,6 +7,7 @@ semantics of priv/Status.cpp:31-110 -- with this library's alignment constants (
 512-byte base)."""
 import ctypes as C
 import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -571,3 +572,12 @@ def test_reshape_of_padded_rows_gives_the_reference_strides(cv, shape_arg, layou
     assert tuple(t.reshape(list(shape_arg), layout_arg).strides) == expected
     with pytest.raises(cv.Error):
         t.reshape([300], "A")  # padded rows cannot become one dense dimension
+
+
+def test_block_pool_of_the_default_allocator(tmp_path):
+    # what it hands out again and when, its bounds, what it gives back, threads: with a counting stand-in for the device
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "block_pool_cases.cpp")
+    exe = str(tmp_path / "block_pool_cases")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cv-cuda_amd", "csrc", "nvcv")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I" + csrc, src, "-o", exe, "-lpthread"], check=True)
+    assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "ok"
