@@ -261,6 +261,7 @@ _sig(nvcv, "nvcvImageBatchVarShapeGetUniqueFormat", ST, H, P(C.c_uint64))
 _sig(nvcv, "nvcvImageBatchVarShapePushImages", ST, H, P(H), C.c_int32)
 PushImageFunc = C.CFUNCTYPE(C.c_void_p, C.c_void_p)
 _sig(nvcv, "nvcvImageBatchVarShapePushImagesCallback", ST, H, PushImageFunc, C.c_void_p)
+_sig(nvcv, "nvcvxImageBatchVarShapePushBuffers", ST, H, C.c_uint64, C.c_void_p, C.c_int32)
 _sig(nvcv, "nvcvImageBatchVarShapePopImages", ST, H, C.c_int32)
 _sig(nvcv, "nvcvImageBatchVarShapeClear", ST, H)
 _sig(nvcv, "nvcvImageBatchVarShapeGetImages", ST, H, C.c_int32, P(H), C.c_int32)

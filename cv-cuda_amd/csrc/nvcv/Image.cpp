@@ -263,6 +263,12 @@ private:
 };
 
 } // namespace
+
+NVCVImageHandle CreateWrappedImage(const NVCVImageData &d)
+{
+    return static_cast<NVCVImageHandle>(ImagePool().create(std::make_unique<WrappedImage>(d, nullptr, nullptr)));
+}
+
 } // namespace nvcvamd
 
 using namespace nvcvamd;

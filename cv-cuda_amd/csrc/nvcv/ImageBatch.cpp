@@ -37,10 +37,11 @@ public:
         }
         try
         {
-            m_devImages   = static_cast<NVCVImageBufferStrided *>(m_alloc.allocDevice(imagesBytes(), m_reqs.alignBytes));
-            m_devFormats  = static_cast<NVCVImageFormat *>(m_alloc.allocDevice(formatsBytes(), m_reqs.alignBytes));
-            m_hostImages  = static_cast<NVCVImageBufferStrided *>(m_alloc.allocPinned(imagesBytes(), m_reqs.alignBytes));
-            m_hostFormats = static_cast<NVCVImageFormat *>(m_alloc.allocPinned(formatsBytes(), m_reqs.alignBytes));
+            // formats in front of images, in one block each: a batch filled once is uploaded by one copy
+            m_devFormats  = static_cast<NVCVImageFormat *>(m_alloc.allocDevice(listsBytes(), m_reqs.alignBytes));
+            m_hostFormats = static_cast<NVCVImageFormat *>(m_alloc.allocPinned(listsBytes(), m_reqs.alignBytes));
+            m_devImages   = reinterpret_cast<NVCVImageBufferStrided *>(reinterpret_cast<uint8_t *>(m_devFormats) + formatsBytes());
+            m_hostImages  = reinterpret_cast<NVCVImageBufferStrided *>(reinterpret_cast<uint8_t *>(m_hostFormats) + formatsBytes());
             m_handles     = static_cast<NVCVImageHandle *>(m_alloc.allocHost(handlesBytes(), m_reqs.alignBytes));
             CheckHip(hipEventCreateWithFlags(&m_uploaded, hipEventDisableTiming), "hipEventCreateWithFlags");
         }
@@ -54,7 +55,9 @@ public:
 
     ~VarShapeBatch() override
     {
-        if (m_uploaded != nullptr)
+        // An upload may still read the pinned lists. The default allocator hands a block out again only when the device has
+        // been idle since it was given back, so only a caller's own allocator has to be waited for here.
+        if (m_uploaded != nullptr && m_hAlloc != nullptr)
         {
             (void)hipEventSynchronize(m_uploaded);
         }
@@ -127,12 +130,21 @@ public:
             // of the arrays that changed since the last export.
             CheckHip(hipStreamWaitEvent(stream, m_uploaded, 0), "hipStreamWaitEvent");
             size_t n = (size_t)(m_num - m_dirtyFrom);
-            CheckHip(hipMemcpyAsync(m_devImages + m_dirtyFrom, m_hostImages + m_dirtyFrom, n * sizeof(*m_devImages),
-                                    hipMemcpyHostToDevice, stream),
-                     "hipMemcpyAsync");
-            CheckHip(hipMemcpyAsync(m_devFormats + m_dirtyFrom, m_hostFormats + m_dirtyFrom, n * sizeof(*m_devFormats),
-                                    hipMemcpyHostToDevice, stream),
-                     "hipMemcpyAsync");
+            if (m_dirtyFrom == 0)
+            {
+                CheckHip(hipMemcpyAsync(m_devFormats, m_hostFormats, (size_t)formatsBytes() + n * sizeof(*m_devImages),
+                                        hipMemcpyHostToDevice, stream),
+                         "hipMemcpyAsync");
+            }
+            else
+            {
+                CheckHip(hipMemcpyAsync(m_devImages + m_dirtyFrom, m_hostImages + m_dirtyFrom, n * sizeof(*m_devImages),
+                                        hipMemcpyHostToDevice, stream),
+                         "hipMemcpyAsync");
+                CheckHip(hipMemcpyAsync(m_devFormats + m_dirtyFrom, m_hostFormats + m_dirtyFrom, n * sizeof(*m_devFormats),
+                                        hipMemcpyHostToDevice, stream),
+                         "hipMemcpyAsync");
+            }
             CheckHip(hipEventRecord(m_uploaded, stream), "hipEventRecord");
             m_dirtyFrom = m_num;
         }
@@ -161,6 +173,50 @@ public:
             for (int i = 0; i < n; ++i)
             {
                 pushOne(images[i]);
+            }
+        }
+        catch (...)
+        {
+            rollback(before);
+            throw;
+        }
+    }
+
+    // Images over n buffers of one plane, owned by the batch alone.
+    void pushBuffers(NVCVImageFormat format, const NVCVImagePlaneStrided *planes, int32_t n)
+    {
+        NotNull(planes, "List of planes");
+        if (n < 0)
+        {
+            throw Error(NVCV_ERROR_INVALID_ARGUMENT, "Number of images cannot be negative");
+        }
+        if ((int64_t)n + m_num > m_reqs.capacity)
+        {
+            throw Error(NVCV_ERROR_OVERFLOW, "Adding %d images to image batch would make its size %d exceed its capacity %d",
+                        n, n + m_num, m_reqs.capacity);
+        }
+        waitUpload();
+        int           before = m_num;
+        NVCVImageData d      = {};
+        d.format             = format;
+        d.bufferType         = NVCV_IMAGE_BUFFER_STRIDED_CUDA;
+        d.buffer.strided.numPlanes = 1;
+        try
+        {
+            for (int i = 0; i < n; ++i)
+            {
+                d.buffer.strided.planes[0] = planes[i];
+                NVCVImageHandle h          = CreateWrappedImage(d);
+                try
+                {
+                    pushOne(h);
+                }
+                catch (...)
+                {
+                    ImagePool().decRef(h);
+                    throw;
+                }
+                ImagePool().decRef(h); // the batch's reference is the only one
             }
         }
         catch (...)
@@ -250,6 +306,11 @@ private:
         return (int64_t)m_reqs.capacity * (int64_t)sizeof(NVCVImageFormat);
     }
 
+    int64_t listsBytes() const
+    {
+        return formatsBytes() + imagesBytes();
+    }
+
     int64_t handlesBytes() const
     {
         return (int64_t)m_reqs.capacity * (int64_t)sizeof(NVCVImageHandle);
@@ -327,10 +388,8 @@ private:
 
     void freeAll() noexcept
     {
-        m_alloc.freeDevice(m_devImages, imagesBytes(), m_reqs.alignBytes);
-        m_alloc.freeDevice(m_devFormats, formatsBytes(), m_reqs.alignBytes);
-        m_alloc.freePinned(m_hostImages, imagesBytes(), m_reqs.alignBytes);
-        m_alloc.freePinned(m_hostFormats, formatsBytes(), m_reqs.alignBytes);
+        m_alloc.freeDevice(m_devFormats, listsBytes(), m_reqs.alignBytes);
+        m_alloc.freePinned(m_hostFormats, listsBytes(), m_reqs.alignBytes);
         m_alloc.freeHost(m_handles, handlesBytes(), m_reqs.alignBytes);
         if (m_uploaded != nullptr)
         {
@@ -399,10 +458,8 @@ NVCVStatus nvcvImageBatchVarShapeCalcRequirements(int32_t capacity, NVCVImageBat
             int64_t align = std::lcm<int64_t>(alignof(NVCVImageBufferStrided), alignof(NVCVImageHandle));
             align         = NextPow2(std::lcm<int64_t>(align, alignof(NVCVImageFormat)));
             r.alignBytes  = (int32_t)align;
-            ReqAddBuffer(r.mem.cudaMem, (int64_t)capacity * sizeof(NVCVImageBufferStrided), align);
-            ReqAddBuffer(r.mem.cudaMem, (int64_t)capacity * sizeof(NVCVImageFormat), align);
-            ReqAddBuffer(r.mem.hostPinnedMem, (int64_t)capacity * sizeof(NVCVImageBufferStrided), align);
-            ReqAddBuffer(r.mem.hostPinnedMem, (int64_t)capacity * sizeof(NVCVImageFormat), align);
+            ReqAddBuffer(r.mem.cudaMem, (int64_t)capacity * (sizeof(NVCVImageFormat) + sizeof(NVCVImageBufferStrided)), align);
+            ReqAddBuffer(r.mem.hostPinnedMem, (int64_t)capacity * (sizeof(NVCVImageFormat) + sizeof(NVCVImageBufferStrided)), align);
             ReqAddBuffer(r.mem.hostMem, (int64_t)capacity * sizeof(NVCVImageHandle), align);
             *reqs = r;
         });
@@ -539,6 +596,12 @@ NVCVStatus nvcvImageBatchVarShapePushImagesCallback(NVCVImageBatchHandle handle,
                                                     void *ctxCallback)
 {
     return Protect([&] { Batch(handle).pushCallback(cbPushImage, ctxCallback); });
+}
+
+NVCVStatus nvcvxImageBatchVarShapePushBuffers(NVCVImageBatchHandle handle, NVCVImageFormat format,
+                                              const NVCVImagePlaneStrided *planes, int32_t numImages)
+{
+    return Protect([&] { Batch(handle).pushBuffers(format, planes, numImages); });
 }
 
 NVCVStatus nvcvImageBatchVarShapePopImages(NVCVImageBatchHandle handle, int32_t numImages)

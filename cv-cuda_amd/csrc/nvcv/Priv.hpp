@@ -328,6 +328,9 @@ public:
     virtual NVCVAllocatorHandle allocHandle() const                  = 0;
 };
 
+// An image over memory that somebody else keeps (validated as nvcvImageWrapDataConstruct does); one reference.
+NVCVImageHandle CreateWrappedImage(const NVCVImageData &d);
+
 void ValidateWrappedTensor(const NVCVTensorData &d);
 
 } // namespace nvcvamd

@@ -78,6 +78,12 @@ NVCV_PUBLIC NVCVStatus nvcvxImageBatchVarShapeGetHostImageList(NVCVImageBatchHan
                                                                const NVCVImageBufferStrided **outList,
                                                                int32_t                       *outNumImages);
 
+/* Extension: appends one image of `format` (one plane) per buffer, which the caller keeps alive while the image is in
+ * use. What nvcvImageWrapDataConstruct and nvcvImageBatchVarShapePushImages do image by image, in one call; the batch
+ * holds the only references. Exceeding the capacity -> OVERFLOW and the batch is left unchanged. */
+NVCV_PUBLIC NVCVStatus nvcvxImageBatchVarShapePushBuffers(NVCVImageBatchHandle handle, NVCVImageFormat format,
+                                                          const NVCVImagePlaneStrided *planes, int32_t numImages);
+
 #ifdef __cplusplus
 }
 #endif

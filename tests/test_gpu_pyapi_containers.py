@@ -302,3 +302,35 @@ def test_wrapped_streams(nvcv):
     out = nvcv.flip(src, 0, stream=wrapped)
     wrapped.sync()
     assert torch.equal(out.torch().cpu(), torch.arange(24, dtype=torch.uint8).reshape(2, 4, 3).flip(0))
+
+
+def test_as_images_of_torch_tensors_in_one_call(nvcv):
+    # the batch made in one call is the one that image by image makes: descriptors, formats, Image objects asked for
+    # later (and kept alive by them), pops and pushes; buffers that need as_image's own look take that way
+    import torch
+    tensors = [torch.randint(0, 256, (5 + i, 7 + 2 * i, 3), dtype=torch.uint8, device="cuda") for i in range(4)]
+    tensors.append(torch.zeros((9, 24, 3), dtype=torch.uint8, device="cuda")[:, :11])  # rows of another pitch
+    for fmt in (None, nvcv.Format.BGR8):
+        one, many = nvcv.as_images(tensors, fmt), nvcv.ImageBatchVarShape(5)
+        many.pushback([nvcv.as_image(t, fmt) for t in tensors])
+        assert one._buffers is not None and len(one) == 5 and one.maxsize == many.maxsize
+        assert one.uniqueformat == many.uniqueformat == (fmt or nvcv.Format.RGB8)
+        for a, b in zip(one, many):
+            p, q = (x.export().buffer.strided.planes[0] for x in (a, b))
+            assert (a.size, a.format, p.rowStride, p.basePtr) == (b.size, b.format, q.rowStride, q.basePtr)
+        assert one[0].cpu().tolist() == tensors[0].cpu().tolist()
+    batch = nvcv.as_images([t.clone() for t in tensors])
+    last = batch.maxsize
+    batch.popback(2)
+    assert len(batch) == 3 and [i.size for i in batch] == [(t.shape[1], t.shape[0]) for t in tensors[:3]] and batch.maxsize != last
+    batch.pushback(nvcv.as_image(tensors[4]))
+    image = batch[1]
+    del batch
+    assert image.cpu().tolist() == tensors[1].cpu().tolist()
+    cleared = nvcv.as_images(tensors)
+    cleared.clear()
+    assert len(cleared) == 0 and list(cleared) == []
+    masks = nvcv.as_images([torch.zeros((4, 6), device="cuda"), torch.zeros((3, 5), device="cuda")])
+    assert masks.uniqueformat == nvcv.Format.F32 and masks[1].size == (5, 3)
+    mixed = nvcv.as_images([tensors[0], torch.zeros((4, 4), dtype=torch.uint8, device="cuda")])
+    assert mixed._buffers is None and mixed.uniqueformat is None
