@@ -74,6 +74,18 @@ class _DevMem:
         self._owner = owner
 
 
+class _DevArray:
+    """The same for a strided array."""
+
+    def __init__(self, ptr, shape, strides, typestr, owner):
+        self.__cuda_array_interface__ = {"shape": tuple(shape), "strides": tuple(strides), "typestr": typestr,
+                                         "data": (ptr, False), "version": 2}
+        self._owner = owner
+
+
+_DIRECT_VIEW = (np.dtype(np.uint8), np.dtype(np.float32))
+
+
 def _bytes_view(ptr, nbytes, owner):
     return torch.as_tensor(_DevMem(ptr, nbytes, owner), device="cuda")
 
@@ -227,8 +239,10 @@ class Tensor(_Handle):
         d = self.export()
         npdt = _DT2NP[d.dtype]
         es = npdt.itemsize
-        shape = [d.shape[i] for i in range(d.rank)]
-        strides = [d.buffer.strides[i] for i in range(d.rank)]
+        shape = d.shape[:d.rank]
+        strides = d.buffer.strides[:d.rank]
+        if 0 not in shape and npdt in _DIRECT_VIEW and all(st % es == 0 for st in strides):
+            return torch.as_tensor(_DevArray(d.buffer.basePtr, shape, strides, npdt.str, self), device="cuda")
         nbytes = max(1, sum((s - 1) * st for s, st in zip(shape, strides)) + es)
         raw = _bytes_view(d.buffer.basePtr, nbytes, self)
         if npdt != np.dtype(np.uint8):

@@ -300,6 +300,10 @@ class _Buffer:
 class Tensor:
     """Tensor(shape, dtype, layout=None) or Tensor(nimages, imgsize=(w, h), format) (python/mod_nvcv/Tensor.cpp)."""
 
+    _key = None    # _Outputs: what the tensor can be handed out again as
+    _seen = False  # something outside this module knows its memory
+    _meta = None   # shape, element type and layout, which a tensor keeps for life
+
     def __init__(self, *args, rowalign=0, _wrap=None, **kw):
         if _wrap is not None:
             self._t = _wrap
@@ -316,33 +320,106 @@ class Tensor:
 
     @property
     def handle(self):
+        self._seen = True
         return self._t.handle
+
+    def _properties(self):
+        if self._meta is None:
+            d = self._t.export()
+            self._meta = (tuple(d.shape[:d.rank]), _DT2NP.get(d.dtype), str(d.layout) or None)
+        return self._meta
 
     @property
     def shape(self):
-        return tuple(self._t.shape)
+        return self._properties()[0]
 
     @property
     def ndim(self):
-        return len(self._t.shape)
+        return len(self._properties()[0])
 
     @property
     def dtype(self):
-        return _DT2NP[self._t.dtype]
+        return self._properties()[1] or _DT2NP[self._t.dtype]
 
     @property
     def layout(self):
-        return self._t.layout or None
+        return self._properties()[2]
 
     def cuda(self):
+        self._seen = True
         return _Buffer(self._t.__cuda_array_interface__, self)
 
     def reshape(self, shape, layout=None):
+        self._seen = True
         return Tensor(_wrap=self._t.reshape(list(shape), layout or ""))
 
     def torch(self):
         """Strided torch view of the tensor's memory (not in the reference: what its tests build by hand)."""
+        self._seen = True
         return self._t.torch_view()
+
+    def __del__(self):
+        if self._key is not None and not self._seen:
+            _outputs.put(self)
+
+
+class _Outputs:
+    """Tensors that operators made for their results and whose owners are gone, for results of the same shape, type and
+    layout: the intermediate results of a chain of operators. (The reference's bindings keep such objects too, in their
+    object cache.) A tensor comes back here only if every use of it was a call of this module on the default stream,
+    where the next user's work is ordered behind the last one's; one whose memory, handle or views were given out goes
+    back to the library's allocator, which knows when the device is done with it. Bounded: beyond `most_bytes` or
+    `most_tensors` everything held goes back to the allocator."""
+    most_bytes, most_tensors = 256 << 20, 64
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._free, self._bytes, self._count = {}, 0, 0
+
+    def get(self, shape, dtype, layout):
+        shape, dtype = tuple(shape), np.dtype(dtype)
+        key = (shape, dtype, layout, torch._C._cuda_getDevice())
+        with self._lock:
+            stack = self._free.get(key)
+            raw = stack.pop() if stack else None
+            if raw is not None:
+                self._bytes -= raw._nbytes
+                self._count -= 1
+        out = Tensor(_wrap=raw if raw is not None else _Tensor.alloc(list(shape), dtype, layout or ""))
+        if raw is not None:
+            out._wrote = _BY_DEFAULT  # another stream's first use of it waits for the default stream's last
+        else:
+            d = out._t.export()
+            out._t._nbytes = d.buffer.strides[0] * d.shape[0] if d.rank else 0
+        out._key, out._meta = key, (shape, dtype, layout or None)
+        return out
+
+    def put(self, tensor):
+        try:
+            if getattr(tensor, "_wrote", _BY_DEFAULT)[0] != 0 or any(k != 0 for k in getattr(tensor, "_read", _NO_READS)):
+                return
+            # (not waited for: the collector may have stepped in while this thread holds the lock)
+            if not self._lock.acquire(blocking=False):
+                return
+            drop = None
+            try:
+                raw = tensor._t
+                if self._count >= self.most_tensors or self._bytes + raw._nbytes > self.most_bytes:
+                    drop, self._free, self._bytes, self._count = self._free, {}, 0, 0
+                if raw._nbytes <= self.most_bytes // 4:
+                    self._free.setdefault(tensor._key, []).append(raw)
+                    self._bytes += raw._nbytes
+                    self._count += 1
+            finally:
+                self._lock.release()
+            del drop
+        except (AttributeError, TypeError):
+            pass  # the interpreter is ending: the module's names are gone
+
+
+_NO_READS = {}
+_BY_DEFAULT = (0, None)
+_outputs = _Outputs()
 
 
 def reshape(tensor, shape, layout=None):
@@ -589,13 +666,13 @@ class ImageBatchVarShape(_ImageBatchVarShape):
     def popback(self, count=1):
         self.pop_back(count)
 
-    @property
-    def maxsize(self):
-        return self.max_size
-
     def pop_back(self, n=1):
         self.images  # (made before the library drops the last of them)
         super().pop_back(n)
+
+    @property
+    def maxsize(self):
+        return self.max_size
 
     @property
     def uniqueformat(self):
@@ -663,7 +740,7 @@ def _submit(stream, reads, writes, op, *args):
                 mark = _new_event()
                 mark.record(_default_stream())
             waiting.wait_event(mark)
-    op(s, *args)
+    op(s, *[a._t if type(a) is Tensor else a for a in args])
     mark = None
     if s:
         mark = _new_event()
@@ -679,7 +756,6 @@ def _submit(stream, reads, writes, op, *args):
 
 
 _events_lock = threading.Lock()
-_NO_READS = {}
 
 
 def _default_stream_key(stream):
@@ -729,7 +805,7 @@ def resize(src, shape=None, interp=Interp.LINEAR, *, sizes=None, stream=None):
         if len(src) != len(sizes):
             raise RuntimeError("Number of input images must be equal to the number of elements in output size list ")
         return resize_into(_same_images(src, sizes=[tuple(s) for s in sizes]), src, interp, stream=stream)
-    return resize_into(Tensor(tuple(shape), src.dtype, src.layout), src, interp, stream=stream)
+    return resize_into(_outputs.get(shape, src.dtype, src.layout), src, interp, stream=stream)
 
 
 _CODE = re.compile(r"^(.*?)2(BGRA|RGBA|BGR|RGB|GRAY|YUV|HSV|HLS|YCrCb|XYZ|Lab|Luv)(.*)$")
@@ -798,7 +874,7 @@ def cvtcolor(src, code, *, stream=None):
             raise RuntimeError("All images in input must have the same single-plane format")
         return cvtcolor_into(_same_images(src, fmt=_cvtcolor_format(fmt, code)), src, code, stream=stream)
     layout = "NHWC" if src.ndim == 4 else "HWC"
-    return cvtcolor_into(Tensor(_cvtcolor_shape(src.shape, code), src.dtype, layout), src, code, stream=stream)
+    return cvtcolor_into(_outputs.get(_cvtcolor_shape(src.shape, code), src.dtype, layout), src, code, stream=stream)
 
 
 def normalize_into(dst, src, base, scale, flags=None, *, globalscale=1.0, globalshift=0.0, epsilon=0.0, stream=None):
@@ -808,7 +884,7 @@ def normalize_into(dst, src, base, scale, flags=None, *, globalscale=1.0, global
 
 
 def normalize(src, base, scale, flags=None, *, globalscale=1.0, globalshift=0.0, epsilon=0.0, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else Tensor(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
     return normalize_into(dst, src, base, scale, flags, globalscale=globalscale, globalshift=globalshift,
                           epsilon=epsilon, stream=stream)
 
@@ -824,7 +900,7 @@ def reformat(src, layout, *, stream=None):
     if sorted(have) != sorted(layout):
         raise ValueError("layout %r is not a permutation of %r" % (layout, have))
     shape = tuple(src.shape[have.index(c)] for c in layout)
-    return reformat_into(Tensor(shape, src.dtype, layout), src, stream=stream)
+    return reformat_into(_outputs.get(shape, src.dtype, layout), src, stream=stream)
 
 
 def convertto_into(dst, src, scale=1, offset=0, *, stream=None):
@@ -833,7 +909,7 @@ def convertto_into(dst, src, scale=1, offset=0, *, stream=None):
 
 
 def convertto(src, dtype, scale=1, offset=0, *, stream=None):
-    return convertto_into(Tensor(src.shape, _np_dtype(dtype), src.layout), src, scale, offset, stream=stream)
+    return convertto_into(_outputs.get(src.shape, _np_dtype(dtype), src.layout), src, scale, offset, stream=stream)
 
 
 def customcrop_into(dst, src, rect, *, stream=None):
@@ -850,7 +926,7 @@ def customcrop(src, rect, *, stream=None):
     shape[wi] = rect.width
     if hi is not None:
         shape[hi] = rect.height
-    return customcrop_into(Tensor(tuple(shape), src.dtype, src.layout), src, rect, stream=stream)
+    return customcrop_into(_outputs.get(shape, src.dtype, src.layout), src, rect, stream=stream)
 
 
 def center_crop_into(dst, src, crop_size, *, stream=None):
@@ -864,7 +940,7 @@ def center_crop(src, crop_size, *, stream=None):
         raise ValueError("Non-supported tensor layout")
     shape = list(src.shape)
     shape[wi], shape[hi] = int(crop_size[0]), int(crop_size[1])
-    return center_crop_into(Tensor(tuple(shape), src.dtype, src.layout), src, crop_size, stream=stream)
+    return center_crop_into(_outputs.get(shape, src.dtype, src.layout), src, crop_size, stream=stream)
 
 
 def flip_into(dst, src, flipCode, *, stream=None):
@@ -877,7 +953,7 @@ def flip_into(dst, src, flipCode, *, stream=None):
 
 
 def flip(src, flipCode, *, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else Tensor(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
     return flip_into(dst, src, flipCode, stream=stream)
 
 
@@ -912,7 +988,7 @@ def warp_affine_into(dst, src, xform, flags, *, border_mode=Border.CONSTANT, bor
 
 
 def warp_affine(src, xform, flags, *, border_mode=Border.CONSTANT, border_value=0, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else Tensor(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
     return warp_affine_into(dst, src, xform, flags, border_mode=border_mode, border_value=border_value, stream=stream)
 
 
@@ -922,7 +998,7 @@ def warp_perspective_into(dst, src, xform, flags, *, border_mode, border_value, 
 
 
 def warp_perspective(src, xform, flags, *, border_mode, border_value, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else Tensor(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
     return warp_perspective_into(dst, src, xform, flags, border_mode=border_mode, border_value=border_value,
                                  stream=stream)
 
@@ -959,7 +1035,7 @@ def resize_crop_convert_reformat(src, resize_dim, interp, crop_rect, *, layout="
     if out_layout not in ("HWC", "NHWC", "CHW", "NCHW"):
         raise Error(7, "Output tensor must have layout 'HWC', 'NHWC', 'CHW', or 'NCHW'.")
     shape = tuple(nhwc["NHWC".index(c)] for c in out_layout)
-    dst = Tensor(shape, _np_dtype(data_type) if data_type else src_dtype, out_layout)
+    dst = _outputs.get(shape, _np_dtype(data_type) if data_type else src_dtype, out_layout)
     return resize_crop_convert_reformat_into(dst, src, resize_dim, interp, (rect.x, rect.y), manip=manip, scale=scale,
                                              offset=offset, srcCast=srcCast, stream=stream)
 
@@ -975,6 +1051,6 @@ def crop_flip_normalize_reformat_into(dst, src, rect, flip_code, base, scale, gl
 def crop_flip_normalize_reformat(src, out_shape, out_dtype, out_layout, rect, flip_code, base, scale, globalscale=1.0,
                                  globalshift=0.0, epsilon=0.0, flags=None, border=Border.CONSTANT, bvalue=0, *,
                                  stream=None):
-    dst = Tensor(tuple(out_shape), _np_dtype(out_dtype), out_layout)
+    dst = _outputs.get(out_shape, _np_dtype(out_dtype), out_layout)
     return crop_flip_normalize_reformat_into(dst, src, rect, flip_code, base, scale, globalscale, globalshift, epsilon,
                                              flags, border, bvalue, stream=stream)

@@ -209,3 +209,69 @@ def test_submit_orders_the_default_stream_by_events_recorded_when_needed(api, mo
     assert default.waited == [7, 7]
     api._submit(default, [b], [c], lambda s: None)  # its own result, and c, which only it has read since
     assert default.waited == [7, 7, 7]  # c was written by `side`
+
+
+def test_results_come_back_only_from_the_default_stream_and_unseen(api, monkeypatch):
+    # which of an operator's result tensors are handed out again (no GPU: the library's tensors are stand-ins)
+    import gc
+
+    class Raw:
+        made = 0
+
+        def __init__(self):
+            Raw.made += 1
+            self.handle = object()
+
+        @classmethod
+        def alloc(cls, shape, dtype, layout):
+            raw = cls()
+            raw.size = int(np.prod(shape)) * np.dtype(dtype).itemsize
+            return raw
+
+        def export(self):
+            class D:
+                rank, shape = 1, [1]
+
+                class buffer:
+                    strides = [self.size]
+            return D
+
+        def torch_view(self):
+            return "view"
+
+    monkeypatch.setattr(api, "_Tensor", Raw)
+    monkeypatch.setattr(api.torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    outputs = api._Outputs()
+    monkeypatch.setattr(api, "_outputs", outputs)
+
+    def used(mark=(0, None), reads=()):
+        t = outputs.get((2, 4), np.float32, "NC")
+        t._wrote, t._read = mark, {k: None for k in reads}
+        return t
+
+    t = used()
+    raw = t._t
+    del t
+    again = used(reads=[0])
+    assert again._t is raw and Raw.made == 1
+    other = outputs.get((2, 4), np.uint8, "NC")
+    assert Raw.made == 2 and other._t is not raw
+    del again
+    fresh = outputs.get((2, 4), np.float32, "NC")
+    assert fresh._t is raw and fresh._wrote == (0, None)  # a side stream's first use waits for the default stream
+    for spoil in (lambda t: t.torch(), lambda t: t.handle, lambda t: setattr(t, "_wrote", (7, None)),
+                  lambda t: t._read.update({7: None})):
+        t = used()
+        raw = t._t
+        spoil(t)
+        del t
+        gc.collect()
+        assert outputs.get((2, 4), np.float32, "NC")._t is not raw
+    outputs.most_bytes = 4096
+    keep = [outputs.get((256,), np.uint8, "N") for _ in range(40)]
+    del keep
+    assert outputs._bytes <= 4096 and outputs._count <= 16
+    big = outputs.get((2048,), np.uint8, "N")
+    raw = big._t
+    del big
+    assert outputs.get((2048,), np.uint8, "N")._t is not raw  # more than a quarter of the bound
