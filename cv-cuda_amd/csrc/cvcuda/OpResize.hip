@@ -9,7 +9,7 @@
 // point on those indices and weights (bilinear: FixedPointBlend.hpp; bicubic: kFixedCubic; box filter:
 // kAreaFixed), at most 1 from the reference's goldens.
 //
-// Seven kernel shapes, all with streaming stores, var-shape batches on a packed tile grid:
+// Eight kernel shapes, all with streaming stores, var-shape batches on a packed tile grid:
 //  * pixels of up to 8 bytes: wave patches (64 columns x 4 rows per wave; adjacent taps in one load,
 //    row terms computed once per wave, 4x4 lane transposes so that every lane stores whole dwords);
 //  * 8-bit bilinear at horizontal scales up to 2: a lane owns 2 columns x 4 rows (image batches x 2; 4 x 8 when
@@ -21,6 +21,8 @@
 //  * bicubic reductions >= 2x of 12/16-byte pixels: tap-major loads exchanged through LDS;
 //  * AREA of 8-bit pixels at reductions of up to 3: fixed-point row sums, a wave owns 64 columns x 16 rows and
 //    produces vertically adjacent rows in pairs from the source rows they share;
+//  * AREA of 8-bit tensors at larger reductions: one lane per output pixel, a row of its box in one window, rows in
+//    batches;
 //  * bilinear one-channel float tensors whose rows are not reduced, launches of 512 blocks and more: whole rows
 //    gathered in LDS and written out on 64-byte boundaries;
 //  * everything else (12/16-byte pixels, other AREA): one lane per output pixel, a 256-thread block covers
@@ -35,6 +37,7 @@
 #include <cvcuda/OpResize.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace cvamd {
@@ -3091,6 +3094,202 @@ __global__ __launch_bounds__(256) void ResizeCubicStagedKernel(const ResizeArgs 
 }
 
 // ---------------------------------------------------------------------------------------------
+// AREA of 8-bit pixels at reductions of more than the fixed-point form's 3 along an axis (up to kAreaWindowMost
+// horizontally), tensors. Bound by reading the source. The sums are ResizeValue's, term by term in its order; what
+// changes is how the source arrives. There a lane walks its box a few pixels per load and waits for each load in turn, and
+// the launch takes the time of that chain. Here a row of the box is one window of K pixels from its first (partial or
+// whole) pixel on, in up to three loads of 16 bytes from dword boundaries, and the windows of kAreaBatch rows are
+// requested before the first is used (with windows a pixel wider, 3 rows: 39.7 us in the first case below, 4: 40.3, 6: 38.6, but 92 / 98 / 101 us in
+// the second). Bytes of the window that are not whole pixels of the box are masked to 0, which a sum of non-negative terms
+// does not notice, so every lane adds K pixels; the left partial pixel is the window's first, the right one is a load of its
+// own (its place in the window differs from lane to lane); PARTIAL: the scale has such pixels. u8x3 32 x 1080p -> 320 x 180
+// 56.6 -> 38.1 us (5.4 TB/s), 16 x 4K -> 500 x 281 176.5 -> 83 us, 32 x 1080p -> 571 x 323 142 -> 77 us, one 2363 x 1415 ->
+// 355 x 153 15.9 -> 8.2 us; u8x4 16 x 4K -> 350 x 201 216 -> 117 us; u8x1 32 x 1080p -> 311 x 177 46.4 -> 24.9 us.
+constexpr float kAreaWindowMost = 12.f;
+constexpr int kAreaBatch = 3;
+
+template<int C, int K>
+struct AreaWindow
+{
+    static constexpr int kBytes = K * C, kDwords = (kBytes + 3) / 4; // brought to the front
+    static constexpr int kLoad  = C == 4 ? K : (kBytes + 3 + 3) / 4;  // the dwords that hold them at any offset
+    uint32_t d[kLoad];
+    uint32_t right;
+};
+
+template<int C, int K, bool PARTIAL>
+__device__ __forceinline__ void LoadAreaWindow(const uint8_t *row, uint32_t at, uint32_t rightAt, AreaWindow<C, K> &w)
+{
+    struct __attribute__((packed, aligned(1))) Dwords
+    {
+        uint32_t d[AreaWindow<C, K>::kLoad];
+    };
+    const Dwords v = *reinterpret_cast<const Dwords *>(row + at);
+    __builtin_memcpy(w.d, &v, sizeof(v));
+    if constexpr (PARTIAL)
+    {
+        w.right = C == 1 ? row[rightAt] : LoadU32Unaligned(row + rightAt);
+    }
+}
+
+// The same for the image's last row, behind which nothing may be read: dwords that end behind the row are moved back.
+template<int C, int K, bool PARTIAL>
+__device__ __forceinline__ void LoadAreaWindowGuarded(const uint8_t *row, uint32_t at, uint32_t rightAt, uint32_t rowBytes,
+                                                      AreaWindow<C, K> &w)
+{
+    auto dword = [&](uint32_t from)
+    {
+        const uint32_t back = min(from, rowBytes - 4), by = from - back;
+        return by < 4 ? LoadU32Unaligned(row + back) >> (8 * by) : 0u;
+    };
+#pragma unroll
+    for (int i = 0; i < AreaWindow<C, K>::kLoad; ++i)
+    {
+        w.d[i] = dword(at + 4 * i);
+    }
+    if constexpr (PARTIAL)
+    {
+        w.right = C == 1 ? row[rightAt] : dword(rightAt);
+    }
+}
+
+template<int C, int K, bool PARTIAL>
+__global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a)
+{
+    using Window = AreaWindow<C, K>;
+    const Plane p    = GetPlanes<false>(a, blockIdx.z);
+    const int   lane = threadIdx.x & 63, dx = blockIdx.x * kTileW + lane;
+    const int   dy   = blockIdx.y * kTileH + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (dx >= p.dstW || dy >= p.dstH)
+    {
+        return;
+    }
+    // ResizeValue's terms; the vertical ones are the same in all lanes
+    const float fsx1 = dx * p.scaleX, fsx2 = fsx1 + p.scaleX, fsy1 = dy * p.scaleY, fsy2 = fsy1 + p.scaleY;
+    const int   xmin = (int)ceilf(fsx1), xmax = (int)floorf(fsx2);
+    const int   ymin = __builtin_amdgcn_readfirstlane((int)ceilf(fsy1)), ymax = __builtin_amdgcn_readfirstlane((int)floorf(fsy2));
+    const bool  hasLeft = xmin > fsx1, hasRight = xmax < fsx2 && xmax < p.srcW;
+    const float scale = 1.f / (fminf(p.scaleX, p.srcW - fsx1) * fminf(p.scaleY, p.srcH - fsy1));
+    const float left = hasLeft ? xmin - fsx1 : 0.f, right = hasRight ? fsx2 - xmax : 0.f;
+
+    const uint32_t rowBytes = (uint32_t)p.srcW * C, off = (uint32_t)(xmin - (hasLeft ? 1 : 0)) * C;
+    const uint32_t rightAt = (uint32_t)min(xmax, p.srcW - 1) * C;
+    // whole pixels: bytes first .. last of the window
+    const int first = hasLeft ? C : 0, last = first + (min(xmax, p.srcW) - xmin) * C;
+    uint32_t  mask[Window::kDwords];
+#pragma unroll
+    for (int i = 0; i < Window::kDwords; ++i)
+    {
+        const int lo = min(max(first - 4 * i, 0), 4), hi = min(max(last - 4 * i, 0), 4);
+        mask[i] = (uint32_t)((1ull << (8 * hi)) - (1ull << (8 * lo)));
+        mask[i] = hi > lo ? mask[i] : 0u;
+    }
+
+    // rows in the order of the sums: the whole ones, the partial one above, the partial one below
+    const int whole = max(min(ymax, p.srcH) - ymin, 0);
+    const int above = ymin > fsy1 ? 1 : 0, below = ymax < fsy2 && ymax < p.srcH ? 1 : 0; // (uniform)
+    const int rows  = __builtin_amdgcn_readfirstlane(whole + above + below);
+    float     sum[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+    {
+        sum[c] = 0.f;
+    }
+    [[maybe_unused]] auto addPixel = [&](uint32_t q, float w)
+    {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+        {
+            sum[c] += (float)((q >> (8 * c)) & 0xFF) * w;
+        }
+    };
+#pragma unroll 1
+    for (int j0 = 0; j0 < rows; j0 += kAreaBatch)
+    {
+        Window   w[kAreaBatch];
+        uint32_t shift[kAreaBatch]; // of the window's first byte in its first dword (the low two bits)
+#pragma unroll
+        for (int b = 0; b < kAreaBatch; ++b)
+        {
+            const int j = min(j0 + b, rows - 1); // (a repeated row is not added)
+            const int y = j < whole ? ymin + j : (j == whole && above ? ymin - 1 : ymax);
+            const uint8_t *row = p.src + (int64_t)y * p.srcRow;
+            if (y == p.srcH - 1)
+            {
+                LoadAreaWindowGuarded<C, K, PARTIAL>(row, off & ~3u, rightAt, rowBytes, w[b]);
+                shift[b] = off;
+            }
+            else if constexpr (C == 4)
+            {
+                LoadAreaWindow<C, K, PARTIAL>(row, off, rightAt, w[b]);
+            }
+            else
+            {
+                // from the dword of memory that holds the first byte on
+                const uint32_t mis = (uint32_t)reinterpret_cast<uintptr_t>(row) & 3u;
+                shift[b]           = off + mis;
+                LoadAreaWindow<C, K, PARTIAL>(row - mis, shift[b] & ~3u, rightAt + mis, w[b]);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kAreaBatch; ++b)
+        {
+            const int j = j0 + b;
+            if (j >= rows)
+            {
+                break;
+            }
+            const bool top = j == whole && above, bottom = j >= whole && !top;
+            const float wy = top ? ymin - fsy1 : fsy2 - ymax; // (used for the partial rows only)
+            const float wi = j < whole ? scale : wy * scale;
+            const float wl = j < whole ? left * scale : wy * left * scale, wr = j < whole ? right * scale : wy * right * scale;
+            uint32_t    r[Window::kDwords + 1];
+#pragma unroll
+            for (int i = 0; i < Window::kDwords; ++i)
+            {
+                r[i] = C == 4 ? w[b].d[i] : __builtin_amdgcn_alignbyte(w[b].d[min(i + 1, Window::kLoad - 1)], w[b].d[i], shift[b]);
+            }
+            [[maybe_unused]] const uint32_t px0 = r[0];
+#pragma unroll
+            for (int i = 0; i < Window::kDwords; ++i)
+            {
+                r[i] &= mask[i];
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+            {
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                {
+                    const int byte = k * C + c;
+                    sum[c] += (float)((r[byte / 4] >> (8 * (byte % 4))) & 0xFF) * wi;
+                }
+            }
+            if constexpr (PARTIAL)
+            {
+                if (bottom)
+                {
+                    addPixel(w[b].right, wr);
+                    addPixel(px0, wl);
+                }
+                else
+                {
+                    addPixel(px0, wl);
+                    addPixel(w[b].right, wr);
+                }
+            }
+        }
+    }
+    Pixel<uint8_t, C> out;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+    {
+        out.v[c] = SaturateCast<uint8_t>(sum[c]);
+    }
+    StorePx<uint8_t, C>(p.dst + (int64_t)dy * p.dstRow, dx, out);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Bilinear resize of one-channel float pixels where rows are not reduced (maps and masks brought to their frames'
 // size). Bound by the output's writes. Rows of such outputs rarely start at a multiple of 64 bytes (a dense row of 1917
 // floats), and then every store instruction of a wave ends in two partly written 64-byte sectors that its neighbours
@@ -3274,6 +3473,29 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             hipLaunchKernelGGL((ResizeAreaFixedTensorKernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, kAreaRowsPerWave, flat),
                                dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeAreaFixedTensorKernel");
+            return;
+        }
+    }
+    if constexpr (kAreaFixed<T, C, INTERP>)
+    {
+        // Wider boxes than kAreaWindowMost, enlargements and rows shorter than a window keep the one-pixel form.
+        if (a.scaleX > 1.f && a.scaleX <= kAreaWindowMost && a.scaleY > 1.f && a.srcW * C >= 64)
+        {
+            const float s = a.scaleX;
+            // whole scales have no partial columns and exactly s pixels per row; between them the box has at most floor(s)
+            // whole pixels beside the partial first one, and one more where its end rounds up to a whole number
+            auto kernel = std::ceil(s) == s
+                            ? (s <= 4.f   ? ResizeAreaWindowKernel<C, 4, false>
+                               : s <= 6.f ? ResizeAreaWindowKernel<C, 6, false>
+                               : s <= 8.f ? ResizeAreaWindowKernel<C, 8, false>
+                                          : ResizeAreaWindowKernel<C, 12, false>)
+                            : (s < 4.f   ? ResizeAreaWindowKernel<C, 5, true>
+                               : s < 5.f ? ResizeAreaWindowKernel<C, 6, true>
+                               : s < 6.f ? ResizeAreaWindowKernel<C, 7, true>
+                               : s < 8.f ? ResizeAreaWindowKernel<C, 9, true>
+                                         : ResizeAreaWindowKernel<C, 13, true>);
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
+            CheckLaunch("ResizeAreaWindowKernel");
             return;
         }
     }

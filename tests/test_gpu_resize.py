@@ -378,6 +378,27 @@ def test_area_tensor(cv, orc, gpu, row):
             assert np.abs(res.astype(np.int64) - golden.astype(np.int64)).max() <= 1
 
 
+# the window form of larger reductions: whole scales of every window size, scales just below and above them, the widest,
+# axes that differ (one of them within the fixed-point form's 3), boxes at the right and lower edge, output columns that
+# leave most of a wave idle; dense odd rows and views whose rows start anywhere
+@pytest.mark.parametrize("sw,sh,dw,dh", [(256, 64, 64, 16), (390, 66, 65, 11), (512, 40, 64, 5), (780, 60, 65, 5), (257, 65, 64, 16),
+                                         (391, 67, 79, 11), (511, 41, 86, 5), (600, 50, 76, 9), (779, 61, 65, 5), (100, 90, 33, 8),
+                                         (133, 99, 129, 9), (67, 31, 20, 30), (64, 200, 16, 20), (90, 13, 8, 4), (1201, 45, 101, 4)])
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("kind", ["dense", "view"])
+def test_area_larger_reductions(cv, orc, gpu, sw, sh, dw, dh, c, kind):
+    src = make_input(orc, (2, sh, sw, c), np.uint8, 0xA3EA + sw + dh)
+    lead, pitch = (0, sw * c) if kind == "dense" else (3, sw * c + 5)
+    # exactly the rows and nothing behind the last one
+    buf = torch.zeros(lead + (2 * sh - 1) * pitch + sw * c, dtype=torch.uint8, device="cuda")
+    torch.as_strided(buf, (2, sh, sw, c), (sh * pitch, pitch, c, 1), lead).copy_(torch.from_numpy(src).cuda())
+    tin = cv.Tensor.wrap(buf.data_ptr() + lead, [2, sh, sw, c], [sh * pitch, pitch, c, 1], np.uint8, "NHWC", keep=buf)
+    out = torch.zeros((2, dh, dw, c), dtype=torch.uint8, device="cuda")
+    cv.Resize()(None, tin, cv.Tensor.from_torch(out, "NHWC"), AREA)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), AREA, threads=8))
+
+
 def test_area_sources_one_and_two_pixels_wide(cv, orc, gpu):
     # u8x3 rows shorter than the 4- and 8-byte tap loads: 1 x 1, 1 x H, 2 x 1 and W x 1 sources, every
     # interpolation (the tap loads of the last row must not be moved in front of the row)
