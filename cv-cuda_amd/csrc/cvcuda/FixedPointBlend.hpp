@@ -125,13 +125,17 @@ __device__ __forceinline__ int Dot2I16(uint32_t a, uint32_t b, int c)
     return __builtin_amdgcn_sdot2(x, y, c, false);
 }
 
-// a.lo * b.lo + a.hi * b.hi with nothing added: the three-operand form with the constant 0 (for a sum
-// that starts here the compiler picks the accumulate-in-place form and spends a move on clearing it).
-__device__ __forceinline__ int Dot2I16(uint32_t a, uint32_t b)
+// A row's four taps of one channel (two pairs) times the packed weights, as a float. The sum lies between -0.19 and 1.19
+// times 255 * 2^14, so accumulated on the bit pattern of 2^23 + 2^20, whose unit in the last place is 1, it is the
+// mantissa of a float that is that much too large, and a subtraction (exact) takes the place of v_cvt_f32_i32: the
+// vector unit issues additions, multiplications, logic and right shifts of 32 bits at 1.6 times the rate of everything
+// else (conversions, permutes, dot products ...: 590 G wave-instructions/s) and partly beside it. The start is an operand
+// of the three-operand form (the compiler would move it into the accumulator of the two-operand one).
+__device__ __forceinline__ float RowSumQ14(uint32_t taps01, uint32_t taps23, uint32_t p01, uint32_t p23)
 {
-    int d;
-    asm("v_dot2_i32_i16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
-    return d;
+    int h;
+    asm("v_dot2_i32_i16 %0, %1, %2, %3" : "=v"(h) : "v"(taps01), "v"(p01), "s"(0x4B100000u));
+    return __int_as_float(Dot2I16(taps23, p23, h)) - 9437184.f;
 }
 
 } // namespace cvamd

@@ -937,8 +937,8 @@ __device__ __forceinline__ uint32_t CubicRowsQ14(const Plane &p, int y0, uint32_
 #pragma unroll
         for (int c = 0; c < C; ++c)
         {
-            const int h = Dot2I16(QuadTapPair<C>(r[j], 2, c), w23, Dot2I16(QuadTapPair<C>(r[j], 0, c), w01));
-            acc[c]      = j == 0 ? (float)h * w : fmaf((float)h, w, acc[c]);
+            const float h = RowSumQ14(QuadTapPair<C>(r[j], 0, c), QuadTapPair<C>(r[j], 2, c), w01, w23);
+            acc[c]        = j == 0 ? h * w : fmaf(h, w, acc[c]);
         }
     }
     uint32_t q = 0;
@@ -973,7 +973,7 @@ __device__ __forceinline__ void CubicRowPairQ14(const Plane &p, int y0, uint32_t
 #pragma unroll
         for (int c = 0; c < C; ++c)
         {
-            const float h = (float)Dot2I16(QuadTapPair<C>(r[j], 2, c), w23, Dot2I16(QuadTapPair<C>(r[j], 0, c), w01));
+            const float h = RowSumQ14(QuadTapPair<C>(r[j], 0, c), QuadTapPair<C>(r[j], 2, c), w01, w23);
             if (j < 4)
             {
                 accA[c] = j == 0 ? h * wyA[0] : fmaf(h, wyA[j], accA[c]);
@@ -1360,7 +1360,7 @@ __device__ __forceinline__ void CubicRowSumsQ14(const RawQuadWindow<C> &w, uint3
 #pragma unroll
     for (int c = 0; c < C; ++c)
     {
-        h[c] = (float)Dot2I16(QuadTapPair<C>(r, 2, c), w23, Dot2I16(QuadTapPair<C>(r, 0, c), w01));
+        h[c] = RowSumQ14(QuadTapPair<C>(r, 0, c), QuadTapPair<C>(r, 2, c), w01, w23);
     }
 }
 

@@ -234,6 +234,73 @@ __device__ __forceinline__ uint32_t PixelOffset(const Img &im, int x, int y)
     return (uint32_t)__mul24(y, im.row) + (uint32_t)x * PIXEL_BYTES;
 }
 
+// 1 / x, correctly rounded, for 2^-123 <= |x| < 2^123: the hardware's approximation (within one unit in the last place) and
+// one correction by the residual, which fused multiply-adds form and apply without rounding in between (P. Markstein,
+// Computation of elementary functions on the IBM RISC System/6000 processor, 1990). Equal to the quotient for all 2^23
+// mantissas of both signs at every exponent in the range on gfx950.
+__device__ __forceinline__ float ReciprocalInRange(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
+}
+
+// The source coordinates of a lane's samples at the destination pixels (dx[k], dy[k]), as MapCoord gives them. A perspective's
+// quotients are 3 instructions instead of 10 where all of them are in ReciprocalInRange's range (16 x 1240 x 1754 u8x3
+// bicubic: see BlendCubicQ14).
+template<bool PERSPECTIVE, int N>
+__device__ __forceinline__ void MapCoords(const float (&m)[9], const int (&dx)[N], const int (&dy)[N], float (&sx)[N], float (&sy)[N])
+{
+    static_assert(N == 4);
+    if constexpr (PERSPECTIVE)
+    {
+        float    coeff[N];
+        uint32_t low = 0xffffffffu, high = 0;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            coeff[k] = m[6] * dx[k] + m[7] * dy[k] + m[8];
+            low      = min(low, __float_as_uint(coeff[k]) & 0x7fffffffu);
+            high     = max(high, __float_as_uint(coeff[k]) & 0x7fffffffu);
+        }
+        if (low >= (4u << 23) && high < (250u << 23))
+        {
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+            {
+                coeff[k] = ReciprocalInRange(coeff[k]);
+            }
+        }
+        else
+        {
+#pragma nounroll
+            for (int k = 0; k < N; ++k)
+            {
+                const float q = 1.0f / (k == 0 ? coeff[0] : k == 1 ? coeff[1] : k == 2 ? coeff[2] : coeff[3]);
+#pragma unroll
+                for (int j = 0; j < N; ++j)
+                {
+                    coeff[j] = j == k ? q : coeff[j];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            sx[k] = coeff[k] * (m[0] * dx[k] + m[1] * dy[k] + m[2]);
+            sy[k] = coeff[k] * (m[3] * dx[k] + m[4] * dy[k] + m[5]);
+        }
+    }
+    else
+    {
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            sx[k] = m[0] * dx[k] + m[1] * dy[k] + m[2];
+            sy[k] = m[3] * dx[k] + m[4] * dy[k] + m[5];
+        }
+    }
+}
+
 template<bool PERSPECTIVE>
 __device__ __forceinline__ void MapCoord(const float (&m)[9], int dx, int dy, float &sx, float &sy)
 {
@@ -558,9 +625,8 @@ __device__ __forceinline__ uint32_t BlendCubicQ14(const uint32_t (&r)[4][C], flo
 #pragma unroll
         for (int j = 0; j < 4; ++j)
         {
-            int h = Dot2I16(BytePair(r[j], c, c + C), p01);
-            h     = Dot2I16(BytePair(r[j], c + 2 * C, c + 3 * C), p23, h);
-            acc   = j == 0 ? (float)h * wy[0] : __builtin_fmaf((float)h, wy[j], acc);
+            const float h = RowSumQ14(BytePair(r[j], c, c + C), BytePair(r[j], c + 2 * C, c + 3 * C), p01, p23);
+            acc           = j == 0 ? h * wy[0] : __builtin_fmaf(h, wy[j], acc);
         }
         q = __builtin_amdgcn_cvt_pk_u8_f32(acc, c, q);
     }
@@ -956,6 +1022,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     // m maps to source coordinates times kCoordScale; so do sx, sy and the limits
     constexpr float kScale = kCoordScale<T, INTERP>;
     const float     limX = InsideLimit<INTERP>(im.w, kWideTapLoads<T, C>) * kScale, limY = InsideLimit<INTERP>(im.h, false) * kScale;
+    int         px[kPxPerLane], py[kPxPerLane]; // the lane's destination pixels
     float       sx[kPxPerLane], sy[kPxPerLane];
     uint32_t    q[D][kPxPerLane]; // q[d][k]: dword d of this lane's pixel in patch k
     // rows too long or too many for 24-bit offset arithmetic go through the generic path
@@ -966,11 +1033,11 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     for (int k = 0; k < kPxPerLane; ++k)
     {
         const int patch = wave * kPxPerLane + k;
-        const int px = (patch % kPatchesX) * kPatch + lx, py = (patch / kPatchesX) * kPatch + ly;
         // pixels of the tile beyond the image edge repeat the edge pixel's sample; they are never stored
-        const int dx = min(tx * kTileW + px, dstW - 1), dy = min(ty * kTileH + py, dstH - 1);
-        MapCoord<PERSP>(m, dx, dy, sx[k], sy[k]);
+        px[k] = min(tx * kTileW + (patch % kPatchesX) * kPatch + lx, dstW - 1);
+        py[k] = min(ty * kTileH + (patch / kPatchesX) * kPatch + ly, dstH - 1);
     }
+    MapCoords<PERSP>(m, px, py, sx, sy);
     allInside = allInside & TapsInside<INTERP>(limX, limY, sx, sy);
     if (allInside)
     {
@@ -1121,8 +1188,8 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         QuadTranspose(q[d], lx & 3);
     }
     const int patch = wave * kPxPerLane + (lx & 3);
-    const int px0 = (patch % kPatchesX) * kPatch + (lx & 4), py = (patch / kPatchesX) * kPatch + ly;
-    const int dy = ty * kTileH + py, dx0 = tx * kTileW + px0;
+    const int px0 = (patch % kPatchesX) * kPatch + (lx & 4);
+    const int dy = ty * kTileH + (patch / kPatchesX) * kPatch + ly, dx0 = tx * kTileW + px0;
     if (dy >= dstH || dx0 >= dstW)
     {
         return;
