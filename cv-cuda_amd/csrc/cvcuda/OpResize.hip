@@ -232,6 +232,12 @@ __device__ __forceinline__ void LoadTapPairBytes(const uint8_t *row, int xoff, b
     }
 }
 
+// Bytes from the dword boundary in front of a row to the row (wave-uniform).
+__device__ __forceinline__ uint32_t RowMisalignment(const uint8_t *row)
+{
+    return (uint32_t)reinterpret_cast<uintptr_t>(row) & 3u;
+}
+
 // Four horizontally adjacent 8-bit pixels as raw bytes (the box filter's and the bicubic blend's row window): the
 // D dwords that hold the 4 pixels at byte offset `at` + `shift` of the row (shift 0 .. 3; 4 channels: none),
 // brought to the front: pixel k, channel c in byte k * C + c.
@@ -251,26 +257,26 @@ __device__ __forceinline__ void LoadQuadWindow(const uint8_t *row, uint32_t at, 
     }
     else
     {
-        // the load runs up to 4 bytes past the window, harmless except behind the image's last row, where it is
-        // moved back to end with the row (GUARDED: the rows passed may include that one)
-        bool whole = false;
-        if (GUARDED && lastRow)
+        // From the dword of memory that holds the first byte, whatever the row's address (wave-uniform): loads counted from
+        // an odd row are not dword aligned, and the vector memory path takes those apart (32 x 1921 x 1081 -> 1280 x 720,
+        // box filter: 137 us counted from the row, 78 us so; 1920 x 1080 takes 61-63 us either way).
+        // The load runs up to 4 bytes past the window, harmless except behind the image's last row, where it is
+        // counted from the row and moved back to end with it (GUARDED: the rows passed may include that one).
+        const bool     guard = GUARDED && lastRow;
+        const uint32_t mis = guard ? 0u : RowMisalignment(row), o = at + shift + mis;
+        uint32_t       from = o & ~3u;
+        if (GUARDED)
         {
-            const uint32_t back = min(at, rowBytes - 4 * D);
-            shift += at - back; // up to 4
-            at    = back;
-            whole = shift == 4;
-            shift = whole ? 0 : shift;
+            from = lastRow ? min(from, rowBytes - 4 * D) : from;
         }
-        const Window w = *reinterpret_cast<const Window *>(row + at);
+        const Window   w     = *reinterpret_cast<const Window *>(row - mis + from);
+        const uint32_t sh    = o - from; // 4 at most, and only if moved back
+        const bool     whole = GUARDED && sh == 4;
 #pragma unroll
         for (int i = 0; i < C; ++i)
         {
-            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], shift);
-            if constexpr (GUARDED)
-            {
-                r[i] = whole ? w.d[i + 1] : r[i];
-            }
+            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], sh);
+            r[i] = whole ? w.d[i + 1] : r[i];
         }
     }
 }
@@ -1324,16 +1330,16 @@ struct RawQuadWindow
     uint32_t d[C == 4 ? 4 : C + 1];
 };
 
-// (row: wave-uniform; at: the lane's byte offset in it - the load then takes the row as its scalar base and the
-// lane needs no address arithmetic)
+// (row: wave-uniform; off: the window's byte offset in it - the load then takes the row as its scalar base. mis: the row's
+// RowMisalignment, so that the load starts at a dword of memory)
 template<int C>
-__device__ __forceinline__ RawQuadWindow<C> RequestQuadWindow(const uint8_t *row, uint32_t at)
+__device__ __forceinline__ RawQuadWindow<C> RequestQuadWindow(const uint8_t *row, uint32_t off, uint32_t mis)
 {
     struct __attribute__((packed, aligned(1))) Window
     {
         uint32_t d[C == 4 ? 4 : C + 1];
     };
-    const Window     w = *reinterpret_cast<const Window *>(row + at);
+    const Window     w = *reinterpret_cast<const Window *>(row - mis + (C == 4 ? off : (off + mis) & ~3u));
     RawQuadWindow<C> r;
     __builtin_memcpy(&r, &w, sizeof(r));
     return r;
@@ -1381,8 +1387,12 @@ __device__ __forceinline__ void CubicRowSumsQ14(const RawQuadWindow<C> &w, uint3
 // A strip takes this form when its windows advance as said from each output row to the next and stay clear of the
 // image's last row; others (the image's top and bottom, other scales) go one output row at a time with guarded
 // loads. The launch requires sources wide enough for the window loads (16 bytes a row, 8 for one channel).
-template<int C, int S>
-__device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y0)
+// ODD: the source's rows need not start at dwords of memory, and each window is placed by its row's address (32 x 1921 x
+// 1081 x 3 -> 1280 x 720: 160 us with loads counted from the row, 82 us so; to 1931 x 1081 from 1281 x 721: 227 and 140).
+// That costs two vector and a few scalar instructions per row, so that aligned rows keep a form of their own (1920 x
+// 1080: 79 us, with the other 83).
+template<int C, int S, bool ODD>
+__device__ __forceinline__ void ResizeCubicStripRowsU8(const Plane &p, int x0, int y0)
 {
     static_assert(S == 4 || S == 8);
     constexpr bool kReducing = S == 4;
@@ -1428,7 +1438,9 @@ __device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y
         }
         return;
     }
-    auto request = [&](int row) { return RequestQuadWindow<C>(p.src + (int64_t)row * p.srcRow, cq.at); };
+    const uint32_t off       = ODD ? cq.at + cq.shift : cq.at;
+    auto           misplaced = [&](int row) { return ODD ? RowMisalignment(p.src + (int64_t)row * p.srcRow) : 0u; };
+    auto           request = [&](int row) { return RequestQuadWindow<C>(p.src + (int64_t)row * p.srcRow, off, misplaced(row)); };
 
     float acc[S][C] = {};
     // The weight of source row j in output row r, whose second tap is row sr: tap j - (sr - 1) where that is 0 .. 3,
@@ -1453,7 +1465,7 @@ __device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y
     auto add = [&](int K, const RawQuadWindow<C> &w, int j, int r, const int (&sr)[S], int outputs, int sure)
     {
         float h[C];
-        CubicRowSumsQ14<C>(w, cq.shift, cq.w01, cq.w23, h);
+        CubicRowSumsQ14<C>(w, ODD ? off + misplaced(j) : cq.shift, cq.w01, cq.w23, h);
 #pragma unroll
         for (int i = 0; i < S; ++i)
         {
@@ -1552,6 +1564,17 @@ __device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y
             }
         }
     }
+}
+
+template<int C, int S>
+__device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y0)
+{
+    if (C != 4 && ((reinterpret_cast<uintptr_t>(p.src) | (uint32_t)p.srcRow) & 3) != 0)
+    {
+        ResizeCubicStripRowsU8<C, S, C != 4>(p, x0, y0);
+        return;
+    }
+    ResizeCubicStripRowsU8<C, S, false>(p, x0, y0);
 }
 
 // 8-bit bilinear at horizontal scales up to 2. The cost of the wave-patch form there is the number

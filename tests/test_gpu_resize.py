@@ -399,6 +399,25 @@ def test_area_larger_reductions(cv, orc, gpu, sw, sh, dw, dh, c, kind):
     np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), AREA, threads=8))
 
 
+# the row windows of the bicubic strips, the bicubic patches and the box filter, on dense images whose rows start at every
+# byte of a dword in turn, from every start of the first: the buffer ends with the image, whose last rows are read
+@pytest.mark.parametrize("c", [3, 1])
+@pytest.mark.parametrize("lead", [0, 1, 2, 3])
+@pytest.mark.parametrize("shape", [(1535, 703, 1021, 467, CUBIC, 6), (701, 101, 1285, 151, CUBIC, 1), (703, 90, 401, 57, AREA, 2),
+                                   (131, 37, 67, 19, AREA, 1), (67, 19, 66, 18, CUBIC, 2), (701, 501, 1003, 751, CUBIC, 5)],
+                         ids=lambda sh: "%dx%d-%dx%d-i%d-n%d" % sh)
+def test_rows_from_every_byte_of_a_dword(cv, orc, gpu, shape, lead, c):
+    sw, sh, dw, dh, interp, n = shape
+    src = make_input(orc, (n, sh, sw, c), np.uint8, 0xD0D + sw + lead)
+    buf = torch.zeros(lead + src.size, dtype=torch.uint8, device="cuda")
+    buf[lead:].copy_(torch.from_numpy(src.reshape(-1)))
+    tin = cv.Tensor.wrap(buf.data_ptr() + lead, [n, sh, sw, c], [sh * sw * c, sw * c, c, 1], np.uint8, "NHWC", keep=buf)
+    tout = cv.Tensor.alloc([n, dh, dw, c], np.uint8, "NHWC")
+    cv.Resize()(None, tin, tout, interp)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(tout.numpy(), orc.resize_shipped(src, (dh, dw), interp, threads=8))
+
+
 def test_area_sources_one_and_two_pixels_wide(cv, orc, gpu):
     # u8x3 rows shorter than the 4- and 8-byte tap loads: 1 x 1, 1 x H, 2 x 1 and W x 1 sources, every
     # interpolation (the tap loads of the last row must not be moved in front of the row)
