@@ -387,7 +387,7 @@ class _Outputs:
                 self._count -= 1
         out = Tensor(_wrap=raw if raw is not None else _Tensor.alloc(list(shape), dtype, layout or ""))
         if raw is not None:
-            out._wrote = _BY_DEFAULT  # another stream's first use of it waits for the default stream's last
+            out._wrote = (-key[3], None)  # another stream's first use of it waits for the default stream's last
         else:
             d = out._t.export()
             out._t._nbytes = d.buffer.strides[0] * d.shape[0] if d.rank else 0
@@ -396,7 +396,8 @@ class _Outputs:
 
     def put(self, tensor):
         try:
-            if getattr(tensor, "_wrote", _BY_DEFAULT)[0] != 0 or any(k != 0 for k in getattr(tensor, "_read", _NO_READS)):
+            by = -tensor._key[3]
+            if getattr(tensor, "_wrote", (by, None))[0] != by or any(k != by for k in getattr(tensor, "_read", _NO_READS)):
                 return
             # (not waited for: the collector may have stepped in while this thread holds the lock)
             if not self._lock.acquire(blocking=False):
@@ -418,8 +419,15 @@ class _Outputs:
 
 
 _NO_READS = {}
-_BY_DEFAULT = (0, None)
 _outputs = _Outputs()
+
+
+def _result(shape, dtype, layout, stream):
+    """A tensor for an operator's result. Only a call on the default stream takes one that is handed out again: another
+    stream would have to wait for the default stream's last use of it, which one that is being captured cannot."""
+    if _default_stream_key(stream) is None:
+        return Tensor(tuple(shape), dtype, layout)
+    return _outputs.get(shape, dtype, layout)
 
 
 def reshape(tensor, shape, layout=None):
@@ -706,7 +714,7 @@ def _submit(stream, reads, writes, op, *args):
     """Runs op(stream, *args) with the ordering the reference's bindings give their containers (its ResourceGuard,
     python/mod_nvcv/ResourceGuard.hpp): work on one stream that reads what another stream wrote, or writes what
     another stream still reads or writes, waits for that work first. Each container remembers, per stream, a mark of
-    its last write and of the reads since: an event recorded behind the work, or None for the default stream, which
+    its last write and of the reads since: an event recorded behind the work, or None for a device's default stream, which
     is never destroyed and never captured: its event is recorded when (and only if) another stream has to wait. Recorded
     behind every launch it cost 6 us of a 9 us pass with a small kernel and 2.6 us of the device's time with a large one."""
     key = _default_stream_key(stream)
@@ -723,22 +731,22 @@ def _submit(stream, reads, writes, op, *args):
             wrote = getattr(obj, "_wrote", None)
             if wrote is not None and wrote[0] != key:
                 waits = waits or []
-                waits.append(wrote[1])
+                waits.append(wrote)
         for obj in writes:
             wrote = getattr(obj, "_wrote", None)
             if wrote is not None and wrote[0] != key:
                 waits = waits or []
-                waits.append(wrote[1])
+                waits.append(wrote)
             for other, mark in getattr(obj, "_read", _NO_READS).items():
                 if other != key:
                     waits = waits or []
-                    waits.append(mark)
+                    waits.append((other, mark))
     if waits:
-        waiting = s if s else _default_stream()
-        for mark in waits:
+        waiting = s if s else _default_stream(-key)
+        for other, mark in waits:
             if mark is None:
                 mark = _new_event()
-                mark.record(_default_stream())
+                mark.record(_default_stream(-other))
             waiting.wait_event(mark)
     op(s, *[a._t if type(a) is Tensor else a for a in args])
     mark = None
@@ -759,18 +767,20 @@ _events_lock = threading.Lock()
 
 
 def _default_stream_key(stream):
-    """0, the default stream's handle, where `stream` (None: the current one) is the default stream; else None. What
-    Stream.current gives, without making its objects."""
+    """Where `stream` (None: the current one, what Stream.current gives, without making its objects) is a device's default
+    stream: 0 for the first device's and -n for device n's, as no other stream's handle is; else None."""
     if stream is None:
         stack = getattr(Stream._tls, "stack", None)
         if not stack:
-            return 0 if torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()) == 0 else None
+            device = torch._C._cuda_getDevice()
+            return -device if torch._C._cuda_getCurrentRawStream(device) == 0 else None
         stream = stack[-1]
-    return 0 if getattr(stream, "_s", stream).cuda_stream == 0 else None
+    stream = getattr(stream, "_s", stream)
+    return -getattr(stream, "device_index", 0) if stream.cuda_stream == 0 else None
 
 
-def _default_stream():
-    return torch.cuda.default_stream()
+def _default_stream(device):
+    return torch.cuda.default_stream(device)
 
 
 def _new_event():
@@ -805,7 +815,7 @@ def resize(src, shape=None, interp=Interp.LINEAR, *, sizes=None, stream=None):
         if len(src) != len(sizes):
             raise RuntimeError("Number of input images must be equal to the number of elements in output size list ")
         return resize_into(_same_images(src, sizes=[tuple(s) for s in sizes]), src, interp, stream=stream)
-    return resize_into(_outputs.get(shape, src.dtype, src.layout), src, interp, stream=stream)
+    return resize_into(_result(shape, src.dtype, src.layout, stream), src, interp, stream=stream)
 
 
 _CODE = re.compile(r"^(.*?)2(BGRA|RGBA|BGR|RGB|GRAY|YUV|HSV|HLS|YCrCb|XYZ|Lab|Luv)(.*)$")
@@ -874,7 +884,7 @@ def cvtcolor(src, code, *, stream=None):
             raise RuntimeError("All images in input must have the same single-plane format")
         return cvtcolor_into(_same_images(src, fmt=_cvtcolor_format(fmt, code)), src, code, stream=stream)
     layout = "NHWC" if src.ndim == 4 else "HWC"
-    return cvtcolor_into(_outputs.get(_cvtcolor_shape(src.shape, code), src.dtype, layout), src, code, stream=stream)
+    return cvtcolor_into(_result(_cvtcolor_shape(src.shape, code), src.dtype, layout, stream), src, code, stream=stream)
 
 
 def normalize_into(dst, src, base, scale, flags=None, *, globalscale=1.0, globalshift=0.0, epsilon=0.0, stream=None):
@@ -884,7 +894,7 @@ def normalize_into(dst, src, base, scale, flags=None, *, globalscale=1.0, global
 
 
 def normalize(src, base, scale, flags=None, *, globalscale=1.0, globalshift=0.0, epsilon=0.0, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
     return normalize_into(dst, src, base, scale, flags, globalscale=globalscale, globalshift=globalshift,
                           epsilon=epsilon, stream=stream)
 
@@ -900,7 +910,7 @@ def reformat(src, layout, *, stream=None):
     if sorted(have) != sorted(layout):
         raise ValueError("layout %r is not a permutation of %r" % (layout, have))
     shape = tuple(src.shape[have.index(c)] for c in layout)
-    return reformat_into(_outputs.get(shape, src.dtype, layout), src, stream=stream)
+    return reformat_into(_result(shape, src.dtype, layout, stream), src, stream=stream)
 
 
 def convertto_into(dst, src, scale=1, offset=0, *, stream=None):
@@ -909,7 +919,7 @@ def convertto_into(dst, src, scale=1, offset=0, *, stream=None):
 
 
 def convertto(src, dtype, scale=1, offset=0, *, stream=None):
-    return convertto_into(_outputs.get(src.shape, _np_dtype(dtype), src.layout), src, scale, offset, stream=stream)
+    return convertto_into(_result(src.shape, _np_dtype(dtype), src.layout, stream), src, scale, offset, stream=stream)
 
 
 def customcrop_into(dst, src, rect, *, stream=None):
@@ -926,7 +936,7 @@ def customcrop(src, rect, *, stream=None):
     shape[wi] = rect.width
     if hi is not None:
         shape[hi] = rect.height
-    return customcrop_into(_outputs.get(shape, src.dtype, src.layout), src, rect, stream=stream)
+    return customcrop_into(_result(shape, src.dtype, src.layout, stream), src, rect, stream=stream)
 
 
 def center_crop_into(dst, src, crop_size, *, stream=None):
@@ -940,7 +950,7 @@ def center_crop(src, crop_size, *, stream=None):
         raise ValueError("Non-supported tensor layout")
     shape = list(src.shape)
     shape[wi], shape[hi] = int(crop_size[0]), int(crop_size[1])
-    return center_crop_into(_outputs.get(shape, src.dtype, src.layout), src, crop_size, stream=stream)
+    return center_crop_into(_result(shape, src.dtype, src.layout, stream), src, crop_size, stream=stream)
 
 
 def flip_into(dst, src, flipCode, *, stream=None):
@@ -953,7 +963,7 @@ def flip_into(dst, src, flipCode, *, stream=None):
 
 
 def flip(src, flipCode, *, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
     return flip_into(dst, src, flipCode, stream=stream)
 
 
@@ -988,7 +998,7 @@ def warp_affine_into(dst, src, xform, flags, *, border_mode=Border.CONSTANT, bor
 
 
 def warp_affine(src, xform, flags, *, border_mode=Border.CONSTANT, border_value=0, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
     return warp_affine_into(dst, src, xform, flags, border_mode=border_mode, border_value=border_value, stream=stream)
 
 
@@ -998,7 +1008,7 @@ def warp_perspective_into(dst, src, xform, flags, *, border_mode, border_value, 
 
 
 def warp_perspective(src, xform, flags, *, border_mode, border_value, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _outputs.get(src.shape, src.dtype, src.layout)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
     return warp_perspective_into(dst, src, xform, flags, border_mode=border_mode, border_value=border_value,
                                  stream=stream)
 
@@ -1035,7 +1045,7 @@ def resize_crop_convert_reformat(src, resize_dim, interp, crop_rect, *, layout="
     if out_layout not in ("HWC", "NHWC", "CHW", "NCHW"):
         raise Error(7, "Output tensor must have layout 'HWC', 'NHWC', 'CHW', or 'NCHW'.")
     shape = tuple(nhwc["NHWC".index(c)] for c in out_layout)
-    dst = _outputs.get(shape, _np_dtype(data_type) if data_type else src_dtype, out_layout)
+    dst = _result(shape, _np_dtype(data_type) if data_type else src_dtype, out_layout, stream)
     return resize_crop_convert_reformat_into(dst, src, resize_dim, interp, (rect.x, rect.y), manip=manip, scale=scale,
                                              offset=offset, srcCast=srcCast, stream=stream)
 
@@ -1051,6 +1061,6 @@ def crop_flip_normalize_reformat_into(dst, src, rect, flip_code, base, scale, gl
 def crop_flip_normalize_reformat(src, out_shape, out_dtype, out_layout, rect, flip_code, base, scale, globalscale=1.0,
                                  globalshift=0.0, epsilon=0.0, flags=None, border=Border.CONSTANT, bvalue=0, *,
                                  stream=None):
-    dst = _outputs.get(out_shape, _np_dtype(out_dtype), out_layout)
+    dst = _result(out_shape, _np_dtype(out_dtype), out_layout, stream)
     return crop_flip_normalize_reformat_into(dst, src, rect, flip_code, base, scale, globalscale, globalshift, epsilon,
                                              flags, border, bvalue, stream=stream)

@@ -194,7 +194,7 @@ def test_submit_orders_the_default_stream_by_events_recorded_when_needed(api, mo
 
     default, side, other = FakeStream(0), FakeStream(7), FakeStream(9)
     monkeypatch.setattr(api, "_torch_stream", lambda s: s)
-    monkeypatch.setattr(api, "_default_stream", lambda: default)
+    monkeypatch.setattr(api, "_default_stream", lambda device: default)
     monkeypatch.setattr(api, "_new_event", FakeEvent)
     a, b, c = Box(), Box(), Box()
     handles = []
@@ -275,3 +275,46 @@ def test_results_come_back_only_from_the_default_stream_and_unseen(api, monkeypa
     raw = big._t
     del big
     assert outputs.get((2048,), np.uint8, "N")._t is not raw  # more than a quarter of the bound
+
+
+def test_default_streams_of_two_devices_are_told_apart(api, monkeypatch):
+    # a wait for work on the second device's default stream is for an event recorded there, whatever device is current
+    class FakeStream:
+        def __init__(self, key, device):
+            self.cuda_stream, self.device_index, self.waited = key, device, []
+
+        def wait_event(self, event):
+            self.waited.append(event.stream)
+
+    class FakeEvent:
+        def record(self, stream):
+            self.stream = (stream.cuda_stream, stream.device_index)
+
+    class Box:
+        pass
+
+    default = [FakeStream(0, 0), FakeStream(0, 1)]
+    monkeypatch.setattr(api, "_torch_stream", lambda s: s)
+    monkeypatch.setattr(api, "_default_stream", lambda device: default[device])
+    monkeypatch.setattr(api, "_new_event", FakeEvent)
+    a, side = Box(), FakeStream(7, 0)
+    api._submit(default[1], [], [a], lambda s: None)
+    api._submit(side, [a], [], lambda s: None)
+    assert side.waited == [(0, 1)]
+    api._submit(default[1], [a], [], lambda s: None)
+    assert not default[1].waited
+    api._submit(default[0], [], [a], lambda s: None)
+    assert default[0].waited == [(0, 1), (7, 0), (0, 1)]
+
+
+def test_results_on_other_streams_are_always_new(api, monkeypatch):
+    # a call on another stream (one that is being captured cannot wait for the default stream) takes no kept result
+    class FakeStream:
+        def __init__(self, key):
+            self.cuda_stream, self.device_index = key, 0
+
+    made = []
+    monkeypatch.setattr(api, "Tensor", lambda *args: made.append(args) or "new")
+    monkeypatch.setattr(api._outputs, "get", lambda *args: "kept")
+    assert api._result([2, 3], np.uint8, "HW", FakeStream(7)) == "new" and made == [((2, 3), np.uint8, "HW")]
+    assert api._result([2, 3], np.uint8, "HW", FakeStream(0)) == "kept"
