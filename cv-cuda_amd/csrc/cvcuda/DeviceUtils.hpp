@@ -146,43 +146,6 @@ __device__ __forceinline__ void StoreDwordsNT(uint8_t *p, const uint32_t (&w)[N]
     }
 }
 
-// 8 bytes starting at the arbitrary byte address base + off, fetched as 3 ALIGNED dwords and funnel-
-// shifted into place. The texture path serves a misaligned multi-dword load at a fraction of the
-// rate of an aligned one (measured on a gather of u8x3 pixel pairs: 31 vs 22 cycles per wave-load),
-// which costs more than the two extra shifts. Reads the aligned window [p & ~3, (p & ~3) + 12) for
-// p = base + off: up to 3 bytes before p (same dword as p, so never another page) and up to 6 bytes
-// after the data; the caller keeps that tail inside its allocation. base must be uniform over the
-// wave: its misalignment is folded into the 32-bit offset, so the per-lane address arithmetic is one
-// mask (the load takes the aligned base from scalar registers plus a 32-bit lane offset) instead of
-// 64-bit adds per lane.
-__device__ __forceinline__ uint64_t LoadU64Window(const uint8_t *base, uint32_t off)
-{
-    struct alignas(4) W3
-    {
-        uint32_t d[3];
-    };
-    const uint32_t mis = (uint32_t)reinterpret_cast<uintptr_t>(base) & 3u;
-    const uint32_t o   = off + mis;
-    const W3       w   = *reinterpret_cast<const W3 *>((base - mis) + (o & ~3u));
-    const uint32_t lo  = __builtin_amdgcn_alignbyte(w.d[1], w.d[0], o); // shifts by the bytes in bits 1:0
-    const uint32_t hi  = __builtin_amdgcn_alignbyte(w.d[2], w.d[1], o);
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// 4 bytes starting at the arbitrary byte address base + off, the same way: 2 aligned dwords and one
-// funnel shift. Reads up to 3 bytes before and up to 4 bytes after the data.
-__device__ __forceinline__ uint32_t LoadU32Window(const uint8_t *base, uint32_t off)
-{
-    struct alignas(4) W2
-    {
-        uint32_t d[2];
-    };
-    const uint32_t mis = (uint32_t)reinterpret_cast<uintptr_t>(base) & 3u;
-    const uint32_t o   = off + mis;
-    const W2       w   = *reinterpret_cast<const W2 *>((base - mis) + (o & ~3u));
-    return __builtin_amdgcn_alignbyte(w.d[1], w.d[0], o);
-}
-
 // The constant a caller gives for pixels outside the image, as an element of type T: truncated toward
 // zero and saturated to T's range (floats pass through).
 template<class T>

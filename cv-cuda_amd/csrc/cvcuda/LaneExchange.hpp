@@ -40,7 +40,7 @@ __device__ __forceinline__ void QuadTranspose(uint32_t (&r)[4], int i)
     }
 }
 
-// 4 pixels of PB bytes, each held zero-extended in ceil(PB/4) dwords (q[d][k] = dword d of pixel k),
+// 4 pixels of PB bytes, each held in ceil(PB/4) dwords (q[d][k] = dword d of pixel k; zero-extended where PB is 2 or 6),
 // packed back to back into PB dwords.
 template<int PB>
 __device__ __forceinline__ void PackQuad(const uint32_t (&q)[(PB + 3) / 4][4], uint32_t (&w)[PB])
@@ -59,7 +59,8 @@ __device__ __forceinline__ void PackQuad(const uint32_t (&q)[(PB + 3) / 4][4], u
     }
     else if constexpr (PB == 1)
     {
-        w[0] = q[0][0] | (q[0][1] << 8) | (q[0][2] << 16) | (q[0][3] << 24);
+        w[0] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(q[0][3], q[0][2], 0x0c0c0400u),
+                                     __builtin_amdgcn_perm(q[0][1], q[0][0], 0x0c0c0400u), 0x05040100u);
     }
     else if constexpr (PB == 2)
     {
@@ -68,9 +69,10 @@ __device__ __forceinline__ void PackQuad(const uint32_t (&q)[(PB + 3) / 4][4], u
     }
     else if constexpr (PB == 3)
     {
-        w[0] = q[0][0] | (q[0][1] << 24);
-        w[1] = (q[0][1] >> 8) | (q[0][2] << 16);
-        w[2] = (q[0][2] >> 16) | (q[0][3] << 8);
+        // bytes 0 1 2 of each
+        w[0] = __builtin_amdgcn_perm(q[0][1], q[0][0], 0x04020100u);
+        w[1] = __builtin_amdgcn_perm(q[0][2], q[0][1], 0x05040201u);
+        w[2] = __builtin_amdgcn_perm(q[0][3], q[0][2], 0x06050402u);
     }
     else
     {

@@ -13,7 +13,7 @@
 // one operator handle may therefore be in flight at once. Var-shape batches run on a packed tile grid.
 //
 // Kernel shape. A 256-thread block produces a 64 x 16 pixel tile of the destination; each of its four
-// waves works on its own 32 x 8 part, no LDS and no barrier.
+// waves works on its own 32 x 8 part, no barrier.
 // Gather: the cost of the gather is set by how many distinct cache lines one wave-wide load touches,
 // and under a rotation every source row a wave's footprint crosses is another line; so a wave samples
 // compact 8 x 8 pixel patches (one lane per pixel, ~10 source rows per load where a 64 x 1 strip would
@@ -21,9 +21,9 @@
 // whose loads are in flight together. Taps that lie inside the source image - nearly all of them -
 // skip the border logic and fetch the horizontally adjacent taps of a row with one load (u8x3: the 6
 // bytes of two pixels from an aligned 12-byte window).
-// Store: a 4x4 transpose inside every group of 4 lanes (cross-lane moves) turns "one pixel in each of 4
-// patches" into "4 consecutive pixels of one row in one patch", which the lane writes as whole dwords;
-// single-byte stores scattered over 8 rows are several times slower.
+// Store: "one pixel in each of 4 patches" becomes "4 consecutive pixels of one row", which the lane writes as whole
+// dwords (through LDS, or by a 4x4 transpose inside every group of 4 lanes); single-byte stores scattered over 8 rows
+// are several times slower.
 #include "DeviceUtils.hpp"
 #include "FixedPointBlend.hpp"
 #include "LaneExchange.hpp"
@@ -44,7 +44,8 @@ constexpr int kPatch     = 8;  // gather granule: a wave samples kPatch x kPatch
 constexpr int kPxPerLane = 4;  // steps per wave
 constexpr int kTileW     = 64; // = 8 patches
 constexpr int kTileH     = 16; // = 2 patches; 16 patches / 4 waves = kPxPerLane
-constexpr int kPatchesX  = kTileW / kPatch;
+constexpr int kWaveW     = kPatch * kPxPerLane; // a wave's patches lie side by side
+constexpr int kWavesX    = kTileW / kWaveW;
 constexpr int kThreads   = kTileW * kTileH / kPxPerLane;
 
 struct WarpArgs
@@ -170,31 +171,28 @@ __device__ __forceinline__ void CubicCoeffsFused(float d, float scale, float (&w
     w[3] = scale - w[0] - w[1] - w[2];
 }
 
-// u8x3 taps are fetched through aligned dword windows (8 bytes for one pixel, 12 for two), which
-// read up to 6 bytes = 2 pixels past them. Inside the image that is harmless; taps within 2 pixels
-// of the end of the last row, after which the image ends, are kept off this path by TapsInside.
+// Taps of 1 and 3 bytes are fetched through dword-aligned windows, as many dwords as hold the taps of a row wherever they
+// start (single bytes as they are). Windows read up to 2 pixels (u8x3) past the taps, 6 (u8x1 bilinear) or 4 (bicubic):
+// harmless inside the image; taps that close to the end of a row, and so of the image, are kept off this path by TapsInside.
 template<class T, int C>
-constexpr bool kWideTapLoads = std::is_same_v<T, uint8_t> && C == 3;
+constexpr bool kWideTapLoads = std::is_same_v<T, uint8_t> && (C == 1 || C == 3);
+
+template<class T, int C, int INTERP>
+constexpr int kTapOverrun = !kWideTapLoads<T, C>          ? 0
+                          : C == 3                        ? 2
+                          : INTERP == NVCV_INTERP_NEAREST ? 0
+                          : INTERP == NVCV_INTERP_LINEAR  ? 6
+                                                          : 4;
 
 // One pixel at base + off, known to be inside the image.
 template<class T, int C>
 __device__ __forceinline__ void LoadPixelInside(const uint8_t *base, uint32_t off, T (&out)[C])
 {
-    if constexpr (kWideTapLoads<T, C>)
-    {
-        const uint32_t q = LoadU32Window(base, off);
-        out[0]           = (uint8_t)q;
-        out[1]           = (uint8_t)(q >> 8);
-        out[2]           = (uint8_t)(q >> 16);
-    }
-    else
-    {
-        const Vec<T, C> v = *reinterpret_cast<const Vec<T, C> *>(base + off);
+    const Vec<T, C> v = *reinterpret_cast<const Vec<T, C> *>(base + off);
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-        {
-            out[c] = v.v[c];
-        }
+    for (int c = 0; c < C; ++c)
+    {
+        out[c] = v.v[c];
     }
 }
 
@@ -202,26 +200,12 @@ __device__ __forceinline__ void LoadPixelInside(const uint8_t *base, uint32_t of
 template<class T, int C>
 __device__ __forceinline__ void LoadPairInside(const uint8_t *base, uint32_t off, float (&p0)[C], float (&p1)[C])
 {
-    if constexpr (kWideTapLoads<T, C>)
-    {
-        const uint64_t q  = LoadU64Window(base, off);
-        const uint32_t lo = (uint32_t)q, hi = (uint32_t)(q >> 32);
-        p0[0] = (float)(lo & 0xFF);
-        p0[1] = (float)((lo >> 8) & 0xFF);
-        p0[2] = (float)((lo >> 16) & 0xFF);
-        p1[0] = (float)(lo >> 24);
-        p1[1] = (float)(hi & 0xFF);
-        p1[2] = (float)((hi >> 8) & 0xFF);
-    }
-    else
-    {
-        const Vec<T, 2 * C> v = *reinterpret_cast<const Vec<T, 2 * C> *>(base + off);
+    const Vec<T, 2 * C> v = *reinterpret_cast<const Vec<T, 2 * C> *>(base + off);
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-        {
-            p0[c] = (float)v.v[c];
-            p1[c] = (float)v.v[C + c];
-        }
+    for (int c = 0; c < C; ++c)
+    {
+        p0[c] = (float)v.v[c];
+        p1[c] = (float)v.v[C + c];
     }
 }
 
@@ -465,9 +449,9 @@ __device__ __forceinline__ void SampleWithBorder(const Img &im, const WarpArgs &
     }
 }
 
-// True when every tap of the sample at (sx, sy) lies inside the image (and, with WIDE loads, none of
-// them is among the image's last two columns: the window loads read 2 pixels past a tap pair, which
-// must not run off the end of the last row). limX / limY come from InsideLimits. For an integer k,
+// True when every tap of the sample at (sx, sy) lies inside the image (and none of them is among
+// the image's last kTapOverrun columns: the window loads read that far past a row's taps, which must not run off the end
+// of the last row). limX / limY come from InsideLimits. For an integer k,
 // floor(v) < k <=> v < k, so the test is 0 <= v - lo < lim per axis, done as ONE unsigned comparison
 // of the float's bit pattern: non-negative floats order like their bits, negative ones and NaNs have
 // patterns above every finite positive limit (-0.0 fails too and takes the generic path, which
@@ -492,11 +476,11 @@ __device__ __forceinline__ bool TapsInside(float limX, float limY, const float (
 // Exclusive upper limit of floor(v) - lo along an axis of `size` pixels; 0 (no sample passes) when the
 // image is smaller than the tap span.
 template<int INTERP>
-__device__ __forceinline__ float InsideLimit(int size, bool wide)
+__device__ __forceinline__ float InsideLimit(int size, int overrun)
 {
     constexpr int lo = INTERP == NVCV_INTERP_CUBIC ? 1 : 0;
     constexpr int hi = INTERP == NVCV_INTERP_CUBIC ? 2 : (INTERP == NVCV_INTERP_LINEAR ? 1 : 0);
-    return (float)max(size - hi - lo - (wide ? 2 : 0), 0);
+    return (float)max(size - hi - lo - overrun, 0);
 }
 
 // Same arithmetic as SampleWithBorder for a sample whose taps are all inside the image: no border
@@ -582,29 +566,70 @@ __device__ __forceinline__ void SampleInside(const Img &im, float sx, float sy, 
     }
 }
 
-// Four horizontally adjacent u8 pixels at base + off (all inside the image) as raw bytes in C dwords.
-// u8x3: one aligned 16-byte window, funnel-shifted (see LoadU64Window); reads up to 3 bytes before and
-// 4 bytes after the 12.
-template<int C>
-__device__ __forceinline__ void LoadQuadBytes(const uint8_t *base, uint32_t off, uint32_t (&r)[C])
+// A uniform address that stays one: without this the compiler adds the row's part to each lane's 64-bit address.
+__device__ __forceinline__ const uint8_t *UniformRow(const uint8_t *row)
 {
-    if constexpr (kWideTapLoads<uint8_t, C>)
+    uintptr_t at = reinterpret_cast<uintptr_t>(row);
+    asm("" : "+s"(at));
+    return AsGlobal(reinterpret_cast<const uint8_t *>(at));
+}
+
+// The rows y .. y + ROWS - 1 of a u8 image, from pixel x on (TAPS pixels, all inside the image), as raw bytes: r[j] holds row
+// j's. Per sample this is two multiply-adds for the offset, whose start (uniform) takes in what is added to x and y, and, where
+// the rows' addresses agree in their low two bits (SAME: a row pitch of whole dwords), one mask: a row's address is its own
+// uniform base plus that one offset. Written with the compiler's choice of instructions and the row pitch added per lane,
+// the kernel had a fifth more vector instructions (bilinear; bicubic a ninth). Single-channel taps, which had been fetched as
+// 2- and 4-byte loads at any address, gain most, by the loads: one that is not dword aligned is taken apart (a gather of
+// u8x3 pixel pairs: 31 against 22 cycles per wave). 24 x 1283 x 721 u8x1 bilinear 54.3 -> 43.0 us, bicubic 131.3 -> 100.7;
+// 16 x 1280 x 720 u8x3 bicubic 68.4 -> 64.6, bilinear 30.1 -> 29.2 (its gathers and their latency are left).
+template<int C, int TAPS, int ROWS, bool SAME>
+__device__ __forceinline__ void LoadTapRows(const Img &im, int x, int y, int x0, int y0, uint32_t (&r)[ROWS][(C * TAPS + 3) / 4])
+{
+    constexpr int  N       = (C * TAPS + 3) / 4;
+    constexpr bool kWindow = kWideTapLoads<uint8_t, C> && C * TAPS > 1;
+    constexpr int  kLoad   = kWindow ? (C * TAPS + 3 + 3) / 4 : N; // dwords that hold C * TAPS bytes at any of the 4 places
+    struct alignas(4) W
     {
-        struct alignas(4) W4
+        uint32_t d[kLoad];
+    };
+    const uint32_t mis0  = kWindow ? (uint32_t)reinterpret_cast<uintptr_t>(im.base) & 3u : 0u;
+    const int      start = y0 * im.row + x0 * C + (int)mis0;
+    uint32_t       o;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(o) : "v"(x), "n"(C), "s"(start));
+    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(o) : "v"(y), "s"(im.row), "v"(o));
+    W w[ROWS];
+    if constexpr (kWindow)
+    {
+        uint32_t       shift[ROWS];
+        const uint8_t *base = im.base - mis0;
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j)
         {
-            uint32_t d[4];
-        };
-        const uint32_t mis = (uint32_t)reinterpret_cast<uintptr_t>(base) & 3u;
-        const uint32_t o   = off + mis;
-        const W4       w   = *reinterpret_cast<const W4 *>((base - mis) + (o & ~3u));
-        r[0]               = __builtin_amdgcn_alignbyte(w.d[1], w.d[0], o);
-        r[1]               = __builtin_amdgcn_alignbyte(w.d[2], w.d[1], o);
-        r[2]               = __builtin_amdgcn_alignbyte(w.d[3], w.d[2], o);
+            // (in a row pitch that is not of whole dwords, row j's base starts at a dword and its offset grows by the rest)
+            const uint32_t rest = SAME ? 0u : (mis0 + (uint32_t)(j * im.row)) & 3u;
+            shift[j]            = SAME ? o : o - mis0 + rest;
+            const uint8_t *row  = UniformRow(SAME ? base + j * im.row : im.base + j * im.row - rest);
+            w[j]                = *reinterpret_cast<const W *>(row + (shift[j] & ~3u));
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+        {
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+            {
+                r[j][i] = __builtin_amdgcn_alignbyte(i + 1 < kLoad ? w[j].d[i + 1] : w[j].d[i], w[j].d[i], shift[j]);
+            }
+        }
     }
     else
     {
-        const Vec<uint8_t, 4 * C> v = *reinterpret_cast<const Vec<uint8_t, 4 * C> *>(base + off);
-        __builtin_memcpy(r, &v, 4 * C);
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+        {
+            const Vec<uint8_t, C * TAPS> v = *reinterpret_cast<const Vec<uint8_t, C * TAPS> *>(UniformRow(im.base + j * im.row) + o);
+            r[j][N - 1]                    = 0;
+            __builtin_memcpy(r[j], &v, C * TAPS);
+        }
     }
 }
 
@@ -634,60 +659,36 @@ __device__ __forceinline__ uint32_t BlendCubicQ14(const uint32_t (&r)[4][C], flo
 }
 
 // The same for a sample whose 16 taps are inside the image.
-template<int C>
+template<int C, bool SAME>
 __device__ __forceinline__ uint32_t SampleInsideCubicQ14(const Img &im, float sx, float sy)
 {
-    uint32_t o = PixelOffset<C>(im, (int)floorf(sx) - 1, (int)floorf(sy) - 1);
     uint32_t r[4][C];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-    {
-        LoadQuadBytes<C>(im.base, o, r[j]);
-        o += (uint32_t)im.row;
-    }
+    LoadTapRows<C, 4, 4, SAME>(im, (int)floorf(sx), (int)floorf(sy), -1, -1, r);
     return BlendCubicQ14<C>(r, sx, sy);
-}
-
-// The two horizontally adjacent u8 pixels at base + off (both inside the image) as raw bytes: byte i of
-// the 64-bit value {w[1]:w[0]} is channel i % C of pixel i / C.
-template<int C>
-__device__ __forceinline__ void LoadPairBytes(const uint8_t *base, uint32_t off, uint32_t (&w)[2])
-{
-    if constexpr (kWideTapLoads<uint8_t, C>)
-    {
-        const uint64_t q = LoadU64Window(base, off);
-        w[0]             = (uint32_t)q;
-        w[1]             = (uint32_t)(q >> 32);
-    }
-    else
-    {
-        const Vec<uint8_t, 2 * C> v = *reinterpret_cast<const Vec<uint8_t, 2 * C> *>(base + off);
-        w[0] = w[1] = 0;
-        __builtin_memcpy(w, &v, 2 * C);
-    }
 }
 
 // SampleWithBorder's fixed-point bilinear sum for a sample whose taps are all inside the image, whose
 // coordinates are not negative and below 2^16, given in units of 2^-15 pixel: floor and fraction come
 // from one float -> integer conversion, the taps of a row from one window, the two taps of a channel
 // from one byte permute. Returns the pixel's dword.
-template<int C>
+template<int C, bool SAME>
 __device__ __forceinline__ uint32_t SampleInsideQ15(const Img &im, float sx, float sy)
 {
     const uint32_t X = (uint32_t)(int)sx, Y = (uint32_t)(int)sy;
-    uint32_t       top, bottom;
-    WeightPairsQ15(X & (kQ15 - 1), Y & (kQ15 - 1), top, bottom);
-    const uint32_t o = PixelOffset<C>(im, (int)(X >> 15), (int)(Y >> 15));
-    uint32_t       r0[2], r1[2];
-    LoadPairBytes<C>(im.base, o, r0);
-    LoadPairBytes<C>(im.base, o + (uint32_t)im.row, r1);
+    const uint32_t ax = X & (kQ15 - 1), ay = Y & (kQ15 - 1);
+    // WeightPairsQ15 with the sum 2^15 + 65535 ax as one instruction, its constant in a register (the compiler sees two
+    // constants, which that instruction does not take, and writes one more; the resize kernels lose by it)
+    const uint32_t bottom = __umul24((__umul24(ax, ay) + (kQ15 >> 1)) >> 15, 65535u) + ay;
+    uint32_t       top;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(top) : "v"(ax), "s"(65535u), "v"(kQ15));
+    top -= bottom;
+    uint32_t r[2][(2 * C + 3) / 4];
+    LoadTapRows<C, 2, 2, SAME>(im, (int)(X >> 15), (int)(Y >> 15), 0, 0, r);
     uint32_t q = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c)
     {
-        // bytes c and c + C of the row's 8 -> (left | right << 16); selector 0x0c gives a zero byte
-        const uint32_t sel = 0x0c000c00u | (uint32_t)c | ((uint32_t)(c + C) << 16);
-        q = BlendQ15(__builtin_amdgcn_perm(r0[1], r0[0], sel), __builtin_amdgcn_perm(r1[1], r1[0], sel), top, bottom, c, q);
+        q = BlendQ15(BytePair(r[0], c, c + C), BytePair(r[1], c, c + C), top, bottom, c, q);
     }
     return q;
 }
@@ -826,35 +827,28 @@ __device__ __forceinline__ uint32_t SampleNearBorderNearest(const Img &im, const
 {
     const int      x = FloorToInt(sx + .5f), y = FloorToInt(sy + .5f);
     const uint32_t p = LoadPixelGuarded<C>(im, (uint32_t)__mul24(Fold(fy, y), im.row), Fold(fx, x));
-    // (the bytes above the pixel's must be 0: the stores merge neighbouring pixels' dwords)
-    return constant && !((uint32_t)x < (uint32_t)im.w && (uint32_t)y < (uint32_t)im.h) ? borderPx : p & (0xffffffffu >> (32 - 8 * C));
+    return constant && !((uint32_t)x < (uint32_t)im.w && (uint32_t)y < (uint32_t)im.h) ? borderPx : p;
 }
 
-// The dwords of the pixel that SampleInside gives. u8 channels are rounded, saturated and placed into
-// their byte by one instruction each (v_cvt_pk_u8_f32 with a byte select and the dword so far), where
-// packing converted bytes takes as many shifts and merges again.
-template<class T, int C, int INTERP>
+// The dwords of the pixel that SampleInside gives; what lies above the pixel's bytes is not looked at. u8 channels are
+// rounded, saturated and placed into their byte by one instruction each (v_cvt_pk_u8_f32 with a byte select and the dword
+// so far), where packing converted bytes takes as many shifts and merges again. SAME: see LoadTapRows.
+template<class T, int C, int INTERP, bool SAME>
 __device__ __forceinline__ void SampleInsidePacked(const Img &im, float sx, float sy, uint32_t (&w)[(C * sizeof(T) + 3) / 4])
 {
     if constexpr (kFixedPoint<T, INTERP>)
     {
-        w[0] = SampleInsideQ15<C>(im, sx, sy);
+        w[0] = SampleInsideQ15<C, SAME>(im, sx, sy);
     }
     else if constexpr (kFixedPointCubic<T, INTERP>)
     {
-        w[0] = SampleInsideCubicQ14<C>(im, sx, sy);
+        w[0] = SampleInsideCubicQ14<C, SAME>(im, sx, sy);
     }
-    else if constexpr (std::is_same_v<T, uint8_t> && INTERP != NVCV_INTERP_NEAREST)
+    else if constexpr (std::is_same_v<T, uint8_t>)
     {
-        float acc[C];
-        SampleInside<float, C, INTERP, T>(im, sx, sy, acc);
-        uint32_t q = 0;
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-        {
-            q = __builtin_amdgcn_cvt_pk_u8_f32(acc[c], c, q);
-        }
-        w[0] = q;
+        uint32_t r[1][1];
+        LoadTapRows<C, 1, 1, SAME>(im, (int)floorf(sx + .5f), (int)floorf(sy + .5f), 0, 0, r);
+        w[0] = r[0][0];
     }
     else
     {
@@ -1018,10 +1012,12 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 
     // ---- gather: lane (lx, ly) of wave w samples its pixel in patches 4w .. 4w+3 (side by side: a
     // wave covers 32 columns x 8 rows)
-    const int wave = threadIdx.x >> 6, lx = threadIdx.x & (kPatch - 1), ly = (threadIdx.x >> 3) & (kPatch - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lx = threadIdx.x & (kPatch - 1),
+              ly = (threadIdx.x >> 3) & (kPatch - 1);
+    const int x0 = tx * kTileW + wave % kWavesX * kWaveW, y0 = ty * kTileH + wave / kWavesX * kPatch;
     // m maps to source coordinates times kCoordScale; so do sx, sy and the limits
     constexpr float kScale = kCoordScale<T, INTERP>;
-    const float     limX = InsideLimit<INTERP>(im.w, kWideTapLoads<T, C>) * kScale, limY = InsideLimit<INTERP>(im.h, false) * kScale;
+    const float     limX = InsideLimit<INTERP>(im.w, kTapOverrun<T, C, INTERP>) * kScale, limY = InsideLimit<INTERP>(im.h, 0) * kScale;
     int         px[kPxPerLane], py[kPxPerLane]; // the lane's destination pixels
     float       sx[kPxPerLane], sy[kPxPerLane];
     uint32_t    q[D][kPxPerLane]; // q[d][k]: dword d of this lane's pixel in patch k
@@ -1032,20 +1028,30 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
     for (int k = 0; k < kPxPerLane; ++k)
     {
-        const int patch = wave * kPxPerLane + k;
         // pixels of the tile beyond the image edge repeat the edge pixel's sample; they are never stored
-        px[k] = min(tx * kTileW + (patch % kPatchesX) * kPatch + lx, dstW - 1);
-        py[k] = min(ty * kTileH + (patch / kPatchesX) * kPatch + ly, dstH - 1);
+        px[k] = min(x0 + k * kPatch + lx, dstW - 1);
+        py[k] = min(y0 + ly, dstH - 1);
     }
     MapCoords<PERSP>(m, px, py, sx, sy);
     allInside = allInside & TapsInside<INTERP>(limX, limY, sx, sy);
     if (allInside)
     {
         uint32_t w[kPxPerLane][D];
-#pragma unroll
-        for (int k = 0; k < kPxPerLane; ++k)
+        if (!kWideTapLoads<T, C> || INTERP == NVCV_INTERP_NEAREST || (im.row & 3) == 0) // uniform
         {
-            SampleInsidePacked<T, C, INTERP>(im, sx[k], sy[k], w[k]);
+#pragma unroll
+            for (int k = 0; k < kPxPerLane; ++k)
+            {
+                SampleInsidePacked<T, C, INTERP, true>(im, sx[k], sy[k], w[k]);
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int k = 0; k < kPxPerLane; ++k)
+            {
+                SampleInsidePacked<T, C, INTERP, false>(im, sx[k], sy[k], w[k]);
+            }
         }
 #pragma unroll
         for (int k = 0; k < kPxPerLane; ++k)
@@ -1090,6 +1096,8 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                         SampleAllOutside<T, C, INTERP>(a, sx[k], sy[k], v);
                         q[0][k] = 0;
                         __builtin_memcpy(&q[0][k], v, C);
+                        // (a dword from here on: the compiler carried its bytes apart through all paths, 28 instructions)
+                        asm("" : "+v"(q[0][k]));
                     }
                     else
                     {
@@ -1125,9 +1133,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         {
             // position and coordinates recomputed rather than indexed, results placed by selects: a
             // run-time index would put the arrays in scratch memory
-            const int patch = wave * kPxPerLane + k;
-            const int px = (patch % kPatchesX) * kPatch + lx, py = (patch / kPatchesX) * kPatch + ly;
-            const int dx = min(tx * kTileW + px, dstW - 1), dy = min(ty * kTileH + py, dstH - 1);
+            const int dx = min(x0 + k * kPatch + lx, dstW - 1), dy = min(y0 + ly, dstH - 1);
             float     bx, by;
             MapCoord<PERSP>(m, dx, dy, bx, by);
             bx *= 1.f / kScale;
@@ -1146,6 +1152,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
             for (int d = 0; d < D; ++d)
             {
+                asm("" : "+v"(w[d]));
 #pragma unroll
                 for (int j = 0; j < kPxPerLane; ++j)
                 {
@@ -1164,9 +1171,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
         for (int k = 0; k < kPxPerLane; ++k)
         {
-            const int patch = wave * kPxPerLane + k;
-            const int px = (patch % kPatchesX) * kPatch + lx, py = (patch / kPatchesX) * kPatch + ly;
-            const int dx = tx * kTileW + px, dy = ty * kTileH + py;
+            const int dx = x0 + k * kPatch + lx, dy = y0 + ly;
             if (dx < dstW && dy < dstH)
             {
                 uint32_t w[D];
@@ -1180,21 +1185,45 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         }
         return;
     }
-    // Smaller pixels: the 4 lanes lx & ~3 .. | 3 hold columns 4g .. 4g+3 (g = lx >> 2) of row ly in each of the
-    // wave's 4 patches; after a 4x4 transpose lane i = lx & 3 holds those 4 columns of patch 4w + i
-#pragma unroll
-    for (int d = 0; d < D; ++d)
+    // Smaller pixels change lanes so that a lane holds 4 consecutive pixels of a row. One dword each: through the wave's own
+    // part of LDS (rows of 40 dwords: every quarter of a wave on banks of its own), after which lane (lx, ly) holds columns
+    // 4 lx .. 4 lx + 3 of row ly. These kernels wait for vector instructions; moves and selects between lanes took 20 of
+    // them, and left a row's pieces in another order than the lanes'.
+    int dx0;
+    if constexpr (D == 1)
     {
-        QuadTranspose(q[d], lx & 3);
+        __shared__ __align__(16) uint32_t exchange[kThreads / 64][kPatch][40];
+#pragma unroll
+        for (int k = 0; k < kPxPerLane; ++k)
+        {
+            exchange[wave][ly][k * kPatch + lx] = q[0][k];
+        }
+        WaveExchangeFence();
+        const uint4 r = *reinterpret_cast<const uint4 *>(&exchange[wave][ly][4 * lx]);
+        q[0][0]       = r.x;
+        q[0][1]       = r.y;
+        q[0][2]       = r.z;
+        q[0][3]       = r.w;
+        dx0           = x0 + 4 * lx;
     }
-    const int patch = wave * kPxPerLane + (lx & 3);
-    const int px0 = (patch % kPatchesX) * kPatch + (lx & 4);
-    const int dy = ty * kTileH + (patch / kPatchesX) * kPatch + ly, dx0 = tx * kTileW + px0;
+    else
+    {
+        // the 4 lanes lx & ~3 .. | 3 hold columns 4g .. 4g+3 (g = lx >> 2) of row ly in each of the wave's 4 patches; after
+        // a 4x4 transpose lane i = lx & 3 holds those 4 columns of patch 4w + i
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+        {
+            QuadTranspose(q[d], lx & 3);
+        }
+        dx0 = x0 + (lx & 3) * kPatch + (lx & 4);
+    }
+    const int dy = y0 + ly;
     if (dy >= dstH || dx0 >= dstW)
     {
         return;
     }
-    uint8_t *to = dst + (int64_t)dy * dstRow + (int64_t)dx0 * PB;
+    // (the wave's rows start at one address, and a lane's bytes are less than 2 GiB behind it: an image's are)
+    uint8_t *to = dst + (int64_t)y0 * dstRow + (int64_t)x0 * PB + (uint32_t)(ly * dstRow + (dx0 - x0) * PB);
     if (dx0 + 4 <= dstW)
     {
         uint32_t w[PB];

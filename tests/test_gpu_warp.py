@@ -95,6 +95,27 @@ def test_mirroring_and_repeating_borders_near_and_far(cv, orc, gpu, c):
         np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((c, interp, border)))
 
 
+# row windows of dense images whose rows start at every byte of a dword in turn, from every start of the first; widths about
+# the tap blocks' and the windows' own (samples whose window would pass the row's end take the border's forms). The buffer
+# ends with the last image.
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("lead", [0, 1, 2, 3])
+@pytest.mark.parametrize("size", [(1, 9), (4, 4), (7, 5), (11, 6), (61, 40), (70, 41)], ids=lambda s: "%dx%d" % s)
+def test_rows_from_every_byte_of_a_dword(cv, orc, gpu, size, lead, c):
+    w, h = size
+    src = orc.fill_u8((2, h, w, c), 0xD0D + w + lead)
+    buf = torch.zeros(lead + src.size, dtype=torch.uint8, device="cuda")
+    buf[lead:].copy_(torch.from_numpy(src.reshape(-1)))
+    tin = cv.Tensor.wrap(buf.data_ptr() + lead, [2, h, w, c], [h * w * c, w * c, c, 1], np.uint8, "NHWC", keep=buf)
+    for interp, border in itertools.product((NEAREST, LINEAR, CUBIC), (0, 1, 2, 3, 4)):
+        for m in (rotation(w, h, 4.0, 1.02), [1.0, 0.0, 0.3, 0.0, 1.0, -0.6], rotation(w, h, 21.0, 0.7)):
+            tout = cv.Tensor.alloc([2, h + 3, w + 5, c], np.uint8, "NHWC")
+            cv.WarpAffine(0)(None, tin, tout, m, interp, border, (9, 200, 31, 77))
+            torch.cuda.synchronize()
+            dev = orc.warp(src, (h + 3, w + 5), orc.invert_affine(m), interp, border, (9, 200, 31, 77), variant=device_variant(interp))
+            np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((size, lead, c, interp, border, m)))
+
+
 def rotation(w, h, deg, s):
     t = np.deg2rad(deg)
     c, sn = s * np.cos(t), s * np.sin(t)
