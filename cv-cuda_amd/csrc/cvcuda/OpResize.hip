@@ -3128,6 +3128,8 @@ __global__ __launch_bounds__(256) void ResizeCubicStagedKernel(const ResizeArgs 
 // own (its place in the window differs from lane to lane); PARTIAL: the scale has such pixels. u8x3 32 x 1080p -> 320 x 180
 // 56.6 -> 38.1 us (5.4 TB/s), 16 x 4K -> 500 x 281 176.5 -> 83 us, 32 x 1080p -> 571 x 323 142 -> 77 us, one 2363 x 1415 ->
 // 355 x 153 15.9 -> 8.2 us; u8x4 16 x 4K -> 350 x 201 216 -> 117 us; u8x1 32 x 1080p -> 311 x 177 46.4 -> 24.9 us.
+// Those figures are with windows a pixel wider at scales between whole numbers; as the dispatch has them now, 64 x 1283 x 721
+// u8x3 -> 321 x 181 61.8 -> 52.9 us, -> 279 x 157 52.6 -> 50.1, -> 138 x 78 49.1 -> 45.0; u8x4 (48 images) 54.4 -> 46.1 us.
 constexpr float kAreaWindowMost = 12.f;
 constexpr int kAreaBatch = 3;
 
@@ -3505,18 +3507,17 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         if (a.scaleX > 1.f && a.scaleX <= kAreaWindowMost && a.scaleY > 1.f && a.srcW * C >= 64)
         {
             const float s = a.scaleX;
-            // whole scales have no partial columns and exactly s pixels per row; between them the box has at most floor(s)
-            // whole pixels beside the partial first one, and one more where its end rounds up to a whole number
-            auto kernel = std::ceil(s) == s
-                            ? (s <= 4.f   ? ResizeAreaWindowKernel<C, 4, false>
-                               : s <= 6.f ? ResizeAreaWindowKernel<C, 6, false>
-                               : s <= 8.f ? ResizeAreaWindowKernel<C, 8, false>
-                                          : ResizeAreaWindowKernel<C, 12, false>)
-                            : (s < 4.f   ? ResizeAreaWindowKernel<C, 5, true>
-                               : s < 5.f ? ResizeAreaWindowKernel<C, 6, true>
-                               : s < 6.f ? ResizeAreaWindowKernel<C, 7, true>
-                               : s < 8.f ? ResizeAreaWindowKernel<C, 9, true>
-                                         : ResizeAreaWindowKernel<C, 13, true>);
+            // A box touches at most ceil(s) pixels per row besides the partial last one, which is not in the window: whole
+            // scales s whole ones; between whole numbers floor(s) whole ones behind a partial first, or floor(s) + 1 without
+            // one where the box's end rounds up (behind a partial first one it would have to round by more than the spacing
+            // of the floats there).
+            const bool partial = std::ceil(s) != s;
+            auto       kernel  = s <= 4.f   ? (partial ? ResizeAreaWindowKernel<C, 4, true> : ResizeAreaWindowKernel<C, 4, false>)
+                               : s <= 5.f   ? (partial ? ResizeAreaWindowKernel<C, 5, true> : ResizeAreaWindowKernel<C, 5, false>)
+                               : s <= 6.f   ? (partial ? ResizeAreaWindowKernel<C, 6, true> : ResizeAreaWindowKernel<C, 6, false>)
+                               : s <= 8.f   ? (partial ? ResizeAreaWindowKernel<C, 8, true> : ResizeAreaWindowKernel<C, 8, false>)
+                               : s <= 10.f  ? (partial ? ResizeAreaWindowKernel<C, 10, true> : ResizeAreaWindowKernel<C, 10, false>)
+                                            : (partial ? ResizeAreaWindowKernel<C, 12, true> : ResizeAreaWindowKernel<C, 12, false>);
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
             CheckLaunch("ResizeAreaWindowKernel");
             return;
