@@ -61,14 +61,23 @@ public:
         }
         if (p != nullptr)
         {
-            std::lock_guard<std::mutex> lock(m_mutex);
-            m_inUse[p] = {want, dev};
+            try
+            {
+                std::lock_guard<std::mutex> lock(m_mutex);
+                m_inUse[p] = {want, dev};
+            }
+            catch (...) // no host memory
+            {
+                Source::free(p);
+                return nullptr;
+            }
         }
         return p;
     }
 
-    void free(void *p)
+    void free(void *p) noexcept
     {
+        try
         {
             std::lock_guard<std::mutex> lock(m_mutex);
             auto                        it = m_inUse.find(p);
@@ -79,12 +88,17 @@ public:
                 Device &d = m_devices[b.device];
                 if (b.size <= m_limit / 4 && d.held + b.size <= m_limit)
                 {
+                    size_t &ofSize = d.waitingOfSize[b.size];
                     d.waiting.push_back({b.size, p});
-                    ++d.waitingOfSize[b.size];
+                    ++ofSize;
                     d.held += b.size;
                     return;
                 }
             }
+        }
+        catch (...)
+        {
+            // no host memory to remember it by
         }
         Source::free(p); // beyond the limit, or not from here
     }
@@ -107,9 +121,14 @@ private:
         int64_t                                  held = 0;      // bytes of ready and waiting
     };
 
-    // Sizes of eight steps per power of two (at most an eighth more than asked for), 4 KiB and more.
+    // Sizes of eight steps per power of two (at most an eighth more than asked for), 4 KiB and more. Sizes that no memory
+    // has are left as they are, for the allocation to refuse.
     static int64_t RoundUp(int64_t size)
     {
+        if (size >= int64_t(1) << 48)
+        {
+            return size;
+        }
         int64_t step = 4096;
         while (step * 16 <= size)
         {
@@ -128,12 +147,12 @@ private:
             return nullptr;
         }
         // the last in first out: the most likely to be in the caches
-        void *p = it->second.back();
+        void *p    = it->second.back();
+        m_inUse[p] = {size, dev};
         it->second.pop_back();
         size_t &unused = d.unused[size];
         unused         = unused < it->second.size() ? unused : it->second.size();
         d.held -= size;
-        m_inUse[p] = {size, dev};
         return p;
     }
 

@@ -144,6 +144,16 @@ int main()
         pool.free(std::malloc(16)); // not from here: passed on
     }
     {
+        // sizes that no memory has are refused
+        Reset();
+        BlockPool<Counting> pool(1 << 20);
+        for (int bits = 50; bits < 64; ++bits)
+        {
+            volatile int64_t size = (int64_t)((uint64_t(1) << bits) - 1);
+            REQUIRE(pool.alloc(size) == nullptr);
+        }
+    }
+    {
         // threads
         Reset();
         BlockPool<Counting>      pool(1 << 22);
