@@ -150,6 +150,22 @@ def test_random_rotations_tensor(cv, orc, gpu, dt, c, interp):
                 assert np.abs(res.astype(np.int16) - gold.astype(np.int16)).max() <= 1
 
 
+# 12- and 16-byte pixels leave the wave 16 bytes per lane: widths about a wave's 32 columns, rows that end in 1 to 3 dwords
+@pytest.mark.parametrize("c", [3, 4])
+@pytest.mark.parametrize("dw,dh", [(1, 1), (3, 9), (31, 8), (33, 17), (62, 5), (64, 16), (67, 23)])
+def test_wide_pixels_at_the_tile_edges(cv, orc, gpu, dw, dh, c):
+    src = orc.fill_f32((2, 21, 37, c), 5 + dw)
+    m = rotation(37, 21, 12.0, 0.9)
+    buf = torch.full((2 * dh * dw * c + 8,), -7.0, device="cuda")
+    tout = cv.Tensor.wrap(buf.data_ptr() + 16, [2, dh, dw, c], [dh * dw * c * 4, dw * c * 4, c * 4, 4], np.float32, "NHWC", keep=buf)
+    cv.WarpAffine(0)(None, cv.Tensor.from_numpy(src, "NHWC"), tout, m, NEAREST, 1, (0, 0, 0, 0))
+    torch.cuda.synchronize()
+    res = buf.cpu().numpy()
+    dev = orc.warp(src, (dh, dw), orc.invert_affine(m), NEAREST, 1, (0, 0, 0, 0), variant=1)
+    np.testing.assert_array_equal(res[4:-4].reshape(dev.shape), dev)
+    assert (res[:4] == -7).all() and (res[-4:] == -7).all()
+
+
 def make_c4_batch(cv, K, orc, n, seed):
     rng = np.random.default_rng(seed)
     bi, bo, hosts, outs, mats = cv.ImageBatchVarShape(n), cv.ImageBatchVarShape(n), [], [], []
