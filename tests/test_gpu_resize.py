@@ -399,6 +399,18 @@ def test_area_larger_reductions(cv, orc, gpu, sw, sh, dw, dh, c, kind):
     np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), AREA, threads=8))
 
 
+# every width of the window, at whole scales and just above and below them (the widest boxes of a width)
+@pytest.mark.parametrize("sw,dw", [(300, 75), (299, 75), (301, 75), (375, 75), (374, 75), (376, 75), (449, 75), (451, 75),
+                                   (599, 75), (601, 75), (675, 75), (749, 75), (751, 75), (899, 75), (900, 75)])
+@pytest.mark.parametrize("c", [1, 3, 4])
+def test_area_window_widths(cv, orc, gpu, sw, dw, c):
+    src = make_input(orc, (2, 47, sw, c), np.uint8, 0xA0 + sw)
+    tout = cv.Tensor.alloc([2, 11, dw, c], np.uint8, "NHWC")
+    cv.Resize()(None, cv.Tensor.from_numpy(src, "NHWC"), tout, AREA)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(tout.numpy(), orc.resize_shipped(src, (11, dw), AREA, threads=8))
+
+
 # the row windows of the bicubic strips, the bicubic patches and the box filter, on dense images whose rows start at every
 # byte of a dword in turn, from every start of the first: the buffer ends with the image, whose last rows are read
 @pytest.mark.parametrize("c", [3, 1])
@@ -589,3 +601,40 @@ def test_negative_cases(cv, gpu):
             __import__("cvcuda_amd")._capi.cvcuda.cvcudaResizeSubmit(cv.ResizeCropConvertReformat().handle, None,
                                                                      a.handle, a.handle, LINEAR))
     assert e.value.status == 9  # handle of another operator -> NOT_COMPATIBLE
+
+
+# float boxes, their rows summed by column first: every number of pieces per lane, reductions that are whole along one axis,
+# both or none, the last rows and columns, rows that end inside a lane's 16 bytes; an infinity outside a box does not reach
+# it. Against the box filter in 64 bits over the same float32 edges: a result is a sum of ny products, then of nx, times a
+# scale of 4 roundings, each off by at most 2^-24 of itself, all of them positive.
+@pytest.mark.parametrize("sw,sh,dw,dh", [(67, 41, 61, 37), (128, 66, 64, 33), (131, 50, 66, 25), (198, 47, 66, 30), (263, 83, 66, 21),
+                                         (264, 84, 66, 21), (397, 61, 66, 9), (527, 33, 66, 4), (791, 40, 66, 3), (792, 36, 66, 3),
+                                         (20, 19, 13, 7), (16, 64, 2, 5), (601, 40, 151, 9), (1537, 30, 128, 3)])
+@pytest.mark.parametrize("c", [1, 3, 4])
+def test_area_of_floats(cv, orc, gpu, sw, sh, dw, dh, c):
+    src = orc.fill_f32((2, sh, sw, c), 0xF0 + sw)
+    src = np.abs(src)
+    src[1, 0, 0, 0] = np.inf
+    buf = torch.zeros(src.size, dtype=torch.float32, device="cuda")
+    buf.copy_(torch.from_numpy(src.reshape(-1)))
+    tin = cv.Tensor.wrap(buf.data_ptr(), [2, sh, sw, c], [sh * sw * c * 4, sw * c * 4, c * 4, 4], np.float32, "NHWC", keep=buf)
+    tout = cv.Tensor.alloc([2, dh, dw, c], np.float32, "NHWC")
+    cv.Resize()(None, tin, tout, AREA)
+    torch.cuda.synchronize()
+    res = tout.numpy()
+
+    def shares(size, new):  # [new, size] of each source pixel in each box, from float32 edges, over the box's nominal size
+        scale = np.float32(size) / np.float32(new)
+        lo = np.arange(new, dtype=np.float32) * scale
+        hi = np.minimum(lo + scale, np.float32(size))
+        i = np.arange(size, dtype=np.float64)
+        covered = np.clip(np.minimum(i + 1, hi[:, None]) - np.maximum(i, lo[:, None]), 0, None)
+        return covered / np.minimum(scale, np.float32(size) - lo)[:, None].astype(np.float64)
+
+    wy, wx = shares(sh, dh), shares(sw, dw)
+    clean = np.where(np.isinf(src), 0, src).astype(np.float64)
+    ref = np.einsum("yh,nhwc,xw->nyxc", wy, clean, wx)
+    assert np.isinf(res[1, 0, 0, 0])
+    res[1, 0, 0, 0] = ref[1, 0, 0, 0]
+    bound = 2.0 ** -24 * (2 * (np.ceil(sh / dh) + np.ceil(sw / dw)) + 12)
+    assert (np.abs(res - ref) <= bound * np.abs(ref)).all(), np.max(np.abs(res - ref) / np.abs(ref)) / bound
