@@ -638,3 +638,42 @@ def test_area_of_floats(cv, orc, gpu, sw, sh, dw, dh, c):
     res[1, 0, 0, 0] = ref[1, 0, 0, 0]
     bound = 2.0 ** -24 * (2 * (np.ceil(sh / dh) + np.ceil(sw / dw)) + 12)
     assert (np.abs(res - ref) <= bound * np.abs(ref)).all(), np.max(np.abs(res - ref) / np.abs(ref)) / bound
+
+
+# bicubic floats in strips of 16 rows (launches of 2048 strips and more): enlarged, the same size, reduced by almost 2, strips
+# cut off by the lower edge, sources of 4 pixels along an axis. Against the formula in 64 bits over the float32 weights: two
+# sums of 4 products each.
+@pytest.mark.parametrize("sw,sh,dw,dh,n", [(131, 97, 197, 145, 60), (130, 33, 131, 33, 230), (200, 63, 101, 32, 512), (4, 4, 65, 17, 512),
+                                           (67, 50, 64, 49, 512), (301, 7, 151, 250, 48)])
+@pytest.mark.parametrize("c", [1, 3, 4])
+def test_bicubic_float_strips(cv, orc, gpu, sw, sh, dw, dh, n, c):
+    assert ((dw + 63) // 64) * ((dh + 15) // 16) * n >= 2048
+    one = orc.fill_f32((3, sh, sw, c), 0xCC + sw)
+    src = torch.from_numpy(one).cuda().repeat((n + 2) // 3, 1, 1, 1)[:n].contiguous()
+    tin = cv.Tensor.wrap(src.data_ptr(), [n, sh, sw, c], [sh * sw * c * 4, sw * c * 4, c * 4, 4], np.float32, "NHWC", keep=src)
+    tout = cv.Tensor.alloc([n, dh, dw, c], np.float32, "NHWC")
+    cv.Resize()(None, tin, tout, CUBIC)
+    torch.cuda.synchronize()
+    res = tout.numpy()
+
+    def axis(size, new, horizontal):
+        f = np.float32
+        at = (np.arange(new, dtype=f) + f(.5)) * (f(size) / f(new)) - f(.5)
+        s = np.floor(at).astype(np.int64)
+        d = at - s.astype(f)
+        if horizontal:
+            d = np.where((s < 1) | (s >= size - 3), f(0), d)
+        s = np.clip(s, 1, size - 3)
+        a, d, one, e = f(-.75), d.astype(f), f(1), f(1) - d.astype(f)
+        w = [((a * (d + one) - 5 * a) * (d + one) + 8 * a) * (d + one) - 4 * a, ((a + f(2)) * d - (a + f(3))) * d * d + one,
+             ((a + f(2)) * e - (a + f(3))) * e * e + one]
+        assert all(x.dtype == f for x in w)
+        m = np.zeros((new, size))
+        for i, wi in enumerate(w + [one - w[0] - w[1] - w[2]]):
+            m[np.arange(new), s - 1 + i] += wi.astype(np.float64)
+        return m
+
+    ref = np.abs(np.einsum("yh,nhwc,xw->nyxc", axis(sh, dh, False), one.astype(np.float64), axis(sw, dw, True)))
+    ref = np.concatenate([ref] * ((n + 2) // 3))[:n]
+    # the weights of an axis add up to at most 1.375 in magnitude; 4 products and 3 additions, twice
+    assert np.abs(res - ref).max() <= 2 * 7 * 2.0 ** -24 * 1.375 ** 2 * np.abs(one).max()
