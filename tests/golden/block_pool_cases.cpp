@@ -20,6 +20,11 @@ struct Counting
         {
             return nullptr;
         }
+        // (more than any device has: a sanitizer's malloc would end the program for it)
+        if (size >= size_t(1) << 40)
+        {
+            return nullptr;
+        }
         ++g_allocs;
         return std::malloc(size);
     }
