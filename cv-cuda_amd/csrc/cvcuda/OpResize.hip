@@ -3465,11 +3465,29 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
     {
         return;
     }
-    const AxisTerms<4> col = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleX, min(dx, p.dstW - 1), p.srcW, true);
-    const uint32_t     at  = (uint32_t)(col.s - 1) * (uint32_t)sizeof(Pixel<float, C>); // taps col.s - 1 .. col.s + 2, inside the row
+    AxisTerms<4>   col = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleX, min(dx, p.dstW - 1), p.srcW, true);
+    const uint32_t at  = (uint32_t)(col.s - 1) * (uint32_t)sizeof(Pixel<float, C>); // taps col.s - 1 .. col.s + 2, inside the row
+
+    // Weights along a row add up to as much as 1.375 in magnitude, so a row of the type's extreme values would overflow
+    // also where its own weight is 0. Halves here, doubled again with the row's weights (both exact).
+    auto rowTerms = [&](int dy)
+    {
+        AxisTerms<4> r = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleY, dy, p.srcH, false);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+        {
+            r.w[i] *= 2.f;
+        }
+        return r;
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        col.w[i] *= 0.5f;
+    }
 
     auto load = [&](int y) { return *reinterpret_cast<const Taps *>(p.src + (int64_t)min(y, p.srcH - 1) * p.srcRow + at); };
-    float h[4][C]; // of source rows first .. first + 3
+    float h[4][C]; // halves of the sums of source rows first .. first + 3
     auto  rowSum = [&](const Taps &t, float (&out)[C])
     {
 #pragma unroll
@@ -3483,7 +3501,7 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
         }
     };
 
-    AxisTerms<4> row   = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleY, y0, p.srcH, false);
+    AxisTerms<4> row   = rowTerms(y0);
     int          first = __builtin_amdgcn_readfirstlane(row.s) - 1;
     {
         Taps t[4];
@@ -3521,7 +3539,7 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
         {
             break;
         }
-        row = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleY, dy, p.srcH, false);
+        row              = rowTerms(dy);
         const int target = __builtin_amdgcn_readfirstlane(row.s) - 1;
 #pragma unroll 1
         for (; first < target; ++first) // (up to twice; rows never go back)

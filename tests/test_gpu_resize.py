@@ -677,3 +677,20 @@ def test_bicubic_float_strips(cv, orc, gpu, sw, sh, dw, dh, n, c):
     ref = np.concatenate([ref] * ((n + 2) // 3))[:n]
     # the weights of an axis add up to at most 1.375 in magnitude; 4 products and 3 additions, twice
     assert np.abs(res - ref).max() <= 2 * 7 * 2.0 ** -24 * 1.375 ** 2 * np.abs(one).max()
+
+
+# rows of zeros between rows of the type's lowest value: the horizontal sums of the latter pass the type's range, the rows
+# between must not see it (vertical weights of exactly 0 there)
+@pytest.mark.parametrize("c", [1, 3, 4])
+def test_bicubic_float_strips_next_to_extreme_values(cv, gpu, c):
+    n, sw, sh, dw = 230, 43, 33, 129
+    src = torch.zeros((n, sh, sw, c), dtype=torch.float32, device="cuda")
+    src[:, 1::2] = torch.finfo(torch.float32).min
+    tin = cv.Tensor.from_torch(src, "NHWC")
+    out = torch.full((n, sh, dw, c), -7.0, device="cuda")
+    cv.Resize()(None, tin, cv.Tensor.from_torch(out, "NHWC"), CUBIC)
+    torch.cuda.synchronize()
+    # (the last rows' taps are moved into the image, but their fraction stays 0, so every row is one source row)
+    rows = out.cpu().numpy()
+    assert not np.isnan(rows).any()
+    assert (rows[:, 2:sh - 3:2] == 0).all()
