@@ -9,7 +9,7 @@
 // point on those indices and weights (bilinear: FixedPointBlend.hpp; bicubic: kFixedCubic; box filter:
 // kAreaFixed), at most 1 from the reference's goldens.
 //
-// Eight kernel shapes, all with streaming stores, var-shape batches on a packed tile grid:
+// Ten kernel shapes, all with streaming stores, var-shape batches on a packed tile grid:
 //  * pixels of up to 8 bytes: wave patches (64 columns x 4 rows per wave; adjacent taps in one load,
 //    row terms computed once per wave, 4x4 lane transposes so that every lane stores whole dwords);
 //  * 8-bit bilinear at horizontal scales up to 2: a lane owns 2 columns x 4 rows (image batches x 2; 4 x 8 when
@@ -29,7 +29,7 @@
 //    columns (ResizeAreaFloatKernel);
 //  * bicubic float tensors at scales below 2, large launches: a wave owns 64 columns x 16 rows and forms every source
 //    row's sums once (ResizeCubicStripF32Kernel);
-//  * everything else (12/16-byte pixels, other AREA): one lane per output pixel, a 256-thread block covers
+//  * everything else (other 12/16-byte pixels, other AREA): one lane per output pixel, a 256-thread block covers
 //    64 columns x 4 rows, pixels moved as whole C-channel vectors.
 #include "DeviceUtils.hpp"
 #include "FixedPointBlend.hpp"
