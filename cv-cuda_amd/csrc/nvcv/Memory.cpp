@@ -274,10 +274,13 @@ int CurrentDevice()
     return device;
 }
 
+// Waits for all of the device's work. By hipFree, which does (57 ms behind 57 ms of another stream's work, whatever the block's
+// size): hipDeviceSynchronize invalidates every graph capture of the process, also one of another thread in the relaxed or
+// thread-local mode, in which tensors may be made and dropped meanwhile.
 bool SynchronizeDevice()
 {
-    // not possible while a stream of the device is being captured
-    if (hipDeviceSynchronize() != hipSuccess)
+    void *p = nullptr;
+    if (hipMalloc(&p, 1) != hipSuccess || hipFree(p) != hipSuccess)
     {
         (void)hipGetLastError();
         return false;
@@ -300,8 +303,7 @@ struct PinnedMemory
 
     static void free(void *p)
     {
-        (void)SynchronizeDevice(); // a copy may still read or write it
-        (void)hipHostFree(p);
+        (void)hipHostFree(p); // (waits for the device, as hipFree does)
     }
 
     static int device()

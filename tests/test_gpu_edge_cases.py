@@ -1,5 +1,7 @@
 """Edge cases shared by the operators: empty image batches, one-pixel images, rows whose width is not
 a multiple of anything, odd base addresses and pitches (views into a larger buffer)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -144,6 +146,39 @@ def test_submits_captured_in_a_hip_graph_replay_correctly(cv, K, orc, gpu):
         want = orc.normalize(x, np.array([[[[0.4, 0.5, 0.6]]]], np.float32), np.array([[[[0.2, 0.3, 0.4]]]], np.float32),
                              1.0, 0.0, 0.0, True).transpose(0, 3, 1, 2)
         assert (np.abs(got3 - want) <= 1e-5 * np.maximum(1.0, np.abs(want))).all()
+
+
+@pytest.mark.parametrize("mode,where", [("relaxed", "same thread"), ("relaxed", "another thread"), ("thread_local", "another thread")])
+def test_containers_made_and_dropped_while_a_graph_is_captured(cv, gpu, mode, where):
+    # more tensors and batches than the default allocator keeps waiting, by the capturing thread where the capture's mode
+    # lets it allocate and by another one: the capture goes on, and the graph replays what was captured
+    x, errors = torch.zeros(8, device="cuda"), []
+
+    def churn():
+        try:
+            for i in range(80):
+                cv.Tensor.alloc([16, 16, 3], np.uint8, "HWC")
+                cv.Tensor.alloc([300 << 20], np.uint8, "N") if i % 40 == 0 else None  # larger than what is kept
+                cv.ImageBatchVarShape(4)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode=mode):
+        x.add_(1)
+        if where == "same thread":
+            churn()
+        else:
+            thread = threading.Thread(target=churn)
+            thread.start()
+            thread.join()
+        x.add_(1)
+    assert not errors, errors
+    for replay in range(1, 4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert x.tolist() == [2.0 * replay] * 8
 
 
 def test_image_batch_descriptors_must_be_uploaded_before_graph_capture(cv, K, orc, gpu):
