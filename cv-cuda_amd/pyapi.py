@@ -359,7 +359,7 @@ class Tensor:
         return self._t.torch_view()
 
     def __del__(self):
-        if self._key is not None and not self._seen:
+        if self._key is not None and not self._seen and _outputs is not None:  # (None: the interpreter is ending)
             _outputs.put(self)
 
 

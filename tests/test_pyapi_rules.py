@@ -3,6 +3,9 @@ first name of the reference's headers, as its table of output formats does, pyth
 the output shapes and formats of cvtcolor (CvtColorUtil.cpp:244-330) and the argument checks the reference's bindings
 make themselves."""
 import importlib
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -318,3 +321,22 @@ def test_results_on_other_streams_are_always_new(api, monkeypatch):
     monkeypatch.setattr(api._outputs, "get", lambda *args: "kept")
     assert api._result([2, 3], np.uint8, "HW", FakeStream(7)) == "new" and made == [((2, 3), np.uint8, "HW")]
     assert api._result([2, 3], np.uint8, "HW", FakeStream(0)) == "kept"
+
+
+def test_results_alive_at_the_end_of_the_program_say_nothing():
+    # a module's result tensors that outlive this package's module globals: nothing on stderr
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    program = """
+import sys
+sys.path.insert(0, %r)
+from __graft_entry__ import load_package
+load_package()
+import cvcuda_amd.pyapi as api
+class Raw:
+    _nbytes = 1
+result = api.Tensor(_wrap=Raw())
+result._key, result._wrote = ((1,), "u1", "N", 0), (0, None)
+api.kept = result
+""" % root
+    r = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "Exception ignored" not in r.stderr, r.stderr
