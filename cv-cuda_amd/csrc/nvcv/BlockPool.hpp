@@ -38,33 +38,39 @@ public:
 
     void *alloc(int64_t size)
     {
-        const int     dev  = Source::device();
-        const int64_t want = RoundUp(size);
-        if (want <= m_limit / 4)
+        const int     dev     = Source::device();
+        const int64_t rounded = RoundUp(size);
+        const bool    kept    = rounded <= m_limit / 4;
+        if (kept)
         {
-            if (void *p = take(dev, want))
+            if (void *p = take(dev, rounded))
             {
                 return p;
             }
-            if (worthSynchronizing(dev, want) && recycle(dev))
+            if (worthSynchronizing(dev, rounded) && recycle(dev))
             {
-                if (void *p = take(dev, want))
+                if (void *p = take(dev, rounded))
                 {
                     return p;
                 }
             }
         }
-        void *p = Source::alloc((size_t)want);
+        // what is never kept is not rounded either: a tensor of half the device's memory would ask for an eighth more
+        void *p = Source::alloc((size_t)(kept ? rounded : size));
         if (p == nullptr && giveBack(dev))
         {
-            p = Source::alloc((size_t)want);
+            p = Source::alloc((size_t)(kept ? rounded : size));
         }
-        if (p != nullptr)
+        if (p == nullptr && kept && rounded != size)
+        {
+            return Source::alloc((size_t)size); // (not remembered, so freed at once)
+        }
+        if (p != nullptr && kept)
         {
             try
             {
                 std::lock_guard<std::mutex> lock(m_mutex);
-                m_inUse[p] = {want, dev};
+                m_inUse[p] = {rounded, dev};
             }
             catch (...) // no host memory
             {
@@ -86,7 +92,7 @@ public:
                 const Block b = it->second;
                 m_inUse.erase(it);
                 Device &d = m_devices[b.device];
-                if (b.size <= m_limit / 4 && d.held + b.size <= m_limit)
+                if (d.held + b.size <= m_limit)
                 {
                     size_t &ofSize = d.waitingOfSize[b.size];
                     d.waiting.push_back({b.size, p});
@@ -100,7 +106,7 @@ public:
         {
             // no host memory to remember it by
         }
-        Source::free(p); // beyond the limit, or not from here
+        Source::free(p); // beyond the limit, larger than what is kept, or not from here
     }
 
 private:
@@ -121,8 +127,8 @@ private:
         int64_t                                  held = 0;      // bytes of ready and waiting
     };
 
-    // Sizes of eight steps per power of two (at most an eighth more than asked for), 4 KiB and more. Sizes that no memory
-    // has are left as they are, for the allocation to refuse.
+    // Sizes of eight steps per power of two (at most an eighth more than asked for from 32 KiB on, and whole multiples of 4 KiB
+    // below). Sizes that no memory has are left as they are, for the allocation to refuse.
     static int64_t RoundUp(int64_t size)
     {
         if (size >= int64_t(1) << 48)

@@ -10,13 +10,15 @@
 using nvcvamd::BlockPool;
 
 static std::atomic<int64_t> g_allocs{0}, g_frees{0}, g_syncs{0};
+static std::atomic<int64_t> g_asked{0}, g_most{INT64_MAX}; // bytes of the last request; the largest request there is memory for
 static std::atomic<bool>    g_full{false}, g_busy{false};
 
 struct Counting
 {
     static void *alloc(size_t size)
     {
-        if (g_full && g_allocs - g_frees > 0)
+        g_asked = (int64_t)size;
+        if ((g_full && g_allocs - g_frees > 0) || (int64_t)size > g_most)
         {
             return nullptr;
         }
@@ -26,7 +28,7 @@ struct Counting
             return nullptr;
         }
         ++g_allocs;
-        return std::malloc(size);
+        return std::malloc(size < 65536 ? size : 65536); // (larger ones are not written)
     }
     static void free(void *p)
     {
@@ -58,6 +60,7 @@ static void Reset()
 {
     g_allocs = g_frees = g_syncs = 0;
     g_full = g_busy = false;
+    g_most          = INT64_MAX;
 }
 
 int main()
@@ -157,6 +160,22 @@ int main()
             volatile int64_t size = (int64_t)((uint64_t(1) << bits) - 1);
             REQUIRE(pool.alloc(size) == nullptr);
         }
+    }
+    {
+        // what is never kept is asked for as it is; what is kept too, where there is no memory for the rounded size
+        Reset();
+        BlockPool<Counting> pool(1 << 20);
+        for (int64_t size : {(int64_t(1) << 18) + 1, (int64_t(1) << 32) + 1, int64_t(0x123456789)})
+        {
+            void *p = pool.alloc(size);
+            REQUIRE(p != nullptr && g_asked == size);
+            pool.free(p);
+        }
+        g_most  = 70000;
+        void *p = pool.alloc(70000), *q = pool.alloc(70001);
+        REQUIRE(p != nullptr && g_asked == 70001 && q == nullptr);
+        pool.free(p);
+        REQUIRE(g_allocs == 4 && g_frees == 4);
     }
     {
         // threads
