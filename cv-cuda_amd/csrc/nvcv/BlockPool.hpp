@@ -5,12 +5,13 @@
 // which the kernels take 28). A block given back here is not waited for: it goes to `waiting`, whatever stream may
 // still use it, and becomes `ready` only after a synchronisation of the whole device that began after it was given
 // back. That synchronisation is made on the allocating side, when no ready block fits and either kMostWaiting blocks of
-// the size wait or half of the pool's limit is waiting or ready: once in dozens of allocations, by which time most of
-// the blocks are idle.
+// the size wait or half of the pool's limit is waiting or ready: once in 32 allocations of blocks of up to a 64th of the
+// limit, by which time most of them are idle, and in as many as fit half of the limit of larger ones (200 MiB under 1 GiB:
+// every third).
 //
-// Bounds: the blocks held and not in use never exceed `limit` (a block beyond it is freed at once, as is one larger
-// than a quarter of it); at every synchronisation the blocks that were ready since the one before and found no use are
-// freed; when the device is out of memory all of them are. Safe with any number of threads (one lock, not held across the
+// Bounds: the blocks held and not in use never exceed `limit` (where one more would, others are freed to make room;
+// one larger than a quarter of it is not kept); at every synchronisation the blocks that were ready since the one
+// before and found no use are freed; when the device is out of memory all of them are. Safe with any number of threads (one lock, not held across the
 // synchronisation) and streams. At the end of the process the blocks are left to the runtime, which may be gone by then.
 #ifndef NVCVAMD_BLOCKPOOL_HPP
 #define NVCVAMD_BLOCKPOOL_HPP
@@ -83,6 +84,7 @@ public:
 
     void free(void *p) noexcept
     {
+        std::vector<void *> drop;
         try
         {
             std::lock_guard<std::mutex> lock(m_mutex);
@@ -90,23 +92,29 @@ public:
             if (it != m_inUse.end())
             {
                 const Block b = it->second;
+                Device     &d = m_devices[b.device];
+                d.waiting.reserve(d.waiting.size() + 1);
+                size_t &ofSize = d.waitingOfSize[b.size];
                 m_inUse.erase(it);
-                Device &d = m_devices[b.device];
-                if (d.held + b.size <= m_limit)
-                {
-                    size_t &ofSize = d.waitingOfSize[b.size];
-                    d.waiting.push_back({b.size, p});
-                    ++ofSize;
-                    d.held += b.size;
-                    return;
-                }
+                makeRoom(d, b.size, drop);
+                d.waiting.push_back({b.size, p});
+                ++ofSize;
+                d.held += b.size;
+                p = nullptr;
             }
         }
         catch (...)
         {
             // no host memory to remember it by
         }
-        Source::free(p); // beyond the limit, larger than what is kept, or not from here
+        for (void *q : drop)
+        {
+            Source::free(q);
+        }
+        if (p != nullptr)
+        {
+            Source::free(p); // larger than what is kept, or not from here
+        }
     }
 
 private:
@@ -141,6 +149,50 @@ private:
             step *= 2;
         }
         return size <= step ? step : (size + step - 1) / step * step;
+    }
+
+    // Takes out blocks until one of `size` fits under the limit: ready ones first, of other sizes before its own, then those
+    // that have waited longest (freeing them waits for the device, as freeing the new one would). The new one stays: the
+    // sizes that a program frees now are those it asks for next, and what is left of earlier ones would stay for good
+    // if it had no way out but another request for its own size (256, 240, 224 and 208 MiB freed once under a limit of 1 GiB:
+    // 104 MiB were allocated and freed anew every time from then on).
+    void makeRoom(Device &d, int64_t size, std::vector<void *> &drop)
+    {
+        if (d.held + size <= m_limit)
+        {
+            return;
+        }
+        size_t most = d.waiting.size();
+        for (auto &r : d.ready)
+        {
+            most += r.second.size();
+        }
+        drop.reserve(most); // (nothing below throws)
+        for (int own = 0; own < 2; ++own)
+        {
+            for (auto &r : d.ready)
+            {
+                while (d.held + size > m_limit && !r.second.empty() && (r.first == size) == (own == 1))
+                {
+                    drop.push_back(r.second.front());
+                    r.second.erase(r.second.begin());
+                    auto unused = d.unused.find(r.first);
+                    if (unused != d.unused.end() && unused->second > 0)
+                    {
+                        --unused->second; // (the front ones)
+                    }
+                    d.held -= r.first;
+                }
+            }
+        }
+        size_t n = 0;
+        for (; d.held + size > m_limit && n < d.waiting.size(); ++n)
+        {
+            drop.push_back(d.waiting[n].second);
+            --d.waitingOfSize.find(d.waiting[n].first)->second;
+            d.held -= d.waiting[n].first;
+        }
+        d.waiting.erase(d.waiting.begin(), d.waiting.begin() + n);
     }
 
     void *take(int dev, int64_t size)

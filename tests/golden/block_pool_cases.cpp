@@ -111,7 +111,8 @@ int main()
         {
             pool.free(m);
         }
-        REQUIRE(g_frees - before == 12 - 4); // 2 x 256 KiB are held already: 4 x 128 KiB fit under 1 MiB
+        // 8 x 128 KiB are 1 MiB: the 2 x 256 KiB held already and the 4 of them that waited longest make room
+        REQUIRE(g_frees - before == 2 + 4);
     }
     {
         // blocks that find no use between two synchronisations are freed; a device that cannot be synchronised now
@@ -150,6 +151,21 @@ int main()
         void *w = pool.alloc(1 << 16 | 1);
         REQUIRE(w != nullptr && g_allocs - g_frees == 1);
         pool.free(std::malloc(16)); // not from here: passed on
+    }
+    {
+        // sizes that nothing asks for any more do not keep others out
+        Reset();
+        BlockPool<Counting> pool(1 << 30);
+        for (int64_t mib : {256, 240, 224, 208})
+        {
+            pool.free(pool.alloc(mib << 20));
+        }
+        for (int i = 0; i < 1000; ++i)
+        {
+            pool.free(pool.alloc(104 << 20));
+        }
+        REQUIRE(g_allocs <= 4 + 6 && g_syncs > 0); // (half of the limit holds 5 x 104 MiB)
+        REQUIRE(g_frees >= 4);                     // and the others are gone
     }
     {
         // sizes that no memory has are refused
