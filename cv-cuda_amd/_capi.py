@@ -221,6 +221,7 @@ for _t in ("Allocator", "Tensor", "Image", "ImageBatch"):
         _sig(nvcv, "nvcv%s%s" % (_t, _f), ST, H, P(C.c_int))
     _sig(nvcv, "nvcv%sSetUserPointer" % _t, ST, H, C.c_void_p)
     _sig(nvcv, "nvcv%sGetUserPointer" % _t, ST, H, P(C.c_void_p))
+_sig(nvcv, "nvcvxAllocatorReleaseUnused", ST)
 _sig(nvcv, "nvcvAllocatorAllocHostMemory", ST, H, P(C.c_void_p), C.c_int64, C.c_int32)
 _sig(nvcv, "nvcvAllocatorFreeHostMemory", ST, H, C.c_void_p, C.c_int64, C.c_int32)
 # tensor

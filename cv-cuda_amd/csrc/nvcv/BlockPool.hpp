@@ -11,7 +11,7 @@
 //
 // Bounds: the blocks held and not in use never exceed `limit` (where one more would, others are freed to make room;
 // one larger than a quarter of it is not kept); at every synchronisation the blocks that were ready since the one
-// before and found no use are freed; when the device is out of memory all of them are. Safe with any number of threads (one lock, not held across the
+// before and found no use are freed; when the device is out of memory, or release() is called, all of them are. Safe with any number of threads (one lock, not held across the
 // synchronisation) and streams. At the end of the process the blocks are left to the runtime, which may be gone by then.
 #ifndef NVCVAMD_BLOCKPOOL_HPP
 #define NVCVAMD_BLOCKPOOL_HPP
@@ -114,6 +114,23 @@ public:
         if (p != nullptr)
         {
             Source::free(p); // larger than what is kept, or not from here
+        }
+    }
+
+    // Frees every block that is not in use, of all devices.
+    void release()
+    {
+        std::vector<void *> drop;
+        {
+            std::lock_guard<std::mutex> lock(m_mutex);
+            for (auto &d : m_devices)
+            {
+                takeAll(d.second, drop);
+            }
+        }
+        for (void *p : drop)
+        {
+            Source::free(p);
         }
     }
 
@@ -283,22 +300,27 @@ private:
         return true;
     }
 
+    // Takes out every block of the device that is not in use.
+    static void takeAll(Device &d, std::vector<void *> &drop)
+    {
+        for (auto &r : d.ready)
+        {
+            drop.insert(drop.end(), r.second.begin(), r.second.end());
+        }
+        for (auto &b : d.waiting)
+        {
+            drop.push_back(b.second);
+        }
+        d = {};
+    }
+
     // Frees every block that is not in use; false if there was none. (Freeing waits for the device's work by itself.)
     bool giveBack(int dev)
     {
         std::vector<void *> drop;
         {
             std::lock_guard<std::mutex> lock(m_mutex);
-            Device                     &d = m_devices[dev];
-            for (auto &r : d.ready)
-            {
-                drop.insert(drop.end(), r.second.begin(), r.second.end());
-            }
-            for (auto &b : d.waiting)
-            {
-                drop.push_back(b.second);
-            }
-            d = {};
+            takeAll(m_devices[dev], drop);
         }
         for (void *p : drop)
         {

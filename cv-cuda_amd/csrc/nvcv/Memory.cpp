@@ -634,6 +634,16 @@ NVCVStatus nvcvAllocatorGetUserPointer(NVCVAllocatorHandle handle, void **outUse
     return Protect([&] { *NotNull(outUserPtr, "Pointer to output") = AllocatorPool().get(handle)->userPtr; });
 }
 
+NVCVStatus nvcvxAllocatorReleaseUnused(void)
+{
+    return Protect(
+        []
+        {
+            DevicePool().release();
+            PinnedPool().release();
+        });
+}
+
 #define NVCVAMD_ALLOC_PAIR(Name, allocFn, freeFn)                                                                  \
     NVCVStatus nvcvAllocatorAlloc##Name(NVCVAllocatorHandle halloc, void **ptr, int64_t sizeBytes, int32_t alignBytes) \
     {                                                                                                              \

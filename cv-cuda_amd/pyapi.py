@@ -313,10 +313,11 @@ class Tensor:
         vals = dict(zip(names, args))
         vals.update(kw)
         if names[0] == "nimages":
-            self._t = _Tensor.for_images(vals["nimages"], tuple(vals["imgsize"]), int(vals["format"]), row_align=rowalign)
+            self._t = _allocated(_Tensor.for_images, vals["nimages"], tuple(vals["imgsize"]), int(vals["format"]),
+                                 row_align=rowalign)
         else:
-            self._t = _Tensor.alloc(list(vals["shape"]), _np_dtype(vals["dtype"]), vals.get("layout") or "",
-                                    row_align=rowalign)
+            self._t = _allocated(_Tensor.alloc, list(vals["shape"]), _np_dtype(vals["dtype"]), vals.get("layout") or "",
+                                 row_align=rowalign)
 
     @property
     def handle(self):
@@ -369,7 +370,8 @@ class _Outputs:
     object cache.) A tensor comes back here only if every use of it was a call of this module on the default stream,
     where the next user's work is ordered behind the last one's; one whose memory, handle or views were given out goes
     back to the library's allocator, which knows when the device is done with it. Bounded: beyond `most_bytes` or
-    `most_tensors` everything held goes back to the allocator."""
+    `most_tensors` everything held goes back to the allocator, as it does when the device is out of memory and in
+    `clear_cache()`."""
     most_bytes, most_tensors = 256 << 20, 64
 
     def __init__(self):
@@ -385,7 +387,7 @@ class _Outputs:
             if raw is not None:
                 self._bytes -= raw._nbytes
                 self._count -= 1
-        out = Tensor(_wrap=raw if raw is not None else _Tensor.alloc(list(shape), dtype, layout or ""))
+        out = Tensor(_wrap=raw if raw is not None else _allocated(_Tensor.alloc, list(shape), dtype, layout or ""))
         if raw is not None:
             out._wrote = (-key[3], None)  # another stream's first use of it waits for the default stream's last
         else:
@@ -418,8 +420,33 @@ class _Outputs:
             pass  # the interpreter is ending: the module's names are gone
 
 
+    def clear(self):
+        """Gives everything held back to the allocator; False if there was nothing."""
+        with self._lock:
+            drop, self._free, self._bytes, self._count = self._free, {}, 0, 0
+        return any(drop.values())
+
+
 _NO_READS = {}
 _outputs = _Outputs()
+
+
+def _allocated(make, *args, **kw):
+    """make(...) of an object with memory of its own; once more without the results that are kept where there is none."""
+    try:
+        return make(*args, **kw)
+    except Error as e:
+        if e.status != 7 or not _outputs.clear():  # NVCV_ERROR_OUT_OF_MEMORY
+            raise
+    return make(*args, **kw)
+
+
+def clear_cache():
+    """Gives the memory that is kept for later objects back to the system: operators' results that are handed out again,
+    and the blocks of the library's allocator (the reference's bindings empty their object cache under this name,
+    python/mod_nvcv/Cache.cpp)."""
+    _outputs.clear()
+    check(_nv.nvcvxAllocatorReleaseUnused())
 
 
 def _result(shape, dtype, layout, stream):
@@ -465,7 +492,7 @@ class Image(_Image):
 
     def __init__(self, size=None, format=None, rowalign=0, *, _handle=None):
         if _handle is None:
-            made = _Image.alloc(tuple(size), int(format), row_align=rowalign)
+            made = _allocated(_Image.alloc, tuple(size), int(format), row_align=rowalign)
             _handle, made.handle = made.handle, None  # the handle moves to this object
         _Image.__init__(self, _handle)
 
@@ -652,6 +679,9 @@ def as_images(buffers, format=None):
 class ImageBatchVarShape(_ImageBatchVarShape):
     """ImageBatchVarShape(capacity) (python/mod_nvcv/ImageBatch.cpp)."""
     _buffers = None  # the buffers of the first images, where these have no Image objects yet
+
+    def __init__(self, capacity):
+        _allocated(super().__init__, capacity)
 
     @property
     def images(self):

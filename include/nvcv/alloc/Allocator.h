@@ -75,6 +75,10 @@ NVCV_PUBLIC NVCVStatus nvcvAllocatorAllocCudaMemory(NVCVAllocatorHandle halloc, 
 NVCV_PUBLIC NVCVStatus nvcvAllocatorFreeCudaMemory(NVCVAllocatorHandle halloc, void *ptr, int64_t sizeBytes,
                                                    int32_t alignBytes);
 
+/* Extension: gives the blocks that the default allocator keeps of freed objects (at most 1 GiB of device and 64 MiB of
+ * pinned memory per device) back to the system. Waits for the work of the devices that hold any. */
+NVCV_PUBLIC NVCVStatus nvcvxAllocatorReleaseUnused(void);
+
 NVCV_PUBLIC const char *nvcvResourceTypeGetName(NVCVResourceType resource);
 
 #ifdef __cplusplus

@@ -168,6 +168,33 @@ int main()
         REQUIRE(g_frees >= 4);                     // and the others are gone
     }
     {
+        // everything kept is given back when asked for, ready and waiting; what is in use is not
+        Reset();
+        BlockPool<Counting> pool(1 << 20);
+        void               *a[40];
+        for (auto &p : a)
+        {
+            p = pool.alloc(5000);
+        }
+        for (auto &p : a)
+        {
+            pool.free(p);
+        }
+        int *used = static_cast<int *>(pool.alloc(5000)); // 39 are ready
+        for (int i = 0; i < 3; ++i)
+        {
+            pool.free(pool.alloc(70000 + 20000 * i)); // others wait
+        }
+        pool.release();
+        REQUIRE(g_allocs - g_frees == 1);
+        *used = 1;
+        pool.free(used);
+        pool.release();
+        pool.release();
+        REQUIRE(g_allocs == g_frees);
+        REQUIRE(pool.alloc(5000) != nullptr);
+    }
+    {
         // sizes that no memory has are refused
         Reset();
         BlockPool<Counting> pool(1 << 20);

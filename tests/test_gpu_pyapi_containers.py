@@ -334,3 +334,16 @@ def test_as_images_of_torch_tensors_in_one_call(nvcv):
     assert masks.uniqueformat == nvcv.Format.F32 and masks[1].size == (5, 3)
     mixed = nvcv.as_images([tensors[0], torch.zeros((4, 4), dtype=torch.uint8, device="cuda")])
     assert mixed._buffers is None and mixed.uniqueformat is None
+
+
+def test_kept_memory_is_given_back(nvcv):
+    # results that were dropped and blocks of freed tensors stay with the process until clear_cache()
+    import torch
+    src = nvcv.as_tensor(torch.zeros((4, 1000, 1000, 3), dtype=torch.uint8, device="cuda"), "NHWC")
+    kept = [nvcv.flip(src, 0) for _ in range(4)] + [nvcv.Tensor((4, 1000, 1000, 3), "u1", "NHWC") for _ in range(4)]
+    torch.cuda.synchronize()
+    del kept
+    before = torch.cuda.mem_get_info()[0]
+    nvcv.clear_cache()
+    assert torch.cuda.mem_get_info()[0] - before >= 8 * 12_000_000
+    assert nvcv.flip(src, 0).torch().sum().item() == 0

@@ -323,6 +323,78 @@ def test_results_on_other_streams_are_always_new(api, monkeypatch):
     assert api._result([2, 3], np.uint8, "HW", FakeStream(0)) == "kept"
 
 
+def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
+    # an allocation that finds no memory is tried once more without the kept results, which it would otherwise never reach;
+    # clear_cache() gives them and the library's blocks back (no GPU: the library's tensors are stand-ins)
+    class Raw:
+        alive, most = 0, 3
+
+        def __init__(self):
+            Raw.alive += 1
+
+        def __del__(self):
+            Raw.alive -= 1
+
+        @classmethod
+        def alloc(cls, shape, dtype=None, layout=None, row_align=0):
+            if cls.alive >= cls.most:
+                raise api.Error(7, "no memory")
+            if shape == [0]:
+                raise api.Error(2, "empty")
+            return cls()
+
+        for_images = alloc
+
+        def export(self):
+            class D:
+                rank, shape = 1, [1]
+
+                class buffer:
+                    strides = [1]
+            return D
+
+    class Picture(api._Image):
+        @staticmethod
+        def alloc(size, fmt, row_align=0):
+            made = Raw.alloc(size)
+            made.handle = api.C.c_void_p()
+            return made
+
+    outputs = api._Outputs()
+    monkeypatch.setattr(api, "_Tensor", Raw)
+    monkeypatch.setattr(api, "_Image", Picture)
+    monkeypatch.setattr(api, "_outputs", outputs)
+    monkeypatch.setattr(api.torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+
+    def fill():
+        kept = [outputs.get((n,), np.uint8, "N") for n in (1, 2, 3)]
+        for t in kept:
+            t._wrote = (0, None)
+        del kept, t
+        assert Raw.alive == outputs._count == 3
+
+    for make in (lambda: outputs.get((9,), np.uint8, "N"), lambda: api.Tensor((4,), np.uint8, "N"),
+                 lambda: api.Tensor(2, (4, 4), api.Format.U8), lambda: api.Image((4, 4), api.Format.U8)):
+        fill()
+        made = make()
+        assert outputs._count == 0
+        del made
+        outputs.clear()
+        assert Raw.alive == 0
+    held = [api.Tensor((n,), np.uint8, "N") for n in (4, 5, 6)]
+    with pytest.raises(api.Error) as e:  # nothing left to give back
+        api.Tensor((7,), np.uint8, "N")
+    assert e.value.status == 7
+    del held, e
+    fill()
+    Raw.most = 9
+    with pytest.raises(api.Error) as e:
+        api.Tensor((0,), np.uint8, "N")
+    assert e.value.status == 2 and outputs._count == 3  # another error than want of memory
+    api.clear_cache()
+    assert Raw.alive == outputs._count == outputs._bytes == 0
+
+
 def test_results_alive_at_the_end_of_the_program_say_nothing():
     # a module's result tensors that outlive this package's module globals: nothing on stderr
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
