@@ -16,6 +16,11 @@ def api(cv):
     return importlib.import_module("cvcuda_amd.pyapi")
 
 
+@pytest.fixture(autouse=True)
+def no_default_stream_is_followed(api, monkeypatch):
+    monkeypatch.setattr(api, "_followed", {})
+
+
 def test_enumerations(api, K):
     assert api.Interp.LINEAR == K.INTERP_LINEAR and api.Interp.WARP_INVERSE_MAP == K.WARP_INVERSE_MAP == 16
     assert api.Border.REFLECT101 == K.BORDER_REFLECT101 and api.ChannelManip.REVERSE == K.CHANNEL_REVERSE
@@ -212,6 +217,57 @@ def test_submit_orders_the_default_stream_by_events_recorded_when_needed(api, mo
     assert default.waited == [7, 7]
     api._submit(default, [b], [c], lambda s: None)  # its own result, and c, which only it has read since
     assert default.waited == [7, 7, 7]  # c was written by `side`
+
+
+def test_a_stream_that_follows_the_default_one_waits_for_what_it_reads_alone(api, monkeypatch):
+    # a program that prepares the next batch on the default stream while another stream works on the last one: from the
+    # second wait on, the other stream waits for the write it reads and not for what the default stream was given since; a
+    # program that stops doing so gets no events again. No GPU: a stand-in device that counts the default stream's work.
+    class FakeStream:
+        def __init__(self, key):
+            self.cuda_stream, self.device_index, self.work, self.waited = key, 0, 0, []
+
+        def wait_event(self, event):
+            self.waited.append((event.stream.cuda_stream, event.at))
+
+    class FakeEvent:
+        made = 0
+
+        def __init__(self):
+            FakeEvent.made += 1
+
+        def record(self, stream):
+            self.stream, self.at = stream, stream.work
+
+    class Box:
+        pass
+
+    default, side = FakeStream(0), FakeStream(7)
+    monkeypatch.setattr(api, "_torch_stream", lambda s: s)
+    monkeypatch.setattr(api, "_default_stream", lambda device: default)
+    monkeypatch.setattr(api, "_new_event", FakeEvent)
+
+    def launch(s):
+        assert s == 0
+        default.work += 1
+
+    def one_batch():
+        batch, other = Box(), Box()
+        api._submit(default, [], [batch], launch)
+        written = default.work
+        for _ in range(5):
+            api._submit(default, [other], [other], launch)
+        api._submit(side, [batch], [], lambda s: None)
+        return written
+
+    assert one_batch() == 1 and side.waited == [(0, 6)]
+    for _ in range(3):
+        written = one_batch()
+        assert side.waited[-1] == (0, written)
+    other, before = Box(), FakeEvent.made
+    for _ in range(2000):
+        api._submit(default, [other], [other], launch)
+    assert FakeEvent.made - before == api._FOLLOWED_CALLS < 2000
 
 
 def test_results_come_back_only_from_the_default_stream_and_unseen(api, monkeypatch):
