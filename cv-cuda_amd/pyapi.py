@@ -676,6 +676,9 @@ def as_images(buffers, format=None):
     return batch
 
 
+_images_lock = threading.RLock()
+
+
 class ImageBatchVarShape(_ImageBatchVarShape):
     """ImageBatchVarShape(capacity) (python/mod_nvcv/ImageBatch.cpp)."""
     _buffers = None  # the buffers of the first images, where these have no Image objects yet
@@ -686,12 +689,15 @@ class ImageBatchVarShape(_ImageBatchVarShape):
     @property
     def images(self):
         if self._buffers is not None:
-            buffers, self._buffers = self._buffers, None
-            handles = (C.c_void_p * len(buffers))()
-            check(_nv.nvcvImageBatchVarShapeGetImages(self.handle, 0, handles, len(buffers)))
-            self._images = [Image(_handle=C.c_void_p(h)) for h in handles]
-            for image, buffer in zip(self._images, buffers):
-                image._keep.append(buffer)
+            # (threads that read one batch at a time find the whole list or wait for it; the buffers are held until then)
+            with _images_lock:
+                if self._buffers is not None:
+                    handles = (C.c_void_p * len(self._buffers))()
+                    check(_nv.nvcvImageBatchVarShapeGetImages(self.handle, 0, handles, len(self._buffers)))
+                    made = [Image(_handle=C.c_void_p(h)) for h in handles]
+                    for image, buffer in zip(made, self._buffers):
+                        image._keep.append(buffer)
+                    self._images, self._buffers = made, None
         return self._images
 
     @images.setter

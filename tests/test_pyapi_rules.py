@@ -270,6 +270,40 @@ def test_a_stream_that_follows_the_default_one_waits_for_what_it_reads_alone(api
     assert FakeEvent.made - before == api._FOLLOWED_CALLS < 2000
 
 
+def test_images_of_a_batch_asked_for_by_several_threads(api, monkeypatch):
+    # a batch made in one call makes its Image objects when they are asked for: every thread gets all of them, the same
+    # ones, and a failure loses no buffer (no GPU: the library's call is a stand-in that takes its time)
+    import threading
+    import time
+    import types
+
+    calls = []
+
+    def get_images(handle, first, handles, n):
+        calls.append(n)
+        time.sleep(0.05)
+        return status[0]
+
+    monkeypatch.setattr(api, "_nv", types.SimpleNamespace(nvcvImageBatchVarShapeGetImages=get_images))
+    batch = api.ImageBatchVarShape.__new__(api.ImageBatchVarShape)
+    batch.handle, batch.images = None, []
+    buffers = batch._buffers = [object() for _ in range(5)]
+    status = [2]
+    with pytest.raises(api.Error):
+        batch.images
+    assert batch._buffers is buffers and calls == [5]
+    status = [0]
+    got = []
+    threads = [threading.Thread(target=lambda: got.append(list(batch.images))) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 8 and calls == [5, 5]
+    assert [i._keep for i in got[0]] == [[b] for b in buffers] and batch._buffers is None
+    assert all([id(i) for i in g] == [id(i) for i in got[0]] for g in got)
+
+
 def test_results_come_back_only_from_the_default_stream_and_unseen(api, monkeypatch):
     # which of an operator's result tensors are handed out again (no GPU: the library's tensors are stand-ins)
     import gc
