@@ -130,7 +130,7 @@ public:
             // of the arrays that changed since the last export.
             CheckHip(hipStreamWaitEvent(stream, m_uploaded, 0), "hipStreamWaitEvent");
             size_t n = (size_t)(m_num - m_dirtyFrom);
-            if (m_dirtyFrom == 0)
+            if (m_dirtyFrom == 0 && uploadedAtOnce(n * sizeof(*m_devImages), formatsBytes() - n * sizeof(*m_devFormats)))
             {
                 CheckHip(hipMemcpyAsync(m_devFormats, m_hostFormats, (size_t)formatsBytes() + n * sizeof(*m_devImages),
                                         hipMemcpyHostToDevice, stream),
@@ -309,6 +309,15 @@ private:
     int64_t listsBytes() const
     {
         return formatsBytes() + imagesBytes();
+    }
+
+    // Whether all formats, with `room` bytes behind those of the images held, and the images' `bytes` go in one copy. A
+    // copy takes 3.0 us up to 16 KiB and 9.3 us and 18 us per MiB beyond, and two small ones 5.8 us: a batch with room for a
+    // million images would spend 156 us on its first one.
+    bool uploadedAtOnce(int64_t bytes, int64_t room) const
+    {
+        constexpr int64_t kSmallCopy = 16384;
+        return formatsBytes() + bytes <= kSmallCopy || (bytes > kSmallCopy && room <= 131072);
     }
 
     int64_t handlesBytes() const

@@ -6,6 +6,7 @@ src/nvcv/src/priv/Tensor.cpp:172-185, validation of TensorWrapDataStrided.cpp:35
 semantics of priv/Status.cpp:31-110 -- with this library's alignment constants (128-byte rows,
 512-byte base)."""
 import ctypes as C
+import glob
 import os
 import subprocess
 
@@ -581,3 +582,21 @@ def test_block_pool_of_the_default_allocator(tmp_path):
     csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cv-cuda_amd", "csrc", "nvcv")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I" + csrc, src, "-o", exe, "-lpthread"], check=True)
     assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "ok"
+
+
+def test_what_an_image_batch_uploads(tmp_path):
+    # the device's lists follow the host's, and the room of a batch that is not full is not copied: the library's sources
+    # over a stand-in for the HIP runtime
+    here = os.path.dirname(os.path.abspath(__file__))
+    root = os.path.dirname(here)
+    exe = str(tmp_path / "image_batch_upload")
+    csrc = os.path.join(root, "cv-cuda_amd", "csrc")
+    sources = [os.path.join(here, "golden", "image_batch_upload.cpp")] + sorted(glob.glob(os.path.join(csrc, "nvcv", "*.cpp")))
+    objects = [str(tmp_path / (os.path.basename(s) + ".o")) for s in sources]
+    builds = [subprocess.Popen(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                                "-I" + os.path.join(root, "include"), "-I" + csrc, "-c", s, "-o", o])
+              for s, o in zip(sources, objects)]
+    assert [b.wait() for b in builds] == [0] * len(builds)
+    subprocess.run(["g++"] + objects + ["-o", exe, "-lpthread"], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.stdout.strip() == "ok", r.stdout
