@@ -43,6 +43,7 @@ public:
             m_devImages   = reinterpret_cast<NVCVImageBufferStrided *>(reinterpret_cast<uint8_t *>(m_devFormats) + formatsBytes());
             m_hostImages  = reinterpret_cast<NVCVImageBufferStrided *>(reinterpret_cast<uint8_t *>(m_hostFormats) + formatsBytes());
             m_handles     = static_cast<NVCVImageHandle *>(m_alloc.allocHost(handlesBytes(), m_reqs.alignBytes));
+            CheckHip(hipGetDevice(&m_device), "hipGetDevice");
             CheckHip(hipEventCreateWithFlags(&m_uploaded, hipEventDisableTiming), "hipEventCreateWithFlags");
         }
         catch (...)
@@ -55,9 +56,10 @@ public:
 
     ~VarShapeBatch() override
     {
-        // An upload may still read the pinned lists. The default allocator hands a block out again only when the device has
-        // been idle since it was given back, so only a caller's own allocator has to be waited for here.
-        if (m_uploaded != nullptr && m_hAlloc != nullptr)
+        // An upload may still read the pinned lists. The default allocator hands a block out again only when the device on
+        // which it was made has been idle since it was given back, so only a caller's own allocator, and an upload by a
+        // stream of another device, have to be waited for here.
+        if (m_uploaded != nullptr && (m_hAlloc != nullptr || m_uploadedElsewhere))
         {
             (void)hipEventSynchronize(m_uploaded);
         }
@@ -129,6 +131,13 @@ public:
             // Order after any earlier upload (possibly issued on another stream), then copy the tail
             // of the arrays that changed since the last export.
             CheckHip(hipStreamWaitEvent(stream, m_uploaded, 0), "hipStreamWaitEvent");
+            hipDevice_t device = m_device;
+            if (hipStreamGetDevice(stream, &device) != hipSuccess)
+            {
+                (void)hipGetLastError();
+                device = -1;
+            }
+            m_uploadedElsewhere |= device != m_device;
             size_t n = (size_t)(m_num - m_dirtyFrom);
             if (m_dirtyFrom == 0 && uploadedAtOnce(n * sizeof(*m_devImages), formatsBytes() - n * sizeof(*m_devFormats)))
             {
@@ -432,6 +441,8 @@ private:
     NVCVImageFormat        *m_hostFormats = nullptr;
     NVCVImageHandle        *m_handles     = nullptr;
     hipEvent_t              m_uploaded    = nullptr;
+    int                     m_device      = 0; // of the lists and the event
+    bool                    m_uploadedElsewhere = false;
 
     int32_t         m_num        = 0;
     int32_t         m_dirtyFrom  = 0;

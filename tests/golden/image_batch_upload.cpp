@@ -1,5 +1,6 @@
 // What an image batch uploads, over a stand-in for the HIP runtime whose device memory is the host's: the lists on the device
 // are those on the host after every export, and a batch with room for many more images than it holds does not copy that room.
+// A batch that ends waits for its upload where the allocator of its lists does not.
 #include <hip/hip_runtime_api.h>
 
 #include <nvcv/Image.h>
@@ -10,7 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 
-static int64_t g_copied = 0, g_copies = 0;
+static int64_t g_copied = 0, g_copies = 0, g_waits = 0;
 
 extern "C"
 {
@@ -58,8 +59,14 @@ hipError_t hipEventRecord(hipEvent_t, hipStream_t)
 {
     return hipSuccess;
 }
+hipError_t hipStreamGetDevice(hipStream_t stream, hipDevice_t *d)
+{
+    *d = stream == reinterpret_cast<hipStream_t>(0x1000) ? 1 : 0;
+    return hipSuccess;
+}
 hipError_t hipEventSynchronize(hipEvent_t)
 {
+    ++g_waits;
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned)
@@ -127,6 +134,32 @@ int main()
             REQUIRE(nvcvImageBatchExportData(batch, nullptr, &data) == NVCV_SUCCESS && g_copied == 0);
         }
         REQUIRE(nvcvImageBatchDecRef(batch, nullptr) == NVCV_SUCCESS);
+    }
+    // uploaded by its own device's stream, by another's, and by either with lists from the caller's own allocator
+    for (int own = 0; own < 2; ++own)
+    {
+        for (uintptr_t stream : {uintptr_t(0), uintptr_t(0x2000), uintptr_t(0x1000)})
+        {
+            const int                          capacity = 4;
+            NVCVImageBatchVarShapeRequirements reqs;
+            NVCVImageBatchHandle               batch     = nullptr;
+            NVCVAllocatorHandle                allocator = nullptr;
+            NVCVResourceAllocator              host      = {};
+            host.resType         = NVCV_RESOURCE_MEM_HOST_PINNED;
+            host.res.mem.fnAlloc = [](void *, int64_t size, int32_t) { return std::malloc((size_t)size); };
+            host.res.mem.fnFree  = [](void *, void *p, int64_t, int32_t) { std::free(p); };
+            REQUIRE(own == 0 || nvcvAllocatorConstructCustom(&host, 1, &allocator) == NVCV_SUCCESS);
+            REQUIRE(nvcvImageBatchVarShapeCalcRequirements(capacity, &reqs) == NVCV_SUCCESS);
+            REQUIRE(nvcvImageBatchVarShapeConstruct(&reqs, allocator, &batch) == NVCV_SUCCESS);
+            NVCVImagePlaneStrided plane = {5, 7, 256, reinterpret_cast<NVCVByte *>(0x1000)};
+            REQUIRE(nvcvxImageBatchVarShapePushBuffers(batch, NVCV_IMAGE_FORMAT_U8, &plane, 1) == NVCV_SUCCESS);
+            NVCVImageBatchData data;
+            REQUIRE(nvcvImageBatchExportData(batch, reinterpret_cast<hipStream_t>(stream), &data) == NVCV_SUCCESS);
+            g_waits = 0;
+            REQUIRE(nvcvImageBatchDecRef(batch, nullptr) == NVCV_SUCCESS);
+            REQUIRE((g_waits > 0) == (own == 1 || stream == 0x1000));
+            REQUIRE(own == 0 || nvcvAllocatorDecRef(allocator, nullptr) == NVCV_SUCCESS);
+        }
     }
     std::puts("ok");
     return 0;
