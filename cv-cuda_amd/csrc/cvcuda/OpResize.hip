@@ -3440,6 +3440,32 @@ __global__ __launch_bounds__(256) void ResizeAreaFloatKernel(const ResizeArgs a)
     }
 }
 
+// 16-byte pieces per lane that hold the columns of 64 boxes, those that edges between two columns add and one for their
+// rounding; and the kernel for so many, of those that scales of more than 1 and up to kAreaWindowMost need (1 to 4, 1 to 10
+// and 2 to 13 for 1, 3 and 4 channels).
+template<int C>
+constexpr int AreaFloatPieces(float scaleX)
+{
+    const float columns = scaleX * kTileW;
+    const int   whole   = (int)columns;
+    return ((whole + (columns > (float)whole ? 1 : 0) + 3) * C + 255) / 256;
+}
+
+using AreaFloatKernelPtr = void (*)(const ResizeArgs);
+
+template<int C, int KCHUNKS = AreaFloatPieces<C>(kAreaWindowMost)>
+AreaFloatKernelPtr AreaFloatKernel(int pieces)
+{
+    if constexpr (KCHUNKS > ((kTileW + 1 + 3) * C + 255) / 256)
+    {
+        if (pieces < KCHUNKS)
+        {
+            return AreaFloatKernel<C, KCHUNKS - 1>(pieces);
+        }
+    }
+    return ResizeAreaFloatKernel<C, KCHUNKS>;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Bicubic resize of float tensors at scales below 2 along both axes, large launches. One pixel at a time the 16 taps of every
 // output pixel are loaded and weighted, four fifths of them again for its neighbour below. Here a lane owns a column of
@@ -3782,17 +3808,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         if (a.scaleX > 1.f && a.scaleX <= kAreaWindowMost && a.scaleY > 1.f && a.srcW >= 16)
         {
-            // 16-byte pieces per lane that hold the columns of 64 boxes, those that edges between two columns add and one
-            // for their rounding
-            using Kernel = void (*)(const ResizeArgs);
-            static constexpr Kernel kKernels[] = {ResizeAreaFloatKernel<C, 1>, ResizeAreaFloatKernel<C, 2>, ResizeAreaFloatKernel<C, 3>,
-                                                  ResizeAreaFloatKernel<C, 4>, ResizeAreaFloatKernel<C, 5>, ResizeAreaFloatKernel<C, 6>,
-                                                  ResizeAreaFloatKernel<C, 7>, ResizeAreaFloatKernel<C, 8>, ResizeAreaFloatKernel<C, 9>,
-                                                  ResizeAreaFloatKernel<C, 10>, ResizeAreaFloatKernel<C, 11>, ResizeAreaFloatKernel<C, 12>,
-                                                  ResizeAreaFloatKernel<C, 13>};
-            const int    pieces = DivUp(((int)std::ceil(a.scaleX * kTileW) + 3) * C, 256); // at most 12.05 for 4 channels
-            const Kernel kernel = kKernels[pieces - 1];
-            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
+            hipLaunchKernelGGL(AreaFloatKernel<C>(AreaFloatPieces<C>(a.scaleX)), grid, dim3(256), 0, stream, a);
             CheckLaunch("ResizeAreaFloatKernel");
             return;
         }
