@@ -609,7 +609,9 @@ def test_negative_cases(cv, gpu):
 # scale of 4 roundings, each off by at most 2^-24 of itself, all of them positive.
 @pytest.mark.parametrize("sw,sh,dw,dh", [(67, 41, 61, 37), (128, 66, 64, 33), (131, 50, 66, 25), (198, 47, 66, 30), (263, 83, 66, 21),
                                          (264, 84, 66, 21), (397, 61, 66, 9), (527, 33, 66, 4), (791, 40, 66, 3), (792, 36, 66, 3),
-                                         (20, 19, 13, 7), (16, 64, 2, 5), (601, 40, 151, 9), (1537, 30, 128, 3)])
+                                         (20, 19, 13, 7), (16, 64, 2, 5), (601, 40, 151, 9), (1537, 30, 128, 3),
+                                         (329, 31, 66, 8), (330, 36, 66, 9), (461, 40, 66, 6), (462, 50, 66, 7), (594, 30, 66, 4),
+                                         (659, 33, 66, 5), (660, 30, 66, 3), (725, 45, 66, 4), (726, 44, 66, 4)])
 @pytest.mark.parametrize("c", [1, 3, 4])
 def test_area_of_floats(cv, orc, gpu, sw, sh, dw, dh, c):
     src = orc.fill_f32((2, sh, sw, c), 0xF0 + sw)
@@ -694,3 +696,32 @@ def test_bicubic_float_strips_next_to_extreme_values(cv, gpu, c):
     rows = out.cpu().numpy()
     assert not np.isnan(rows).any()
     assert (rows[:, 2:sh - 3:2] == 0).all()
+
+
+# the forms of float tensors on sources and results that are views (rows 4 bytes off a 16-byte boundary in another pitch): the
+# dense result, bit for bit, and nothing outside the rows
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("n,sw,sh,dw,dh,interp", [(2, 131, 50, 66, 25, AREA), (2, 263, 83, 66, 21, AREA), (2, 20, 19, 13, 7, AREA),
+                                                  (2, 791, 40, 66, 3, AREA), (60, 131, 97, 197, 145, CUBIC), (512, 67, 50, 64, 49, CUBIC),
+                                                  (512, 4, 4, 65, 17, CUBIC)])
+def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
+    src = torch.from_numpy(orc.fill_f32((2, sh, sw, c), 0xF1 + sw)).cuda().repeat(n // 2, 1, 1, 1)
+    results = []
+    for lead, extra in ((0, 0), (1, 3), (3, 5)):
+        def view(h, w, fill):
+            pitch = w * c + extra
+            # (the source's buffer ends with its last row)
+            buf = torch.full((lead + n * h * pitch - extra,), fill, device="cuda")
+            t = torch.as_strided(buf, (n, h, w, c), (h * pitch, pitch, c, 1), lead)
+            return buf, t, cv.Tensor.wrap(buf.data_ptr() + 4 * lead, [n, h, w, c], [4 * h * pitch, 4 * pitch, 4 * c, 4], np.float32,
+                                          "NHWC", keep=buf)
+        _, s, tin = view(sh, sw, 99.0)
+        s.copy_(src)
+        buf, d, tout = view(dh, dw, -7.0)
+        cv.Resize()(None, tin, tout, interp)
+        torch.cuda.synchronize()
+        results.append(d.clone())
+        d.fill_(-7.0)
+        assert bool((buf == -7.0).all()), "floats outside the rows written"
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+    assert not torch.isnan(results[0]).any()

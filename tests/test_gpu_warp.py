@@ -166,6 +166,35 @@ def test_wide_pixels_at_the_tile_edges(cv, orc, gpu, dw, dh, c):
     assert (res[:4] == -7).all() and (res[-4:] == -7).all()
 
 
+# the same for the other interpolations and borders, and for sources and results that are views: rows 4 bytes off a 16-byte
+# boundary in another pitch. A view's result is the dense one's, bit for bit
+@pytest.mark.parametrize("c", [3, 4])
+@pytest.mark.parametrize("interp", [NEAREST, LINEAR, CUBIC])
+@pytest.mark.parametrize("border", [0, 1, 2, 3, 4])
+def test_wide_pixels_in_views(cv, orc, gpu, c, interp, border):
+    for sw, sh, dw, dh, deg, scale in ((37, 21, 33, 17, 12.0, 0.9), (90, 70, 131, 41, -31.0, 1.4)):
+        src = orc.fill_f32((2, sh, sw, c), 5 + dw + border)
+        m, colour = rotation(sw, sh, deg, scale), (0.25, -3.0, 7.5, 0.125)
+        results = []
+        for lead, extra in ((0, 0), (1, 3)):
+            def view(h, w, fill):
+                buf = torch.full((2 * h * (w * c + extra) + 2 * lead + 8,), fill, device="cuda")
+                t = torch.as_strided(buf, (2, h, w, c), (h * (w * c + extra), w * c + extra, c, 1), lead)
+                return buf, t, cv.Tensor.wrap(buf.data_ptr() + 4 * lead, [2, h, w, c],
+                                              [4 * h * (w * c + extra), 4 * (w * c + extra), 4 * c, 4], np.float32, "NHWC", keep=buf)
+            _, s, tin = view(sh, sw, 99.0)
+            s.copy_(torch.from_numpy(src))
+            buf, d, tout = view(dh, dw, -7.0)
+            cv.WarpAffine(0)(None, tin, tout, m, interp, border, colour)
+            torch.cuda.synchronize()
+            results.append(d.cpu().numpy().copy())
+            d.fill_(-7.0)
+            assert bool((buf == -7.0).all()), "floats outside the rows written"
+        np.testing.assert_array_equal(results[0], results[1])
+        dev = orc.warp(src, (dh, dw), orc.invert_affine(m), interp, border, colour, variant=1)
+        assert np.abs(results[0] - dev).max() <= 1e-3
+
+
 def make_c4_batch(cv, K, orc, n, seed):
     rng = np.random.default_rng(seed)
     bi, bo, hosts, outs, mats = cv.ImageBatchVarShape(n), cv.ImageBatchVarShape(n), [], [], []
@@ -274,6 +303,42 @@ def test_warp_perspective(cv, K, orc, gpu):
     ref = orc.warp(src, (50, 90), H, LINEAR, 1, perspective=True, variant=2)
     for i in range(2):
         np.testing.assert_array_equal(outs[i].plane_view(0, np.uint8, 3).cpu().numpy(), ref[i])
+
+
+# a perspective's quotients against the correctly rounded ones, for every mantissa of the third row and both signs: 1 / x is
+# carried into the result by a bilinear sample of a row of 0, 1, 2, ... at (2^n / x, 0), which float32 holds exactly
+# (24 bits in all: the products of the integer part and the fraction are exact, and so is their sum). In the range of
+# exponents that takes the shorter form, its ends, and outside it
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("e", [-126, -124, -123, -64, 0, 1, 77, 121, 122, 123, 126])
+def test_perspective_quotients(cv, gpu, e, sign):
+    n = min(20, 127 - e)  # (2^(n + e) is a float32)
+    ramp = torch.arange((1 << n) + 8, dtype=torch.float32, device="cuda").repeat(3, 1)[None, :, :, None].contiguous()
+    w, h = 4096, 2048
+    out = torch.zeros((1, h, w, 1), device="cuda")
+    x0 = sign * 2.0 ** e
+    # (a quotient below 0 times -0 is 0, and 0 is inside the image)
+    m = [0.0, 0.0, sign * 2.0 ** (n + e)] + [sign * 0.0] * 3 + [x0 * 2.0 ** -23, x0 * 2.0 ** -11, x0]
+    cv.WarpPerspective(0)(None, cv.Tensor.from_torch(ramp, "NHWC"), cv.Tensor.from_torch(out, "NHWC"), m, LINEAR | INVERSE_MAP, 1,
+                          (0, 0, 0, 0))
+    torch.cuda.synchronize()
+    x = (np.float32(x0) * (1 + np.arange(w * h, dtype=np.float64) * 2.0 ** -23)).astype(np.float32)
+    want = np.float64(np.float32(1) / x) * (sign * 2.0 ** (n + e))
+    np.testing.assert_array_equal(out.cpu().numpy().reshape(-1), want)
+
+
+def test_perspective_quotients_in_and_out_of_range_in_one_wave(cv, gpu):
+    # third rows on both sides of 2^123, and of 2^-123, within the samples of one lane
+    ramp = torch.arange(40, dtype=torch.float32, device="cuda").repeat(3, 1)[None, :, :, None].contiguous()
+    for e, num in ((118, 123), (-125, -120)):
+        out = torch.zeros((1, 8, 64, 1), device="cuda")
+        m = [0.0, 0.0, 2.0 ** num, 0.0, 0.0, 0.0, 2.0 ** e, 0.0, 2.0 ** e]
+        cv.WarpPerspective(0)(None, cv.Tensor.from_torch(ramp, "NHWC"), cv.Tensor.from_torch(out, "NHWC"), m, LINEAR | INVERSE_MAP, 1,
+                              (0, 0, 0, 0))
+        torch.cuda.synchronize()
+        x = (2.0 ** e * np.arange(1, 65)).astype(np.float32)
+        want = np.float64(np.float32(1) / x) * 2.0 ** num
+        np.testing.assert_array_equal(out.cpu().numpy().reshape(8, 64), np.tile(want, (8, 1)))
 
 
 # seeded random cases: every element type and channel count, interpolation and border mode; sources and outputs from 1
