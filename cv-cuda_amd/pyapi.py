@@ -371,33 +371,22 @@ class _Outputs:
     where the next user's work is ordered behind the last one's; one whose memory, handle or views were given out goes
     back to the library's allocator, which knows when the device is done with it. Bounded: beyond `most_bytes` or
     `most_tensors` everything held goes back to the allocator, as it does when the device is out of memory and in
-    `clear_cache()`; what `most_calls` calls have not asked for goes back by itself."""
-    most_bytes, most_tensors, most_calls = 256 << 20, 64, 1024
+    `clear_cache()`."""
+    most_bytes, most_tensors = 256 << 20, 64
 
     def __init__(self):
         self._lock = threading.Lock()
         self._free, self._bytes, self._count = {}, 0, 0
-        self._asked, self._calls = set(), 0  # what was asked for since the last look
 
     def get(self, shape, dtype, layout):
         shape, dtype = tuple(shape), np.dtype(dtype)
         key = (shape, dtype, layout, torch._C._cuda_getDevice())
-        old = None
         with self._lock:
-            self._asked.add(key)
-            self._calls += 1
-            if self._calls >= self.most_calls:
-                old = [self._free.pop(k) for k in list(self._free) if k not in self._asked]
-                for raw in [r for s in old for r in s]:
-                    self._bytes -= raw._nbytes
-                    self._count -= 1
-                self._asked, self._calls = set(), 0
             stack = self._free.get(key)
             raw = stack.pop() if stack else None
             if raw is not None:
                 self._bytes -= raw._nbytes
                 self._count -= 1
-        del old
         out = Tensor(_wrap=raw if raw is not None else _allocated(_Tensor.alloc, list(shape), dtype, layout or ""))
         if raw is not None:
             out._wrote = (-key[3], None)  # another stream's first use of it waits for the default stream's last
