@@ -92,10 +92,9 @@ public:
             if (it != m_inUse.end())
             {
                 const Block b = it->second;
-                Device     &d = m_devices[b.device];
-                d.waiting.reserve(d.waiting.size() + 1);
-                size_t &ofSize = d.waitingOfSize[b.size];
                 m_inUse.erase(it);
+                Device &d      = m_devices[b.device];
+                size_t &ofSize = d.waitingOfSize[b.size];
                 makeRoom(d, b.size, drop);
                 d.waiting.push_back({b.size, p});
                 ++ofSize;

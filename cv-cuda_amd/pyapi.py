@@ -419,7 +419,6 @@ class _Outputs:
         except (AttributeError, TypeError):
             pass  # the interpreter is ending: the module's names are gone
 
-
     def clear(self):
         """Gives everything held back to the allocator; False if there was nothing."""
         with self._lock:
@@ -781,10 +780,11 @@ def _submit(stream, reads, writes, op, *args):
                 if other != key:
                     waits = waits or []
                     waits.append((other, mark))
-        for other, _ in waits or ():
-            if other <= 0:
-                _followed[other] = _FOLLOWED_CALLS
-        if not s and _followed.get(key):
+        if waits:
+            for other, _ in waits:
+                if other <= 0:
+                    _followed[other] = _FOLLOWED_CALLS
+        if _followed and not s and _followed.get(key):
             _followed[key] -= 1
             s = _default_stream(-key)
     if waits:
