@@ -243,9 +243,15 @@ __device__ __forceinline__ uint32_t RowMisalignment(const uint8_t *row)
 }
 
 // Four horizontally adjacent 8-bit pixels as raw bytes (the box filter's and the bicubic blend's row window): the
-// D dwords that hold the 4 pixels at byte offset `at` + `shift` of the row (shift 0 .. 3; 4 channels: none),
-// brought to the front: pixel k, channel c in byte k * C + c.
-template<int C, bool GUARDED>
+// D dwords that hold the 4 pixels at byte offset `at` + `shift` of the row (`at` a multiple of 4, shift 0 .. 3; 4 channels:
+// any, none), brought to the front: pixel k, channel c in byte k * C + c.
+// ODD: rows may start at other places than dwords of memory. Loads counted from an odd row are not dword aligned, and the
+// vector memory path takes those apart (32 x 1921 x 1081 -> 1280 x 720, box filter: 137 us counted from the row, 78 us from the
+// dword of memory); finding that dword costs two vector and a few scalar instructions per row, which images whose rows are
+// aligned do without (64 x 256 x 256 u8x3 -> 224 x 224 bicubic 15.9 us with them, 14.0 without; 16 x 720p -> 1080p u8x1 50.3
+// and 46.9). The launch chooses (RowsAreOdd): one kernel that holds both forms takes the registers of the larger (16 x 1080p
+// -> 1000 x 500 u8x1, box filter: 22.4 us, 31.3 in one kernel).
+template<int C, bool GUARDED, bool ODD>
 __device__ __forceinline__ void LoadQuadWindow(const uint8_t *row, uint32_t at, uint32_t shift, bool lastRow, uint32_t rowBytes,
                                                uint32_t (&r)[C])
 {
@@ -261,26 +267,33 @@ __device__ __forceinline__ void LoadQuadWindow(const uint8_t *row, uint32_t at, 
     }
     else
     {
-        // From the dword of memory that holds the first byte, whatever the row's address (wave-uniform): loads counted from
-        // an odd row are not dword aligned, and the vector memory path takes those apart (32 x 1921 x 1081 -> 1280 x 720,
-        // box filter: 137 us counted from the row, 78 us so; 1920 x 1080 takes 61-63 us either way).
-        // The load runs up to 4 bytes past the window, harmless except behind the image's last row, where it is
-        // counted from the row and moved back to end with it (GUARDED: the rows passed may include that one).
-        const bool     guard = GUARDED && lastRow;
-        const uint32_t mis = guard ? 0u : RowMisalignment(row), o = at + shift + mis;
-        uint32_t       from = o & ~3u;
-        if (GUARDED)
+        // the load runs up to 4 bytes past the window, harmless except behind the image's last row, where it is counted
+        // from the row and moved back to end with it (GUARDED: the rows passed may include that one)
+        bool whole = false;
+        if (GUARDED && lastRow) // wave-uniform
         {
-            from = lastRow ? min(from, rowBytes - 4 * D) : from;
+            const uint32_t back = min(at, rowBytes - 4 * D);
+            shift += at - back; // up to 4
+            at    = back;
+            whole = shift == 4;
+            shift = whole ? 0 : shift;
         }
-        const Window   w     = *reinterpret_cast<const Window *>(row - mis + from);
-        const uint32_t sh    = o - from; // 4 at most, and only if moved back
-        const bool     whole = GUARDED && sh == 4;
+        else if constexpr (ODD)
+        {
+            const uint32_t mis = RowMisalignment(row);
+            shift += at + mis; // (its low two bits count)
+            at    = shift & ~3u;
+            row -= mis;
+        }
+        const Window w = *reinterpret_cast<const Window *>(row + at);
 #pragma unroll
         for (int i = 0; i < C; ++i)
         {
-            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], sh);
-            r[i] = whole ? w.d[i + 1] : r[i];
+            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], shift);
+            if constexpr (GUARDED)
+            {
+                r[i] = whole ? w.d[i + 1] : r[i];
+            }
         }
     }
 }
@@ -926,7 +939,7 @@ __device__ __forceinline__ float ReadLane(float v, int lane)
 // The 8-bit bicubic sum of one output pixel per lane: rows y0 .. y0 + 3 (clamped into the image), their windows of 4
 // pixels at `at` + `shift`, the packed horizontal weights and the vertical ones times 2^-14 (wave-uniform). All four
 // windows are requested before the first sum.
-template<int C, bool GUARDED>
+template<int C, bool GUARDED, bool ODD>
 __device__ __forceinline__ uint32_t CubicRowsQ14(const Plane &p, int y0, uint32_t at, uint32_t shift, uint32_t rowBytes,
                                                  uint32_t w01, uint32_t w23, const float (&wy)[4])
 {
@@ -937,7 +950,7 @@ __device__ __forceinline__ uint32_t CubicRowsQ14(const Plane &p, int y0, uint32_
     {
         const int      yy   = GUARDED ? max(0, min(y0 + j, p.srcH - 1)) : y0 + j;
         const uint8_t *line = GUARDED ? p.src + (int64_t)yy * p.srcRow : first + (int64_t)j * p.srcRow;
-        LoadQuadWindow<C, GUARDED>(line, at, shift, yy == p.srcH - 1, rowBytes, r[j]);
+        LoadQuadWindow<C, GUARDED, ODD>(line, at, shift, yy == p.srcH - 1, rowBytes, r[j]);
     }
     float acc[C];
 #pragma unroll
@@ -964,7 +977,7 @@ __device__ __forceinline__ uint32_t CubicRowsQ14(const Plane &p, int y0, uint32_
 // lie inside the image, clear of its last row: the N source rows from y0 on are loaded once, each row's sums are
 // formed once, and each pixel adds its own four in ascending order - the sums and their order are those of
 // CubicRowsQ14, so the result is the same bit for bit. At scale 1.5 that is 5 or 6 row sums where two pixels took 8.
-template<int C, int N>
+template<int C, int N, bool ODD>
 __device__ __forceinline__ void CubicRowPairQ14(const Plane &p, int y0, uint32_t at, uint32_t shift, uint32_t rowBytes,
                                                 uint32_t w01, uint32_t w23, const float (&wyA)[4], const float (&wyB)[4],
                                                 uint32_t (&out)[2])
@@ -974,7 +987,7 @@ __device__ __forceinline__ void CubicRowPairQ14(const Plane &p, int y0, uint32_t
 #pragma unroll
     for (int j = 0; j < N; ++j)
     {
-        LoadQuadWindow<C, false>(first + (int64_t)j * p.srcRow, at, shift, false, rowBytes, r[j]);
+        LoadQuadWindow<C, false, ODD>(first + (int64_t)j * p.srcRow, at, shift, false, rowBytes, r[j]);
     }
     float accA[C], accB[C];
 #pragma unroll
@@ -1031,7 +1044,7 @@ __device__ __forceinline__ CubicColumnQ14 CubicColumn(const AxisTerms<4> &col)
 // already in units of 2^-14) of the 8-bit bicubic form, clear of the image's last row: output rows in pairs that
 // share the source rows between their windows (wave-uniform choice by how far the windows are apart; farther than
 // 2: one by one).
-template<int C>
+template<int C, bool ODD>
 __device__ __forceinline__ void CubicPatchPairsQ14(const Plane &p, const AxisTerms<4> &col, const AxisTerms<4> &rows,
                                                    uint32_t (&q)[4])
 {
@@ -1045,20 +1058,20 @@ __device__ __forceinline__ void CubicPatchPairsQ14(const Plane &p, const AxisTer
         uint32_t   two[2];
         if (apart == 1)
         {
-            CubicRowPairQ14<C, 5>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w, rowB.w, two);
+            CubicRowPairQ14<C, 5, ODD>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w, rowB.w, two);
         }
         else if (apart == 2)
         {
-            CubicRowPairQ14<C, 6>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w, rowB.w, two);
+            CubicRowPairQ14<C, 6, ODD>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w, rowB.w, two);
         }
         else if (apart == 0)
         {
-            CubicRowPairQ14<C, 4>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w, rowB.w, two);
+            CubicRowPairQ14<C, 4, ODD>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w, rowB.w, two);
         }
         else
         {
-            two[0] = CubicRowsQ14<C, false>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w);
-            two[1] = CubicRowsQ14<C, false>(p, rowB.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowB.w);
+            two[0] = CubicRowsQ14<C, false, ODD>(p, rowA.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowA.w);
+            two[1] = CubicRowsQ14<C, false, ODD>(p, rowB.s - 1, cq.at, cq.shift, rb, cq.w01, cq.w23, rowB.w);
         }
         q[k]     = two[0];
         q[k + 1] = two[1];
@@ -1069,7 +1082,7 @@ __device__ __forceinline__ void CubicPatchPairsQ14(const Plane &p, const AxisTer
 // be among the rows read, so every tap load tests for it (its loads must not run past the image's end); the caller
 // settles that once per wave patch, because a wave-uniform test in front of a load keeps the compiler from requesting
 // the next load before this one has returned.
-template<class T, int C, int INTERP, bool VARSHAPE, bool GUARDED>
+template<class T, int C, int INTERP, bool VARSHAPE, bool GUARDED, bool ODD>
 __device__ __forceinline__ Pixel<T, C> SampleWide(const Plane &p, const AxisTerms<kWeights<INTERP>> &col,
                                                   const AxisTerms<kWeights<INTERP>> &row)
 {
@@ -1130,7 +1143,7 @@ __device__ __forceinline__ Pixel<T, C> SampleWide(const Plane &p, const AxisTerm
         // (the column's part of this does not depend on the row and is computed once per lane)
         const CubicColumnQ14 cq = CubicColumn<C>(col);
         // rows row.s - 1 .. row.s + 2, inside the image for sources of 4 rows and more; four windows together
-        const uint32_t q = CubicRowsQ14<C, GUARDED>(p, row.s - 1, cq.at, cq.shift, (uint32_t)rowBytes, cq.w01, cq.w23, row.w);
+        const uint32_t q = CubicRowsQ14<C, GUARDED, ODD>(p, row.s - 1, cq.at, cq.shift, (uint32_t)rowBytes, cq.w01, cq.w23, row.w);
         __builtin_memcpy(&out, &q, PB);
     }
     else
@@ -1239,7 +1252,7 @@ __device__ __forceinline__ void StoreWavePatch(const Plane &p, int x0, int y0, i
 // wave-uniform. Sampling: lane l owns column x0 + l and computes its 4 rows (the column terms are
 // shared; neighbouring lanes read neighbouring source pixels whatever the scale). Storing: after
 // the 4x4 transposes lane l owns row y0 + (l & 3), columns x0 + 4 * (l >> 2) .. + 3.
-template<class T, int C, int INTERP, bool VARSHAPE>
+template<class T, int C, int INTERP, bool VARSHAPE, bool ODD = false>
 __device__ __forceinline__ void ResizeWavePatch(const Plane &p, int x0, int y0)
 {
     constexpr int PB = sizeof(Pixel<T, C>), D = (PB + 3) / 4;
@@ -1278,7 +1291,7 @@ __device__ __forceinline__ void ResizeWavePatch(const Plane &p, int x0, int y0)
 #pragma unroll
             for (int k = 0; k < 4; ++k)
             {
-                const Pixel<T, C> out  = SampleWide<T, C, INTERP, VARSHAPE, decltype(guarded)::value>(p, col, FromLane(rows, k));
+                const Pixel<T, C> out  = SampleWide<T, C, INTERP, VARSHAPE, decltype(guarded)::value, ODD>(p, col, FromLane(rows, k));
                 uint32_t          w[D] = {};
                 __builtin_memcpy(w, &out, PB);
 #pragma unroll
@@ -1294,7 +1307,7 @@ __device__ __forceinline__ void ResizeWavePatch(const Plane &p, int x0, int y0)
         }
         else if constexpr (INTERP == NVCV_INTERP_CUBIC && kFixedCubic<T>)
         {
-            CubicPatchPairsQ14<C>(p, col, rows, q[0]);
+            CubicPatchPairsQ14<C, ODD>(p, col, rows, q[0]);
         }
         else
         {
@@ -1391,12 +1404,10 @@ __device__ __forceinline__ void CubicRowSumsQ14(const RawQuadWindow<C> &w, uint3
 // A strip takes this form when its windows advance as said from each output row to the next and stay clear of the
 // image's last row; others (the image's top and bottom, other scales) go one output row at a time with guarded
 // loads. The launch requires sources wide enough for the window loads (16 bytes a row, 8 for one channel).
-// ODD: the source's rows need not start at dwords of memory, and each window is placed by its row's address (32 x 1921 x
-// 1081 x 3 -> 1280 x 720: 160 us with loads counted from the row, 82 us so; to 1931 x 1081 from 1281 x 721: 227 and 140).
-// That costs two vector and a few scalar instructions per row, so that aligned rows keep a form of their own (1920 x
-// 1080: 79 us, with the other 83).
+// ODD: see LoadQuadWindow (32 x 1921 x 1081 x 3 -> 1280 x 720: 160 us with loads counted from the row, 82 us so; to 1931 x 1081 from
+// 1281 x 721: 227 and 140; aligned, 1920 x 1080: 79 us, with the other form 83).
 template<int C, int S, bool ODD>
-__device__ __forceinline__ void ResizeCubicStripRowsU8(const Plane &p, int x0, int y0)
+__device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y0)
 {
     static_assert(S == 4 || S == 8);
     constexpr bool kReducing = S == 4;
@@ -1436,7 +1447,7 @@ __device__ __forceinline__ void ResizeCubicStripRowsU8(const Plane &p, int x0, i
                 const int   r     = g + k;
                 const float wy[4] = {ReadLane(wLane, 4 * r), ReadLane(wLane, 4 * r + 1), ReadLane(wLane, 4 * r + 2),
                                      ReadLane(wLane, 4 * r + 3)};
-                q[0][k] = CubicRowsQ14<C, true>(p, second(r) - 1, cq.at, cq.shift, (uint32_t)p.srcW * C, cq.w01, cq.w23, wy);
+                q[0][k] = CubicRowsQ14<C, true, ODD>(p, second(r) - 1, cq.at, cq.shift, (uint32_t)p.srcW * C, cq.w01, cq.w23, wy);
             }
             StoreWavePatch<uint8_t, C>(p, x0, y0 + g, lane, q);
         }
@@ -1568,17 +1579,6 @@ __device__ __forceinline__ void ResizeCubicStripRowsU8(const Plane &p, int x0, i
             }
         }
     }
-}
-
-template<int C, int S>
-__device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y0)
-{
-    if (C != 4 && ((reinterpret_cast<uintptr_t>(p.src) | (uint32_t)p.srcRow) & 3) != 0)
-    {
-        ResizeCubicStripRowsU8<C, S, C != 4>(p, x0, y0);
-        return;
-    }
-    ResizeCubicStripRowsU8<C, S, false>(p, x0, y0);
 }
 
 // 8-bit bilinear at horizontal scales up to 2. The cost of the wave-patch form there is the number
@@ -2592,13 +2592,13 @@ __global__ __launch_bounds__(256) void ResizeNearestStripsU8VarShapeKernel(const
 
 constexpr int kPatchTileW = 64, kPatchTileH = 16; // block = 4 waves stacked vertically
 
-template<class T, int C, int INTERP>
+template<class T, int C, int INTERP, bool ODD>
 __global__ __launch_bounds__(256) void ResizePatchTensorKernel(const ResizeArgs a, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     // blocks are 4 waves, or single waves when the whole launch is small
     const WaveTile t = WaveTileOf(flat);
-    ResizeWavePatch<T, C, INTERP, false>(p, t.x * kPatchTileW, t.y * 4);
+    ResizeWavePatch<T, C, INTERP, false, ODD>(p, t.x * kPatchTileW, t.y * 4);
 }
 
 // Which of the bicubic strip forms an image takes by its vertical scale and row length: 4 (reducing by up to 2), 8
@@ -2614,7 +2614,7 @@ __host__ __device__ __forceinline__ int CubicStripForm(int srcW, int srcH, int d
 }
 
 // Large image batches: a 64 x 64 tile per block, a strip per wave where the image's scale allows, else four patches.
-template<int C>
+template<int C, bool ODD>
 __global__ __launch_bounds__(256) void ResizeCubicStripU8VarShapeKernel(const ResizeArgs a, const VarTiles tiles)
 {
     const TileCoord tc   = LocateTile(tiles, blockIdx.x);
@@ -2623,38 +2623,38 @@ __global__ __launch_bounds__(256) void ResizeCubicStripU8VarShapeKernel(const Re
     const int       form = CubicStripForm<C>(p.srcW, p.srcH, p.dstH);
     if (form == 4)
     {
-        ResizeCubicStripU8<C, 4>(p, x0, y0);
+        ResizeCubicStripU8<C, 4, ODD>(p, x0, y0);
     }
     else if (form == 8)
     {
-        ResizeCubicStripU8<C, 8>(p, x0, y0);
+        ResizeCubicStripU8<C, 8, ODD>(p, x0, y0);
     }
     else
     {
 #pragma unroll 1
         for (int g = 0; g < kCubicStripRows; g += 4)
         {
-            ResizeWavePatch<uint8_t, C, NVCV_INTERP_CUBIC, true>(p, x0, y0 + g);
+            ResizeWavePatch<uint8_t, C, NVCV_INTERP_CUBIC, true, ODD>(p, x0, y0 + g);
         }
     }
 }
 
 // 8-bit bicubic strips: block = 4 waves stacked vertically (64 columns x 64 rows) or, reducing wide images, side by side.
-template<int C, int S>
+template<int C, int S, bool ODD>
 __global__ __launch_bounds__(256) void ResizeCubicStripU8Kernel(const ResizeArgs a, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeCubicStripU8<C, S>(p, t.x * kPatchTileW, t.y * kCubicStripRows);
+    ResizeCubicStripU8<C, S, ODD>(p, t.x * kPatchTileW, t.y * kCubicStripRows);
 }
 
-template<class T, int C, int INTERP>
+template<class T, int C, int INTERP, bool ODD>
 __global__ __launch_bounds__(256) void ResizePatchVarShapeKernel(const ResizeArgs a, const VarTiles tiles, const int flat)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
     const Plane     p  = GetPlanes<true>(a, tc.image);
     const WaveTile  t  = VarWaveTileOf(tc, flat);
-    ResizeWavePatch<T, C, INTERP, true>(p, t.x * kPatchTileW, t.y * 4);
+    ResizeWavePatch<T, C, INTERP, true, ODD>(p, t.x * kPatchTileW, t.y * 4);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2764,7 +2764,7 @@ __device__ __forceinline__ void AreaSumRows(const uint32_t (&r)[N][C], uint32_t 
     }
 }
 
-template<int C, int N, int K, bool GUARDED>
+template<int C, int N, int K, bool GUARDED, bool ODD>
 __device__ __forceinline__ void AreaFixedPixels(const uint8_t *row, int srcRow, int lastRowIn, uint32_t at, uint32_t shift,
                                                 uint32_t rowBytes, uint32_t w01, uint32_t w23, const float (&wy)[K][4],
                                                 const float (&start)[K], uint32_t (&out)[K])
@@ -2773,14 +2773,14 @@ __device__ __forceinline__ void AreaFixedPixels(const uint8_t *row, int srcRow, 
 #pragma unroll
     for (int j = 0; j < N; ++j)
     {
-        LoadQuadWindow<C, GUARDED>(row + (int64_t)j * srcRow, at, shift, j == lastRowIn, rowBytes, r[j]);
+        LoadQuadWindow<C, GUARDED, ODD>(row + (int64_t)j * srcRow, at, shift, j == lastRowIn, rowBytes, r[j]);
     }
     AreaSumRows<C, N, K>(r, w01, w23, wy, start, out);
 }
 
 // Two such pairs of output pixels (4 vertically adjacent ones) from 3 source rows each, none of them the image's last:
 // the six windows are requested together. A pair that needs only 2 rows passes a third of weight 0.
-template<int C>
+template<int C, bool ODD>
 __device__ __forceinline__ void AreaFixedTwoPairs(const uint8_t *rowA, const uint8_t *rowB, int srcRow, uint32_t at, uint32_t shift,
                                                   uint32_t rowBytes, uint32_t w01, uint32_t w23, const float (&wyA)[2][4],
                                                   const float (&wyB)[2][4], const float (&startA)[2], const float (&startB)[2],
@@ -2790,18 +2790,18 @@ __device__ __forceinline__ void AreaFixedTwoPairs(const uint8_t *rowA, const uin
 #pragma unroll
     for (int j = 0; j < 3; ++j)
     {
-        LoadQuadWindow<C, false>(rowA + (int64_t)j * srcRow, at, shift, false, rowBytes, ra[j]);
+        LoadQuadWindow<C, false, ODD>(rowA + (int64_t)j * srcRow, at, shift, false, rowBytes, ra[j]);
     }
 #pragma unroll
     for (int j = 0; j < 3; ++j)
     {
-        LoadQuadWindow<C, false>(rowB + (int64_t)j * srcRow, at, shift, false, rowBytes, rb[j]);
+        LoadQuadWindow<C, false, ODD>(rowB + (int64_t)j * srcRow, at, shift, false, rowBytes, rb[j]);
     }
     AreaSumRows<C, 3, 2>(ra, w01, w23, wyA, startA, &out[0]);
     AreaSumRows<C, 3, 2>(rb, w01, w23, wyB, startB, &out[2]);
 }
 
-template<int C, int K, bool GUARDED>
+template<int C, int K, bool GUARDED, bool ODD>
 __device__ __forceinline__ void AreaFixedRowsOf(int n, const uint8_t *row, int srcRow, int lastRowIn, uint32_t at, uint32_t shift,
                                                 uint32_t rowBytes, uint32_t w01, uint32_t w23, const float (&wy)[K][4],
                                                 const float (&start)[K], uint32_t (&out)[K])
@@ -2809,40 +2809,40 @@ __device__ __forceinline__ void AreaFixedRowsOf(int n, const uint8_t *row, int s
     // (wave-uniform)
     if (n == 3)
     {
-        AreaFixedPixels<C, 3, K, GUARDED>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
+        AreaFixedPixels<C, 3, K, GUARDED, ODD>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
     }
     else if (n == 2)
     {
-        AreaFixedPixels<C, 2, K, GUARDED>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
+        AreaFixedPixels<C, 2, K, GUARDED, ODD>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
     }
     else if (n == 4)
     {
-        AreaFixedPixels<C, 4, K, GUARDED>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
+        AreaFixedPixels<C, 4, K, GUARDED, ODD>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
     }
     else
     {
-        AreaFixedPixels<C, 1, K, GUARDED>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
+        AreaFixedPixels<C, 1, K, GUARDED, ODD>(row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
     }
 }
 
 // n source rows from `row` on; lastRowIn: which of them is the image's last row (n or more: none).
-template<int C, int K>
+template<int C, int K, bool ODD>
 __device__ __forceinline__ void AreaFixedRows(int n, const uint8_t *row, int srcRow, int lastRowIn, uint32_t at, uint32_t shift,
                                               uint32_t rowBytes, uint32_t w01, uint32_t w23, const float (&wy)[K][4],
                                               const float (&start)[K], uint32_t (&out)[K])
 {
     if (C != 4 && lastRowIn < n) // wave-uniform, once per image and column tile
     {
-        AreaFixedRowsOf<C, K, true>(n, row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
+        AreaFixedRowsOf<C, K, true, ODD>(n, row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
     }
     else
     {
-        AreaFixedRowsOf<C, K, false>(n, row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
+        AreaFixedRowsOf<C, K, false, ODD>(n, row, srcRow, lastRowIn, at, shift, rowBytes, w01, w23, wy, start, out);
     }
 }
 
 // The tile of 64 columns x 16 rows whose top left pixel is (x0, y0), both wave-uniform (y0 even).
-template<int C>
+template<int C, bool ODD>
 __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, int y0)
 {
     if (x0 >= p.dstW || y0 >= p.dstH)
@@ -2900,7 +2900,7 @@ __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, 
                 wy[1][j] = ReadLane(pw[j], i + 1);
             }
             const float start[2] = {ReadLane(rowStart, i), ReadLane(rowStart, i + 1)};
-            AreaFixedRows<C, 2>(n, p.src + (int64_t)first * p.srcRow, p.srcRow, p.srcH - 1 - first, at, shift, rowBytes, w01,
+            AreaFixedRows<C, 2, ODD>(n, p.src + (int64_t)first * p.srcRow, p.srcRow, p.srcH - 1 - first, at, shift, rowBytes, w01,
                                 w23, wy, start, two);
             out[0] = two[0];
             out[1] = two[1];
@@ -2919,7 +2919,7 @@ __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, 
                 }
                 uint32_t    one[1];
                 const float start[1] = {ReadLane(rowStart, i + k)};
-                AreaFixedRows<C, 1>(__builtin_amdgcn_readlane(ownRows, i + k), p.src + (int64_t)first * p.srcRow, p.srcRow,
+                AreaFixedRows<C, 1, ODD>(__builtin_amdgcn_readlane(ownRows, i + k), p.src + (int64_t)first * p.srcRow, p.srcRow,
                                     p.srcH - 1 - first, at, shift, rowBytes, w01, w23, wy, start, one);
                 out[k] = one[0];
             }
@@ -2947,7 +2947,7 @@ __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, 
             }
             const float startA[2] = {ReadLane(rowStart, i), ReadLane(rowStart, i + 1)};
             const float startB[2] = {ReadLane(rowStart, i + 2), ReadLane(rowStart, i + 3)};
-            AreaFixedTwoPairs<C>(p.src + (int64_t)firstA * p.srcRow, p.src + (int64_t)firstB * p.srcRow, p.srcRow, at, shift,
+            AreaFixedTwoPairs<C, ODD>(p.src + (int64_t)firstA * p.srcRow, p.src + (int64_t)firstB * p.srcRow, p.srcRow, at, shift,
                                  rowBytes, w01, w23, wyA, wyB, startA, startB, q[0]);
         }
         else
@@ -2975,15 +2975,15 @@ __device__ __forceinline__ void ResizeAreaPlainWaveTile(const Plane &p, int x0, 
     }
 }
 
-template<int C>
+template<int C, bool ODD>
 __global__ __launch_bounds__(256) void ResizeAreaFixedTensorKernel(const ResizeArgs a, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeAreaFixedWaveTile<C>(p, t.x * kAreaTileW, t.y * kAreaRowsPerWave);
+    ResizeAreaFixedWaveTile<C, ODD>(p, t.x * kAreaTileW, t.y * kAreaRowsPerWave);
 }
 
-template<int C>
+template<int C, bool ODD>
 __global__ __launch_bounds__(256) void ResizeAreaVarShapeKernel(const ResizeArgs a, const VarTiles tiles)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
@@ -2991,7 +2991,7 @@ __global__ __launch_bounds__(256) void ResizeAreaVarShapeKernel(const ResizeArgs
     const int       x0 = tc.tx * kAreaTileW, y0 = tc.ty * kAreaTileH + (threadIdx.x >> 6) * kAreaRowsPerWave;
     if (AreaFixedDomain(p.scaleX, p.scaleY, p.srcW * C, p.srcH))
     {
-        ResizeAreaFixedWaveTile<C>(p, x0, y0);
+        ResizeAreaFixedWaveTile<C, ODD>(p, x0, y0);
     }
     else
     {
@@ -3710,6 +3710,21 @@ __global__ __launch_bounds__(256) void ResizeLinearRowsKernel(const ResizeArgs a
     }
 }
 
+// Whether rows of the sources start at other places than dwords of memory, where a kernel has a form for that
+// (LoadQuadWindow): any row of a tensor, any image of a batch.
+template<int C>
+bool RowsAreOdd(const ResizeArgs &a)
+{
+    return C != 4 && ((reinterpret_cast<uintptr_t>(a.srcBase) | (uint64_t)a.srcSampleStride | (uint32_t)a.srcRowStride) & 3) != 0;
+}
+
+template<int C>
+bool RowsAreOdd(const NVCVImageBufferStrided *src, int count)
+{
+    return C != 4 && std::any_of(src, src + count, [](const NVCVImageBufferStrided &i)
+                                 { return ((reinterpret_cast<uintptr_t>(i.planes[0].basePtr) | (uint32_t)i.planes[0].rowStride) & 3) != 0; });
+}
+
 // Which (type, channels, interpolation) run as wave patches.
 template<class T, int C, int INTERP>
 constexpr bool kPatchForm = INTERP != NVCV_INTERP_AREA && sizeof(Pixel<T, C>) <= 8;
@@ -3776,7 +3791,8 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         if (AreaFixedDomain(a.scaleX, a.scaleY, a.srcW * C, a.srcH))
         {
             const bool flat = FlatBlocks(a.dstW, kAreaTileW);
-            hipLaunchKernelGGL((ResizeAreaFixedTensorKernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, kAreaRowsPerWave, flat),
+            auto kernel = RowsAreOdd<C>(a) ? ResizeAreaFixedTensorKernel<C, C != 4> : ResizeAreaFixedTensorKernel<C, false>;
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, kAreaRowsPerWave, flat),
                                dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeAreaFixedTensorKernel");
             return;
@@ -3824,14 +3840,10 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         {
             const bool flat = form == 4 && FlatBlocks(a.dstW, kPatchTileW); // (enlarging: stacked, see WaveTileOf)
             const dim3 sgrid = WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, kCubicStripRows, flat);
-            if (form == 4)
-            {
-                hipLaunchKernelGGL((ResizeCubicStripU8Kernel<C, 4>), sgrid, dim3(256), 0, stream, a, (int)flat);
-            }
-            else
-            {
-                hipLaunchKernelGGL((ResizeCubicStripU8Kernel<C, 8>), sgrid, dim3(256), 0, stream, a, (int)flat);
-            }
+            const bool odd = RowsAreOdd<C>(a);
+            auto kernel = form == 4 ? (odd ? ResizeCubicStripU8Kernel<C, 4, C != 4> : ResizeCubicStripU8Kernel<C, 4, false>)
+                                    : (odd ? ResizeCubicStripU8Kernel<C, 8, C != 4> : ResizeCubicStripU8Kernel<C, 8, false>);
+            hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeCubicStripU8Kernel");
             return;
         }
@@ -3860,7 +3872,9 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         const int64_t blocks = (int64_t)DivUp(a.dstW, kPatchTileW) * DivUp(a.dstH, kPatchTileH) * N;
         const int     waves  = blocks < 8 * 256 ? 1 : 4;
         const bool    flat   = waves == 4 && FlatBlocks(a.dstW, kPatchTileW);
-        hipLaunchKernelGGL((ResizePatchTensorKernel<T, C, INTERP>), WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, 4, flat, waves),
+        constexpr bool kOdd   = INTERP == NVCV_INTERP_CUBIC && kFixedCubic<T> && C != 4;
+        auto           kernel = kOdd && RowsAreOdd<C>(a) ? ResizePatchTensorKernel<T, C, INTERP, kOdd> : ResizePatchTensorKernel<T, C, INTERP, false>;
+        hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, 4, flat, waves),
                            dim3(64 * waves), 0, stream, a, (int)flat);
         CheckLaunch("ResizePatchTensorKernel");
         return;
@@ -3938,7 +3952,8 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
             int total = BuildVarTiles(tiles, dstHost, first, count, kAreaTileW, kAreaTileH);
             if (total > 0)
             {
-                hipLaunchKernelGGL((ResizeAreaVarShapeKernel<C>), dim3(total), dim3(256), 0, stream, a, tiles);
+                auto kernel = RowsAreOdd<C>(srcHost + first, count) ? ResizeAreaVarShapeKernel<C, C != 4> : ResizeAreaVarShapeKernel<C, false>;
+                hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a, tiles);
                 CheckLaunch("ResizeAreaVarShapeKernel");
             }
             continue;
@@ -3975,7 +3990,9 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
             int total = 2 * stripPixels > allPixels ? BuildVarTiles(tiles, dstHost, first, count, kPatchTileW, 4 * kCubicStripRows) : 0;
             if (total >= 8 * 256)
             {
-                hipLaunchKernelGGL((ResizeCubicStripU8VarShapeKernel<C>), dim3(total), dim3(256), 0, stream, a, tiles);
+                auto kernel = RowsAreOdd<C>(srcHost + first, count) ? ResizeCubicStripU8VarShapeKernel<C, C != 4>
+                                                                    : ResizeCubicStripU8VarShapeKernel<C, false>;
+                hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a, tiles);
                 CheckLaunch("ResizeCubicStripU8VarShapeKernel");
                 continue;
             }
@@ -3986,7 +4003,10 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
             int        total = buildTiles(kPatchTileW, 4, flat);
             if (total > 0)
             {
-                hipLaunchKernelGGL((ResizePatchVarShapeKernel<T, C, INTERP>), dim3(total), dim3(256), 0, stream, a,
+                constexpr bool kOdd   = INTERP == NVCV_INTERP_CUBIC && kFixedCubic<T> && C != 4;
+                auto           kernel = kOdd && RowsAreOdd<C>(srcHost + first, count) ? ResizePatchVarShapeKernel<T, C, INTERP, kOdd>
+                                                                                      : ResizePatchVarShapeKernel<T, C, INTERP, false>;
+                hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a,
                                    tiles, (int)flat);
                 CheckLaunch("ResizePatchVarShapeKernel");
             }
