@@ -23,7 +23,7 @@
 //    produces vertically adjacent rows in pairs from the source rows they share;
 //  * AREA of 8-bit tensors at larger reductions: one lane per output pixel, a row of its box in one window, rows in
 //    batches;
-//  * bilinear one-channel float tensors whose rows are not reduced, launches of 512 blocks and more: whole rows
+//  * bilinear one-channel float tensors whose rows are not reduced, launches of 704 blocks and more: whole rows
 //    gathered in LDS and written out on 64-byte boundaries;
 //  * AREA of float tensors at reductions: a wave sums the rows of 64 boxes column by column, then each lane its box's
 //    columns (ResizeAreaFloatKernel);
@@ -3617,6 +3617,8 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
 // 53.5 us, cached stores, which the L2 merges to 3.13 M requests, 79 us (they evict the source rows).
 constexpr int kRowsPerGroup = 4;
 
+constexpr int kLdsBytes = 163840; // of a CU
+
 // Source rows from the first on that kRowsPerGroup output rows span, 3 to 5; 0: more than 5 (rows reduced). A place is
 // a rounded product and a rounded difference, each off by at most 2^-11 below 8192: two of them by less than the margin.
 static inline int LinearRowsSources(const ResizeArgs &a)
@@ -3873,10 +3875,19 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         const int groups = chunks >= 3 ? 1 : chunks == 2 ? 2 : 4;
         const int lds = (groups * kRowsPerGroup * (((a.dstW + 15) & ~15) + 16) + 16) * 4;
         const dim3 rgrid(DivUp(a.dstH, groups * kRowsPerGroup), N);
-        // Two blocks and more per CU: below that the wave patches spread further (one 513 x 289 -> 1917 x 1079, 270 blocks:
-        // 5.3 us as patches, 6.3 as rows; 4 x 1280 x 720 -> 1281 x 722, 724 blocks: 8.9 and 8.5). Rows of up to 4000 floats:
-        // from there on the LDS holds one block per CU (4 x 1901 x 900 -> 3841 x 1922, two per CU: 45.6 and 43.2 us).
-        if (sources != 0 && a.srcW >= 2 && a.srcH >= 2 && lds <= 65536 && (int64_t)rgrid.x * N >= 512)
+        const int64_t blocks = (int64_t)rgrid.x * N;
+        // us as patches / as rows:
+        // - Close to three blocks and more per CU: below that the wave patches spread further (one 513 x 289 -> 1917 x 1079, 270
+        //   blocks: 5.3 / 6.3; 3 x 1281 x 721, 543: 7.0 / 7.9; 4 x 1026 x 578, 580: 5.9 / 6.5; 4 x 1281 x 721, 724: 8.8 / 8.2).
+        // - Rows that fill a wave's 256 columns well: 2929 x 64 x 64 18.0 / 29.7; 244 x 128 x 128 7.7 / 8.3, from 64 x 64 7.2 / 7.1,
+        //   732 of these 17.5 / 14.9; 156 x 160 x 160 8.4 / 7.8.
+        // - Three blocks per CU and more in the LDS (one 1080p -> 4K, two per CU: 13.2 / 19.7, 4 of these 45.6 / 49.3), and with
+        //   three no second round of blocks that is nearly empty (2 x 2560 x 1440, 720 blocks for 768 places: 12.3 / 10.6; 2 x
+        //   2816 x 1584, 792: 14.9 / 17.2; 4 of these 26.6 / 26.0).
+        const bool wide   = a.dstW >= 144 || (a.dstW >= 96 && a.dstW >= 2 * a.srcW && (int64_t)a.dstW * a.dstH * N >= 4000000);
+        const int  perCu  = kLdsBytes / lds;
+        const bool rounds = perCu >= 4 || (perCu == 3 && (blocks <= 3 * 256 || blocks >= 6 * 256));
+        if (sources != 0 && a.srcW >= 2 && a.srcH >= 2 && blocks >= 704 && wide && rounds)
         {
             auto kernel = sources == 3 ? ResizeLinearRowsKernel<3> : sources == 4 ? ResizeLinearRowsKernel<4> : ResizeLinearRowsKernel<5>;
             hipLaunchKernelGGL(kernel, rgrid, dim3(256), lds, stream, a, chunks, groups);

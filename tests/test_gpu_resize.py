@@ -478,11 +478,12 @@ def test_area_varshape(cv, K, orc, gpu, dt, c):
             assert bad.mean() <= (0.0 if (sw, sh, dw, dh) in sizes[:3] else 0.02), (sw, sh, dw, dh, bad.mean())
 
 
-# one-channel float maps whose rows are not reduced, in launches large enough for the whole-rows form: 1, 2 and 3 pieces
-# of 256 columns (4, 2 and 1 groups of 4 rows per block) with remainders, 3, 4 and 5 source rows per group, the smallest
-# source, equal heights; dense odd rows, the library's padded rows, and views whose rows start 4 bytes off
+# one-channel float maps whose rows are not reduced, in launches that take the whole-rows form and some that do not (too few
+# blocks, too narrow): 1, 2, 3 and 12 pieces of 256 columns (4, 2 and 1 groups of 4 rows per block) with remainders, 3, 4 and 5
+# source rows per group, the smallest source and the narrowest rows, equal heights; dense odd rows, the library's padded rows, and views whose rows start 4 bytes off
 @pytest.mark.parametrize("n,sw,sh,dw,dh", [(512, 2, 2, 5, 7), (300, 40, 9, 257, 21), (256, 30, 20, 256, 33), (130, 100, 13, 700, 61),
-                                           (50, 1301, 41, 1025, 41), (90, 5, 50, 513, 73), (520, 9, 5, 13, 6)])
+                                           (50, 1301, 41, 1025, 41), (90, 5, 50, 513, 73), (520, 9, 5, 13, 6),
+                                           (704, 2, 2, 145, 7), (70, 1301, 41, 1025, 41), (704, 40, 5, 97, 64), (150, 1500, 20, 3001, 41)])
 @pytest.mark.parametrize("kind", ["dense", "padded", "view"])
 def test_linear_float_maps_by_whole_rows(cv, orc, gpu, n, sw, sh, dw, dh, kind):
     src = make_input(orc, (n, sh, sw, 1), np.float32, 0xF10A + sw + dw)
