@@ -3132,6 +3132,12 @@ __global__ __launch_bounds__(256) void ResizeCubicStagedKernel(const ResizeArgs 
 // own (its place in the window differs from lane to lane); PARTIAL: the scale has such pixels. u8x3 32 x 1080p -> 320 x 180
 // 56.6 -> 38.1 us (5.4 TB/s), 16 x 4K -> 500 x 281 176.5 -> 83 us, 32 x 1080p -> 571 x 323 142 -> 77 us, one 2363 x 1415 ->
 // 355 x 153 15.9 -> 8.2 us; u8x4 16 x 4K -> 350 x 201 216 -> 117 us; u8x1 32 x 1080p -> 311 x 177 46.4 -> 24.9 us.
+// REST: the rows that are left after whole batches are a batch of their own size, instead of one that asks for its last row
+// again. Boxes whose rows are no multiple of 3 gain (4 x 720p u8x3 -> 492 x 180 7.4 -> 6.3 us, 2 x 4K u8x1 -> 549 x 1080 8.1 -> 7.0), but
+// three and four channels pay with registers, so there it is for whole vertical scales alone (64 x 396 x 300 u8x3 -> 66 x 50
+// 8.4 us without, 9.2 with it), of four channels at horizontal scales of more than 3 (64 x 400 x 296 -> 200 x 37 10.4 and 11.3; 16 x
+// 720p -> 160 x 180 11.9 and 11.2); and one channel does without it where the boxes are whole batches (16 x 720p -> 160 x 240
+// 6.2 and 6.5).
 // Those figures are with windows a pixel wider at scales between whole numbers; as the dispatch has them now, 64 x 1283 x 721
 // u8x3 -> 321 x 181 61.8 -> 52.9 us, -> 279 x 157 52.6 -> 50.1, -> 138 x 78 49.1 -> 45.0; u8x4 (48 images) 54.4 -> 46.1 us.
 constexpr float kAreaWindowMost = 12.f;
@@ -3182,7 +3188,7 @@ __device__ __forceinline__ void LoadAreaWindowGuarded(const uint8_t *row, uint32
     }
 }
 
-template<int C, int K, bool PARTIAL>
+template<int C, int K, bool PARTIAL, bool REST>
 __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a)
 {
     using Window = AreaWindow<C, K>;
@@ -3232,15 +3238,16 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
             sum[c] += (float)((q >> (8 * c)) & 0xFF) * w;
         }
     };
-#pragma unroll 1
-    for (int j0 = 0; j0 < rows; j0 += kAreaBatch)
+    // rows j0 .. j0 + B - 1
+    auto addRows = [&](auto batch, int j0)
     {
-        Window   w[kAreaBatch];
-        uint32_t shift[kAreaBatch]; // of the window's first byte in its first dword (the low two bits)
+        constexpr int B = decltype(batch)::value;
+        Window        w[B];
+        uint32_t      shift[B]; // of the window's first byte in its first dword (the low two bits)
 #pragma unroll
-        for (int b = 0; b < kAreaBatch; ++b)
+        for (int b = 0; b < B; ++b)
         {
-            const int j = min(j0 + b, rows - 1); // (a repeated row is not added)
+            const int j = REST ? j0 + b : min(j0 + b, rows - 1); // (a repeated row is not added)
             const int y = j < whole ? ymin + j : (j == whole && above ? ymin - 1 : ymax);
             const uint8_t *row = p.src + (int64_t)y * p.srcRow;
             if (y == p.srcH - 1)
@@ -3261,10 +3268,10 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
             }
         }
 #pragma unroll
-        for (int b = 0; b < kAreaBatch; ++b)
+        for (int b = 0; b < B; ++b)
         {
             const int j = j0 + b;
-            if (j >= rows)
+            if (!REST && j >= rows)
             {
                 break;
             }
@@ -3308,6 +3315,24 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
                 }
             }
         }
+    };
+    int j0 = 0;
+#pragma unroll 1
+    for (; REST ? j0 + kAreaBatch <= rows : j0 < rows; j0 += kAreaBatch)
+    {
+        addRows(std::integral_constant<int, kAreaBatch>{}, j0);
+    }
+    if constexpr (REST)
+    {
+        static_assert(kAreaBatch == 3);
+        if (rows - j0 == 2) // (uniform)
+        {
+            addRows(std::integral_constant<int, 2>{}, j0);
+        }
+        else if (rows - j0 == 1)
+        {
+            addRows(std::integral_constant<int, 1>{}, j0);
+        }
     }
     Pixel<uint8_t, C> out;
 #pragma unroll
@@ -3316,6 +3341,40 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
         out.v[c] = SaturateCast<uint8_t>(sum[c]);
     }
     StorePx<uint8_t, C>(p.dst + (int64_t)dy * p.dstRow, dx, out);
+}
+
+// The kernel whose window holds a row of boxes `s` wide.
+using AreaKernelPtr = void (*)(const ResizeArgs);
+
+template<int C, bool PARTIAL, bool REST>
+AreaKernelPtr AreaWindowKernel(float s)
+{
+    return s <= 4.f   ? ResizeAreaWindowKernel<C, 4, PARTIAL, REST>
+         : s <= 5.f   ? ResizeAreaWindowKernel<C, 5, PARTIAL, REST>
+         : s <= 6.f   ? ResizeAreaWindowKernel<C, 6, PARTIAL, REST>
+         : s <= 8.f   ? ResizeAreaWindowKernel<C, 8, PARTIAL, REST>
+         : s <= 10.f  ? ResizeAreaWindowKernel<C, 10, PARTIAL, REST>
+                      : ResizeAreaWindowKernel<C, 12, PARTIAL, REST>;
+}
+
+// Where one lane per output pixel that walks its box is still the faster form: it reads four pixels per load, so boxes up to 2
+// wide are one load a row, and boxes 4 and 8 wide have no rest. Its waves also hold fewer registers, which counts in large
+// launches. us by pixels / by windows: boxes up to 2 wide and few rows high, 16 x 720p -> 853 x 180 u8x3 22.3 / 24.5, u8x4 21.8 / 26.7
+// (one 640 x 480 of these, 210 blocks, 4.8 / 4.5 and 4.3 / 3.8; 4 x 720p u8x3 -> 674 x 225 9.5 / 8.9; 2 x 4K u8x4 -> 2258 x 240, 9 rows,
+// 22.5 / 21.6); 4 wide, 16 x 720p -> 320 x 180 u8x3 9.6 / 10.4, -> 320 x 90 9.0 / 10.4, -> 320 x 288 11.0 / 11.1 (90 blocks, one 640 x
+// 480 -> 160 x 120, 3.4 / 3.4); 8 wide, one 1080p -> 240 x 540 u8x3 3.4 / 4.0, u8x4 3.1 / 3.5, 16 x 720p -> 160 x 360 u8x4 13.0 / 11.7.
+// One channel has no such sizes.
+template<int C>
+bool AreaPixelsAreFasterU8(const ResizeArgs &a, int64_t blocks)
+{
+    const float sx = a.scaleX, sy = a.scaleY;
+    if (C == 3)
+    {
+        return (sx < 2.f && sx * sy <= 6.5f && blocks >= 4096)
+            || (sx == 4.f && blocks >= 512 && (sy <= 2.f || sy >= 3.5f) && (sy <= 5.f || blocks >= 1360))
+            || ((sx == 8.f || sx == 12.f) && sy <= 2.f && blocks >= 256);
+    }
+    return C == 4 && ((sx <= 2.f && sx * sy <= 8.5f && blocks >= 1024) || (sx == 8.f && sy == 2.f && blocks >= 256 && blocks < 1024));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -3821,20 +3880,18 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     if constexpr (kAreaFixed<T, C, INTERP>)
     {
         // Wider boxes than kAreaWindowMost, enlargements and rows shorter than a window keep the one-pixel form.
-        if (a.scaleX > 1.f && a.scaleX <= kAreaWindowMost && a.scaleY > 1.f && a.srcW * C >= 64)
+        if (a.scaleX > 1.f && a.scaleX <= kAreaWindowMost && a.scaleY > 1.f && a.srcW * C >= 64
+            && !AreaPixelsAreFasterU8<C>(a, (int64_t)grid.x * grid.y * N))
         {
-            const float s = a.scaleX;
             // A box touches at most ceil(s) pixels per row besides the partial last one, which is not in the window: whole
             // scales s whole ones; between whole numbers floor(s) whole ones behind a partial first, or floor(s) + 1 without
             // one where the box's end rounds up (behind a partial first one it would have to round by more than the spacing
             // of the floats there).
-            const bool partial = std::ceil(s) != s;
-            auto       kernel  = s <= 4.f   ? (partial ? ResizeAreaWindowKernel<C, 4, true> : ResizeAreaWindowKernel<C, 4, false>)
-                               : s <= 5.f   ? (partial ? ResizeAreaWindowKernel<C, 5, true> : ResizeAreaWindowKernel<C, 5, false>)
-                               : s <= 6.f   ? (partial ? ResizeAreaWindowKernel<C, 6, true> : ResizeAreaWindowKernel<C, 6, false>)
-                               : s <= 8.f   ? (partial ? ResizeAreaWindowKernel<C, 8, true> : ResizeAreaWindowKernel<C, 8, false>)
-                               : s <= 10.f  ? (partial ? ResizeAreaWindowKernel<C, 10, true> : ResizeAreaWindowKernel<C, 10, false>)
-                                            : (partial ? ResizeAreaWindowKernel<C, 12, true> : ResizeAreaWindowKernel<C, 12, false>);
+            const bool partial = std::ceil(a.scaleX) != a.scaleX;
+            const bool wholeY  = std::ceil(a.scaleY) == a.scaleY, batches = wholeY && std::fmod(a.scaleY, (float)kAreaBatch) == 0.f;
+            const bool rest    = C == 1 ? !batches : wholeY && !batches && (C == 3 || a.scaleX > 3.f);
+            auto       kernel  = partial ? (rest ? AreaWindowKernel<C, true, true>(a.scaleX) : AreaWindowKernel<C, true, false>(a.scaleX))
+                                         : (rest ? AreaWindowKernel<C, false, true>(a.scaleX) : AreaWindowKernel<C, false, false>(a.scaleX));
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
             CheckLaunch("ResizeAreaWindowKernel");
             return;

@@ -411,6 +411,32 @@ def test_area_window_widths(cv, orc, gpu, sw, dw, c):
     np.testing.assert_array_equal(tout.numpy(), orc.resize_shipped(src, (11, dw), AREA, threads=8))
 
 
+# boxes of 4 to 11 rows: whole batches of the window form's rows, and one and two rows behind them, with partial rows and not
+@pytest.mark.parametrize("sh", [44, 55, 66, 77, 88, 99, 110, 121, 43, 56, 87, 100])
+@pytest.mark.parametrize("c,dw", [(1, 45), (3, 45), (3, 62), (4, 45), (4, 78)])
+def test_area_window_rows(cv, orc, gpu, sh, c, dw):
+    src = make_input(orc, (2, sh, 315, c), np.uint8, 0xA7 + sh)
+    tout = cv.Tensor.alloc([2, 11, dw, c], np.uint8, "NHWC")
+    cv.Resize()(None, cv.Tensor.from_numpy(src, "NHWC"), tout, AREA)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(tout.numpy(), orc.resize_shipped(src, (11, dw), AREA, threads=8))
+
+
+# boxes that are walked one lane per pixel in launches of many blocks and by windows in smaller ones: just below and at the
+# numbers of blocks where that changes (an image of 8 rows is two blocks)
+@pytest.mark.parametrize("n,sw,sh,dw,dh,c", [(255, 80, 32, 20, 8, 3), (256, 80, 32, 20, 8, 3), (680, 80, 48, 20, 8, 3),
+                                             (128, 160, 16, 20, 8, 3), (128, 240, 16, 20, 8, 3), (127, 160, 16, 20, 8, 3),
+                                             (63, 30, 832, 20, 256, 3), (64, 30, 832, 20, 256, 3), (511, 30, 40, 20, 8, 4),
+                                             (512, 30, 40, 20, 8, 4), (512, 40, 33, 20, 8, 4), (127, 160, 16, 20, 8, 4),
+                                             (128, 160, 16, 20, 8, 4), (512, 160, 16, 20, 8, 4)])
+def test_area_small_boxes_in_large_launches(cv, orc, gpu, n, sw, sh, dw, dh, c):
+    src = make_input(orc, (n, sh, sw, c), np.uint8, 0xA9 + n)
+    tout = cv.Tensor.alloc([n, dh, dw, c], np.uint8, "NHWC")
+    cv.Resize()(None, cv.Tensor.from_numpy(src, "NHWC"), tout, AREA)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(tout.numpy(), orc.resize_shipped(src, (dh, dw), AREA, threads=8))
+
+
 # the row windows of the bicubic strips, the bicubic patches and the box filter, on dense images whose rows start at every
 # byte of a dword in turn, from every start of the first: the buffer ends with the image, whose last rows are read
 @pytest.mark.parametrize("c", [3, 1])
