@@ -11,8 +11,9 @@
 //
 // Bounds: the blocks held and not in use never exceed `limit` (where one more would, others are freed to make room;
 // one larger than a quarter of it is not kept); at every synchronisation the blocks that were ready since the one
-// before and found no use are freed; when the device is out of memory, or release() is called, all of them are. Safe with any number of threads (one lock, not held across the
-// synchronisation) and streams. At the end of the process the blocks are left to the runtime, which may be gone by then.
+// before and found no use are freed; when the device is out of memory, or release() is called, all of them are. Safe with
+// any number of threads (one lock, not held across the synchronisation) and streams. At the end of the process the blocks
+// are left to the runtime, which may be gone by then.
 #ifndef NVCVAMD_BLOCKPOOL_HPP
 #define NVCVAMD_BLOCKPOOL_HPP
 

@@ -276,7 +276,9 @@ int CurrentDevice()
 
 // Waits for all of the device's work. By hipFree, which does (57 ms behind 57 ms of another stream's work, whatever the block's
 // size): hipDeviceSynchronize invalidates every graph capture of the process, also one of another thread in the relaxed or
-// thread-local mode, in which tensors may be made and dropped meanwhile.
+// thread-local mode, in which tensors may be made and dropped meanwhile. The price: hipFree also lets go of every command given
+// since the last wait, 0.65 us of host time each, which hipDeviceSynchronize does not (behind 128 launches 111 against 29 us; four
+// operators that allocate their results 47.7 -> 48.9 us a pass, an image batch made for each pass 92 -> 96).
 bool SynchronizeDevice()
 {
     void *p = nullptr;
