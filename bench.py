@@ -840,7 +840,7 @@ WORKLOADS.update({k: (lambda *a, k=k: StreamMix(*a, k)) for k in StreamMix.SPECS
 # wave-instruction per CU and cycle; "vmem-issue": the texture addresser is busy for most of the launch (gathers and
 # loads that are not dword aligned cost cache accesses, not bytes); "launch-latency": the launch floor plus one ramp
 # of memory latency is more than half of the time (batch 8).
-BOUNDS = {"warp-affine-varshape": "valu-issue", "warp-affine-tensor-linear": "valu-issue",
+BOUNDS = {"warp-affine-varshape": "valu-issue", "warp-affine-tensor-linear": "vmem-issue",
           "warp-affine-tensor-cubic": "valu-issue", "warp-affine-tensor-nearest": "vmem-issue",
           "resize-area-720p": "valu-issue", "resize-cubic-720p": "valu-issue", "cvtcolor-bgr2hsv": "valu-issue",
           "resize-linear-720p": "valu-issue", "resize-linear-upscale": "valu-issue", "resize-cubic-upscale": "valu-issue",

@@ -581,7 +581,8 @@ __device__ __forceinline__ const uint8_t *UniformRow(const uint8_t *row)
 // the kernel had a fifth more vector instructions (bilinear; bicubic a ninth). Single-channel taps, which had been fetched as
 // 2- and 4-byte loads at any address, gain most, by the loads: one that is not dword aligned is taken apart (a gather of
 // u8x3 pixel pairs: 31 against 22 cycles per wave). 24 x 1283 x 721 u8x1 bilinear 54.3 -> 43.0 us, bicubic 131.3 -> 100.7;
-// 16 x 1280 x 720 u8x3 bicubic 68.4 -> 64.6, bilinear 30.1 -> 29.2 (its gathers and their latency are left).
+// 16 x 1280 x 720 u8x3 bicubic 68.4 -> 64.6, bilinear 30.1 -> 29.2 (which the L1 accesses of its gathers
+// bound now: 54 us of the 63 that 32 x 1280 x 780 take, against 45 of issue).
 template<int C, int TAPS, int ROWS, bool SAME>
 __device__ __forceinline__ void LoadTapRows(const Img &im, int x, int y, int x0, int y0, uint32_t (&r)[ROWS][(C * TAPS + 3) / 4])
 {
