@@ -269,27 +269,19 @@ __device__ __forceinline__ void LoadQuadWindow(const uint8_t *row, uint32_t at, 
     {
         // the load runs up to 4 bytes past the window, harmless except behind the image's last row, where it is counted
         // from the row and moved back to end with it (GUARDED: the rows passed may include that one)
-        bool whole = false;
-        if (GUARDED && lastRow) // wave-uniform
-        {
-            const uint32_t back = min(at, rowBytes - 4 * D);
-            shift += at - back; // up to 4
-            at    = back;
-            whole = shift == 4;
-            shift = whole ? 0 : shift;
-        }
-        else if constexpr (ODD)
-        {
-            const uint32_t mis = RowMisalignment(row);
-            shift += at + mis; // (its low two bits count)
-            at    = shift & ~3u;
-            row -= mis;
-        }
-        const Window w = *reinterpret_cast<const Window *>(row + at);
+        // (wave-uniform, but without a branch: with one the compiler kept the places of all of a pixel's rows, 117 registers
+        // for 61)
+        const bool     guard = GUARDED && lastRow;
+        const uint32_t mis   = ODD && !guard ? RowMisalignment(row) : 0u, o = at + shift + mis;
+        uint32_t       from  = ODD ? o & ~3u : at;
+        from                 = guard ? min(from, rowBytes - 4 * D) : from;
+        const Window   w     = *reinterpret_cast<const Window *>(row - mis + from);
+        const uint32_t sh    = GUARDED ? o - from : ODD ? o : shift; // (its low two bits count; 4 only if moved back)
+        const bool     whole = GUARDED && sh == 4;
 #pragma unroll
         for (int i = 0; i < C; ++i)
         {
-            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], shift);
+            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], sh);
             if constexpr (GUARDED)
             {
                 r[i] = whole ? w.d[i + 1] : r[i];
