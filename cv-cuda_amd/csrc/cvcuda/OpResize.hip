@@ -3349,6 +3349,21 @@ AreaKernelPtr AreaWindowKernel(float s)
                       : ResizeAreaWindowKernel<C, 12, PARTIAL, REST>;
 }
 
+// Whether rows of the sources start at other places than dwords of memory, where a kernel has a form for that
+// (LoadQuadWindow): any row of a tensor, any image of a batch.
+template<int C>
+bool RowsAreOdd(const ResizeArgs &a)
+{
+    return C != 4 && ((reinterpret_cast<uintptr_t>(a.srcBase) | (uint64_t)a.srcSampleStride | (uint32_t)a.srcRowStride) & 3) != 0;
+}
+
+template<int C>
+bool RowsAreOdd(const NVCVImageBufferStrided *src, int count)
+{
+    return C != 4 && std::any_of(src, src + count, [](const NVCVImageBufferStrided &i)
+                                 { return ((reinterpret_cast<uintptr_t>(i.planes[0].basePtr) | (uint32_t)i.planes[0].rowStride) & 3) != 0; });
+}
+
 // Where one lane per output pixel that walks its box is still the faster form: it reads four pixels per load, so boxes up to 2
 // wide are one load a row, and boxes 4 and 8 wide have no rest. Its waves also hold fewer registers, which counts in large
 // launches. us by pixels / by windows: boxes up to 2 wide and few rows high, 16 x 720p -> 853 x 180 u8x3 22.3 / 24.5, u8x4 21.8 / 26.7
@@ -3360,7 +3375,8 @@ template<int C>
 bool AreaPixelsAreFasterU8(const ResizeArgs &a, int64_t blocks)
 {
     const float sx = a.scaleX, sy = a.scaleY;
-    if (C == 3)
+    // (pixels of odd rows are not read four at a time at dwords: 16 x 1080p u8x3 -> 480 x 272 25.8 us, by windows 23.3)
+    if (C == 3 && !RowsAreOdd<C>(a))
     {
         return (sx < 2.f && sx * sy <= 6.5f && blocks >= 4096)
             || (sx == 4.f && blocks >= 512 && (sy <= 2.f || sy >= 3.5f) && (sy <= 5.f || blocks >= 1360))
@@ -3779,21 +3795,6 @@ __global__ __launch_bounds__(256) void ResizeLinearRowsKernel(const ResizeArgs a
             }
         }
     }
-}
-
-// Whether rows of the sources start at other places than dwords of memory, where a kernel has a form for that
-// (LoadQuadWindow): any row of a tensor, any image of a batch.
-template<int C>
-bool RowsAreOdd(const ResizeArgs &a)
-{
-    return C != 4 && ((reinterpret_cast<uintptr_t>(a.srcBase) | (uint64_t)a.srcSampleStride | (uint32_t)a.srcRowStride) & 3) != 0;
-}
-
-template<int C>
-bool RowsAreOdd(const NVCVImageBufferStrided *src, int count)
-{
-    return C != 4 && std::any_of(src, src + count, [](const NVCVImageBufferStrided &i)
-                                 { return ((reinterpret_cast<uintptr_t>(i.planes[0].basePtr) | (uint32_t)i.planes[0].rowStride) & 3) != 0; });
 }
 
 // Which (type, channels, interpolation) run as wave patches.
