@@ -574,20 +574,29 @@ __device__ __forceinline__ const uint8_t *UniformRow(const uint8_t *row)
     return AsGlobal(reinterpret_cast<const uint8_t *>(at));
 }
 
+// How the taps of a row are read: windows whose rows' addresses differ in their low two bits, or agree in them (a row pitch
+// of whole dwords); or a load of the taps alone at any address (single-channel pixels, see NarrowTapsPay).
+enum RowForm
+{
+    kOddRows,
+    kSameRows,
+    kNarrowTaps
+};
+
 // The rows y .. y + ROWS - 1 of a u8 image, from pixel x on (TAPS pixels, all inside the image), as raw bytes: r[j] holds row
 // j's. Per sample this is two multiply-adds for the offset, whose start (uniform) takes in what is added to x and y, and, where
-// the rows' addresses agree in their low two bits (SAME: a row pitch of whole dwords), one mask: a row's address is its own
+// the rows' addresses agree in their low two bits, one mask: a row's address is its own
 // uniform base plus that one offset. Written with the compiler's choice of instructions and the row pitch added per lane,
 // the kernel had a fifth more vector instructions (bilinear; bicubic a ninth). Single-channel taps, which had been fetched as
 // 2- and 4-byte loads at any address, gain most, by the loads: one that is not dword aligned is taken apart (a gather of
 // u8x3 pixel pairs: 31 against 22 cycles per wave). 24 x 1283 x 721 u8x1 bilinear 54.3 -> 43.0 us, bicubic 131.3 -> 100.7;
 // 16 x 1280 x 720 u8x3 bicubic 68.4 -> 64.6, bilinear 30.1 -> 29.2 (which the L1 accesses of its gathers
 // bound now: 54 us of the 63 that 32 x 1280 x 780 take, against 45 of issue).
-template<int C, int TAPS, int ROWS, bool SAME>
+template<int C, int TAPS, int ROWS, int FORM>
 __device__ __forceinline__ void LoadTapRows(const Img &im, int x, int y, int x0, int y0, uint32_t (&r)[ROWS][(C * TAPS + 3) / 4])
 {
     constexpr int  N       = (C * TAPS + 3) / 4;
-    constexpr bool kWindow = kWideTapLoads<uint8_t, C> && C * TAPS > 1;
+    constexpr bool kWindow = kWideTapLoads<uint8_t, C> && C * TAPS > 1 && FORM != kNarrowTaps, SAME = FORM == kSameRows;
     constexpr int  kLoad   = kWindow ? (C * TAPS + 3 + 3) / 4 : N; // dwords that hold C * TAPS bytes at any of the 4 places
     struct alignas(4) W
     {
@@ -660,11 +669,11 @@ __device__ __forceinline__ uint32_t BlendCubicQ14(const uint32_t (&r)[4][C], flo
 }
 
 // The same for a sample whose 16 taps are inside the image.
-template<int C, bool SAME>
+template<int C, int FORM>
 __device__ __forceinline__ uint32_t SampleInsideCubicQ14(const Img &im, float sx, float sy)
 {
     uint32_t r[4][C];
-    LoadTapRows<C, 4, 4, SAME>(im, (int)floorf(sx), (int)floorf(sy), -1, -1, r);
+    LoadTapRows<C, 4, 4, FORM>(im, (int)floorf(sx), (int)floorf(sy), -1, -1, r);
     return BlendCubicQ14<C>(r, sx, sy);
 }
 
@@ -672,7 +681,7 @@ __device__ __forceinline__ uint32_t SampleInsideCubicQ14(const Img &im, float sx
 // coordinates are not negative and below 2^16, given in units of 2^-15 pixel: floor and fraction come
 // from one float -> integer conversion, the taps of a row from one window, the two taps of a channel
 // from one byte permute. Returns the pixel's dword.
-template<int C, bool SAME>
+template<int C, int FORM>
 __device__ __forceinline__ uint32_t SampleInsideQ15(const Img &im, float sx, float sy)
 {
     const uint32_t X = (uint32_t)(int)sx, Y = (uint32_t)(int)sy;
@@ -684,7 +693,7 @@ __device__ __forceinline__ uint32_t SampleInsideQ15(const Img &im, float sx, flo
     asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(top) : "v"(ax), "s"(65535u), "v"(kQ15));
     top -= bottom;
     uint32_t r[2][(2 * C + 3) / 4];
-    LoadTapRows<C, 2, 2, SAME>(im, (int)(X >> 15), (int)(Y >> 15), 0, 0, r);
+    LoadTapRows<C, 2, 2, FORM>(im, (int)(X >> 15), (int)(Y >> 15), 0, 0, r);
     uint32_t q = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c)
@@ -947,22 +956,22 @@ __device__ __forceinline__ uint32_t SampleNearBorderNearest(const Img &im, const
 
 // The dwords of the pixel that SampleInside gives; what lies above the pixel's bytes is not looked at. u8 channels are
 // rounded, saturated and placed into their byte by one instruction each (v_cvt_pk_u8_f32 with a byte select and the dword
-// so far), where packing converted bytes takes as many shifts and merges again. SAME: see LoadTapRows.
-template<class T, int C, int INTERP, bool SAME>
+// so far), where packing converted bytes takes as many shifts and merges again. FORM: see LoadTapRows.
+template<class T, int C, int INTERP, int FORM>
 __device__ __forceinline__ void SampleInsidePacked(const Img &im, float sx, float sy, uint32_t (&w)[(C * sizeof(T) + 3) / 4])
 {
     if constexpr (kFixedPoint<T, INTERP>)
     {
-        w[0] = SampleInsideQ15<C, SAME>(im, sx, sy);
+        w[0] = SampleInsideQ15<C, FORM>(im, sx, sy);
     }
     else if constexpr (kFixedPointCubic<T, INTERP>)
     {
-        w[0] = SampleInsideCubicQ14<C, SAME>(im, sx, sy);
+        w[0] = SampleInsideCubicQ14<C, FORM>(im, sx, sy);
     }
     else if constexpr (std::is_same_v<T, uint8_t>)
     {
         uint32_t r[1][1];
-        LoadTapRows<C, 1, 1, SAME>(im, (int)floorf(sx + .5f), (int)floorf(sy + .5f), 0, 0, r);
+        LoadTapRows<C, 1, 1, FORM>(im, (int)floorf(sx + .5f), (int)floorf(sy + .5f), 0, 0, r);
         w[0] = r[0][0];
     }
     else
@@ -1118,6 +1127,18 @@ __device__ __forceinline__ bool NearBorderForm(const Img &im, const WarpArgs &a,
     }
 }
 
+// Whether single-channel taps are read alone, at any address, and not in windows of dwords: where lanes next to each other
+// lie more along the source's columns than along its rows, and a window's second dword is another one to fetch for every
+// lane. 16 x 1280 x 720 u8x1, windows / taps alone, at 0.3 rad 30.3 / 38.0 us bilinear, at 0.65 36.1 / 37.9, at 0.8 37.5 / 35.6, at a
+// quarter turn 36.2 / 22.2 (4 x 1283 x 721, rows of odd pitch, 11.3 / 13.6, 13.2 / 12.9, 13.3 / 11.4, 11.5 / 8.5); bicubic, whose windows are
+// two dwords for four taps, at 0.8 66.5 / 77.4, at 1.0 68.2 / 59.6, at a quarter turn 67.7 / 38.4. (Below the line the taps
+// alone were measured with the row pitch added per lane.)
+template<int INTERP>
+__device__ __forceinline__ bool NarrowTapsPay(const float (&m)[9])
+{
+    return fabsf(m[3]) > (INTERP == NVCV_INTERP_LINEAR ? 1.f : 1.5f) * fabsf(m[0]);
+}
+
 // One 64 x 16 tile of the destination image `dst` (tile coordinates tx, ty), all 256 threads.
 template<class T, int C, int INTERP, bool PERSP>
 __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const float (&m)[9], uint8_t *dst, int dstRow,
@@ -1152,21 +1173,25 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     if (allInside)
     {
         uint32_t w[kPxPerLane][D];
-        if (!kWideTapLoads<T, C> || INTERP == NVCV_INTERP_NEAREST || (im.row & 3) == 0) // uniform
+        auto sample = [&](auto form)
         {
 #pragma unroll
             for (int k = 0; k < kPxPerLane; ++k)
             {
-                SampleInsidePacked<T, C, INTERP, true>(im, sx[k], sy[k], w[k]);
+                SampleInsidePacked<T, C, INTERP, decltype(form)::value>(im, sx[k], sy[k], w[k]);
             }
+        };
+        if (std::is_same_v<T, uint8_t> && C == 1 && INTERP != NVCV_INTERP_NEAREST && NarrowTapsPay<INTERP>(m)) // uniform
+        {
+            sample(std::integral_constant<int, kNarrowTaps>{});
+        }
+        else if (!kWideTapLoads<T, C> || INTERP == NVCV_INTERP_NEAREST || (im.row & 3) == 0) // uniform
+        {
+            sample(std::integral_constant<int, kSameRows>{});
         }
         else
         {
-#pragma unroll
-            for (int k = 0; k < kPxPerLane; ++k)
-            {
-                SampleInsidePacked<T, C, INTERP, false>(im, sx[k], sy[k], w[k]);
-            }
+            sample(std::integral_constant<int, kOddRows>{});
         }
 #pragma unroll
         for (int k = 0; k < kPxPerLane; ++k)
@@ -1297,7 +1322,8 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     // ---- store. Pixels of 12 and 16 bytes go through the wave's own part of LDS and leave as the rows they form, 16 bytes
     // per lane: 384 or 512 contiguous bytes of each row. One pixel per lane wrote 96 or 128 bytes of 8 rows per instruction,
     // with a partly written sector at both ends of most: 4 x 1283 x 721 f32x3 nearest 30.5 -> 19.4 us, bilinear 28.4 -> 24.3;
-    // f32x4 33.1 -> 22.0 and 30.4 -> 27.3 (of rows that start at sectors, 1280 x 720: f32x3 22.3 -> 16.6, f32x4 as before).
+    // f32x4 33.1 -> 22.0 and 30.4 -> 27.3 (of rows that start at sectors, 1280 x 720: f32x3 22.3 -> 16.6, f32x4 5 % slower when
+    // small, one 1280 x 720 5.4 -> 5.7, and as before when large; a second form of the store for these cost all others 3 to 5 %).
     if constexpr (PB >= 12)
     {
         constexpr int kChunks = kWaveW * PB / 16, kPitch = kWaveW * D + (D == 4 ? 32 : 0); // (neighbouring rows on other banks)

@@ -116,6 +116,27 @@ def test_rows_from_every_byte_of_a_dword(cv, orc, gpu, size, lead, c):
             np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((size, lead, c, interp, border, m)))
 
 
+# single-channel taps read alone where the map turns by more than 45 degrees (bicubic: 56), in windows below that, from rows that
+# start at every byte of a dword and up to the last bytes of the smallest sources
+@pytest.mark.parametrize("lead", [0, 1, 2, 3])
+@pytest.mark.parametrize("size", [(2, 2), (4, 4), (5, 9), (7, 5), (64, 40), (71, 43)], ids=lambda s: "%dx%d" % s)
+def test_single_channel_quarter_turns(cv, orc, gpu, size, lead):
+    w, h = size
+    src = orc.fill_u8((2, h, w, 1), 0x90 + w + lead)
+    buf = torch.zeros(lead + src.size, dtype=torch.uint8, device="cuda")
+    buf[lead:].copy_(torch.from_numpy(src.reshape(-1)))
+    tin = cv.Tensor.wrap(buf.data_ptr() + lead, [2, h, w, 1], [h * w, w, 1, 1], np.uint8, "NHWC", keep=buf)
+    for deg in (44.0, 46.0, 55.0, 58.0, 90.0, 133.0, 270.0):
+        for scale in (0.9, 1.7):
+            m = rotation(w, h, deg, scale)
+            for interp in (LINEAR, CUBIC):
+                tout = cv.Tensor.alloc([2, h + 3, w + 5, 1], np.uint8, "NHWC")
+                cv.WarpAffine(0)(None, tin, tout, m, interp, 1, (0, 0, 0, 0))
+                torch.cuda.synchronize()
+                dev = orc.warp(src, (h + 3, w + 5), orc.invert_affine(m), interp, 1, (0, 0, 0, 0), variant=device_variant(interp))
+                np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((deg, scale, interp)))
+
+
 # three channels under the replicating border in launches of 256 blocks and more, which take the windows next to the edge (smaller
 # ones take tap by tap): the smallest sources that have room for a window, dense rows that start at every byte of a dword
 @pytest.mark.parametrize("lead", [0, 1, 2, 3])
