@@ -834,14 +834,16 @@ __device__ __forceinline__ uint32_t SampleNearBorderCubicQ14(const Img &im, cons
 // other, which a launch that fills the chip hides and a small one waits for. One and four channels gain at any size. Three
 // channels, whose windows take the most instructions, gain under a replicating border from 256 blocks on (one 320 x 240, 75
 // blocks, 6.9 us with SampleNearBorderCubicQ14 and 8.1 with windows; one 640 x 480, 300 blocks, 9.9 and 9.2; 32 x 1280 x 780 202
-// and 158) and not under a constant one, where lanes outside the image take no part and the colour's share is work of its
-// own (one 320 x 240 6.4 and 8.0; one 1080p 14.5 and 15.6, 4 x 1283 x 721 20.5 and 22.0, 16 x 500 x 333 22.4 and 21.7, 32 x 1280 x
-// 780 113.7 and 112.5).
+// and 158), and under a constant one, where lanes outside the image take no part and the colour's share is work of its own,
+// only in large launches of small images, of which the edge is the larger part (32 x 256 x 256 20.7 and 19.3, in perspective 26.6
+// and 22.5; 16 x 500 x 333 24.4 and 23.6; but one 320 x 240 6.4 and 8.0; one 1080p 14.5 and 15.6, 4 x 1283 x 721 20.5 and 22.0, 32 x
+// 1280 x 780 113.7 and 112.5).
 template<int C>
 __device__ __forceinline__ bool ClampedCubicPays(const Img &im, bool constant)
 {
     return im.w >= 4 && __mul24(im.h - 1, im.row) + im.w * C >= 16
-        && (C != 3 || (!constant && gridDim.x * gridDim.y * gridDim.z >= 256));
+        && (C != 3 || gridDim.x * gridDim.y * gridDim.z >= (constant ? 2048u : 256u))
+        && (C != 3 || !constant || __umul24(im.w, im.h) <= 1u << 18);
 }
 
 // SampleNearBorderCubicQ14 under a constant or replicating border: 4 loads per sample instead of 16. A row is the window of

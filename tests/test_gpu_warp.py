@@ -137,23 +137,24 @@ def test_single_channel_quarter_turns(cv, orc, gpu, size, lead):
                 np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((deg, scale, interp)))
 
 
-# three channels under the replicating border in launches of 256 blocks and more, which take the windows next to the edge (smaller
-# ones take tap by tap): the smallest sources that have room for a window, dense rows that start at every byte of a dword
+# three channels under the replicating border in launches of 256 blocks and more, and under the constant one of 2048, which take the
+# windows next to the edge (smaller ones take tap by tap): the smallest sources that have room for a window, dense rows that start at every byte of a dword
 @pytest.mark.parametrize("lead", [0, 1, 2, 3])
 @pytest.mark.parametrize("size", [(4, 4), (5, 2), (7, 5), (37, 21), (70, 41)], ids=lambda s: "%dx%d" % s)
 def test_bicubic_windows_of_large_launches(cv, orc, gpu, size, lead):
-    (w, h), n, c = size, 32, 3
+    (w, h), n, c = size, 205, 3
     dw, dh = 66, 66  # 2 x 5 tiles
     src = orc.fill_u8((n, h, w, c), 0xB1C + w + lead)
     buf = torch.zeros(lead + src.size, dtype=torch.uint8, device="cuda")
     buf[lead:].copy_(torch.from_numpy(src.reshape(-1)))
     tin = cv.Tensor.wrap(buf.data_ptr() + lead, [n, h, w, c], [h * w * c, w * c, c, 1], np.uint8, "NHWC", keep=buf)
     for m in (rotation(w, h, 4.0, 1.02), [dw / w, 0.0, 0.3, 0.0, dh / h, -0.6], rotation(w, h, 21.0, 2.7)):
-        tout = cv.Tensor.alloc([n, dh, dw, c], np.uint8, "NHWC")
-        cv.WarpAffine(0)(None, tin, tout, m, CUBIC, 1, (0, 0, 0, 0))
-        torch.cuda.synchronize()
-        dev = orc.warp(src, (dh, dw), orc.invert_affine(m), CUBIC, 1, (0, 0, 0, 0), variant=device_variant(CUBIC))
-        np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str(m))
+        for border, color in ((0, (9, 200, 77, 0)), (1, (0, 0, 0, 0))):
+            tout = cv.Tensor.alloc([n, dh, dw, c], np.uint8, "NHWC")
+            cv.WarpAffine(0)(None, tin, tout, m, CUBIC, border, color)
+            torch.cuda.synchronize()
+            dev = orc.warp(src, (dh, dw), orc.invert_affine(m), CUBIC, border, color, variant=device_variant(CUBIC), threads=8)
+            np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((border, m)))
 
 
 def rotation(w, h, deg, s):
