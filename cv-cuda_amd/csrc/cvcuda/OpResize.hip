@@ -3521,8 +3521,8 @@ constexpr int AreaFloatPieces(float scaleX)
 // Boxes of few whole columns, where one lane per output pixel is still the faster form (it has no partial columns to add, and
 // neighbouring lanes' boxes fill the lines they touch). One channel, whose pixels that form reads four at a time: 24 x 720p
 // -> 320 x 180 15.0 us against 17.5 by column sums, one 4K -> 960 x 1440 8.4 and 10.5, -> 480 x 270 7.6 and 8.1 (one 720p ->
-// 160 x 90, few blocks: 4.3 and 4.1), -> 1920 x 1080 10.4 and 11.1 (4 x 720p -> 640 x 360 5.8 and 5.7). Three and four channels while the memory-side cache holds the source: f32x4 one 720p
-// -> 640 x 360 3.7 and 4.65, -> 320 x 180 4.5 and 5.2, 4 x 720p -> 640 x 553 16.1 and 17.2, but -> 320 x 480 20.5 and 16.4;
+// 160 x 90, few blocks: 4.3 and 4.1), -> 1920 x 1080 10.4 and 11.1 (4 x 720p -> 640 x 360 5.8 and 5.7). Three and four channels
+// while the memory-side cache holds the source: f32x4 one 720p -> 640 x 360 3.7 and 4.65, -> 320 x 180 4.5 and 5.2, 4 x 720p -> 640 x 553 16.1 and 17.2, but -> 320 x 480 20.5 and 16.4;
 // 24 x 720p -> 640 x 553 95.7 and 86.1; f32x3 8 x 720p -> 640 x 553 23.4 and 26.6, one 720p -> 426 x 240 4.2 and 4.3.
 template<int C>
 bool AreaPixelsAreFaster(const ResizeArgs &a, int64_t blocks, int64_t srcBytes)
@@ -3532,8 +3532,11 @@ bool AreaPixelsAreFaster(const ResizeArgs &a, int64_t blocks, int64_t srcBytes)
     {
         return s == 4.f || ((s == 5.f || s == 8.f) && blocks >= 512) || (s == 2.f && a.scaleY == 2.f && blocks >= 4096);
     }
-    // (twice as wide and more than four times as high: 480p f32x3 -> 320 x 87 3.8 and 3.5, 4 x 720p -> 640 x 130 10.0 and 10.5)
-    return s == 2.f ? srcBytes <= 128 << 20 && (a.scaleY <= 4.f || srcBytes >= 32 << 20) : (s == 3.f || s == 4.f) && srcBytes <= 16 << 20;
+    // (twice as wide and more than four times as high: 480p f32x3 -> 320 x 87 3.8 and 3.5, 4 x 720p -> 640 x 130 10.0 and 10.5;
+    // three channels and partial rows: one 720p -> 640 x 232 4.54 and 4.21, 4 x 500 x 332 -> 250 x 107 4.6 and 4.4, whole ones
+    // -> 640 x 360 3.7 and 4.06, -> 250 x 166 3.9 and 4.3)
+    const bool rows = C == 4 || a.scaleY <= 2.f || std::ceil(a.scaleY) == a.scaleY;
+    return s == 2.f ? srcBytes <= 128 << 20 && ((a.scaleY <= 4.f && rows) || srcBytes >= 32 << 20) : (s == 3.f || s == 4.f) && srcBytes <= 16 << 20;
 }
 
 using AreaFloatKernelPtr = void (*)(const ResizeArgs);
