@@ -198,6 +198,25 @@ __device__ __forceinline__ int BorderIndex(int border, int c, int s)
     }
 }
 
+// Division of numbers below 2^31 by a number known on the host, as a multiplication (Granlund and Montgomery,
+// "Division by Invariant Integers using Multiplication", 1994, figure 4.1).
+struct DivBy
+{
+    uint32_t d, mul, shift;
+
+    explicit DivBy(uint32_t by)
+        : d(by)
+        , shift(by > 1 ? 32 - (uint32_t)__builtin_clz(by - 1) : 0)
+    {
+        mul = (uint32_t)(((1ull << 32) * ((1ull << shift) - by)) / by + 1);
+    }
+
+    __device__ __forceinline__ uint32_t Quotient(uint32_t n) const
+    {
+        return (__umulhi(n, mul) + n) >> shift;
+    }
+};
+
 // MI355X hands the workgroups of a launch to its 8 XCDs round-robin (hardware id % 8) and every
 // XCD has an L2 of its own.
 constexpr uint32_t kXcdCount = 8;

@@ -29,7 +29,7 @@ namespace {
 // YUV 4:2:0 -> RGB
 constexpr int kYuvBlockW = 8;               // pixels per lane and row (a lane converts a kYuvBlockW x 2 block)
 constexpr int kYuvTileW  = 64 * kYuvBlockW; // pixels per wave and row
-constexpr int kYuvTileH  = 8;               // image batches: rows per block, 4 waves x 2 rows (tensors: 4 waves side by side)
+constexpr int kYuvTileH  = 8;               // rows per block of tiles: 4 waves x 2 rows
 
 struct YuvArgs
 {
@@ -159,6 +159,37 @@ __device__ __forceinline__ void ConvertBlock(const uint8_t *src, int srcRow, uin
     }
 }
 
+// The chroma terms and the rounding constant of YuvToRgb's three sums, once per chroma sample (4 pixels share them), already
+// in output channel order; integer addition is associative, so the results are the same.
+__device__ __forceinline__ void ChromaTerms(int uu, int vv, int bidx, int &c0, int &c1, int &c2)
+{
+    const int rC = 1673527 * vv + (1 << 19);
+    const int bC = 2116026 * uu + (1 << 19);
+    c0           = bidx == 0 ? bC : rC;
+    c1           = -852492 * vv - 409993 * uu + (1 << 19);
+    c2           = bidx == 0 ? rC : bC;
+}
+
+// kYuvBlockW pixels of one row from their lumas and the terms of their chroma samples.
+template<int DCN>
+__device__ __forceinline__ void ConvertRun(const uint8_t (&luma)[kYuvBlockW], const int (&c0)[kYuvBlockW / 2],
+                                           const int (&c1)[kYuvBlockW / 2], const int (&c2)[kYuvBlockW / 2],
+                                           uint8_t (&out)[kYuvBlockW * DCN])
+{
+#pragma unroll
+    for (int i = 0; i < kYuvBlockW; ++i)
+    {
+        const int t      = max(0, (int)luma[i] - 16) * 1220542;
+        out[i * DCN + 0] = (uint8_t)min(max((t + c0[i >> 1]) >> 20, 0), 255);
+        out[i * DCN + 1] = (uint8_t)min(max((t + c1[i >> 1]) >> 20, 0), 255);
+        out[i * DCN + 2] = (uint8_t)min(max((t + c2[i >> 1]) >> 20, 0), 255);
+        if constexpr (DCN == 4)
+        {
+            out[i * DCN + 3] = 255;
+        }
+    }
+}
+
 // A kYuvBlockW x 2 block that lies wholly inside the row (x + kYuvBlockW <= W): every access is a vector
 // of whole dwords (luma 8 bytes per row, chroma 8 or 4 + 4 bytes, 24 or 32 output bytes per row).
 template<int DCN, bool SEMIPLANAR>
@@ -197,18 +228,11 @@ __device__ __forceinline__ void ConvertWideBlock(const uint8_t *src, int srcRow,
             vv[k] = (int)pv[k] - 128;
         }
     }
-    // The chroma terms and the rounding constant of YuvToRgb's three sums, once per chroma sample (4
-    // pixels share them), already in output channel order; integer addition is associative, so the
-    // results are the same.
     int c0[NC], c1[NC], c2[NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k)
     {
-        const int rC = 1673527 * vv[k] + (1 << 19);
-        const int bC = 2116026 * uu[k] + (1 << 19);
-        c0[k]        = bidx == 0 ? bC : rC;
-        c1[k]        = -852492 * vv[k] - 409993 * uu[k] + (1 << 19);
-        c2[k]        = bidx == 0 ? rC : bC;
+        ChromaTerms(uu[k], vv[k], bidx, c0[k], c1[k], c2[k]);
     }
 #pragma unroll
     for (int ry = 0; ry < 2; ++ry)
@@ -220,18 +244,7 @@ __device__ __forceinline__ void ConvertWideBlock(const uint8_t *src, int srcRow,
         }
         uint8_t luma[BW], out[BW * DCN];
         LoadRun<uint8_t, BW>(src + (int64_t)yy * srcRow + x, luma);
-#pragma unroll
-        for (int i = 0; i < BW; ++i)
-        {
-            const int t      = max(0, (int)luma[i] - 16) * 1220542;
-            out[i * DCN + 0] = (uint8_t)min(max((t + c0[i >> 1]) >> 20, 0), 255);
-            out[i * DCN + 1] = (uint8_t)min(max((t + c1[i >> 1]) >> 20, 0), 255);
-            out[i * DCN + 2] = (uint8_t)min(max((t + c2[i >> 1]) >> 20, 0), 255);
-            if constexpr (DCN == 4)
-            {
-                out[i * DCN + 3] = 255;
-            }
-        }
+        ConvertRun<DCN>(luma, c0, c1, c2, out);
         StoreRowRunNT<uint8_t, BW * DCN>(dst + (int64_t)yy * dstRow + (int64_t)(x - lane * BW) * DCN, out, lane, lanes);
     }
 }
@@ -252,15 +265,143 @@ __device__ __forceinline__ void ConvertLaneBlock(const uint8_t *src, int srcRow,
     }
 }
 
+// Tensors. The 8 x 2 blocks of an image are numbered row pair by row pair and dealt to the lanes in that order, whatever the
+// width: a wave goes on in the next pair of rows where one ends. The last block of a row whose width is no multiple of 8
+// starts at W - 8 and writes the pixels that it shares with its neighbour a second time, with the same values.
+//
+// Bound by HBM where rows are long and by issue where they were short: as tiles of 512 x 8 or 2048 x 2 pixels, a lane past
+// the row's end idled (27 of 64 lanes had work at 208 columns) and a width that is no multiple of 8 sent every wave once
+// more through code for the ragged end. 59 x 564 x 634 39.0 -> 18.6 us (5.1 TB/s), 35 x 292 x 2118
+// 38.5 -> 19.4, 36 x 2916 x 306 29.4 -> 24.2, 32 x 1920 x 1080 49.5 -> 48.1 (6.2 TB/s).
+//
+// Both output rows of a wave go through its LDS and leave as 16-byte pieces, lane after lane (RunIO.hpp on why). A piece lies
+// in one block or in two next to each other; where the second of these is in another row the piece is two of 8 bytes.
 template<int DCN, bool SEMIPLANAR>
-__global__ __launch_bounds__(256) void Yuv420ToRgbTensor(const YuvArgs a, const int flat)
+__global__ __launch_bounds__(256) void Yuv420ToRgbTensor(const YuvArgs a, const DivBy perRow, const uint32_t blocks)
 {
-    // flat: a block's four waves side by side on one pair of rows (2048 columns) instead of 512 columns x 8 rows: 32 x
-    // 1080p 51.5 -> 50.8 us, the two alternating on one machine. The host asks for it where rows fill such blocks to 80 %.
-    // (arithmetic rather than a branch on `flat`, so that the other arguments are loaded at once)
-    const int f = flat != 0;
-    const int x = (int)(blockIdx.x * (64u << (2 * f)) + (threadIdx.x & (63u | (192u * f)))) * kYuvBlockW;
-    const int y = (int)(blockIdx.y * (4 - 3 * f) + (threadIdx.x >> 6) * (1 - f)) * 2;
+    constexpr int BW = kYuvBlockW, NC = BW / 2, RB = BW * DCN;
+    __shared__ __attribute__((aligned(16))) uint8_t stage[4][2 * 64 * RB];
+
+    const int      lane  = threadIdx.x & 63;
+    const uint32_t first = blockIdx.x * 256 + (threadIdx.x & 192); // of the wave
+    if (first >= blocks)
+    {
+        return;
+    }
+    const uint32_t n     = blockIdx.z;
+    const uint32_t block = min(first + lane, blocks - 1), pair = perRow.Quotient(block);
+    const uint32_t x     = min((block - pair * perRow.d) * BW, (uint32_t)a.W - BW);
+    const uint8_t *src   = a.srcBase + n * a.srcSampleStride;
+    uint8_t       *dst   = a.dstBase + n * a.dstSampleStride;
+    const uint32_t at    = 2 * pair * (uint32_t)a.srcRowStride + x;
+
+    uint8_t luma[2][BW];
+    LoadRun<uint8_t, BW>(src + at, luma[0]);
+    LoadRun<uint8_t, BW>(src + (at + (uint32_t)a.srcRowStride), luma[1]);
+    int c0[NC], c1[NC], c2[NC];
+    {
+        uint8_t uv[2][NC];
+        if constexpr (SEMIPLANAR)
+        {
+            uint8_t c[BW];
+            LoadRun<uint8_t, BW>(src + ((uint32_t)a.H + pair) * (uint32_t)a.srcRowStride + x, c);
+#pragma unroll
+            for (int k = 0; k < NC; ++k)
+            {
+                uv[0][k] = a.uidx ? c[2 * k + 1] : c[2 * k];
+                uv[1][k] = a.uidx ? c[2 * k] : c[2 * k + 1];
+            }
+        }
+        else
+        {
+            // each chroma plane is (H/2) x (W/2), stored as H/4 rows of W bytes after the luma rows
+            const uint32_t row = (uint32_t)a.H + (pair >> 1), h4 = (uint32_t)a.H >> 2;
+            const uint32_t uvx = (x >> 1) + ((uint32_t)a.W >> 1) * (pair & 1);
+            LoadRun<uint8_t, NC>(src + (row + h4 * (uint32_t)a.uidx) * (uint32_t)a.srcRowStride + uvx, uv[0]);
+            LoadRun<uint8_t, NC>(src + (row + h4 * (uint32_t)(a.uidx ^ 1)) * (uint32_t)a.srcRowStride + uvx, uv[1]);
+        }
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+        {
+            ChromaTerms(uv[0][k] - 128, uv[1][k] - 128, a.bidx, c0[k], c1[k], c2[k]);
+        }
+    }
+    uint8_t *own = stage[threadIdx.x >> 6];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+    {
+        uint8_t out[RB];
+        ConvertRun<DCN>(luma[r], c0, c1, c2, out);
+        __builtin_memcpy(own + r * 64 * RB + lane * RB, out, RB);
+    }
+    WaveExchangeFence();
+
+    const int lanes = (int)min(64u, blocks - first);
+    const int off   = (int)(2 * pair * (uint32_t)a.dstRowStride + x * DCN); // of the lane's piece in the first of its rows
+    constexpr int kPieces = 64 * RB / 16;                                   // of 16 bytes in one row of the wave
+    // Most waves lie in one row: their pieces follow each other (20 x 2048 x 1024 without this 31.0 us, with it 28.6, and as
+    // tiles 28.9).
+    const int off0 = __builtin_amdgcn_readfirstlane(off);
+    if (lanes == 64 && __builtin_amdgcn_readlane(off, 63) - off0 == 63 * RB
+        && __builtin_amdgcn_readlane((int)pair, 63) == __builtin_amdgcn_readfirstlane((int)pair))
+    {
+        uint8_t *row0 = dst + (uint32_t)off0;
+#pragma unroll
+        for (int j = 0; j < 2 * kPieces / 64; ++j)
+        {
+            const int c = j * 64 + lane, row = c >= kPieces;
+            uint32_t  w[4];
+            __builtin_memcpy(w, own + c * 16, 16);
+            StoreDwordsNT<4>(row0 + (uint32_t)(c * 16 + row * (a.dstRowStride - kPieces * 16)), w);
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 2 * kPieces / 64; ++j)
+    {
+        const int c = j * 64 + lane, row = c >= kPieces, cr = c - row * kPieces;
+        const uint8_t *from = own + c * 16;
+        uint32_t       w[4];
+        __builtin_memcpy(w, from, 16);
+        if constexpr (DCN == 4)
+        {
+            const int at0 = __builtin_amdgcn_ds_bpermute((cr >> 1) * 4, off);
+            if ((cr >> 1) < lanes)
+            {
+                StoreDwordsNT<4>(dst + (uint32_t)(at0 + row * a.dstRowStride + (cr & 1) * 16), w);
+            }
+        }
+        else
+        {
+            // pieces 3q, 3q + 1, 3q + 2 of the row: bytes 0 .. 15 of block 2q, its bytes 16 .. 23 and 0 .. 7 of block 2q + 1,
+            // bytes 8 .. 23 of that
+            const int  q = (cr * 43691) >> 17, k = cr - 3 * q, b0 = 2 * q + (k == 2);
+            const int  first0 = __builtin_amdgcn_ds_bpermute(b0 * 4, off);
+            const int  next   = __builtin_amdgcn_ds_bpermute((2 * q + 1) * 4, off) + row * a.dstRowStride;
+            const int  at0    = first0 + row * a.dstRowStride + (k == 0 ? 0 : (k == 1 ? 16 : 8));
+            const bool whole  = k != 1 || (next == at0 + 8 && 2 * q + 1 < lanes);
+            if (b0 < lanes && whole)
+            {
+                StoreDwordsNT<4>(dst + (uint32_t)at0, w);
+            }
+            else if (b0 < lanes)
+            {
+                StoreDwordsNT<2>(dst + (uint32_t)at0, {w[0], w[1]});
+                if (2 * q + 1 < lanes)
+                {
+                    StoreDwordsNT<2>(dst + (uint32_t)next, {w[2], w[3]});
+                }
+            }
+        }
+    }
+}
+
+// The same in tiles of 512 x 8 pixels: images of fewer than 8 columns, and those whose rows span 2 GiB.
+template<int DCN, bool SEMIPLANAR>
+__global__ __launch_bounds__(256) void Yuv420ToRgbTiles(const YuvArgs a)
+{
+    const int x = (int)(blockIdx.x * 64 + (threadIdx.x & 63)) * kYuvBlockW;
+    const int y = (int)(blockIdx.y * 4 + (threadIdx.x >> 6)) * 2;
     if (x >= a.W || y >= a.H)
     {
         return;
@@ -594,11 +735,19 @@ void LaunchYuv(const YuvArgs &a, int N, const NVCVImageBufferStrided *dstHost, h
 {
     if (dstHost == nullptr)
     {
-        const int64_t span = 4 * kYuvTileW;
-        const bool    flat = DivUp(a.W, (int)span) * span * 4 <= (int64_t)a.W * 5;
-        dim3          grid(DivUp(a.W, flat ? 4 * kYuvTileW : kYuvTileW), DivUp(a.H, flat ? 2 : kYuvTileH), N);
-        hipLaunchKernelGGL((Yuv420ToRgbTensor<DCN, SEMIPLANAR>), grid, dim3(256), 0, stream, a, (int)flat);
-        CheckLaunch("Yuv420ToRgbTensor");
+        const int64_t rows = std::max((int64_t)a.srcRowStride * a.H * 3 / 2, (int64_t)a.dstRowStride * a.H);
+        if (a.W >= kYuvBlockW && rows <= INT32_MAX && std::min(a.srcRowStride, a.dstRowStride) >= 0)
+        {
+            const DivBy    perRow(DivUp(a.W, kYuvBlockW));
+            const uint32_t blocks = perRow.d * (uint32_t)(a.H / 2);
+            hipLaunchKernelGGL((Yuv420ToRgbTensor<DCN, SEMIPLANAR>), dim3(DivUp((int)blocks, 256), 1, N), dim3(256), 0, stream,
+                               a, perRow, blocks);
+            CheckLaunch("Yuv420ToRgbTensor");
+            return;
+        }
+        hipLaunchKernelGGL((Yuv420ToRgbTiles<DCN, SEMIPLANAR>), dim3(DivUp(a.W, kYuvTileW), DivUp(a.H, kYuvTileH), N), dim3(256),
+                           0, stream, a);
+        CheckLaunch("Yuv420ToRgbTiles");
         return;
     }
     for (int first = 0; first < N; first += kMaxTileImages)

@@ -47,6 +47,22 @@ def test_yuv420_to_rgb(cv, K, orc, gpu, name, size):
         assert np.abs(res.astype(np.int16) - gold.astype(np.int16)).max() <= 2
 
 
+@pytest.mark.parametrize("name", ["YUV2RGB_NV12", "YUV2BGRA_NV21", "YUV2BGR_YV12", "YUV2RGBA_YV12"])
+@pytest.mark.parametrize("size", [(8, 4, 1), (10, 4, 2), (14, 8, 3), (18, 132, 2), (62, 40, 1), (504, 8, 1), (512, 8, 2), (514, 12, 1),
+                                  (1030, 8, 2)])
+def test_yuv420_rows_that_end_inside_a_wave(cv, K, orc, gpu, name, size):
+    # blocks of 8 columns are dealt to lanes across rows; the last one of a row overlaps its neighbour
+    w, h, n = size
+    dcn, bgr, uidx, semi = YUV_CODES[name]
+    src = nv12_input(orc, n, w, h, w * 5 + h)
+    for align in (0, 64):
+        tin = cv.Tensor.from_numpy(src, "NHWC", row_align=align)
+        tout = cv.Tensor.alloc([n, h, w, dcn], np.uint8, "NHWC", row_align=align)
+        cv.CvtColor()(None, tin, tout, getattr(K, "COLOR_" + name))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(tout.numpy(), orc.yuv420_to_rgb(src, dcn, bgr, uidx, semi, variant=0))
+
+
 def test_config3_full_size(cv, K, orc, gpu):
     # batch 32, 1080p NV12 -> RGB; Y in [16,235], UV in [16,240]
     src = nv12_input(orc, 32, 1920, 1080, 0xC0FFEE03)
