@@ -760,6 +760,25 @@ __device__ __forceinline__ void RunItems(const View &v, const PixArgs &a, int tx
     }
 }
 
+// Tensors whose rows hold at least one group. The groups of an image are numbered row by row and dealt to the lanes in that
+// order, whatever the width; a row's last group ends where the row does and writes the items that it shares with its neighbour
+// a second time, with the same values. In tiles of 64 groups x 4 rows lanes past a row's end idle, and a partial group sends
+// its wave through the items once more. RGB -> NV12, 25 x 518 x 542: 12.4 -> 9.4 us, 8 x 222 x 1084 9.2 -> 5.8,
+// 20 x 960 x 540 11.8 -> 10.5; 12 x 3840 x 2160 76.5 (5.9 TB/s) as before.
+template<class Op>
+__global__ __launch_bounds__(256) void PixelGroupsTensor(const PixArgs a, const DivBy perRow, const uint32_t groups)
+{
+    const uint32_t g = blockIdx.x * 256 + threadIdx.x;
+    if (g >= groups)
+    {
+        return;
+    }
+    const int      n = blockIdx.z;
+    const View     v = {a.src + n * a.srcN, a.dst + n * a.dstN, a.srcRow, a.dstRow, a.W, a.H};
+    const uint32_t y = perRow.Quotient(g);
+    Op::RunGroup(v, a, min((int)(g - y * perRow.d) * Op::kGroup, a.W / Op::kItemW - Op::kGroup), (int)y);
+}
+
 template<class Op>
 __global__ __launch_bounds__(256) void PixelTensor(const PixArgs a)
 {
@@ -849,6 +868,18 @@ void Launch(const ColorIO &io, PixArgs a, hipStream_t stream)
         if (a.W < Op::kItemW || a.H < Op::kItemH)
         {
             return;
+        }
+        if constexpr (!HasRowStore<Op>::value)
+        {
+            const int     perRow = DivUp(a.W / Op::kItemW, Op::kGroup);
+            const int64_t groups = (int64_t)perRow * (a.H / Op::kItemH);
+            if (a.W / Op::kItemW >= Op::kGroup && groups <= INT32_MAX - 256)
+            {
+                hipLaunchKernelGGL((PixelGroupsTensor<Op>), dim3(DivUp((int)groups, 256), 1, io.N), dim3(256), 0, stream, a,
+                                   DivBy(perRow), (uint32_t)groups);
+                CheckLaunch("PixelGroupsTensor");
+                return;
+            }
         }
         dim3 grid(DivUp(a.W, tileW), DivUp(a.H, tileH), io.N);
         hipLaunchKernelGGL((PixelTensor<Op>), grid, dim3(256), 0, stream, a);
