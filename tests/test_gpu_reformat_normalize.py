@@ -43,6 +43,26 @@ def test_reformat_nhwc_nchw_roundtrip(cv, orc, gpu, dt, shape):
     np.testing.assert_array_equal(tback.numpy(), a)
 
 
+@pytest.mark.parametrize("dt", [np.uint8, np.int16, np.float32, np.float64])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 3), (2, 7, 3, 3), (2, 5, 223, 3), (1, 2, 255, 4), (3, 11, 257, 1), (2, 33, 65, 4), (2, 3, 129, 6)])
+def test_reformat_rows_without_gaps(cv, orc, gpu, dt, shape):
+    # an image whose rows follow each other on both sides is moved as one row; one with gaps on one side is not
+    n, h, w, c = shape
+    a = rand(orc, shape, dt, 7 + w) if dt != np.float64 else orc.fill_f32(shape, 5).astype(np.float64)
+    dense = torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    out = torch.full((n, c, h, w), 3, dtype=dense.dtype, device="cuda")
+    back, wide = torch.full_like(dense, 5), torch.full((n, h, w + 3, c), 9, dtype=dense.dtype, device="cuda")
+    op = cv.Reformat()
+    op(None, cv.Tensor.from_torch(dense, "NHWC"), cv.Tensor.from_torch(out, "NCHW"))
+    op(None, cv.Tensor.from_torch(out, "NCHW"), cv.Tensor.from_torch(back, "NHWC"))
+    op(None, cv.Tensor.from_torch(out, "NCHW"), cv.Tensor.from_torch(wide[:, :, :w], "NHWC"))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy(), a.transpose(0, 3, 1, 2))
+    np.testing.assert_array_equal(back.cpu().numpy(), a)
+    np.testing.assert_array_equal(wide[:, :, :w].cpu().numpy(), a)
+    assert (wide[:, :, w:] == 9).all()
+
+
 def test_reformat_hwc_chw_copy_and_errors(cv, orc, gpu):
     a = rand(orc, (30, 40, 3), np.float32, 9)
     t_hwc = cv.Tensor.from_numpy(a, "HWC")
