@@ -42,11 +42,14 @@ __device__ __forceinline__ void LaneAndRow(const ReformatArgs &a, int &lane, int
 
 // The grid; where rows follow each other without a gap on both sides and do not fill their tiles, the image becomes one row
 // first: no lanes idle past the ends of rows, and one partial run per image. u8x3 NCHW -> NHWC, 25 x 518 x 542: 13.8 -> 9.7 us
-// (4.5 TB/s), 8 x 222 x 1084 5.6 -> 4.2, 20 x 960 x 540 13.7 -> 12.2, 32 x 1920 x 1080 69.0 and 70 (5.7 TB/s).
+// (4.5 TB/s), 8 x 222 x 1084 5.6 -> 4.2, 20 x 960 x 540 13.7 -> 12.2. Rows of whole runs that fill nine tenths of their tiles
+// stay rows where the data is more than the memory-side cache's 256 MB: 32 x 1920 x 1080 68.1 and, as one row, 71.4.
 dim3 GridOf(ReformatArgs &a, int pixelsPerLane, int N)
 {
-    const int64_t tile = 64 * pixelsPerLane;
-    if (a.W % tile != 0 && a.sH == a.W * a.sW && a.dH == a.W * a.dW && (int64_t)a.W * a.H <= INT32_MAX - 4 * tile)
+    const int64_t tile = 64 * pixelsPerLane, padded = (a.W + tile - 1) / tile * tile;
+    const bool    keep = a.W % pixelsPerLane == 0
+                   && (padded == a.W || (padded * 9 <= (int64_t)a.W * 10 && N * (a.sN + a.dN) > ((int64_t)256 << 20)));
+    if (!keep && a.sH == a.W * a.sW && a.dH == a.W * a.dW && (int64_t)a.W * a.H <= INT32_MAX - 4 * tile)
     {
         a.W *= a.H;
         a.H = 1;
