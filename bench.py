@@ -698,9 +698,9 @@ class Streaming:
         "resize-linear-upscale": ("Resize", 32, ("uint8", 3, 720, 1280), ("uint8", 3, "NHWC", 1080, 1920),
                                   "ResizeLinearQuadsU8Kernel<3>", "i32", "Resize LINEAR 1280x720 -> 1920x1080"),
         "resize-cubic-720p": ("Resize", 32, ("uint8", 3), ("uint8", 3, "NHWC", 720, 1280),
-                              "ResizeCubicStripU8Kernel<3,4>", "i32", "Resize CUBIC 1920x1080 -> 1280x720"),
+                              "ResizeCubicWalkU8Kernel<3>", "i32", "Resize CUBIC 1920x1080 -> 1280x720"),
         "resize-cubic-upscale": ("Resize", 32, ("uint8", 3, 720, 1280), ("uint8", 3, "NHWC", 1080, 1920),
-                                 "ResizeCubicStripU8Kernel<3,8>", "i32", "Resize CUBIC 1280x720 -> 1920x1080"),
+                                 "ResizeCubicWalkU8Kernel<3>", "i32", "Resize CUBIC 1280x720 -> 1920x1080"),
         "resize-nearest-upscale": ("Resize", 32, ("uint8", 3, 720, 1280), ("uint8", 3, "NHWC", 1080, 1920),
                                    "ResizeNearestQuadsU8Kernel<3>", "f32", "Resize NEAREST 1280x720 -> 1920x1080"),
         "resize-area-720p": ("Resize", 32, ("uint8", 3), ("uint8", 3, "NHWC", 720, 1280),

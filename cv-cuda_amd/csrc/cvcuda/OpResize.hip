@@ -16,8 +16,8 @@
 //    enlarging by 1.5 or more) and fetches each source row once for all its columns and rows, lane pairs swap a
 //    pixel pair each;
 //    nearest neighbour takes the same strips when enlarging by 1.5 or more;
-//  * 8-bit bicubic tensors of 3 and 4 channels at vertical scales of 1/2 to 2, large launches: a wave owns 64 columns
-//    x 16 rows and forms every source row's sums once, adding them to the output rows in flight;
+//  * 8-bit bicubic at vertical scales up to 4, launches of 1024 waves and more (image batches: 3 and 4 channels, 2048
+//    blocks): a wave walks down the source rows once, keeps the sums of the last four and finishes output rows as it goes;
 //  * bicubic reductions >= 2x of 12/16-byte pixels: tap-major loads exchanged through LDS;
 //  * AREA of 8-bit pixels at reductions of up to 3: fixed-point row sums, a wave owns 64 columns x 16 rows and
 //    produces vertically adjacent rows in pairs from the source rows they share;
@@ -1327,252 +1327,6 @@ __device__ __forceinline__ void ResizeWavePatch(const Plane &p, int x0, int y0)
     StoreWavePatch<T, C>(p, x0, y0, lane, q);
 }
 
-// ---- the 8-bit bicubic form over strips of 16 output rows per wave
-
-constexpr int kCubicStripRows = 16;
-
-// A row window as LoadQuadWindow reads it, in two steps: a strip requests the rows of its next output row before it
-// works on the current one.
-template<int C>
-struct RawQuadWindow
-{
-    uint32_t d[C == 4 ? 4 : C + 1];
-};
-
-// (row: wave-uniform; off: the window's byte offset in it - the load then takes the row as its scalar base. mis: the row's
-// RowMisalignment, so that the load starts at a dword of memory)
-template<int C>
-__device__ __forceinline__ RawQuadWindow<C> RequestQuadWindow(const uint8_t *row, uint32_t off, uint32_t mis)
-{
-    struct __attribute__((packed, aligned(1))) Window
-    {
-        uint32_t d[C == 4 ? 4 : C + 1];
-    };
-    const Window     w = *reinterpret_cast<const Window *>(row - mis + (C == 4 ? off : (off + mis) & ~3u));
-    RawQuadWindow<C> r;
-    __builtin_memcpy(&r, &w, sizeof(r));
-    return r;
-}
-
-// The row's sums of 4 taps times the horizontal weights (units of 2^-14), as CubicRowsQ14 forms them.
-template<int C>
-__device__ __forceinline__ void CubicRowSumsQ14(const RawQuadWindow<C> &w, uint32_t shift, uint32_t w01, uint32_t w23,
-                                                float (&h)[C])
-{
-    uint32_t r[C];
-#pragma unroll
-    for (int i = 0; i < C; ++i)
-    {
-        if constexpr (C == 4)
-        {
-            r[i] = w.d[i];
-        }
-        else
-        {
-            r[i] = __builtin_amdgcn_alignbyte(w.d[i + 1], w.d[i], shift);
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-    {
-        h[c] = RowSumQ14(QuadTapPair<C>(r, 0, c), QuadTapPair<C>(r, 2, c), w01, w23);
-    }
-}
-
-// One wave resizes 64 columns x 16 rows whose top left pixel is (x0, y0), both wave-uniform; lane l owns column
-// x0 + l. The windows of consecutive output rows overlap (reducing by 1.5 they advance by 1 or 2 source rows,
-// enlarging by 0 or 1), so the strip walks down the source rows once: a row's sums are formed once and added, times
-// the row's weight in each, to the output pixels whose windows can hold it - the current output row and the S - 1
-// after it. S = 4 when reducing (all of them while windows advance by at least one row), S = 8 when enlarging (all
-// of them while the window 8 rows down starts 4 or more source rows later: enlargements up to 2). The S running
-// pixels live in fixed registers (output row r in slot r mod S, S steps unrolled); a row outside a pixel's window
-// is added with weight 0, which changes nothing, so the instruction stream does not depend on the scale. An output
-// row is finished when the last row of its window has been added, its slot then starts the pixel S rows down.
-// Every pixel adds its four row sums in ascending order (the first to a zero, which gives the product), as
-// CubicRowsQ14 does: the same result bit for bit. Per output pixel 1.5 row sums when reducing by 1.5 where the patch
-// form takes 2.75, 0.67 when enlarging by 1.5 where it takes 2.25, and the column terms once per 16 rows.
-// The rows a step can add (reducing: two, enlarging: one) are requested two steps ahead, needed or not (no test in
-// front of a load).
-// A strip takes this form when its windows advance as said from each output row to the next and stay clear of the
-// image's last row; others (the image's top and bottom, other scales) go one output row at a time with guarded
-// loads. The launch requires sources wide enough for the window loads (16 bytes a row, 8 for one channel).
-// ODD: see LoadQuadWindow (32 x 1921 x 1081 x 3 -> 1280 x 720: 160 us with loads counted from the row, 82 us so; to 1931 x 1081 from
-// 1281 x 721: 227 and 140; aligned, 1920 x 1080: 79 us, with the other form 83).
-template<int C, int S, bool ODD>
-__device__ __forceinline__ void ResizeCubicStripU8(const Plane &p, int x0, int y0)
-{
-    static_assert(S == 4 || S == 8);
-    constexpr bool kReducing = S == 4;
-    if (x0 >= p.dstW || y0 >= p.dstH)
-    {
-        return;
-    }
-    constexpr int R    = kCubicStripRows;
-    const int     lane = threadIdx.x & 63;
-    const int     dx   = min(x0 + lane, p.dstW - 1); // columns past the output compute a duplicate of the last one
-    const auto    col  = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleX, dx, p.srcW, true);
-    // lane 4 r + t holds the second tap's row of output row y0 + r and its weight for tap t, in units of 2^-14
-    // (the row sums' unit)
-    const auto  rows  = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleY, min(y0 + (lane >> 2), p.dstH - 1), p.srcH, false);
-    const int   t     = lane & 3;
-    const float wLane = (t == 0 ? rows.w[0] : t == 1 ? rows.w[1] : t == 2 ? rows.w[2] : rows.w[3]) * (1.f / 16384.f);
-    const int   apartLane = __shfl_down(rows.s, 4) - rows.s;
-    bool        regular   = lane >= 4 * (R - 1) || (apartLane >= (kReducing ? 1 : 0) && apartLane <= (kReducing ? 2 : 1));
-    if constexpr (!kReducing)
-    {
-        // (every lane takes part in the exchange: a lane that has left reads as 0)
-        const int farLane = __shfl_down(rows.s, 4 * S) - rows.s;
-        regular           = regular & ((lane >= 4 * (R - S)) | (farLane >= 4));
-    }
-    const CubicColumnQ14 cq = CubicColumn<C>(col);
-    auto second = [&](int r) { return __builtin_amdgcn_readlane(rows.s, 4 * min(r, R - 1)); }; // the row of output row r's second tap
-    if (y0 + R > p.dstH || __builtin_amdgcn_ballot_w64(!regular) != 0 || second(R - 1) + 2 >= p.srcH - 1) // wave-uniform
-    {
-        // one output row at a time, every window load guarded against the image's last row
-#pragma unroll 1
-        for (int g = 0; g < R && y0 + g < p.dstH; g += 4)
-        {
-            uint32_t q[1][4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-            {
-                const int   r     = g + k;
-                const float wy[4] = {ReadLane(wLane, 4 * r), ReadLane(wLane, 4 * r + 1), ReadLane(wLane, 4 * r + 2),
-                                     ReadLane(wLane, 4 * r + 3)};
-                q[0][k] = CubicRowsQ14<C, true, ODD>(p, second(r) - 1, cq.at, cq.shift, (uint32_t)p.srcW * C, cq.w01, cq.w23, wy);
-            }
-            StoreWavePatch<uint8_t, C>(p, x0, y0 + g, lane, q);
-        }
-        return;
-    }
-    const uint32_t off       = ODD ? cq.at + cq.shift : cq.at;
-    auto           misplaced = [&](int row) { return ODD ? RowMisalignment(p.src + (int64_t)row * p.srcRow) : 0u; };
-    auto           request = [&](int row) { return RequestQuadWindow<C>(p.src + (int64_t)row * p.srcRow, off, misplaced(row)); };
-
-    float acc[S][C] = {};
-    // The weight of source row j in output row r, whose second tap is row sr: tap j - (sr - 1) where that is 0 .. 3,
-    // else 0. Output rows past the strip (r >= 16, terms of row 15) collect sums that are never stored. The lane is
-    // read either way (no branch; the instruction takes the lane number modulo 64) and the choice is written as scalar
-    // instructions, which the compiler otherwise turns into a move and a select on the vector unit per weight.
-    // always: the tap is known to be one of the four, nothing to choose.
-    auto weight = [&](int j, int sr, int r, bool always)
-    {
-        const int tap = j - sr + 1;
-        const int w   = __builtin_amdgcn_readlane(__float_as_int(wLane), 4 * r + tap);
-        if (always)
-        {
-            return __int_as_float(w);
-        }
-        int chosen;
-        asm("s_cmp_lt_u32 %1, 4\n\ts_cselect_b32 %0, %2, 0" : "=s"(chosen) : "s"(tap), "s"(w) : "scc");
-        return __int_as_float(chosen);
-    };
-    // Source row j, whose window is w, into the output rows r .. r + outputs - 1 (slots K .. ; K is a constant once
-    // unrolled), whose second taps are rows sr[0 ..]; the first `sure` of them hold the row for certain.
-    auto add = [&](int K, const RawQuadWindow<C> &w, int j, int r, const int (&sr)[S], int outputs, int sure)
-    {
-        float h[C];
-        CubicRowSumsQ14<C>(w, ODD ? off + misplaced(j) : cq.shift, cq.w01, cq.w23, h);
-#pragma unroll
-        for (int i = 0; i < S; ++i)
-        {
-            if (i >= outputs)
-            {
-                break;
-            }
-            // taps fall with i: from the first pixel whose window starts below the row on, nothing is added (tested
-            // where it pays: once for pixels 4 - 5 and once for 6 - 7 of the enlarging form; wave-uniform)
-            if ((i == 4 || i == 6) && j - sr[i] + 1 < 0)
-            {
-                break;
-            }
-            const float wi = weight(j, sr[i], r + i, i < sure);
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                acc[(K + i) & (S - 1)][c] = fmaf(h[c], wi, acc[(K + i) & (S - 1)][c]);
-            }
-        }
-    };
-    int sr[S];
-#pragma unroll
-    for (int i = 0; i < S; ++i)
-    {
-        sr[i] = second(i);
-    }
-    // output row 0's window but for its last row
-    {
-        const RawQuadWindow<C> w0 = request(sr[0] - 1), w1 = request(sr[0]), w2 = request(sr[0] + 1);
-        add(0, w0, sr[0] - 1, 0, sr, S, 1);
-        add(0, w1, sr[0], 0, sr, S, 1);
-        add(0, w2, sr[0] + 1, 0, sr, S, 1);
-    }
-    // The step to output row r adds row sr + 2 if the window advanced, and before it row sr + 1 if it advanced by 2.
-    // They are requested two steps ahead (even steps use one set of registers, odd steps the other).
-    constexpr int    M = kReducing ? 2 : 1;
-    RawQuadWindow<C> ahead[2][M];
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-    {
-#pragma unroll
-        for (int m = 0; m < M; ++m)
-        {
-            ahead[e][m] = request(sr[e] + 2 - (M - 1 - m));
-        }
-    }
-    int apart = 1; // the rows before sr[0] + 2 are in already
-#pragma unroll 1
-    for (int g = 0; g < R; g += S)
-    {
-        uint32_t q[1][4];
-#pragma unroll
-        for (int k = 0; k < S; ++k)
-        {
-            const int        r = g + k;
-            RawQuadWindow<C> now[M];
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-            {
-                now[m]           = ahead[k & 1][m];
-                ahead[k & 1][m] = request(sr[2] + 2 - (M - 1 - m));
-            }
-            if constexpr (kReducing)
-            {
-                if (apart == 2)
-                {
-                    add(k, now[0], sr[0] + 1, r, sr, 3, 2); // the row above the window's last is in none of output row r + 3's
-                }
-                add(k, now[1], sr[0] + 2, r, sr, 4, 2);
-            }
-            else
-            {
-                if (apart == 1)
-                {
-                    add(k, now[0], sr[0] + 2, r, sr, S, 1);
-                }
-            }
-            apart = sr[1] - sr[0];
-#pragma unroll
-            for (int i = 0; i + 1 < S; ++i)
-            {
-                sr[i] = sr[i + 1];
-            }
-            sr[S - 1] = second(r + S);
-            q[0][k & 3] = 0;
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                q[0][k & 3] = __builtin_amdgcn_cvt_pk_u8_f32(fabsf(acc[k][c]), c, q[0][k & 3]);
-                acc[k][c]   = 0.f;
-            }
-            if ((k & 3) == 3)
-            {
-                StoreWavePatch<uint8_t, C>(p, x0, y0 + r - 3, lane, q);
-            }
-        }
-    }
-}
-
 // 8-bit bilinear at horizontal scales up to 2. The cost of the wave-patch form there is the number
 // of tap loads (the texture addresser is busy 76-90 % of the time). The taps of two neighbouring
 // output columns lie within 4 source pixels, so here a lane owns 2 columns x 2 rows and fetches each
@@ -2593,51 +2347,263 @@ __global__ __launch_bounds__(256) void ResizePatchTensorKernel(const ResizeArgs 
     ResizeWavePatch<T, C, INTERP, false, ODD>(p, t.x * kPatchTileW, t.y * 4);
 }
 
-// Which of the bicubic strip forms an image takes by its vertical scale and row length: 4 (reducing by up to 2), 8
-// (enlarging by up to 2) or 0 (none: wave patches).
+// ---- the 8-bit bicubic form that walks the source rows once
+//
+// Sizes that it takes: every source row counts (farther apart, rows between the windows would be summed for nothing), loads of
+// 16 bytes (8 for one channel) fit a row, and a lane's columns fit its loads, and half of a wave's lanes
+// have columns (one channel, 128 x 64 x 64 -> 48 x 48: as patches 3.6 us, so 4.7; three channels need a whole tile, see below).
 template<int C>
-__host__ __device__ __forceinline__ int CubicStripForm(int srcW, int srcH, int dstH)
+constexpr int kCubicWalkW = C == 1 ? 256 : 64; // a wave's columns
+
+constexpr int kCubicBatchRows = 16; // image batches: a wave's rows
+
+template<int C>
+__host__ __device__ __forceinline__ bool CubicWalks(int srcW, int srcH, int dstW, int dstH)
 {
-    if (!(C == 3 || C == 4) || srcW < 4 || srcW * C < 16)
-    {
-        return 0;
-    }
-    return (srcH >= dstH && srcH <= 2 * (int64_t)dstH) ? 4 : ((srcH < dstH && 2 * (int64_t)srcH >= dstH) ? 8 : 0);
+    return srcH >= 4 && srcH <= 4 * (int64_t)dstH && srcW * C >= (C == 1 ? 8 : 16)
+        && dstW >= (C == 1 ? 128 : C == 3 ? 64 : 1) && (C != 1 || 10 * (int64_t)srcW <= 39 * (int64_t)dstW);
 }
 
-// Large image batches: a 64 x 64 tile per block, a strip per wave where the image's scale allows, else four patches.
-template<int C, bool ODD>
-__global__ __launch_bounds__(256) void ResizeCubicStripU8VarShapeKernel(const ResizeArgs a, const VarTiles tiles)
+// What a lane knows of its columns, and its part of a source row. One channel: four columns, which lie within 8 source
+// bytes (LOADS = 1, horizontal scales up to 1.3) or two by two (LOADS = 2, up to 3.9): a row is one or two unaligned 8-byte
+// loads, and two byte permutes whose selectors are the column's for all rows bring its taps side by side. Windows of columns
+// near the row's end start 8 bytes before it. Three and four channels: one column, its window as LoadQuadWindow reads it.
+template<int C, int LOADS, bool ODD>
+struct CubicLane
 {
-    const TileCoord tc   = LocateTile(tiles, blockIdx.x);
-    const Plane     p    = GetPlanes<true>(a, tc.image);
-    const int       x0 = tc.tx * kPatchTileW, y0 = tc.ty * 4 * kCubicStripRows + (threadIdx.x >> 6) * kCubicStripRows;
-    const int       form = CubicStripForm<C>(p.srcW, p.srcH, p.dstH);
-    if (form == 4)
+    static constexpr int K = C == 1 ? 4 : 1; // columns
+    static constexpr int D = C == 1 ? 2 : 4; // dwords of a load
+
+    struct Window
     {
-        ResizeCubicStripU8<C, 4, ODD>(p, x0, y0);
-    }
-    else if (form == 8)
+        uint32_t d[LOADS][D];
+    };
+
+    uint32_t at[LOADS], pick[K], w01[K], w23[K]; // pick: one channel: the permute of taps 0 and 1; else the window's byte offset
+
+    __device__ __forceinline__ CubicLane(const Plane &p, int x)
     {
-        ResizeCubicStripU8<C, 8, ODD>(p, x0, y0);
-    }
-    else
-    {
-#pragma unroll 1
-        for (int g = 0; g < kCubicStripRows; g += 4)
+#pragma unroll
+        for (int k = 0; k < K; ++k)
         {
-            ResizeWavePatch<uint8_t, C, NVCV_INTERP_CUBIC, true, ODD>(p, x0, y0 + g);
+            const auto           col = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleX, x + k, p.srcW, true);
+            const CubicColumnQ14 cq  = CubicColumn<C>(col);
+            w01[k]                   = cq.w01;
+            w23[k]                   = cq.w23;
+            if constexpr (C == 1)
+            {
+                const int l = k * LOADS / K;
+                if (k % (K / LOADS) == 0)
+                {
+                    at[l] = (uint32_t)min(col.s - 1, p.srcW - 8);
+                }
+                pick[k] = 0x0c010c00u + ((uint32_t)(col.s - 1) - at[l]) * 0x00010001u;
+            }
+            else
+            {
+                at[0]   = cq.at;
+                pick[0] = cq.at + cq.shift;
+            }
+        }
+    }
+
+    // Where a window of three channels begins: row `row` of the image from its own first dword of memory on, the image's last
+    // row from its first byte on and ending with it at the latest.
+    __device__ __forceinline__ uint32_t Begin(const Plane &p, const uint8_t *line, bool end, uint32_t &mis) const
+    {
+        mis              = ODD && !end ? RowMisalignment(line) : 0u;
+        const uint32_t o = ODD ? (pick[0] + mis) & ~3u : at[0];
+        return min(o, end ? (uint32_t)p.srcW * C - 4 * D : ~0u);
+    }
+
+    __device__ __forceinline__ Window Request(const Plane &p, int row) const
+    {
+        const uint8_t *line = p.src + (int64_t)min(row, p.srcH - 1) * p.srcRow;
+        struct __attribute__((packed, aligned(1))) Bytes
+        {
+            uint32_t d[D];
+        };
+        Window w;
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l)
+        {
+            uint32_t off = at[l], mis = 0;
+            if constexpr (C == 3)
+            {
+                off = Begin(p, line, row >= p.srcH - 1, mis);
+            }
+            // (stays a 32-bit offset to a scalar base: widened ahead of the loop it takes 64-bit sums per lane)
+            asm("" : "+v"(off));
+            const Bytes b = *reinterpret_cast<const Bytes *>(line - mis + off);
+            __builtin_memcpy(w.d[l], &b, sizeof(b));
+        }
+        return w;
+    }
+
+    // The window's sums of 4 taps times the horizontal weights, C for each column (units of 2^-14).
+    __device__ __forceinline__ void Sums(const Plane &p, int row, const Window &w, float (&h)[K * C]) const
+    {
+        if constexpr (C == 1)
+        {
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+            {
+                const uint32_t(&d)[D] = w.d[k * LOADS / K];
+                h[k] = RowSumQ14(__builtin_amdgcn_perm(d[1], d[0], pick[k]), __builtin_amdgcn_perm(d[1], d[0], pick[k] + 0x00020002u),
+                                 w01[k], w23[k]);
+            }
+        }
+        else
+        {
+            uint32_t r[C];
+            if constexpr (C == 4)
+            {
+                __builtin_memcpy(r, w.d[0], sizeof(r));
+            }
+            else
+            {
+                const bool     end  = row >= p.srcH - 1;
+                const uint8_t *line = p.src + (int64_t)min(row, p.srcH - 1) * p.srcRow;
+                uint32_t       mis;
+                const uint32_t begin = Begin(p, line, end, mis), shift = pick[0] + mis - begin; // (4 only if moved back)
+#pragma unroll
+                for (int i = 0; i < C; ++i)
+                {
+                    r[i] = __builtin_amdgcn_alignbyte(w.d[0][i + 1], w.d[0][i], shift);
+                }
+                if (end && shift == 4)
+                {
+                    __builtin_memcpy(r, &w.d[0][1], sizeof(r));
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+            {
+                h[c] = RowSumQ14(QuadTapPair<C>(r, 0, c), QuadTapPair<C>(r, 2, c), w01[0], w23[0]);
+            }
+        }
+    }
+};
+
+// A wave owns 64 lanes' columns x `rows` output rows (64 at most). It walks down the source rows, keeps the sums of the last
+// four in registers (a row's place is its number modulo 4, four steps unrolled) and finishes the output rows whose window ends
+// with the row just added: every sum is formed once per strip, at any scale, and none is added with weight 0. Rows are
+// requested two steps ahead (four were no faster; eight at a time, 22.7 us for 17.2: the registers). The vertical weights wait
+// in LDS, one broadcast read per output row (as v_readlane 8 % slower). Sums, their order and the result are those of
+// CubicRowsQ14 bit for bit.
+// An output row leaves as one dword per lane; three channels: the three bytes of four lanes as three of their dwords.
+template<int C, int LOADS, bool ODD>
+__device__ __forceinline__ void ResizeCubicWalkU8(const Plane &p, int x0, int y0, int rows)
+{
+    using Lane       = CubicLane<C, LOADS, ODD>;
+    constexpr int K  = Lane::K, V = K * C;
+    const int     lane = threadIdx.x & 63, n = min(rows, p.dstH - y0);
+    if (x0 >= p.dstW || n <= 0)
+    {
+        return;
+    }
+    if constexpr (C == 3)
+    {
+        x0 = min(x0, p.dstW - 64); // (the last tile overlaps its neighbour, with the same values; so do one channel's last columns)
+    }
+    const int  x = min(x0 + K * lane, p.dstW - K);
+    const Lane column(p, x);
+    const auto down = FinishedAxis<NVCV_INTERP_CUBIC>(p.scaleY, min(y0 + lane, p.dstH - 1), p.srcH, false); // lane r: output row y0 + r
+    __shared__ float4 weights[4][64];
+    float4           *wy    = weights[threadIdx.x >> 6];
+    constexpr float   kUnit = 1.f / 16384.f; // the row sums'
+    wy[lane] = make_float4(down.w[0] * kUnit, down.w[1] * kUnit, down.w[2] * kUnit, down.w[3] * kUnit);
+    WaveExchangeFence();
+
+    float h[4][V];
+    int   j = __builtin_amdgcn_readlane(down.s, 0) - 1;
+    {
+        const auto r0 = column.Request(p, j), r1 = column.Request(p, j + 1), r2 = column.Request(p, j + 2);
+        column.Sums(p, j, r0, h[0]);
+        column.Sums(p, j + 1, r1, h[1]);
+        column.Sums(p, j + 2, r2, h[2]);
+    }
+    j += 3;
+    typename Lane::Window ahead[2] = {column.Request(p, j), column.Request(p, j + 1)};
+
+    // three channels: lane 4 g + i, i < 3, holds dword i of the group's 12 bytes
+    constexpr uint32_t kThird[4] = {0x04020100u, 0x05040201u, 0x06050402u, 0x06050402u};
+    const int          part      = lane & 3;
+    const uint32_t     third     = part == 0 ? kThird[0] : part == 1 ? kThird[1] : kThird[2];
+    const uint32_t     to        = C == 3 ? (uint32_t)(x0 + (lane & ~3)) * 3 + 4 * part : (uint32_t)x * C;
+    const bool         mine      = C == 3 ? part != 3 : x0 + K * lane < p.dstW;
+    uint8_t           *out       = p.dst + (int64_t)y0 * p.dstRow;
+    int                r = 0, last = j; // the output row to come, and the last row of its window
+    float4             w = wy[0];
+    for (;;)
+    {
+#pragma unroll
+        for (int u = 0; u < 4; ++u, ++j)
+        {
+            const auto now = ahead[u & 1];
+            ahead[u & 1]   = column.Request(p, j + 2);
+            column.Sums(p, j, now, h[(3 + u) & 3]);
+            while (last <= j) // (equal: windows of later rows do not end earlier)
+            {
+                uint32_t q = 0;
+#pragma unroll
+                for (int k = 0; k < V; ++k)
+                {
+                    float v = h[u & 3][k] * w.x;
+                    v       = fmaf(h[(u + 1) & 3][k], w.y, v);
+                    v       = fmaf(h[(u + 2) & 3][k], w.z, v);
+                    v       = fmaf(h[(u + 3) & 3][k], w.w, v);
+                    q       = __builtin_amdgcn_cvt_pk_u8_f32(fabsf(v), k, q);
+                }
+                if constexpr (C == 3)
+                {
+                    const uint32_t next = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q, 0xF9 /* quad_perm 1,2,3,3 */, 0xF, 0xF, false);
+                    q                   = __builtin_amdgcn_perm(next, q, third);
+                }
+                if (mine)
+                {
+                    uint32_t off = to;
+                    asm("" : "+v"(off));
+                    StoreDwordsNT<1>(out + off, {q});
+                }
+                if (++r >= n)
+                {
+                    return;
+                }
+                w = wy[r];
+                out += p.dstRow;
+                last = __builtin_amdgcn_readlane(down.s, r) + 2;
+            }
         }
     }
 }
 
-// 8-bit bicubic strips: block = 4 waves stacked vertically (64 columns x 64 rows) or, reducing wide images, side by side.
-template<int C, int S, bool ODD>
-__global__ __launch_bounds__(256) void ResizeCubicStripU8Kernel(const ResizeArgs a, const int flat)
+template<int C, int LOADS, bool ODD>
+__global__ __launch_bounds__(256) void ResizeCubicWalkU8Kernel(const ResizeArgs a, const int rows, const int flat)
 {
-    const Plane p = GetPlanes<false>(a, blockIdx.z);
+    const Plane    p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeCubicStripU8<C, S, ODD>(p, t.x * kPatchTileW, t.y * kCubicStripRows);
+    ResizeCubicWalkU8<C, LOADS, ODD>(p, t.x * kCubicWalkW<C>, t.y * rows, rows);
+}
+
+// Large image batches: a 64 x 64 tile per block, 16 rows of it per wave, walked where the image's sizes allow, else as four
+// patches.
+template<int C, bool ODD>
+__global__ __launch_bounds__(256) void ResizeCubicWalkU8VarShapeKernel(const ResizeArgs a, const VarTiles tiles)
+{
+    const TileCoord tc = LocateTile(tiles, blockIdx.x);
+    const Plane     p  = GetPlanes<true>(a, tc.image);
+    const int       x0 = tc.tx * kPatchTileW, y0 = (tc.ty * 4 + (int)(threadIdx.x >> 6)) * kCubicBatchRows;
+    if (CubicWalks<C>(p.srcW, p.srcH, p.dstW, p.dstH))
+    {
+        ResizeCubicWalkU8<C, 1, ODD>(p, x0, y0, kCubicBatchRows);
+        return;
+    }
+#pragma unroll 1
+    for (int g = 0; g < kCubicBatchRows; g += 4)
+    {
+        ResizeWavePatch<uint8_t, C, NVCV_INTERP_CUBIC, true, ODD>(p, x0, y0 + g);
+    }
 }
 
 template<class T, int C, int INTERP, bool ODD>
@@ -3903,22 +3869,31 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             return;
         }
     }
-    if constexpr (INTERP == NVCV_INTERP_CUBIC && std::is_same_v<T, uint8_t> && (C == 3 || C == 4))
+    if constexpr (INTERP == NVCV_INTERP_CUBIC && std::is_same_v<T, uint8_t> && (C == 1 || C == 3 || C == 4))
     {
-        // strips of 16 rows per wave where consecutive windows overlap (vertical scales of 1/2 to 2) and the launch
-        // still has 8 waves and more per CU; one channel is as fast or faster as wave patches (16 x 720p -> 1080p
-        // 46.6 us against 50.9 as strips, 1080p -> 720p 27.2 against 28.1)
-        const int64_t strips = (int64_t)DivUp(a.dstW, kPatchTileW) * DivUp(a.dstH, kCubicStripRows) * N;
-        const int     form   = CubicStripForm<C>(a.srcW, a.srcH, a.dstH);
-        if (strips >= 8 * 256 && form != 0)
+        constexpr int tileW = kCubicWalkW<C>;
+        auto          waves = [&](int rows) { return (int64_t)DivUp(a.dstW, tileW) * DivUp(a.dstH, rows) * N; };
+        // Fewer waves than 4 to a CU are left to the patches, whose waves are shorter (us as patches / so: 8 x 224 x 224 x 1 -> 256 x
+        // 256 4.0 / 4.0, 100 x 100 x 3 -> 128 x 128 3.5 / 3.6; 640 x 480 x 3 -> 800 x 600 4.9 / 4.4).
+        if (CubicWalks<C>(a.srcW, a.srcH, a.dstW, a.dstH) && waves(4) >= 4 * 256)
         {
-            const bool flat = form == 4 && FlatBlocks(a.dstW, kPatchTileW); // (enlarging: stacked, see WaveTileOf)
-            const dim3 sgrid = WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, kCubicStripRows, flat);
-            const bool odd = RowsAreOdd<C>(a);
-            auto kernel = form == 4 ? (odd ? ResizeCubicStripU8Kernel<C, 4, C != 4> : ResizeCubicStripU8Kernel<C, 4, false>)
-                                    : (odd ? ResizeCubicStripU8Kernel<C, 8, C != 4> : ResizeCubicStripU8Kernel<C, 8, false>);
-            hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, a, (int)flat);
-            CheckLaunch("ResizeCubicStripU8Kernel");
+            // A wave's first row costs three row sums more than the others, its end leaves the CU to fewer waves. us with 4 / 8 / 16 / 32
+            // rows: 1280 x 720 x 3 -> 1080p 7.6 / 6.8 / 7.4 / 10.8; 64 x 256 x 256 x 3 -> 224 x 224 12.1 / 10.6 / 11.6 / 14.9; 21 x 1119 x
+            // 343 x 3 -> 1140 x 403 27.2 / 21.7 / 20.6 / 23.1; 32 x 1280 x 720 x 3 -> 1080p 139 / 101 / 87 / 79. 32 only where the lines
+            // of memory that output rows end in are not shared with a neighbour that comes to them late (9 x 1515 x 649 x 3 -> 3815 x
+            // 1860, 16 / 32: 74 / 90).
+            int rows = 4;
+            rows     = waves(8) >= 1536 ? 8 : rows;
+            rows     = waves(16) >= 16 * 256 ? 16 : rows;
+            rows     = waves(32) >= 64 * 256 && a.dstH > a.srcH && a.dstRowStride % 64 == 0 ? 32 : rows;
+            // Side by side wherever that leaves few waves without columns: rows that end in the middle of a line of memory want
+            // their neighbour soon (the same, stacked / side by side: 114 / 74; 8 x 1080p x 4 -> 640 x 360 15.5 / 13.8).
+            const bool    flat = DivUp(a.dstW, 4 * tileW) * (int64_t)(4 * tileW) * 4 <= (int64_t)a.dstW * 5;
+            constexpr int kTwo = C == 1 ? 2 : 1;
+            auto kernel = C == 1 ? (10 * (int64_t)a.srcW <= 13 * (int64_t)a.dstW ? ResizeCubicWalkU8Kernel<C, 1, false> : ResizeCubicWalkU8Kernel<C, kTwo, false>)
+                                 : (RowsAreOdd<C>(a) ? ResizeCubicWalkU8Kernel<C, 1, C == 3> : ResizeCubicWalkU8Kernel<C, 1, false>);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, tileW, rows, flat), dim3(256), 0, stream, a, rows, (int)flat);
+            CheckLaunch("ResizeCubicWalkU8Kernel");
             return;
         }
     }
@@ -4062,21 +4037,22 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
         }
         if constexpr (INTERP == NVCV_INTERP_CUBIC && std::is_same_v<T, uint8_t> && (C == 3 || C == 4))
         {
-            // strips where most output pixels belong to images that can take them and every CU still gets 8 blocks
-            int64_t stripPixels = 0, allPixels = 0;
+            // walked where most output pixels belong to images that can be and every CU still gets 8 blocks
+            int64_t walked = 0, all = 0;
             for (int i = first; i < first + count; ++i)
             {
-                const int64_t px = (int64_t)dstHost[i].planes[0].width * dstHost[i].planes[0].height;
-                allPixels += px;
-                stripPixels += CubicStripForm<C>(srcHost[i].planes[0].width, srcHost[i].planes[0].height, dstHost[i].planes[0].height) != 0 ? px : 0;
+                const NVCVImagePlaneStrided &in = srcHost[i].planes[0], &out = dstHost[i].planes[0];
+                const int64_t                px = (int64_t)out.width * out.height;
+                all += px;
+                walked += CubicWalks<C>(in.width, in.height, out.width, out.height) ? px : 0;
             }
-            int total = 2 * stripPixels > allPixels ? BuildVarTiles(tiles, dstHost, first, count, kPatchTileW, 4 * kCubicStripRows) : 0;
+            int total = 2 * walked > all ? BuildVarTiles(tiles, dstHost, first, count, kPatchTileW, 4 * kCubicBatchRows) : 0;
             if (total >= 8 * 256)
             {
-                auto kernel = RowsAreOdd<C>(srcHost + first, count) ? ResizeCubicStripU8VarShapeKernel<C, C != 4>
-                                                                    : ResizeCubicStripU8VarShapeKernel<C, false>;
+                auto kernel = RowsAreOdd<C>(srcHost + first, count) ? ResizeCubicWalkU8VarShapeKernel<C, C != 4>
+                                                                    : ResizeCubicWalkU8VarShapeKernel<C, false>;
                 hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a, tiles);
-                CheckLaunch("ResizeCubicStripU8VarShapeKernel");
+                CheckLaunch("ResizeCubicWalkU8VarShapeKernel");
                 continue;
             }
         }

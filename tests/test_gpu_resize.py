@@ -83,11 +83,11 @@ def test_tensor_cubic_reduction(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
 
 
-# 8-bit bicubic at vertical scales of 1/2 to 2 runs as strips of 16 rows per wave once the launch has 2048 strips: the
-# benchmark's shape, ragged widths and heights, scale 2 exactly (every window advances by 2), 1.25, an enlargement
-# beyond 2 vertically (every strip takes the row-by-row path), horizontal enlargement with vertical reduction
+# 8-bit bicubic at vertical scales up to 4 walks the source rows, 4 to 32 output rows per wave: the benchmark's shape, ragged
+# widths and heights, scale 2 exactly (every window advances by 2), 1.25, an enlargement beyond 2, horizontal enlargement with
+# vertical reduction
 STRIPS = [(sw, sh, dw, dh, CUBIC, n, np.uint8, c)
-          for c in (3, 4, 1)  # (one channel stays with wave patches at these sizes too)
+          for c in (3, 4, 1)
           for (sw, sh, dw, dh, n) in [(1920, 1080, 1280, 720, 3), (1917, 1083, 1283, 719, 3), (1024, 1408, 512, 704, 8),
                                       (1600, 900, 1280, 720, 3), (640, 360, 1000, 1100, 2), (300, 1080, 700, 720, 6),
                                       # enlargements: by 1.5, by 2 exactly (the limit of the enlarging strips), by 1.2 with
@@ -99,6 +99,23 @@ STRIPS = [(sw, sh, dw, dh, CUBIC, n, np.uint8, c)
 @pytest.mark.parametrize("row", STRIPS, ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensor_cubic_u8_strips(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
+
+
+# The same at its limits: outputs one column short of a wave, a wave and one more (the last tile overlaps its neighbour); rows of
+# 16 bytes and of 8; four source rows; vertical scale 4 and a little more; horizontal scales on both sides of 1.3 and 3.9
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("shape", [(40, 30, 63, 67, 64), (40, 30, 64, 67, 64), (40, 30, 65, 67, 32), (200, 31, 257, 61, 64), (254, 64, 255, 64, 64),
+                                   (9, 4, 71, 64, 64), (6, 9, 66, 33, 128), (90, 256, 68, 64, 64), (90, 260, 68, 64, 64), (129, 70, 99, 66, 64),
+                                   (260, 70, 66, 66, 64), (270, 70, 66, 66, 64), (4, 40, 4, 71, 256), (333, 5, 999, 640, 2), (600, 70, 154, 66, 64), (610, 70, 154, 66, 64),
+                                   (9, 40, 128, 64, 64), (165, 40, 127, 64, 64)],
+                         ids=lambda sh: "%dx%d-%dx%d-n%d" % sh)
+def test_tensor_cubic_u8_walks(cv, orc, gpu, shape, c):
+    sw, sh, dw, dh, n = shape
+    src = make_input(orc, (n, sh, sw, c), np.uint8, 0x11 + sw + dw + c)
+    out = torch.full((n, dh, dw, c), 7, dtype=torch.uint8, device="cuda")
+    cv.Resize()(None, cv.Tensor.from_torch(torch.from_numpy(src).cuda(), "NHWC"), cv.Tensor.from_torch(out, "NHWC"), CUBIC)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), CUBIC, threads=8))
 
 
 # 8-bit nearest neighbour enlarging by 1.5 or more horizontally (and not reducing vertically) runs as strips once the
@@ -312,8 +329,8 @@ def test_varshape_nearest_u8_strips(cv, K, orc, gpu, c):
         check(res, a[None], (h, w), NEAREST, orc, varshape=True)
 
 
-# large image batches of 8-bit bicubic resizes of 3 and 4 channels run in the tensor kernels' strips (64 x 64 tiles,
-# 2048 and more): reductions up to 2, enlargements up to 2, and a few images outside both among them
+# large image batches of 8-bit bicubic resizes of 3 and 4 channels walk the source rows like the tensor kernels (64 x 64
+# tiles, 2048 and more): reductions up to 2, enlargements up to 2, and a few images beyond among them
 @pytest.mark.parametrize("c", [3, 4])
 def test_varshape_cubic_u8_strips(cv, K, orc, gpu, c):
     rng = np.random.default_rng(41 + c)
