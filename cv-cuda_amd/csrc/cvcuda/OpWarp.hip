@@ -473,6 +473,13 @@ __device__ __forceinline__ bool TapsInside(float limX, float limY, const float (
     return (ux < __float_as_uint(limX)) & (uy < __float_as_uint(limY)); // bitwise on purpose: no branch
 }
 
+template<int INTERP>
+__device__ __forceinline__ bool TapInside(float limX, float limY, float sx, float sy)
+{
+    constexpr float lo = INTERP == NVCV_INTERP_CUBIC ? 1.f : (INTERP == NVCV_INTERP_NEAREST ? -.5f : 0.f);
+    return (__float_as_uint(sx - lo) < __float_as_uint(limX)) & (__float_as_uint(sy - lo) < __float_as_uint(limY));
+}
+
 // Exclusive upper limit of floor(v) - lo along an axis of `size` pixels; 0 (no sample passes) when the
 // image is smaller than the tap span.
 template<int INTERP>
@@ -830,20 +837,21 @@ __device__ __forceinline__ uint32_t SampleNearBorderCubicQ14(const Img &im, cons
     return BlendCubicQ14<C>(r, sx, sy);
 }
 
-// Whether the image has room for the windows of SampleClampedCubicQ14, and they pay. They take a lane's samples one after the
-// other, which a launch that fills the chip hides and a small one waits for. One and four channels gain at any size. Three
-// channels, whose windows take the most instructions, gain under a replicating border from 256 blocks on (one 320 x 240, 75
-// blocks, 6.9 us with SampleNearBorderCubicQ14 and 8.1 with windows; one 640 x 480, 300 blocks, 9.9 and 9.2; 32 x 1280 x 780 202
-// and 158), and under a constant one, where lanes outside the image take no part and the colour's share is work of its own,
-// only in large launches of small images, of which the edge is the larger part (32 x 256 x 256 20.7 and 19.3, in perspective 26.6
-// and 22.5; 16 x 500 x 333 24.4 and 23.6; but one 320 x 240 6.4 and 8.0; one 1080p 14.5 and 15.6, 4 x 1283 x 721 20.5 and 22.0, 32 x
-// 1280 x 780 113.7 and 112.5).
+// Whether the image has room for the windows of SampleClampedCubicQ14, and they pay where a lane takes its own samples, one
+// after the other, which a launch that fills the chip hides and a small one waits for. One and four channels gain at any
+// size. Three channels, whose windows take the most instructions, gain (under a replicating border; under a constant one waves
+// list their samples at the edge) from 256 blocks on: one 320 x 240, 75 blocks, 6.9 us with SampleNearBorderCubicQ14 and 8.1 with
+// windows; one 640 x 480, 300 blocks, 9.9 and 9.2; 32 x 1280 x 780 202 and 158.
 template<int C>
-__device__ __forceinline__ bool ClampedCubicPays(const Img &im, bool constant)
+__device__ __forceinline__ bool ClampedCubicFits(const Img &im)
 {
-    return im.w >= 4 && __mul24(im.h - 1, im.row) + im.w * C >= 16
-        && (C != 3 || gridDim.x * gridDim.y * gridDim.z >= (constant ? 2048u : 256u))
-        && (C != 3 || !constant || __umul24(im.w, im.h) <= 1u << 18);
+    return im.w >= 4 && __mul24(im.h - 1, im.row) + im.w * C >= 16;
+}
+
+template<int C>
+__device__ __forceinline__ bool ClampedCubicPays(const Img &im)
+{
+    return ClampedCubicFits<C>(im) && (C != 3 || gridDim.x * gridDim.y * gridDim.z >= 256u);
 }
 
 // SampleNearBorderCubicQ14 under a constant or replicating border: 4 loads per sample instead of 16. A row is the window of
@@ -1087,45 +1095,203 @@ __device__ __forceinline__ void SampleAllOutside(const WarpArgs &a, float sx, fl
     }
 }
 
-// 8-bit pixels of 1, 3 or 4 channels have straight-line samplers for samples next to the image's edge.
-template<class T, int C>
-constexpr bool kNearBorderForms = std::is_same_v<T, uint8_t> && (C == 1 || C == 3 || C == 4);
-
-// Whether a lane's samples can take them: an image of 4 bytes or more within the 24-bit offsets (the caller's test),
-// every coordinate small enough for the sampler's integer conversion (bilinear: times 2^15 below 2^30; bicubic:
-// below 2^24; nearest: any) and, for the three modes that mirror or repeat the image, every tap no farther than one
-// image size outside it (BorderFold; with a margin of two pixels for the widest tap window).
+// SampleWithBorder for a sample that NearBorderForm lets through: all taps are requested before the first is used, at indices
+// folded into the image, and replaced by the colour where they were outside under a constant border. The weights and the order
+// of the sum are SampleWithBorder's.
 template<class T, int C, int INTERP>
-__device__ __forceinline__ bool NearBorderForm(const Img &im, const WarpArgs &a, const float (&sx)[kPxPerLane],
-                                               const float (&sy)[kPxPerLane])
+__device__ __forceinline__ void SampleNearBorder(const Img &im, const WarpArgs &a, const BorderFold &fx, const BorderFold &fy, float sx,
+                                                 float sy, T (&out)[C])
 {
-    if constexpr (!kNearBorderForms<T, C>)
+    constexpr int N = INTERP == NVCV_INTERP_CUBIC ? 4 : INTERP == NVCV_INTERP_LINEAR ? 2 : 1;
+    const bool    constant = a.border == NVCV_BORDER_CONSTANT;
+    const float   half = INTERP == NVCV_INTERP_NEAREST ? .5f : 0.f;
+    const int     x1 = FloorToInt(sx + half), y1 = FloorToInt(sy + half), x = x1 - (N == 4), y = y1 - (N == 4);
+    uint32_t      at[N];
+    bool          inX[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
     {
-        return false;
+        at[i]  = (uint32_t)Fold(fx, x + i) * (uint32_t)sizeof(Vec<T, C>);
+        inX[i] = (uint32_t)(x + i) < (uint32_t)im.w;
+    }
+    Vec<T, C> p[N][N];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+    {
+        const uint32_t row = (uint32_t)__mul24(Fold(fy, y + j), im.row);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+        {
+            p[j][i] = *reinterpret_cast<const Vec<T, C> *>(im.base + (row + at[i]));
+        }
+    }
+    float t[N][N][C];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+    {
+        const bool inY = (uint32_t)(y + j) < (uint32_t)im.h;
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+        {
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+            {
+                t[j][i][c] = constant && !(inX[i] && inY) ? (float)BorderValueAs<T>(a.bval[c]) : (float)p[j][i].v[c];
+            }
+        }
+    }
+    if constexpr (INTERP == NVCV_INTERP_NEAREST)
+    {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+        {
+            out[c] = (T)t[0][0][c];
+        }
     }
     else
     {
-        constexpr float kScale = kCoordScale<T, INTERP>;
-        uint32_t        u = 0;
-        float           minX = sx[0], maxX = sx[0], minY = sy[0], maxY = sy[0];
+        float wx[4], wy[4], acc[C];
+        if constexpr (INTERP == NVCV_INTERP_LINEAR)
+        {
+            wx[0] = (x1 + 1) - sx;
+            wx[1] = sx - x1;
+            wy[0] = (y1 + 1) - sy;
+            wy[1] = sy - y1;
+        }
+        else
+        {
+            CubicCoeffs(sx - x1, wx);
+            CubicCoeffs(sy - y1, wy);
+        }
 #pragma unroll
-        for (int k = 0; k < kPxPerLane; ++k)
+        for (int c = 0; c < C; ++c)
         {
-            u    = max(u, max(__float_as_uint(sx[k]) & 0x7fffffffu, __float_as_uint(sy[k]) & 0x7fffffffu));
-            minX = fminf(minX, sx[k]);
-            maxX = fmaxf(maxX, sx[k]);
-            minY = fminf(minY, sy[k]);
-            maxY = fmaxf(maxY, sy[k]);
+            acc[c] = 0.f;
         }
-        const uint32_t limit = INTERP == NVCV_INTERP_LINEAR ? 0x4e800000u : (INTERP == NVCV_INTERP_CUBIC ? 0x4b800000u : 0x7f800000u);
-        bool           ok = u < limit && __mul24(im.h - 1, im.row) + im.w * C >= 4;
-        if (a.border > NVCV_BORDER_REPLICATE) // wave-uniform
+#pragma unroll
+        for (int j = 0; j < N; ++j)
         {
-            // taps reach from floor(v) - 1 to floor(v) + 2 at most: all of them within -(s - 1) .. 2s - 2
-            ok = ok && minX >= (float)(2 - im.w) * kScale && maxX < (float)(2 * im.w - 4) * kScale
-              && minY >= (float)(2 - im.h) * kScale && maxY < (float)(2 * im.h - 4) * kScale;
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+            {
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                {
+                    acc[c] += t[j][i][c] * (wx[i] * wy[j]);
+                }
+            }
         }
-        return ok;
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+        {
+            out[c] = SaturateCast<T>(acc[c]);
+        }
+    }
+}
+
+// 8-bit pixels of 1, 3 or 4 channels have samplers of their own for samples next to the image's edge.
+template<class T, int C>
+constexpr bool kNearBorderForms = std::is_same_v<T, uint8_t> && (C == 1 || C == 3 || C == 4);
+
+// Whether a lane's samples can take those or SampleNearBorder: an image within the 24-bit offsets (the caller's test; for the 8-bit
+// forms also of 4 bytes or more), coordinates small enough for the samplers' integer conversions (8-bit bilinear: times 2^15
+// below 2^30; else below 2^24) and, for the three modes that mirror or repeat the image, every tap no farther than one image
+// size outside it (BorderFold; with a margin of two pixels for the widest tap window).
+template<class T, int C, int INTERP, int N>
+__device__ __forceinline__ bool NearBorderForm(const Img &im, const WarpArgs &a, const float (&sx)[N], const float (&sy)[N])
+{
+    constexpr float kScale = kCoordScale<T, INTERP>;
+    uint32_t        u = 0;
+    float           minX = sx[0], maxX = sx[0], minY = sy[0], maxY = sy[0];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+    {
+        u    = max(u, max(__float_as_uint(sx[k]) & 0x7fffffffu, __float_as_uint(sy[k]) & 0x7fffffffu));
+        minX = fminf(minX, sx[k]);
+        maxX = fmaxf(maxX, sx[k]);
+        minY = fminf(minY, sy[k]);
+        maxY = fmaxf(maxY, sy[k]);
+    }
+    bool ok = u < (kFixedPoint<T, INTERP> ? 0x4e800000u : 0x4b800000u)
+           && (!kNearBorderForms<T, C> || __mul24(im.h - 1, im.row) + im.w * C >= 4);
+    if (a.border > NVCV_BORDER_REPLICATE) // wave-uniform
+    {
+        // taps reach from floor(v) - 1 to floor(v) + 2 at most: all of them within -(s - 1) .. 2s - 2
+        ok = ok && minX >= (float)(2 - im.w) * kScale && maxX < (float)(2 * im.w - 4) * kScale
+          && minY >= (float)(2 - im.h) * kScale && maxY < (float)(2 * im.h - 4) * kScale;
+    }
+    return ok;
+}
+
+// The colour of a constant border as the dwords of a pixel.
+template<class T, int C>
+__device__ __forceinline__ void BorderDwords(const WarpArgs &a, uint32_t (&w)[(C * sizeof(T) + 3) / 4])
+{
+    T v[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+    {
+        v[c] = BorderValueAs<T>(a.bval[c]);
+    }
+#pragma unroll
+    for (int d = 0; d < (int)((C * sizeof(T) + 3) / 4); ++d)
+    {
+        w[d] = 0;
+    }
+    __builtin_memcpy(w, v, C * sizeof(T));
+}
+
+// Which launches' waves list their samples at the image's edge (WarpTile): none, those under a constant border, all. 8-bit
+// bilinear and nearest samples are too few instructions for it (32 x 1280 x 780 u8x3 54 us, listed 60), and so is copying
+// pixels. 8-bit bicubic ones pay where what lies all outside takes no part and with three channels (40 images of 443 .. 974 x 412 ..
+// 446 64.3 -> 60.5, 16 x 201 x 332 in perspective 15.3 -> 12.5; one channel, 49 x 1139 x 681: 98 and, listed, 112; replicating, one
+// 320 x 240 x 3 7.2 and 8.8, 25 x 283 x 733 x 4 31.3 and 32.6).
+enum EdgeLists
+{
+    kNoLists,
+    kConstantBorderLists,
+    kAllLists
+};
+
+template<class T, int C, int INTERP>
+constexpr EdgeLists kEdgeLists = INTERP == NVCV_INTERP_NEAREST        ? kNoLists
+                               : !std::is_same_v<T, uint8_t>          ? kAllLists
+                               : INTERP == NVCV_INTERP_CUBIC && C == 3 ? kConstantBorderLists
+                                                                      : kNoLists;
+
+// A sample at the image's edge that NearBorderForm lets through, as the dwords of its pixel.
+template<class T, int C, int INTERP>
+__device__ __forceinline__ void SampleNearEdge(const Img &im, const WarpArgs &a, uint32_t borderPx, float sx, float sy,
+                                               uint32_t (&w)[(C * sizeof(T) + 3) / 4])
+{
+    const bool       constant = a.border == NVCV_BORDER_CONSTANT;
+    const BorderFold foldX = MakeBorderFold(a.border, im.w), foldY = MakeBorderFold(a.border, im.h);
+    if constexpr (!kNearBorderForms<T, C>)
+    {
+        T v[C];
+        SampleNearBorder<T, C, INTERP>(im, a, foldX, foldY, sx, sy, v);
+#pragma unroll
+        for (int d = 0; d < (int)((C * sizeof(T) + 3) / 4); ++d)
+        {
+            w[d] = 0;
+        }
+        __builtin_memcpy(w, v, C * sizeof(T));
+    }
+    else if constexpr (INTERP == NVCV_INTERP_LINEAR)
+    {
+        w[0] = SampleNearBorderQ15<C>(im, foldX, foldY, constant, borderPx, sx, sy);
+    }
+    else if constexpr (INTERP == NVCV_INTERP_NEAREST)
+    {
+        w[0] = SampleNearBorderNearest<C>(im, foldX, foldY, constant, borderPx, sx, sy);
+    }
+    else if (ClampedCubicFits<C>(im)) // uniform; (a constant border: kListEdges)
+    {
+        w[0] = SampleClampedCubicQ14<C>(im, true, borderPx, sx, sy);
+    }
+    else
+    {
+        w[0] = SampleNearBorderCubicQ14<C>(im, foldX, foldY, true, borderPx, sx, sy);
     }
 }
 
@@ -1142,7 +1308,7 @@ __device__ __forceinline__ bool NarrowTapsPay(const float (&m)[9])
 }
 
 // One 64 x 16 tile of the destination image `dst` (tile coordinates tx, ty), all 256 threads.
-template<class T, int C, int INTERP, bool PERSP>
+template<class T, int C, int INTERP, bool PERSP, bool LIST>
 __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const float (&m)[9], uint8_t *dst, int dstRow,
                                          int dstW, int dstH, int tx, int ty)
 {
@@ -1162,7 +1328,6 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     // rows too long or too many for 24-bit offset arithmetic go through the generic path
     // (and, in fixed point, coordinates too large for coordinate * 2^15 in 31 bits)
     const bool fits = (im.row | im.h) < (1 << 23) && (!kFixedPoint<T, INTERP> || (im.w | im.h) < (1 << 16));
-    bool       allInside = fits;
 #pragma unroll
     for (int k = 0; k < kPxPerLane; ++k)
     {
@@ -1171,8 +1336,13 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         py[k] = min(y0 + ly, dstH - 1);
     }
     MapCoords<PERSP>(m, px, py, sx, sy);
-    allInside = allInside & TapsInside<INTERP>(limX, limY, sx, sy);
-    if (allInside)
+    // the wave's pixels as rows, for the store (kPitch: neighbouring rows on other banks)
+    constexpr int kPitch = kWaveW * D + (D == 1 ? 8 : D == 2 ? 16 : D == 4 ? 24 : 0);
+    __shared__ __align__(16) uint32_t room[kThreads / 64][kPatch][kPitch];
+    auto     &rows = room[wave];
+    const int lane = threadIdx.x & 63;
+
+    auto sampleInside = [&]()
     {
         uint32_t w[kPxPerLane][D];
         auto sample = [&](auto form)
@@ -1204,19 +1374,141 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                 q[d][k] = w[k][d];
             }
         }
-    }
-    else if (fits && NearBorderForm<T, C, INTERP>(im, a, sx, sy))
+    };
+    auto place = [&](int k)
     {
-        // 8-bit pixels under a constant or replicating border: the border logic as selects, all four samples in
-        // flight (the generic loop below costs a wave that straddles the image's edge about 4 times as much)
-        if constexpr (kNearBorderForms<T, C>)
-        {
-            uint32_t borderPx = 0;
 #pragma unroll
-            for (int c = 0; c < C; ++c)
+        for (int d = 0; d < D; ++d)
+        {
+            rows[ly][(k * kPatch + lx) * D + d] = q[d][k];
+        }
+    };
+    if constexpr (LIST)
+    {
+        // ---- a wave that the image's edge passes through: its samples at the edge, usually fewer than 64 of the 256, are listed and,
+        // when all lanes have sampled as in the other waves (those with taps outside at a place inside), handed out to the
+        // lanes again; what is all outside under a constant border takes the colour. Where every lane went through all its four
+        // samples for one of them at the edge, such waves cost 2 to 5 times as much as others, and in a launch of small images a
+        // third are such: 3 x 258 x 271 f32x1 bicubic 16.0 -> 6.7 us, 7 x 318 x 538 f32x4 bilinear 14.6 -> 9.6, 3 x 646 x 752 f32x1 bilinear
+        // 9.7 -> 6.2, 40 x 1021 x 1523 of these 169 -> 145; 38 images of 75 .. 801 x 232 .. 359 u8x3 bicubic 36.3 -> 32.0.
+        const bool whole  = __builtin_amdgcn_ballot_w64(!fits || !TapsInside<INTERP>(limX, limY, sx, sy)) == 0;
+        __shared__ uint8_t list[kThreads / 64][64 * kPxPerLane];
+        uint32_t inside = 0xf, colour[D] = {}; // inside: bit k: sample k
+        int      edges  = 0;
+        if (!whole)
+        {
+            const bool constant = a.border == NVCV_BORDER_CONSTANT;
+            BorderDwords<T, C>(a, colour);
+            inside = 0;
+#pragma unroll
+            for (int k = 0; k < kPxPerLane; ++k)
             {
-                borderPx |= (uint32_t)BorderValueAs<T>(a.bval[c]) << (8 * c);
+                const bool in  = fits && TapInside<INTERP>(limX, limY, sx[k], sy[k]);
+                const bool out = constant && TapsOutside<INTERP>(im, sx[k] * (1.f / kScale), sy[k] * (1.f / kScale));
+                if (out)
+                {
+                    uint32_t w[D]; // (the tap itself, or taps whose weights add up to exactly 1; else their sum)
+                    __builtin_memcpy(w, colour, sizeof(w));
+                    if constexpr (INTERP != NVCV_INTERP_NEAREST && !kFixedPoint<T, INTERP>)
+                    {
+                        T v[C];
+                        SampleAllOutside<T, C, INTERP>(a, sx[k] * (1.f / kScale), sy[k] * (1.f / kScale), v);
+                        __builtin_memcpy(w, v, PB);
+                    }
+#pragma unroll
+                    for (int d = 0; d < D; ++d)
+                    {
+                        rows[ly][(k * kPatch + lx) * D + d] = w[d];
+                    }
+                }
+                const bool     edge = !in && !out && x0 + k * kPatch + lx < dstW && y0 + ly < dstH;
+                const uint64_t mask = __builtin_amdgcn_ballot_w64(edge);
+                if (edge)
+                {
+                    const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+                    list[wave][edges + before] = (uint8_t)(k * 64 + lane);
+                }
+                edges += __builtin_popcountll(mask);
+                inside |= in ? 1u << k : 0u;
+                sx[k] = in ? sx[k] : (INTERP == NVCV_INTERP_CUBIC ? 1.f : 0.f);
+                sy[k] = in ? sy[k] : (INTERP == NVCV_INTERP_CUBIC ? 1.f : 0.f);
             }
+            asm("" : "+v"(inside)); // (one register, not a mask for each sample)
+        }
+
+        if (__builtin_amdgcn_ballot_w64(inside != 0) != 0) // (then the place inside is one)
+        {
+            sampleInside();
+        }
+        if (whole)
+        {
+#pragma unroll
+            for (int k = 0; k < kPxPerLane; ++k)
+            {
+                place(k);
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (int k = 0; k < kPxPerLane; ++k)
+            {
+                if ((inside >> k) & 1)
+                {
+                    place(k);
+                }
+            }
+            WaveExchangeFence();
+            auto edgeSamples = [&](auto nearby) // the listed samples that NearBorderForm lets through, or the others; whether there are others
+            {
+                bool others = false;
+#pragma nounroll
+                for (int i = lane; i < edges; i += 64) // (once for most waves that have any)
+                {
+                    const int id = list[wave][i], at = (id >> 6) * kPatch + (id & (kPatch - 1)), line = (id >> 3) & (kPatch - 1);
+                    float     bx[1], by[1];
+                    MapCoord<PERSP>(m, x0 + at, y0 + line, bx[0], by[0]);
+                    if ((fits && NearBorderForm<T, C, INTERP>(im, a, bx, by)) != nearby.value)
+                    {
+                        others = true;
+                        continue;
+                    }
+                    uint32_t w[D] = {};
+                    if constexpr (nearby.value)
+                    {
+                        SampleNearEdge<T, C, INTERP>(im, a, colour[0], bx[0], by[0], w);
+                    }
+                    else
+                    {
+                        T v[C];
+                        SampleWithBorder<T, C, INTERP>(im, a, bx[0] * (1.f / kScale), by[0] * (1.f / kScale), v);
+                        __builtin_memcpy(w, v, PB);
+                    }
+#pragma unroll
+                    for (int d = 0; d < D; ++d)
+                    {
+                        rows[line][at * D + d] = w[d];
+                    }
+                }
+                return __builtin_amdgcn_ballot_w64(others) != 0;
+            };
+            if (edgeSamples(std::true_type{})) // (two loops: one with both samplers holds the registers of both)
+            {
+                edgeSamples(std::false_type{});
+            }
+        }
+    }
+    else
+    {
+        // Each lane takes its own samples, all four in flight.
+        if (fits & TapsInside<INTERP>(limX, limY, sx, sy))
+        {
+            sampleInside();
+        }
+        else if ((kNearBorderForms<T, C> || INTERP == NVCV_INTERP_NEAREST) && fits && NearBorderForm<T, C, INTERP>(im, a, sx, sy))
+        {
+            uint32_t colour[D];
+            BorderDwords<T, C>(a, colour);
             // under a constant border a lane whose samples lie outside with all their taps needs no pixel: whole
             // waves in the corners a rotation leaves empty
             const bool       constant = a.border == NVCV_BORDER_CONSTANT;
@@ -1232,7 +1524,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
                 for (int k = 0; k < kPxPerLane; ++k)
                 {
-                    if constexpr (INTERP == NVCV_INTERP_CUBIC)
+                    if constexpr (kFixedPointCubic<T, INTERP>)
                     {
                         T v[C];
                         SampleAllOutside<T, C, INTERP>(a, sx[k], sy[k], v);
@@ -1243,11 +1535,15 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                     }
                     else
                     {
-                        q[0][k] = borderPx; // the tap itself, or taps whose weights add up to exactly 1
+#pragma unroll
+                        for (int d = 0; d < D; ++d)
+                        {
+                            q[d][k] = colour[d]; // the tap itself, or taps whose weights add up to exactly 1
+                        }
                     }
                 }
             }
-            else if (INTERP == NVCV_INTERP_CUBIC && a.border <= NVCV_BORDER_REPLICATE && ClampedCubicPays<C>(im, constant)) // uniform
+            else if (INTERP == NVCV_INTERP_CUBIC && a.border <= NVCV_BORDER_REPLICATE && ClampedCubicPays<C>(im)) // uniform
             {
                 // one sample at a time (all four at once took 143 registers, which every wave of the launch would have held;
                 // held to the 64 of full occupancy the u8x3 kernel spills and loses 1 to 2 %)
@@ -1261,11 +1557,11 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                     uint32_t v;
                     if (constant)
                     {
-                        v = SampleClampedCubicQ14<C>(im, true, borderPx, bx, by);
+                        v = SampleClampedCubicQ14<C>(im, true, colour[0], bx, by);
                     }
                     else
                     {
-                        v = SampleClampedCubicQ14<C>(im, false, borderPx, bx, by);
+                        v = SampleClampedCubicQ14<C>(im, false, colour[0], bx, by);
                     }
 #pragma unroll
                     for (int j = 0; j < kPxPerLane; ++j)
@@ -1279,78 +1575,85 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
                 for (int k = 0; k < kPxPerLane; ++k)
                 {
-                    if constexpr (INTERP == NVCV_INTERP_LINEAR)
+                    if constexpr (kFixedPoint<T, INTERP>)
                     {
-                        q[0][k] = SampleNearBorderQ15<C>(im, foldX, foldY, constant, borderPx, sx[k], sy[k]);
+                        q[0][k] = SampleNearBorderQ15<C>(im, foldX, foldY, constant, colour[0], sx[k], sy[k]);
                     }
-                    else if constexpr (INTERP == NVCV_INTERP_CUBIC)
+                    else if constexpr (kFixedPointCubic<T, INTERP>)
                     {
-                        q[0][k] = SampleNearBorderCubicQ14<C>(im, foldX, foldY, constant, borderPx, sx[k], sy[k]);
+                        q[0][k] = SampleNearBorderCubicQ14<C>(im, foldX, foldY, constant, colour[0], sx[k], sy[k]);
+                    }
+                    else if constexpr (kNearBorderForms<T, C>)
+                    {
+                        q[0][k] = SampleNearBorderNearest<C>(im, foldX, foldY, constant, colour[0], sx[k], sy[k]);
                     }
                     else
                     {
-                        q[0][k] = SampleNearBorderNearest<C>(im, foldX, foldY, constant, borderPx, sx[k], sy[k]);
+                        T        v[C];
+                        uint32_t w[D] = {};
+                        SampleNearBorder<T, C, INTERP>(im, a, foldX, foldY, sx[k], sy[k], v);
+                        __builtin_memcpy(w, v, PB);
+#pragma unroll
+                        for (int d = 0; d < D; ++d)
+                        {
+                            q[d][k] = w[d];
+                        }
                     }
                 }
             }
         }
-    }
-    else
-    {
-#pragma nounroll
-        for (int k = 0; k < kPxPerLane; ++k)
+        else
         {
-            // position and coordinates recomputed rather than indexed, results placed by selects: a
-            // run-time index would put the arrays in scratch memory
-            const int dx = min(x0 + k * kPatch + lx, dstW - 1), dy = min(y0 + ly, dstH - 1);
-            float     bx, by;
-            MapCoord<PERSP>(m, dx, dy, bx, by);
-            bx *= 1.f / kScale;
-            by *= 1.f / kScale;
-            T v[C];
-            if (a.border == NVCV_BORDER_CONSTANT && TapsOutside<INTERP>(im, bx, by))
+#pragma nounroll
+            for (int k = 0; k < kPxPerLane; ++k)
             {
-                SampleAllOutside<T, C, INTERP>(a, bx, by, v);
-            }
-            else
-            {
-                SampleWithBorder<T, C, INTERP>(im, a, bx, by, v);
-            }
-            uint32_t w[D] = {};
-            __builtin_memcpy(w, v, PB);
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-            {
-                asm("" : "+v"(w[d]));
-#pragma unroll
-                for (int j = 0; j < kPxPerLane; ++j)
+                // position and coordinates recomputed rather than indexed, results placed by selects: a
+                // run-time index would put the arrays in scratch memory
+                const int dx = min(x0 + k * kPatch + lx, dstW - 1), dy = min(y0 + ly, dstH - 1);
+                float     bx, by;
+                MapCoord<PERSP>(m, dx, dy, bx, by);
+                bx *= 1.f / kScale;
+                by *= 1.f / kScale;
+                T v[C];
+                if (a.border == NVCV_BORDER_CONSTANT && TapsOutside<INTERP>(im, bx, by))
                 {
-                    q[d][j] = k == j ? w[d] : q[d][j];
+                    SampleAllOutside<T, C, INTERP>(a, bx, by, v);
+                }
+                else
+                {
+                    SampleWithBorder<T, C, INTERP>(im, a, bx, by, v);
+                }
+                uint32_t w[D] = {};
+                __builtin_memcpy(w, v, PB);
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                {
+                    asm("" : "+v"(w[d]));
+#pragma unroll
+                    for (int j = 0; j < kPxPerLane; ++j)
+                    {
+                        q[d][j] = k == j ? w[d] : q[d][j];
+                    }
                 }
             }
         }
-    }
-
-    // ---- store. Pixels of 12 and 16 bytes go through the wave's own part of LDS and leave as the rows they form, 16 bytes
-    // per lane: 384 or 512 contiguous bytes of each row. One pixel per lane wrote 96 or 128 bytes of 8 rows per instruction,
-    // with a partly written sector at both ends of most: 4 x 1283 x 721 f32x3 nearest 30.5 -> 19.4 us, bilinear 28.4 -> 24.3;
-    // f32x4 33.1 -> 22.0 and 30.4 -> 27.3 (of rows that start at sectors, 1280 x 720: f32x3 22.3 -> 16.6, f32x4 5 % slower when
-    // small, one 1280 x 720 5.4 -> 5.7, and as before when large; a second form of the store for these cost all others 3 to 5 %).
-    if constexpr (PB >= 12)
-    {
-        constexpr int kChunks = kWaveW * PB / 16, kPitch = kWaveW * D + (D == 4 ? 32 : 0); // (neighbouring rows on other banks)
-        __shared__ __align__(16) uint32_t rows[kThreads / 64][kPatch][kPitch];
 #pragma unroll
         for (int k = 0; k < kPxPerLane; ++k)
         {
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-            {
-                rows[wave][ly][(k * kPatch + lx) * D + d] = q[d][k];
-            }
+            place(k);
         }
-        WaveExchangeFence();
-        const int lane = threadIdx.x & 63, dwords = min(dstW - x0, kWaveW) * D; // of a row
+    }
+    WaveExchangeFence();
+
+    // ---- store. Pixels of 12 and 16 bytes leave as the rows they form, 16 bytes per lane: 384 or 512 contiguous bytes of each
+    // row. One pixel per lane wrote 96 or 128 bytes of 8 rows per instruction, with a partly written sector at both ends of
+    // most: 4 x 1283 x 721 f32x3 nearest 30.5 -> 19.4 us, bilinear 28.4 -> 24.3; f32x4 33.1 -> 22.0 and 30.4 -> 27.3 (of rows that
+    // start at sectors, 1280 x 720: f32x3 22.3 -> 16.6, f32x4 5 % slower when small, one 1280 x 720 5.4 -> 5.7, and as before when
+    // large; a second form of the store for these cost all others 3 to 5 %).
+    if constexpr (PB >= 12)
+    {
+        constexpr int kChunks = kWaveW * PB / 16;
+        const int dwords = min(dstW - x0, kWaveW) * D; // of a row
         uint8_t  *to = dst + (int64_t)y0 * dstRow + (int64_t)x0 * PB;
 #pragma unroll
         for (int i = 0; i < D; ++i)
@@ -1360,7 +1663,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             {
                 continue;
             }
-            const uint4    v    = *reinterpret_cast<const uint4 *>(&rows[wave][row][at]);
+            const uint4    v    = *reinterpret_cast<const uint4 *>(&rows[row][at]);
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
             uint8_t       *p    = to + (uint32_t)(row * dstRow + at * 4);
             if (at + 4 <= dwords)
@@ -1382,37 +1685,21 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         }
         return;
     }
-    // Smaller pixels change lanes so that a lane holds 4 consecutive pixels of a row. One dword each: through the wave's own
-    // part of LDS (rows of 40 dwords: every quarter of a wave on banks of its own), after which lane (lx, ly) holds columns
-    // 4 lx .. 4 lx + 3 of row ly. These kernels wait for vector instructions; moves and selects between lanes took 20 of
-    // them, and left a row's pieces in another order than the lanes'.
-    int dx0;
-    if constexpr (D == 1)
+    // Of smaller pixels lane (lx, ly) stores columns 4 lx .. 4 lx + 3 of row ly. (Through LDS: these kernels wait for vector
+    // instructions; moves and selects between lanes took 20 for each dword of a pixel, and left a row's pieces in another
+    // order than the lanes'.)
+    const int dx0 = x0 + 4 * lx;
+    if constexpr (PB < 12)
     {
-        __shared__ __align__(16) uint32_t exchange[kThreads / 64][kPatch][40];
 #pragma unroll
-        for (int k = 0; k < kPxPerLane; ++k)
+        for (int k = 0; k < 4; ++k)
         {
-            exchange[wave][ly][k * kPatch + lx] = q[0][k];
-        }
-        WaveExchangeFence();
-        const uint4 r = *reinterpret_cast<const uint4 *>(&exchange[wave][ly][4 * lx]);
-        q[0][0]       = r.x;
-        q[0][1]       = r.y;
-        q[0][2]       = r.z;
-        q[0][3]       = r.w;
-        dx0           = x0 + 4 * lx;
-    }
-    else
-    {
-        // the 4 lanes lx & ~3 .. | 3 hold columns 4g .. 4g+3 (g = lx >> 2) of row ly in each of the wave's 4 patches; after
-        // a 4x4 transpose lane i = lx & 3 holds those 4 columns of patch 4w + i
 #pragma unroll
-        for (int d = 0; d < D; ++d)
-        {
-            QuadTranspose(q[d], lx & 3);
+            for (int d = 0; d < D; ++d)
+            {
+                q[d][k] = rows[ly][(4 * lx + k) * D + d];
+            }
         }
-        dx0 = x0 + (lx & 3) * kPatch + (lx & 4);
     }
     const int dy = y0 + ly;
     if (dy >= dstH || dx0 >= dstW)
@@ -1508,7 +1795,7 @@ __device__ __forceinline__ void LoadMatrix(const WarpArgs &a, int image, float s
     }
 }
 
-template<class T, int C, int INTERP, bool PERSP>
+template<class T, int C, int INTERP, bool PERSP, bool LIST>
 __global__ __launch_bounds__(kThreads) void WarpTensor(const WarpArgs a)
 {
     const int n  = blockIdx.z;
@@ -1519,10 +1806,10 @@ __global__ __launch_bounds__(kThreads) void WarpTensor(const WarpArgs a)
     {
         m[i] = a.m[i];
     }
-    WarpTile<T, C, INTERP, PERSP>(im, a, m, a.dst + n * a.dstN, a.dstRow, a.dstW, a.dstH, blockIdx.x, blockIdx.y);
+    WarpTile<T, C, INTERP, PERSP, LIST>(im, a, m, a.dst + n * a.dstN, a.dstRow, a.dstW, a.dstH, blockIdx.x, blockIdx.y);
 }
 
-template<class T, int C, int INTERP, bool PERSP>
+template<class T, int C, int INTERP, bool PERSP, bool LIST>
 __global__ __launch_bounds__(kThreads) void WarpVarShape(const WarpArgs a, const VarTiles tiles)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
@@ -1533,16 +1820,16 @@ __global__ __launch_bounds__(kThreads) void WarpVarShape(const WarpArgs a, const
     float                       m[9];
     LoadMatrix<PERSP>(a, tc.image, kCoordScale<T, INTERP>, m);
     const Img im = {AsGlobal(s.basePtr), s.rowStride, s.width, s.height};
-    WarpTile<T, C, INTERP, PERSP>(im, a, m, AsGlobal(d.basePtr), d.rowStride, d.width, d.height, tc.tx, tc.ty);
+    WarpTile<T, C, INTERP, PERSP, LIST>(im, a, m, AsGlobal(d.basePtr), d.rowStride, d.width, d.height, tc.tx, tc.ty);
 }
 
-template<class T, int C, int INTERP, bool PERSP>
+template<class T, int C, int INTERP, bool PERSP, bool LIST>
 void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, hipStream_t stream)
 {
     if (dstHost == nullptr)
     {
         dim3 grid(DivUp(a.dstW, kTileW), DivUp(a.dstH, kTileH), N);
-        hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST>), grid, dim3(kThreads), 0, stream, a);
         CheckLaunch("WarpTensor");
         return;
     }
@@ -1552,7 +1839,7 @@ void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, 
         int      total = BuildVarTiles(tiles, dstHost, first, std::min(kMaxTileImages, N - first), kTileW, kTileH);
         if (total > 0)
         {
-            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
             CheckLaunch("WarpVarShape");
         }
     }
@@ -1561,13 +1848,16 @@ void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, 
 template<class T, int C, int INTERP>
 void Launch(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, hipStream_t stream)
 {
-    if (a.perspective)
+    constexpr EdgeLists kLists = kEdgeLists<T, C, INTERP>;
+    if (kLists == kAllLists || (kLists == kConstantBorderLists && a.border == NVCV_BORDER_CONSTANT))
     {
-        LaunchMap<T, C, INTERP, true>(a, N, dstHost, stream);
+        constexpr bool kList = kLists != kNoLists;
+        a.perspective ? LaunchMap<T, C, INTERP, true, kList>(a, N, dstHost, stream) : LaunchMap<T, C, INTERP, false, kList>(a, N, dstHost, stream);
     }
     else
     {
-        LaunchMap<T, C, INTERP, false>(a, N, dstHost, stream);
+        constexpr bool kList = kLists == kAllLists;
+        a.perspective ? LaunchMap<T, C, INTERP, true, kList>(a, N, dstHost, stream) : LaunchMap<T, C, INTERP, false, kList>(a, N, dstHost, stream);
     }
 }
 

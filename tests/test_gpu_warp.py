@@ -164,6 +164,30 @@ def rotation(w, h, deg, s):
     return [c, -sn, cx - c * cx + sn * cy, sn, c, cy - sn * cx - c * cy]
 
 
+# waves that the image's edge passes through list their samples there and share them out: images smaller than a wave's part
+# and a little larger, all borders, with many, few and no samples inside
+@pytest.mark.parametrize("size", [(1, 1), (3, 2), (9, 8), (33, 9), (40, 70), (65, 17)], ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("dt", [np.uint8, np.uint16, np.int16, np.float32])
+def test_samples_at_the_edge(cv, orc, gpu, dt, c, size):
+    w, h = size
+    src = (orc.fill_u8((2, h, w, c), 5 + w + c).astype(np.float64) * (200 if dt in (np.uint16, np.int16) else 1)
+           - (20000 if dt == np.int16 else 0)).astype(dt)
+    tin = cv.Tensor.from_numpy(src, "NHWC")
+    dh, dw = h + 11, w + 14
+    tout = cv.Tensor.alloc([2, dh, dw, c], dt, "NHWC")
+    for m in ([0.9, -0.5, 6.3, 0.5, 0.9, -2.7], [1.0, 0.0, -0.5, 0.0, 1.0, 3.0], [0.3, 0.1, 700.0, 0.0, 0.4, -300.0]):
+        for interp in (NEAREST, LINEAR, CUBIC):
+            for border in range(5):
+                cv.WarpAffine(0)(None, tin, tout, m, interp | INVERSE_MAP, border, (9, 200, 31, 77))
+                torch.cuda.synchronize()
+                dev = orc.warp(src, (dh, dw), np.asarray(m, np.float32), interp, border, (9, 200, 31, 77), variant=device_variant(interp, dt))
+                if dt == np.float32:
+                    assert np.abs(tout.numpy() - dev).max() <= 1e-3, (m, interp, border)  # (as above)
+                else:
+                    np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((m, interp, border)))
+
+
 @pytest.mark.parametrize("dt,c", [(np.uint8, 3), (np.uint8, 1), (np.uint8, 4), (np.uint16, 3), (np.int16, 4),
                                   (np.float32, 1), (np.float32, 3)])
 @pytest.mark.parametrize("interp", [NEAREST, LINEAR, CUBIC])
