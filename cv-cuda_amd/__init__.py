@@ -130,6 +130,10 @@ class Tensor(_Handle):
     @classmethod
     def alloc(cls, shape, dtype, layout, base_align=0, row_align=0):
         """Library-allocated tensor (hipMalloc through the default allocator)."""
+        if len(shape) <= capi.NVCV_TENSOR_MAX_RANK and len(layout) <= capi.NVCV_TENSOR_MAX_RANK:
+            status, handle = capi.native.tensor_alloc(shape, _as_dtype(dtype), layout, base_align, row_align)
+            check(status)
+            return cls(handle)
         reqs = cls.requirements(shape, dtype, layout, base_align, row_align)
         h = C.c_void_p()
         check(_nv.nvcvTensorConstruct(C.byref(reqs), None, C.byref(h)))
@@ -388,6 +392,7 @@ class ImageBatchVarShape(_Handle):
 # operators ---------------------------------------------------------------------------------------
 class _Operator:
     _create = None
+    _native = 0  # which of csrc/python/Native.cpp's calls it is (none)
 
     def __init__(self, *args):
         h = C.c_void_p()
@@ -412,6 +417,7 @@ def _h(obj):
 
 class ResizeCropConvertReformat(_Operator):
     _create = "cvcudaResizeCropConvertReformatCreate"
+    _native = 6
 
     def __call__(self, stream, inp, out, resize_dim, interp, crop_pos, manip=K.CHANNEL_NO_OP, scale=1.0,
                  offset=0.0, src_cast=True):
@@ -433,6 +439,7 @@ class ResizeCropConvertReformat(_Operator):
 
 class Resize(_Operator):
     _create = "cvcudaResizeCreate"
+    _native = 1
 
     def __call__(self, stream, inp, out, interp):
         fn = _cv.cvcudaResizeVarShapeSubmit if isinstance(inp, ImageBatchVarShape) else _cv.cvcudaResizeSubmit
@@ -441,6 +448,7 @@ class Resize(_Operator):
 
 class CvtColor(_Operator):
     _create = "cvcudaCvtColorCreate"
+    _native = 2
 
     def __call__(self, stream, inp, out, code):
         fn = _cv.cvcudaCvtColorVarShapeSubmit if isinstance(inp, ImageBatchVarShape) else _cv.cvcudaCvtColorSubmit
@@ -449,6 +457,7 @@ class CvtColor(_Operator):
 
 class Normalize(_Operator):
     _create = "cvcudaNormalizeCreate"
+    _native = 5
 
     def __call__(self, stream, inp, base, scale, out, global_scale=1.0, shift=0.0, epsilon=0.0, flags=0):
         fn = _cv.cvcudaNormalizeVarShapeSubmit if isinstance(inp, ImageBatchVarShape) else _cv.cvcudaNormalizeSubmit
@@ -458,6 +467,7 @@ class Normalize(_Operator):
 
 class Reformat(_Operator):
     _create = "cvcudaReformatCreate"
+    _native = 3
 
     def __call__(self, stream, inp, out):
         check(_cv.cvcudaReformatSubmit(self.handle, stream_ptr(stream), _h(inp), _h(out)))
@@ -465,6 +475,7 @@ class Reformat(_Operator):
 
 class CropFlipNormalizeReformat(_Operator):
     _create = "cvcudaCropFlipNormalizeReformatCreate"
+    _native = 7
 
     def __call__(self, stream, inp, out, crop_rect, border, border_value, flip_code, base, scale, global_scale=1.0,
                  shift=0.0, epsilon=0.0, flags=0):
@@ -475,6 +486,7 @@ class CropFlipNormalizeReformat(_Operator):
 
 class ConvertTo(_Operator):
     _create = "cvcudaConvertToCreate"
+    _native = 4
 
     def __call__(self, stream, inp, out, alpha=1.0, beta=0.0):
         check(_cv.cvcudaConvertToSubmit(self.handle, stream_ptr(stream), _h(inp), _h(out), alpha, beta))
@@ -513,6 +525,7 @@ class Flip(_Operator):
 
 class WarpAffine(_Operator):
     _create = "cvcudaWarpAffineCreate"
+    _native = 8
 
     def __init__(self, max_varshape_batch_size=0):
         super().__init__(max_varshape_batch_size)
@@ -529,6 +542,7 @@ class WarpAffine(_Operator):
 
 class WarpPerspective(_Operator):
     _create = "cvcudaWarpPerspectiveCreate"
+    _native = 9
 
     def __init__(self, max_varshape_batch_size=0):
         super().__init__(max_varshape_batch_size)

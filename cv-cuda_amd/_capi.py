@@ -5,6 +5,8 @@ The two shared libraries are loaded from ./lib next to this file; a missing libr
 process is the one the libraries bind to.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 import torch  # noqa: F401  (loads the HIP runtime once, before our libraries resolve it)
@@ -24,6 +26,22 @@ def _load(name):
 
 nvcv = _load("libnvcv_types.so")
 cvcuda = _load("libcvcuda.so")
+
+
+
+def _load_native():
+    """The Python extension csrc/python/Native.cpp; the libraries it needs are those loaded above."""
+    path = os.path.join(_HERE, "lib", "_cvcuda_native.so")
+    if not os.path.exists(path):
+        raise ImportError(
+            "%s not found: build the native libraries first (python cv-cuda_amd/build.py)" % path)
+    loader = importlib.machinery.ExtensionFileLoader("_cvcuda_native", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_cvcuda_native", path, loader=loader))
+    loader.exec_module(module)
+    return module
+
+
+native = _load_native()
 
 NVCV_TENSOR_MAX_RANK = 15
 NVCV_MAX_PLANE_COUNT = 6

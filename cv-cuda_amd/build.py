@@ -4,6 +4,7 @@
   lib/libcvcuda.so      -- operators: host validation/dispatch + HIP kernels
   lib/libcvamd_bench.so -- kernels the benchmark times beside the operators (a copy-bound twin of the
                            fused kernel); nothing in the two libraries above uses it
+  lib/_cvcuda_native.so -- Python extension: the parts of the Python interface that run in every call
 
 Usage: python cv-cuda_amd/build.py [--force] [-j N] [--sanitize]
 Objects are cached under build/ next to this file and rebuilt when a source or header is newer.
@@ -21,9 +22,11 @@ off because the interpreter's own allocations would drown the report).
 """
 import argparse
 import concurrent.futures
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -74,6 +77,27 @@ def _compile(src, obj, extra, force, newest_header):
     return msgs
 
 
+def _compile_native(src, obj, force, newest_header):
+    """The Python extension, by the host compiler against the headers of Python, torch and the HIP runtime."""
+    if (not force and os.path.exists(obj) and os.path.getmtime(obj) >= os.path.getmtime(src)
+            and os.path.getmtime(obj) >= newest_header):
+        return None
+    torch = _torch_dir()
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wextra", "-Wno-unused-parameter", "-D__HIP_PLATFORM_AMD__",
+           "-DUSE_ROCM", "-I" + INCLUDE]
+    for d in (os.path.join(torch, "include"), os.path.join(torch, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+              sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", d]
+    r = subprocess.run(cmd + ["-c", src, "-o", obj], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("compile failed: %s\n%s" % (" ".join(cmd), r.stdout + r.stderr))
+    return r.stdout + r.stderr
+
+
+def _torch_dir():
+    return importlib.util.find_spec("torch").submodule_search_locations[0]
+
+
 def asan_runtime():
     """Path of the AddressSanitizer runtime of hipcc's clang (to LD_PRELOAD into an uninstrumented python)."""
     r = subprocess.run(["hipcc", "-print-file-name=libclang_rt.asan-x86_64.so"], capture_output=True, text=True)
@@ -101,6 +125,10 @@ def build(force=False, jobs=8, verbose=True, sanitize=False):
             for src, extra in items:
                 obj = os.path.join(objdir, group + "_" + os.path.basename(src) + ".o")
                 tasks.append((group, obj, ex.submit(_compile, src, obj, extra, force, newest_header)))
+        if not sanitize:
+            src = os.path.join(CSRC, "python", "Native.cpp")
+            obj = os.path.join(objdir, "python_Native.cpp.o")
+            tasks.append(("python", obj, ex.submit(_compile_native, src, obj, force, newest_header)))
         for group, obj, fut in tasks:
             msgs = fut.result()
             if verbose and msgs:
@@ -122,6 +150,10 @@ def build(force=False, jobs=8, verbose=True, sanitize=False):
     bench_so = os.path.join(libdir, "libcvamd_bench.so")
     subprocess.run(link + [o for g, o, _ in tasks if g == "bench"] + ["-o", bench_so], check=True)
     if not sanitize:
+        torch_lib = os.path.join(_torch_dir(), "lib")
+        subprocess.run(["g++", "-shared", "-fPIC"] + [o for g, o, _ in tasks if g == "python"]
+                       + ["-o", os.path.join(libdir, "_cvcuda_native.so"), "-L" + libdir, "-lcvcuda", "-lnvcv_types", "-L" + torch_lib,
+                          "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"], check=True)
         build_c_caller(libdir)
     return nvcv_so, cvcuda_so, bench_so
 

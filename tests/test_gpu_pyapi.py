@@ -775,3 +775,113 @@ def test_decoder_and_encoder_edges_of_the_samples(cvcuda, orc, cv):
     np.testing.assert_array_equal(host(hwc_batch), rgb)
     np.testing.assert_array_equal(tensor.cpu().numpy().reshape(n, -1, width),
                                   np.asarray(col.yuv420_from_bgr(rgb, False, 0, False)).reshape(n, -1, width))
+
+
+def _native_calls(api):
+    """(operator, arguments) of every call that the native module makes itself, on fresh containers; the first result last."""
+    import torch
+
+    def t(shape, layout, dtype=torch.uint8):
+        x = torch.arange(int(np.prod(shape)), device="cuda") % 250 + 1
+        return api.as_tensor(x.to(dtype).reshape(shape), layout)
+
+    def images(n=3):
+        return api.as_images([(torch.arange((20 + i) * 30 * 3, device="cuda") % 253).to(torch.uint8).reshape(20 + i, 30, 3) for i in range(n)])
+
+    u8, f32 = t((2, 20, 30, 3), "NHWC"), t((2, 20, 30, 3), "NHWC", torch.float32)
+    base, scale = t((1, 1, 1, 3), "NHWC", torch.float32), t((1, 1, 1, 3), "NHWC", torch.float32)
+    xf = [0.9, -0.1, 2.0, 0.1, 0.9, -1.0]
+    rects, codes = api.as_tensor(torch.tensor([[[[1, 2, 8, 8]]]] * 3, dtype=torch.int32, device="cuda"), "NHWC"), \
+        api.as_tensor(torch.tensor([[0], [1], [-1]], dtype=torch.int32, device="cuda"), "NC")
+    mats = api.as_tensor(torch.tensor([xf] * 3, device="cuda"), "NW")
+    persp = api.as_tensor(torch.tensor([xf + [0.0, 0.0, 1.0]] * 3, device="cuda"), "NW")
+    fused = ((25, 26), 1, (1, 2), 0, 0.5, 0.25, False)
+    return [
+        (api.Resize, (), [u8], t((2, 11, 13, 3), "NHWC"), lambda d: (u8, d, 1)),
+        (api.CvtColor, (), [u8], t((2, 20, 30, 3), "NHWC"), lambda d: (u8, d, int(api.ColorConversion.BGR2RGB))),
+        (api.Reformat, (), [u8], t((2, 3, 20, 30), "NCHW"), lambda d: (u8, d)),
+        (api.ConvertTo, (), [u8], t((2, 20, 30, 3), "NHWC", torch.float32), lambda d: (u8, d, 0.5, 1.0)),
+        (api.Normalize, (), [f32, base, scale], t((2, 20, 30, 3), "NHWC", torch.float32), lambda d: (f32, base, scale, d, 1.0, 0.5, 0.0, 1)),
+        (api.ResizeCropConvertReformat, (), [u8], t((2, 3, 9, 8), "NCHW", torch.float32), lambda d: (u8, d) + fused),
+        (api.WarpAffine, (0,), [u8], t((2, 20, 30, 3), "NHWC"), lambda d: (u8, d, xf, 1, 1, (1.0, 2.0, 3.0, 4.0))),
+        (api.WarpPerspective, (0,), [u8], t((2, 20, 30, 3), "NHWC"), lambda d: (u8, d, xf + [0.0, 0.0, 1.0], 1, 0, (1.0, 2.0, 3.0, 4.0))),
+    ] + [(op, args, [b] + more, d, make) for b in [images()] for op, args, more, d, make in [
+        (api.Resize, (), [], images(), lambda d: (b, d, 1)),
+        (api.CvtColor, (), [], images(), lambda d: (b, d, int(api.ColorConversion.BGR2RGB))),
+        (api.Normalize, (), [base, scale], images(), lambda d: (b, base, scale, d, 1.0, 0.5, 0.0, 0)),
+        (api.ResizeCropConvertReformat, (), [], t((3, 3, 9, 8), "NCHW", torch.float32), lambda d: (b, d) + fused),
+        (api.CropFlipNormalizeReformat, (), [rects, codes, base, scale], t((3, 3, 8, 8), "NCHW", torch.float32),
+         lambda d: (b, d, rects, 0, 0.0, codes, base, scale, 1.0, 0.0, 0.0, 0)),
+        (api.WarpAffine, (3,), [mats], images(), lambda d: (b, d, mats, 1, 0, (0.0,) * 4)),
+        (api.WarpPerspective, (3,), [persp], images(), lambda d: (b, d, persp, 1, 0, (0.0,) * 4))]]
+
+
+def test_native_calls_do_what_submit_does(cvcuda, monkeypatch):
+    import torch
+    api = cvcuda
+
+    # results, and the marks that order streams, of the native path and of _submit; and that the native path took the call
+    def results(d):
+        torch.cuda.synchronize()
+        return [d.torch().cpu()] if isinstance(d, api.Tensor) else [torch.as_tensor(i.cuda(), device="cuda").cpu() for i in d]
+
+    for native, python in zip(_native_calls(api), _native_calls(api)):
+        op, args, reads, dst, make = native
+        handed_on = []
+        monkeypatch.setattr(api, "_submit", lambda *a: handed_on.append(a))
+        api._run(None, reads, [dst], api._op(op, *args), *make(dst))
+        monkeypatch.undo()
+        assert not handed_on, op
+        assert dst._wrote == (0, None) and dst._read == {} and all(r._read == {0: None} for r in reads), op
+        op, args, reads, want, make = python
+        api._submit(None, reads, [want], api._op(op, *args), *make(want))
+        for a, b in zip(results(dst), results(want)):
+            assert torch.equal(a, b), op
+
+
+def test_native_calls_leave_the_rest_to_submit(cvcuda):
+    import torch
+    api = cvcuda
+
+    # waits, other streams and bad arguments: what Python did before, with the errors it raised
+    src = api.as_tensor(torch.zeros((1, 8, 8, 3), dtype=torch.uint8, device="cuda"), "NHWC")
+    dst = api.as_tensor(torch.zeros((1, 4, 4, 3), dtype=torch.uint8, device="cuda"), "NHWC")
+    side = api.Stream()
+    api.resize_into(dst, src, api.Interp.LINEAR, stream=side)
+    assert dst._wrote[0] == side.handle and dst._wrote[1] is not None
+    api.resize_into(dst, src, api.Interp.LINEAR)  # waits for `side`
+    assert dst._wrote[0] == 0 and src._read.keys() == {side.handle, 0}
+    with side:
+        api.resize_into(dst, src, api.Interp.LINEAR)
+    assert dst._wrote[0] == side.handle
+    side.sync()
+    for bad in ((dst, src, 99), (src, api.as_tensor(torch.zeros((1, 4, 4, 4), dtype=torch.uint8, device="cuda"), "NHWC"), 1)):
+        with pytest.raises(api.Error) as e:
+            api.resize_into(*bad)
+        assert e.value.status == 2
+    with pytest.raises(Exception):
+        api.resize_into(dst, None, api.Interp.LINEAR)
+
+
+def test_native_views_and_planes(cvcuda):
+    import torch
+    api = cvcuda
+    t = api.Tensor((2, 5, 7, 3), np.float32, "NHWC")
+    view = t.torch()
+    assert view.shape == (2, 5, 7, 3) and view.dtype == torch.float32 and view.data_ptr() == t.cuda().__cuda_array_interface__["data"][0]
+    assert tuple(s * 4 for s in view.stride()) == tuple(t.cuda().strides)
+    view.fill_(3)
+    del t  # the view keeps the memory
+    others = [api.Tensor((2, 5, 7, 3), np.float32, "NHWC") for _ in range(8)]
+    for o in others:
+        o.torch().fill_(7)
+    assert bool((view == 3).all())
+    whole = torch.zeros((40, 50, 3), dtype=torch.uint8, device="cuda")
+    for buffers in ([whole, whole[3:9, 4:20]], [whole[:, :, 0]], [whole.float(), whole.float()[1:]], (whole, whole[::2])):
+        fmt, planes = api._plane_list(buffers, None)
+        want = b"".join(np.array([b.shape[1], b.shape[0], b.stride(0) * b.element_size(), 0], np.int32).tobytes()
+                        + np.array([b.data_ptr()], np.uint64).tobytes() for b in buffers)
+        assert planes == want and fmt == api._FORMAT_OF_TORCH[(buffers[0].dtype, buffers[0].shape[2] if buffers[0].dim() == 3 else 1)]
+    for buffers in ([], [whole, whole.float()], [whole, whole.cpu()], [whole.float().requires_grad_()], [whole[0, 0]], [whole[:0]],
+                    [whole.double()[:, :, :2]], [np.zeros((4, 4, 3), np.uint8)]):
+        assert api._plane_list(buffers, None) is None
