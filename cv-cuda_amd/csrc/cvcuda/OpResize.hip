@@ -1719,14 +1719,14 @@ __device__ __forceinline__ void ResizeLinearQuadsU8(const Plane &p, int x0, int 
 // would be a wait for those stores to reach memory as well.
 // 1 and 3 channels request only the windows that are needed. With 4-byte pixels the compiler joins a window that exists
 // on one side of the test only to the statement through a register move, which waits for its load, so those request
-// all nine (rows past `last` repeat it: an L1 hit, but a load instruction; 16 x 720p -> 900p u8x3 36.8 us against
+// all W (rows past `last` repeat it: an L1 hit, but a load instruction; 16 x 720p -> 900p u8x3 36.8 us against
 // 31.3). Two whole variants, 5 windows or 9, were slower for every pixel size (65 us for the two-column strips).
-template<int C>
-__device__ __forceinline__ void RequestStripWindows(const uint8_t *at, int rowStride, int last, TapWindow<C> (&win)[9])
+template<int C, int W>
+__device__ __forceinline__ void RequestStripWindows(const uint8_t *at, int rowStride, int last, TapWindow<C> (&win)[W])
 {
-    RawTapWindow<C> raw[9];
+    RawTapWindow<C> raw[W];
 #pragma unroll
-    for (int k = 0; k < 9; ++k)
+    for (int k = 0; k < W; ++k)
     {
         if constexpr (C == 4)
         {
@@ -1741,27 +1741,40 @@ __device__ __forceinline__ void RequestStripWindows(const uint8_t *at, int rowSt
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::"v"(raw[0].d[0]), "v"(raw[1].d[0]), "v"(raw[2].d[0]), "v"(raw[3].d[0]), "v"(raw[4].d[0]), "v"(raw[5].d[0]),
-                 "v"(raw[6].d[0]), "v"(raw[7].d[0]), "v"(raw[8].d[0]));
+    if constexpr (W == 9)
+    {
+        asm volatile("" ::"v"(raw[0].d[0]), "v"(raw[1].d[0]), "v"(raw[2].d[0]), "v"(raw[3].d[0]), "v"(raw[4].d[0]),
+                     "v"(raw[5].d[0]), "v"(raw[6].d[0]), "v"(raw[7].d[0]), "v"(raw[8].d[0]));
+    }
+    else if constexpr (W == 5)
+    {
+        asm volatile("" ::"v"(raw[0].d[0]), "v"(raw[1].d[0]), "v"(raw[2].d[0]), "v"(raw[3].d[0]), "v"(raw[4].d[0]));
+    }
+    else
+    {
+        static_assert(W == 3);
+        asm volatile("" ::"v"(raw[0].d[0]), "v"(raw[1].d[0]), "v"(raw[2].d[0]));
+    }
 #pragma unroll
-    for (int k = 0; k < 9; ++k)
+    for (int k = 0; k < W; ++k)
     {
         win[k] = FinishTapWindow<C>(raw[k]);
     }
 }
 
-// The four-column form over a strip of kStripRows output rows per wave. When not reducing vertically those rows
-// lie between at most kStripRows + 1 consecutive source rows. All their windows are requested up front, a source
+// The four-column form over a strip of R output rows per wave (kStripRows; fewer in small launches). When not reducing
+// vertically those rows lie between at most R + 1 consecutive source rows. All their windows are requested up front, a source
 // row's tap pairs are formed once for every output row that uses it as
-// its upper or its lower row, and the column terms are paid once per 8 rows instead of once per 2. The blend per
+// its upper or its lower row, and the column terms are paid once per R rows instead of once per 2. The blend per
 // output pixel is BilinearQ15 as everywhere. A wave that reaches the image's last source row, reduces vertically
-// (more source rows than fit) or has a lane whose columns do not fit its window runs as four two-row steps.
+// (more source rows than fit) or has a lane whose columns do not fit its window runs as two-row steps.
 constexpr int kStripRows = 8, kStripWindows = kStripRows + 1;
 static_assert(kStripWindows == 9);
 
-template<int C>
+template<int C, int R = kStripRows>
 __device__ __forceinline__ void ResizeLinearQuadStripU8(const Plane &p, int x0, int y0)
 {
+    constexpr int kWindows = R + 1;
     if (x0 >= p.dstW || y0 >= p.dstH)
     {
         return;
@@ -1775,20 +1788,20 @@ __device__ __forceinline__ void ResizeLinearQuadStripU8(const Plane &p, int x0, 
         col[j] = Axis<NVCV_INTERP_LINEAR>(p.scaleX, min(dx0 + j, p.dstW - 1), p.srcW);
     }
     // lane r holds the terms of output row y0 + r
-    const auto     rows   = Axis<NVCV_INTERP_LINEAR>(p.scaleY, min(y0 + (lane & (kStripRows - 1)), p.dstH - 1), p.srcH);
+    const auto     rows   = Axis<NVCV_INTERP_LINEAR>(p.scaleY, min(y0 + (lane & (R - 1)), p.dstH - 1), p.srcH);
     const uint32_t ayLane = FractionQ15(rows.w[0]);
-    const int      yFirst = __builtin_amdgcn_readlane(rows.s, 0), yLast = __builtin_amdgcn_readlane(rows.s, kStripRows - 1) + 1;
+    const int      yFirst = __builtin_amdgcn_readlane(rows.s, 0), yLast = __builtin_amdgcn_readlane(rows.s, R - 1) + 1;
     const bool     narrow = col[3].s - col[0].s <= 2;
-    if (yLast >= p.srcH - 1 || yLast - yFirst >= kStripWindows || __builtin_amdgcn_ballot_w64(!narrow) != 0) // wave-uniform
+    if (yLast >= p.srcH - 1 || yLast - yFirst >= kWindows || __builtin_amdgcn_ballot_w64(!narrow) != 0) // wave-uniform
     {
 #pragma unroll 1
-        for (int k = 0; k < kStripRows; k += 2)
+        for (int k = 0; k < R; k += 2)
         {
             ResizeLinearQuadsU8<C>(p, x0, y0 + k);
         }
         return;
     }
-    TapWindow<C>   win[kStripWindows];
+    TapWindow<C>   win[kWindows];
     const uint8_t *at = p.src + (int64_t)yFirst * p.srcRow + col[0].s * C;
     RequestStripWindows<C>(at, p.srcRow, yLast - yFirst, win);
     // lanes past the last column stay (the row terms are read from lanes 0 .. 7 below); they store nothing
@@ -1857,13 +1870,13 @@ __device__ __forceinline__ void ResizeLinearQuadStripU8(const Plane &p, int x0, 
             }
         }
     };
-    const int nRows = min(kStripRows, p.dstH - y0);
+    const int nRows = min(R, p.dstH - y0);
     int       r     = 0;
     uint8_t  *to    = p.dst + (int64_t)y0 * p.dstRow + (int64_t)dx0 * C;
     uint32_t  top[4][C], bot[4][C];
     pairs(win[0], bot);
 #pragma unroll
-    for (int k = 0; k + 1 < kStripWindows; ++k)
+    for (int k = 0; k + 1 < kWindows; ++k)
     {
         if (r < nRows) // wave-uniform
         {
@@ -1999,27 +2012,26 @@ __device__ __forceinline__ void ResizeNearestQuadStripU8(const Plane &p, int x0,
     }
 }
 
-// The two-column form over strips of kPairStripRows output rows per wave (128 columns x 4 rows). At vertical scales
-// up to 2 those rows lie between at most 9 consecutive source rows: the windows are requested up front, a source row
+// The two-column form over strips of R output rows per wave (128 columns x 4 rows; x 2 in small launches). At vertical
+// scales up to 2 those rows lie between at most 2 R + 1 consecutive source rows: the windows are requested up front, a source row
 // is taken apart into its (first tap | second tap) pairs once for every output row that uses it as its upper or its
-// lower row, and the column terms are paid once per 4 rows instead of once per 2. Every output row is finished on its
+// lower row, and the column terms are paid once for all of them. Every output row is finished on its
 // own: a lane rounds the channels of its 2 pixels straight into the bytes they have in the row, the lanes of a pair
 // swap them, and the even lane stores the 4 pixels as whole dwords. The blend per output pixel is BilinearQ15 as
-// everywhere. A wave that reaches the image's last source row or reduces vertically by more than 2 runs as two
+// everywhere. A wave that reaches the image's last source row or reduces vertically by more than 2 runs as
 // two-row steps.
-constexpr int kPairStripRows = 4, kPairStripWindows = 2 * kPairStripRows + 1;
-static_assert(kPairStripWindows == 9);
+constexpr int kPairStripRows = 4;
 
-template<int C>
+template<int C, int R = kPairStripRows>
 __device__ __forceinline__ void ResizeLinearPairStripU8(const Plane &p, int x0, int y0)
 {
+    constexpr int kPairStripWindows = 2 * R + 1;
     if (x0 >= p.dstW || y0 >= p.dstH)
     {
         return;
     }
-    constexpr int R    = kPairStripRows;
-    const int     lane = threadIdx.x & 63;
-    const int     dx0  = x0 + 2 * lane;
+    const int lane = threadIdx.x & 63;
+    const int dx0  = x0 + 2 * lane;
     // columns and rows past the output compute a duplicate of the last one: every lane takes part in the swap
     const auto colA  = Axis<NVCV_INTERP_LINEAR>(p.scaleX, min(dx0, p.dstW - 1), p.srcW);
     const auto colB  = Axis<NVCV_INTERP_LINEAR>(p.scaleX, min(dx0 + 1, p.dstW - 1), p.srcW);
@@ -2030,8 +2042,11 @@ __device__ __forceinline__ void ResizeLinearPairStripU8(const Plane &p, int x0, 
     const int      yFirst = __builtin_amdgcn_readlane(rows.s, 0), yLast = __builtin_amdgcn_readlane(rows.s, R - 1) + 1;
     if (yLast >= p.srcH - 1 || yLast - yFirst >= kPairStripWindows) // wave-uniform
     {
-        ResizeLinearPairsU8<C, false>(p, x0, y0);
-        ResizeLinearPairsU8<C, false>(p, x0, y0 + 2);
+#pragma unroll
+        for (int r = 0; r < R; r += 2)
+        {
+            ResizeLinearPairsU8<C, false>(p, x0, y0 + r);
+        }
         return;
     }
     TapWindow<C>   win[kPairStripWindows];
@@ -2187,28 +2202,22 @@ static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH,
     return flat ? dim3(DivUp(dstW, waves * waveW), DivUp(dstH, waveH), N) : dim3(DivUp(dstW, waveW), DivUp(dstH, waves * waveH), N);
 }
 
-// Tensors: strips of 4 rows per wave.
-template<int C>
+template<int C, int R>
 __global__ __launch_bounds__(256) void ResizeLinearPairsU8Kernel(const ResizeArgs a, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeLinearPairStripU8<C>(p, t.x * kPairsTileW, t.y * kPairStripRows);
+    ResizeLinearPairStripU8<C, R>(p, t.x * kPairsTileW, t.y * R);
 }
 
-constexpr int kQuadsTileW = 256; // a wave's columns; tensors: block = 4 waves side by side (1024 columns x kQuadsRows rows)
+constexpr int kQuadsTileW = 256; // a wave's columns; tensors: block = 4 waves side by side (1024 columns x a strip's rows)
 
-// Rows per wave of the four-column form (strips for every pixel size; with 16-byte stores that the compiler had
-// split into 12 + 4 bytes, 4-byte pixels were faster in two-row steps: 16 x 720p -> 1080p 43.7 us, now 37.7 as strips).
-template<int C>
-constexpr int kQuadsRows = kStripRows;
-
-template<int C>
+template<int C, int R>
 __global__ __launch_bounds__(256) void ResizeLinearQuadsU8Kernel(const ResizeArgs a, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeLinearQuadStripU8<C>(p, t.x * kQuadsTileW, t.y * kStripRows);
+    ResizeLinearQuadStripU8<C, R>(p, t.x * kQuadsTileW, t.y * R);
 }
 
 template<int C>
@@ -2258,7 +2267,7 @@ __device__ __forceinline__ WaveTile VarWaveTileOf(const TileCoord &tc, int flat)
 template<int C>
 __host__ __device__ __forceinline__ bool QuadStripScale(int srcW, int dstW)
 {
-    return kQuadsRows<C> == kStripRows && srcW >= 4 && 3 * (int64_t)srcW <= 2 * (int64_t)dstW;
+    return srcW >= 4 && 3 * (int64_t)srcW <= 2 * (int64_t)dstW;
 }
 
 template<int C, bool WIDE>
@@ -3812,17 +3821,31 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         if (a.srcW >= 4 && 3 * (int64_t)a.srcW <= 2 * (int64_t)a.dstW)
         {
-            const bool flat = FlatBlocks(a.dstW, kQuadsTileW);
-            hipLaunchKernelGGL((ResizeLinearQuadsU8Kernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, kStripRows, flat), dim3(256), 0,
-                               stream, a, (int)flat);
+            // Few waves run one round of loads and stores behind each other, so the launch's time is a wave's: shorter strips until
+            // the chip is full (us with 8 / 4 / 2 rows, three channels: 224 x 224 -> 336 x 336 7.7 / 4.8 / 4.4; 4 x 224 x 224 -> 448 x
+            // 448 8.2 / 6.6 / 5.2; 720p -> 1080p 8.8 / 6.9 / 7.2; 16 x 320 x 240 -> 640 x 480 11.4 / 11.2 / 11.2), from there on the
+            // source rows that strips share and their column terms count (32 x 224 x 224 -> 448 x 448 12.2 / 13.0 / 13.2; one channel,
+            // 8 x 720p -> 1080p 12.6 / 13.5 / 15.5).
+            const bool    flat   = FlatBlocks(a.dstW, kQuadsTileW);
+            const int64_t strips = (int64_t)DivUp(a.dstW, kQuadsTileW) * DivUp(a.dstH, kStripRows) * N;
+            const int     rows   = strips <= 3 * 256 ? 2 : strips <= 12 * 256 ? 4 : kStripRows;
+            auto          kernel = rows == 2   ? ResizeLinearQuadsU8Kernel<C, 2>
+                                   : rows == 4 ? ResizeLinearQuadsU8Kernel<C, 4>
+                                               : ResizeLinearQuadsU8Kernel<C, kStripRows>;
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeLinearQuadsU8Kernel");
             return;
         }
         if (PairsFormScale<C>(a.srcW, a.dstW))
         {
-            const bool flat = FlatBlocks(a.dstW, kPairsTileW);
-            hipLaunchKernelGGL((ResizeLinearPairsU8Kernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kPairsTileW, kPairStripRows, flat), dim3(256),
-                               0, stream, a, (int)flat);
+            // Shorter strips while waves are few, as above (us with 4 / 2 rows, three channels: 720p -> 640 x 360 4.0 / 3.3; 15 x
+            // 1136 x 166 -> 680 x 99 6.3 / 5.3; 32 x 256 x 256 -> 224 x 224 6.5 / 6.2, 64 of these 9.0 / 9.4; one channel, 4 x 720p ->
+            // 960 x 540 5.0 / 5.0, 16 of these 11.2 / 12.5).
+            const bool    flat   = FlatBlocks(a.dstW, kPairsTileW);
+            const int64_t strips = (int64_t)DivUp(a.dstW, kPairsTileW) * DivUp(a.dstH, kPairStripRows) * N;
+            const int     rows   = strips <= 16 * 256 ? 2 : kPairStripRows;
+            auto          kernel = rows == 2 ? ResizeLinearPairsU8Kernel<C, 2> : ResizeLinearPairsU8Kernel<C, kPairStripRows>;
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPairsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeLinearPairsU8Kernel");
             return;
         }

@@ -118,6 +118,26 @@ def test_tensor_cubic_u8_walks(cv, orc, gpu, shape, c):
     np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), CUBIC, threads=8))
 
 
+# 8-bit bilinear in launches of few waves, whose strips are 2 rows (two columns per lane; four, up to 768 strips of 8) and 4 (four
+# columns, up to 3072): one row, heights one off a strip's, widths one off a wave's and of one column, vertical reductions by 2 (all
+# of a strip's windows), a little more and 5 (steps), and the launches on both sides of each line
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("shape", [(40, 30, 61, 1, 1), (40, 30, 1, 31, 2), (40, 30, 257, 33, 1), (100, 33, 255, 34, 3), (5, 3, 77, 19, 9),
+                                   (400, 60, 127, 30, 3), (250, 70, 129, 35, 2), (130, 70, 126, 33, 2), (130, 70, 128, 14, 2),
+                                   (90, 80, 256, 40, 7), (64, 16, 256, 24, 256), (64, 16, 256, 25, 256), (64, 16, 257, 24, 512),
+                                   (64, 16, 256, 25, 768), (64, 16, 256, 25, 769), (120, 17, 128, 16, 1024), (120, 17, 128, 17, 1024)],
+                         ids=lambda sh: "%dx%d-%dx%d-n%d" % sh)
+def test_tensor_linear_u8_small_launches(cv, orc, gpu, shape, c):
+    sw, sh, dw, dh, n = shape
+    src = make_input(orc, (n, sh, sw, c), np.uint8, 0x51 + sw + dw + c)
+    out = torch.full((n, dh, dw + 3, c), 7, dtype=torch.uint8, device="cuda")
+    cv.Resize()(None, cv.Tensor.from_torch(torch.from_numpy(src).cuda(), "NHWC"), cv.Tensor.from_torch(out[:, :, :dw], "NHWC"), LINEAR)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:, :, :dw], orc.resize_shipped(src, (dh, dw), LINEAR, threads=8))
+    assert (got[:, :, dw:] == 7).all()
+
+
 # 8-bit nearest neighbour enlarging by 1.5 or more horizontally (and not reducing vertically) runs as strips once the
 # launch has 2048 of them: 1.5, 2 and 3 times, ragged sizes, mixed scales (2.5 across, 1 down: every source row once),
 # and a vertical reduction with the same widths (wave patches)
