@@ -1930,12 +1930,12 @@ __device__ __forceinline__ void ResizeLinearQuadStripU8(const Plane &p, int x0, 
 }
 
 // Nearest neighbour when enlarging by 1.5 or more (3 * srcW <= 2 * dstW), in the shape of the four-column strips:
-// the source pixels of four neighbouring output columns lie within 3 source pixels, so a lane owns 4 columns x 8
+// the source pixels of four neighbouring output columns lie within 3 source pixels, so a lane owns 4 columns x R
 // rows, takes them from one window per source row and stores every output row that maps to that source row from
 // the same registers. The wave patches spend one 3-byte load per output pixel there (8 x 720p -> 1080p u8x3: 19.0 us,
-// the bilinear strips 22.9; as strips 16.7). Indices are those of Axis<NEAREST>; waves that reach the image's last row,
+// the bilinear strips 22.9; as strips 13.6). Indices are those of Axis<NEAREST>; waves that reach the image's last row,
 // reduce vertically or have a lane whose columns do not fit its window run as wave patches.
-template<int C>
+template<int C, int R>
 __device__ __forceinline__ void ResizeNearestQuadStripU8(const Plane &p, int x0, int y0)
 {
     if (x0 >= p.dstW || y0 >= p.dstH)
@@ -1951,26 +1951,26 @@ __device__ __forceinline__ void ResizeNearestQuadStripU8(const Plane &p, int x0,
         s[j] = Axis<NVCV_INTERP_NEAREST>(p.scaleX, min(dx0 + j, p.dstW - 1), p.srcW).s;
     }
     // lane r holds the source row of output row y0 + r
-    const int  rowLane = Axis<NVCV_INTERP_NEAREST>(p.scaleY, min(y0 + (lane & (kStripRows - 1)), p.dstH - 1), p.srcH).s;
-    const int  yFirst = __builtin_amdgcn_readlane(rowLane, 0), yLast = __builtin_amdgcn_readlane(rowLane, kStripRows - 1);
+    const int  rowLane = Axis<NVCV_INTERP_NEAREST>(p.scaleY, min(y0 + (lane & (R - 1)), p.dstH - 1), p.srcH).s;
+    const int  yFirst = __builtin_amdgcn_readlane(rowLane, 0), yLast = __builtin_amdgcn_readlane(rowLane, R - 1);
     const bool narrow = s[3] - s[0] <= 3;
-    if (yLast >= p.srcH - 1 || yLast - yFirst >= kStripWindows || __builtin_amdgcn_ballot_w64(!narrow) != 0) // wave-uniform
+    if (yLast >= p.srcH - 1 || yLast - yFirst >= (R + 1) || __builtin_amdgcn_ballot_w64(!narrow) != 0) // wave-uniform
     {
 #pragma unroll 1
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < R; ++i)
         {
             ResizeWavePatch<uint8_t, C, NVCV_INTERP_NEAREST, false>(p, x0 + 64 * (i & 3), y0 + 4 * (i >> 2));
         }
         return;
     }
-    TapWindow<C>   win[kStripWindows];
+    TapWindow<C>   win[(R + 1)];
     const uint8_t *at = p.src + (int64_t)yFirst * p.srcRow + s[0] * C;
     RequestStripWindows<C>(at, p.srcRow, yLast - yFirst, win);
-    const int nRows = min(kStripRows, p.dstH - y0);
+    const int nRows = min(R, p.dstH - y0);
     int       r     = 0;
     uint8_t  *to    = p.dst + (int64_t)y0 * p.dstRow + (int64_t)dx0 * C;
 #pragma unroll
-    for (int k = 0; k < kStripWindows; ++k)
+    for (int k = 0; k < (R + 1); ++k)
     {
         if (r < nRows) // wave-uniform
         {
@@ -2220,12 +2220,12 @@ __global__ __launch_bounds__(256) void ResizeLinearQuadsU8Kernel(const ResizeArg
     ResizeLinearQuadStripU8<C, R>(p, t.x * kQuadsTileW, t.y * R);
 }
 
-template<int C>
+template<int C, int R>
 __global__ __launch_bounds__(256) void ResizeNearestQuadsU8Kernel(const ResizeArgs a, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeNearestQuadStripU8<C>(p, t.x * kQuadsTileW, t.y * kStripRows);
+    ResizeNearestQuadStripU8<C, R>(p, t.x * kQuadsTileW, t.y * R);
 }
 
 // Image batches: the same 128 x 8 tile per block for every image; an image whose horizontal scale is
@@ -2323,22 +2323,22 @@ __host__ __device__ __forceinline__ bool NearestStripScale(int srcW, int srcH, i
     return srcW >= 8 && 3 * (int64_t)srcW <= 2 * (int64_t)dstW && srcH <= dstH;
 }
 
-// Large image batches that are mostly such images: a 256 x 8 tile per wave, a strip or eight patches.
-template<int C>
+// Image batches that are mostly such images: a 256 x R tile per wave (4 or 8 rows), a strip or patches.
+template<int C, int R>
 __global__ __launch_bounds__(256) void ResizeNearestStripsU8VarShapeKernel(const ResizeArgs a, const VarTiles tiles, const int flat)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
     const Plane     p  = GetPlanes<true>(a, tc.image);
     const WaveTile  t  = VarWaveTileOf(tc, flat);
-    const int       x0 = t.x * kStripsWaveW<true>, y0 = t.y * kStripsWaveH<true>;
+    const int       x0 = t.x * kStripsWaveW<true>, y0 = t.y * R;
     if (NearestStripScale<C>(p.srcW, p.srcH, p.dstW, p.dstH))
     {
-        ResizeNearestQuadStripU8<C>(p, x0, y0);
+        ResizeNearestQuadStripU8<C, R>(p, x0, y0);
     }
     else
     {
 #pragma unroll 1
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < R; ++i)
         {
             ResizeWavePatch<uint8_t, C, NVCV_INTERP_NEAREST, true>(p, x0 + (i & 3) * 64, y0 + (i >> 2) * 4);
         }
@@ -2644,8 +2644,18 @@ __global__ __launch_bounds__(256) void ResizePatchVarShapeKernel(const ResizeArg
 template<class T, int C, int INTERP>
 constexpr bool kAreaFixed = std::is_same_v<T, uint8_t> && INTERP == NVCV_INTERP_AREA && (C == 1 || C == 3 || C == 4);
 
-constexpr int kAreaRowsPerWave = 16;
-constexpr int kAreaTileW = 64, kAreaTileH = 4 * kAreaRowsPerWave; // image batches: block = 4 waves stacked vertically; tensors: side by side
+constexpr int kAreaRowsMost = 16; // output rows per wave: 4, 8 or 16
+constexpr int kAreaTileW = 64;    // image batches: block = 4 waves stacked vertically; tensors: side by side
+
+// Rows per wave, given the launch's waves of 16. A wave's steps of 4 rows follow one another, so a launch that does not fill
+// the chip takes as long as one wave: fewer steps each until there are enough of them. us with 16 / 8 / 4 rows, three
+// channels: 224 x 224 -> 112 x 112 7.4 / 5.2 / 3.9; 640 x 480 -> 320 x 240 7.7 / 5.0 / 3.8; 1080p -> 720p 6.2 / 5.5 / 5.2; 32 x 256 x
+// 256 -> 224 x 224 9.5 / 8.6 / 8.3; 16 x 640 x 480 -> 416 x 416 12.8 / 11.2 / 11.6; 8 x 1080p -> 720p 18.0 / 17.4 / 19.4; 16 of these
+// 31.1 / 31.5 / 36.1, one channel 19.7 / 20.9 / 25.5: the column terms are paid per wave.
+int AreaRowsPerWave(int64_t waves)
+{
+    return waves <= 8 * 256 ? 4 : waves <= 32 * 256 ? 8 : kAreaRowsMost;
+}
 
 // Per image: both scales within 1 .. 3 and a source of at least 4 rows of at least 32 bytes.
 __host__ __device__ __forceinline__ bool AreaFixedDomain(float scaleX, float scaleY, int srcRowBytes, int srcH)
@@ -2808,9 +2818,9 @@ __device__ __forceinline__ void AreaFixedRows(int n, const uint8_t *row, int src
     }
 }
 
-// The tile of 64 columns x 16 rows whose top left pixel is (x0, y0), both wave-uniform (y0 even).
+// The tile of 64 columns x `rows` rows whose top left pixel is (x0, y0), both wave-uniform (y0 and rows multiples of 4).
 template<int C, bool ODD>
-__device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, int y0)
+__device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, int y0, int rows)
 {
     if (x0 >= p.dstW || y0 >= p.dstH)
     {
@@ -2837,7 +2847,7 @@ __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, 
     // row between their boxes wherever the scale is not a whole number, so they are produced together from the
     // source rows first(2i) .. first(2i) + n - 1 when those are at most 4 (`pairRows`, else 0): `pw` are this row's
     // weights counted from first(2i). Otherwise each row on its own from its box's first row: `ow`, `ownRows`.
-    const int   dy = min(y0 + (lane & (kAreaRowsPerWave - 1)), p.dstH - 1);
+    const int   dy = min(y0 + (lane & (kAreaRowsMost - 1)), p.dstH - 1);
     const float ownStart = floorf(dy * p.scaleY), pairStart = floorf((dy & ~1) * p.scaleY);
     float       ow[4], pw[4];
     AreaWeights(p.scaleY, dy, p.srcH, 1.f / 32768.f, ownStart, true, ow);
@@ -2850,7 +2860,7 @@ __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, 
     // weights of 0 in front or behind change nothing, so the pair form and the single form start alike
     const float rowStart = -8388608.f * (((ow[0] + ow[1]) + ow[2]) + ow[3]);
 
-    const int rowsHere = min(kAreaRowsPerWave, p.dstH - y0);
+    const int rowsHere = min(rows, p.dstH - y0);
     // output rows i, i + 1 -> out[0], out[1]
     auto rowPair = [&](int i, uint32_t *out)
     {
@@ -2928,7 +2938,7 @@ __device__ __forceinline__ void ResizeAreaFixedWaveTile(const Plane &p, int x0, 
 
 // The same tile outside the fixed-point form's scales (image batches decide per image): one pixel at a time.
 template<int C, bool VARSHAPE>
-__device__ __forceinline__ void ResizeAreaPlainWaveTile(const Plane &p, int x0, int y0)
+__device__ __forceinline__ void ResizeAreaPlainWaveTile(const Plane &p, int x0, int y0, int rows)
 {
     const int dx = x0 + (int)(threadIdx.x & 63);
     if (dx >= p.dstW)
@@ -2936,33 +2946,33 @@ __device__ __forceinline__ void ResizeAreaPlainWaveTile(const Plane &p, int x0, 
         return;
     }
 #pragma unroll 1
-    for (int dy = y0; dy < min(y0 + kAreaRowsPerWave, p.dstH); ++dy)
+    for (int dy = y0; dy < min(y0 + rows, p.dstH); ++dy)
     {
         ResizePixel<uint8_t, C, NVCV_INTERP_AREA, VARSHAPE>(p, dx, dy);
     }
 }
 
 template<int C, bool ODD>
-__global__ __launch_bounds__(256) void ResizeAreaFixedTensorKernel(const ResizeArgs a, const int flat)
+__global__ __launch_bounds__(256) void ResizeAreaFixedTensorKernel(const ResizeArgs a, const int rows, const int flat)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
-    ResizeAreaFixedWaveTile<C, ODD>(p, t.x * kAreaTileW, t.y * kAreaRowsPerWave);
+    ResizeAreaFixedWaveTile<C, ODD>(p, t.x * kAreaTileW, t.y * rows, rows);
 }
 
 template<int C, bool ODD>
-__global__ __launch_bounds__(256) void ResizeAreaVarShapeKernel(const ResizeArgs a, const VarTiles tiles)
+__global__ __launch_bounds__(256) void ResizeAreaVarShapeKernel(const ResizeArgs a, const VarTiles tiles, const int rows)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
     const Plane     p  = GetPlanes<true>(a, tc.image);
-    const int       x0 = tc.tx * kAreaTileW, y0 = tc.ty * kAreaTileH + (threadIdx.x >> 6) * kAreaRowsPerWave;
+    const int       x0 = tc.tx * kAreaTileW, y0 = (tc.ty * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * rows;
     if (AreaFixedDomain(p.scaleX, p.scaleY, p.srcW * C, p.srcH))
     {
-        ResizeAreaFixedWaveTile<C, ODD>(p, x0, y0);
+        ResizeAreaFixedWaveTile<C, ODD>(p, x0, y0, rows);
     }
     else
     {
-        ResizeAreaPlainWaveTile<C, true>(p, x0, y0);
+        ResizeAreaPlainWaveTile<C, true>(p, x0, y0, rows);
     }
 }
 
@@ -3530,18 +3540,16 @@ AreaFloatKernelPtr AreaFloatKernel(int pieces)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Bicubic resize of float tensors at scales below 2 along both axes, large launches. One pixel at a time the 16 taps of every
+// Bicubic resize of float tensors at scales below 2 along both axes. One pixel at a time the 16 taps of every
 // output pixel are loaded and weighted, four fifths of them again for its neighbour below. Here a lane owns a column of
-// kFloatStripRows output rows, forms each source row's weighted sum of four pixels once, keeps the last four of them and
+// `rows` output rows, forms each source row's weighted sum of four pixels once, keeps the last four of them and
 // combines those for every output row between; the next source row is requested before the present rows are combined. Sums
 // of four terms, twice, instead of sixteen: closer to the exact formula (131 x 97 -> 197 x 145: 6.2e-8 of the norm, was
 // 7.7e-8). 4 x 1283 x 721
 // f32x3 -> 1931 x 1081 64.9 -> 36.5 us (4.6 TB/s), -> 1200 x 700 27.3 -> 17.5, -> 963 x 541 19.6 -> 15.9; 2 x f32x4 -> 1280 x
 // 960 21.6 -> 14.4; 12 x f32x1 -> 1931 x 1081 67.3 -> 51.7 (its writes: rows that start at no sector).
-constexpr int kFloatStripRows = 16;
-
 template<int C>
-__global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArgs a)
+__global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArgs a, const int rows)
 {
     struct Taps
     {
@@ -3549,7 +3557,7 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
     };
     const Plane p    = GetPlanes<false>(a, blockIdx.z);
     const int   lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int   dx = blockIdx.x * kTileW + lane, y0 = (blockIdx.y * 4 + wave) * kFloatStripRows;
+    const int   dx = blockIdx.x * kTileW + lane, y0 = (blockIdx.y * 4 + wave) * rows;
     if (y0 >= p.dstH)
     {
         return;
@@ -3606,7 +3614,7 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
         }
     }
     Taps      next = load(first + 4);
-    const int yEnd = min(y0 + kFloatStripRows, p.dstH);
+    const int yEnd = min(y0 + rows, p.dstH);
 #pragma unroll 1
     for (int dy = y0;;)
     {
@@ -3794,25 +3802,41 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     }
     if constexpr (INTERP == NVCV_INTERP_CUBIC && std::is_same_v<T, float> && (C == 1 || C == 3 || C == 4))
     {
-        // launches that give every CU 8 waves; from a scale of 2 on a row sum serves one output row or two
-        const int64_t strips = (int64_t)DivUp(a.dstW, kTileW) * DivUp(a.dstH, kFloatStripRows) * N;
-        if (a.srcW < 2 * (int64_t)a.dstW && a.srcH < 2 * (int64_t)a.dstH && a.srcW >= 4 && a.srcH >= 4 && strips >= 8 * 256)
+        // From a scale of 2 on a row sum serves one output row or two; a few waves leave their CUs idle in both forms, where a wave of one
+        // row ends soonest (us as pixels / so, three channels: 224 x 224 -> 256 x 256 3.0 / 3.5, 320 x 240 -> 400 x 300 4.0 / 3.8; one
+        // channel, the same: 3.7 / 3.1, 4.1 / 3.2).
+        auto waves = [&](int rows) { return (int64_t)DivUp(a.dstW, kTileW) * DivUp(a.dstH, rows) * N; };
+        if (a.srcW < 2 * (int64_t)a.dstW && a.srcH < 2 * (int64_t)a.dstH && a.srcW >= 4 && a.srcH >= 4 && waves(4) >= (C == 1 ? 128 : 512))
         {
-            hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), dim3(DivUp(a.dstW, kTileW), DivUp(a.dstH, 4 * kFloatStripRows), N), dim3(256),
-                               0, stream, a);
+            // Rows per wave: a wave begins with four row sums. us with 4 / 8 / 16, three channels: 640 x 480 -> 800 x 600 4.8 / 5.1 / 7.3;
+            // 8 x 256 x 256 -> 224 x 224 5.2 / 6.0 / 9.2; 32 of these 11.2 / 11.4 / 12.6; 720p -> 1080p 9.4 / 8.8 / 8.9; 2 x 1080p, as many, 21.2 /
+            // 22.2 / 20.3; 4K 30.6 / 27.9 / 26.0; reducing, 4 x 1283 x 721 -> 963 x 541 15.8 / 17.0 / 16.1, four channels 20.3 / 21.5 / 19.4, one
+            // 8.3 / 8.4 / 11.3. Enlarged rows that start at no line of memory are the better the sooner their neighbours follow (20 x 515
+            // x 313 -> 815 x 460, 8 / 16, one channel 15.0 / 18.0, three 29.3 / 33.4, four 34.3 / 40.5; 12 x 1283 x 721 -> 1931 x 1081 39.8 / 53.0,
+            // 112 / 118, 141 / 141).
+            const bool enlarging = a.srcH <= a.dstH, few = waves(8) <= 18 * 256 && (C == 1 || enlarging);
+            const int  rows      = waves(4) <= 30 * 256 ? 4 : few || (enlarging && a.dstRowStride % 64 != 0) ? 8 : 16;
+            hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), dim3(DivUp(a.dstW, kTileW), DivUp(a.dstH, 4 * rows), N), dim3(256), 0, stream, a,
+                               rows);
             CheckLaunch("ResizeCubicStripF32Kernel");
             return;
         }
     }
-    // (8 x 720p -> 1080p: 1 channel 12.4 -> 8.4 us, 3 channels 19.0 -> 16.7 us, 4 channels 21.2 -> 18.7 us)
+    // us as patches / in strips of 4 rows: 4 x 640 x 480 -> 1280 x 720 1 channel 4.4 / 4.2, 3 channels 6.4 / 5.6, 4 channels 5.3 / 5.0; one
+    // 720p -> 1080p, 1080 strips of 8, 4.2 / 3.7, 4.6 / 4.8, 4.5 / 4.0; 16 x 160 x 160 -> 256 x 256, 512 of them, 3.9 / 3.6, 4.3 / 4.7, 4.0 / 3.8;
+    // 4 x 224 x 224 -> 448 x 448, 448, 3.5 / 3.6, 3.8 / 4.5, 3.7 / 3.7.
     if constexpr (std::is_same_v<T, uint8_t> && INTERP == NVCV_INTERP_NEAREST && (C == 1 || C == 3 || C == 4))
     {
         const int64_t strips = (int64_t)DivUp(a.dstW, kQuadsTileW) * DivUp(a.dstH, kStripRows) * N;
-        if (NearestStripScale<C>(a.srcW, a.srcH, a.dstW, a.dstH) && strips >= 8 * 256)
+        if (NearestStripScale<C>(a.srcW, a.srcH, a.dstW, a.dstH) && strips >= (C == 3 ? 6 : 4) * 256)
         {
-            const bool flat = FlatBlocks(a.dstW, kQuadsTileW);
-            hipLaunchKernelGGL((ResizeNearestQuadsU8Kernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, kStripRows, flat), dim3(256), 0,
-                               stream, a, (int)flat);
+            // 4 rows: fewer registers, more waves in flight (8 / 4 rows: 8 x 720p -> 1080p 9.0 / 8.5, 15.3 / 13.6, 17.5 / 15.9; 32 x 224 x 224 ->
+            // 448 x 448 6.1 / 5.3, 8.5 / 7.0, 9.4 / 7.2). One channel's largest launches pay more for the column terms (24 x 720p -> 1080p
+            // 16.0 / 17.0, 32 of these 19.8 / 21.8) unless rows end inside lines of memory (100 x 300 x 300 -> 1000 x 500 20.5 / 18.7).
+            const bool flat   = FlatBlocks(a.dstW, kQuadsTileW);
+            const int  rows   = C == 1 && strips >= 60 * 256 && a.dstRowStride % 64 == 0 ? kStripRows : 4;
+            auto       kernel = rows == 4 ? ResizeNearestQuadsU8Kernel<C, 4> : ResizeNearestQuadsU8Kernel<C, C == 1 ? kStripRows : 4>;
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeNearestQuadsU8Kernel");
             return;
         }
@@ -3856,8 +3880,8 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         {
             const bool flat = FlatBlocks(a.dstW, kAreaTileW);
             auto kernel = RowsAreOdd<C>(a) ? ResizeAreaFixedTensorKernel<C, C != 4> : ResizeAreaFixedTensorKernel<C, false>;
-            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, kAreaRowsPerWave, flat),
-                               dim3(256), 0, stream, a, (int)flat);
+            const int rows = AreaRowsPerWave((int64_t)DivUp(a.dstW, kAreaTileW) * DivUp(a.dstH, kAreaRowsMost) * N);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, rows, flat), dim3(256), 0, stream, a, rows, (int)flat);
             CheckLaunch("ResizeAreaFixedTensorKernel");
             return;
         }
@@ -4030,11 +4054,16 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
         }
         if constexpr (kAreaFixed<T, C, INTERP>)
         {
-            int total = BuildVarTiles(tiles, dstHost, first, count, kAreaTileW, kAreaTileH);
+            int       total = BuildVarTiles(tiles, dstHost, first, count, kAreaTileW, 4 * kAreaRowsMost);
+            const int rows  = AreaRowsPerWave(4 * (int64_t)total);
+            if (rows != kAreaRowsMost)
+            {
+                total = BuildVarTiles(tiles, dstHost, first, count, kAreaTileW, 4 * rows);
+            }
             if (total > 0)
             {
                 auto kernel = RowsAreOdd<C>(srcHost + first, count) ? ResizeAreaVarShapeKernel<C, C != 4> : ResizeAreaVarShapeKernel<C, false>;
-                hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a, tiles);
+                hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a, tiles, rows);
                 CheckLaunch("ResizeAreaVarShapeKernel");
             }
             continue;
@@ -4050,12 +4079,24 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
                 stripPixels += NearestStripScale<C>(sp.width, sp.height, dp.width, dp.height) ? px : 0;
             }
             const bool flat  = flatFor(kStripsWaveW<true>);
-            int        total = 2 * stripPixels > allPixels ? buildTiles(kStripsWaveW<true>, kStripsWaveH<true>, flat) : 0;
-            if (total >= 8 * 256)
+            // (us as patches / 4 rows, three channels: 8 x 640 x 480 -> 1280 x 720 10.8 / 8.0; 32 x 224 x 224 -> 448 x 448 9.8 / 7.1; 8 x
+            // 320 x 240 -> 640 x 480 5.8 / 5.9; 8 / 4 rows: 16 x 720p -> 1080p 24.2 / 20.9, one channel 13.8 / 16.1)
+            if (2 * stripPixels > allPixels)
             {
-                hipLaunchKernelGGL((ResizeNearestStripsU8VarShapeKernel<C>), dim3(total), dim3(256), 0, stream, a, tiles, (int)flat);
-                CheckLaunch("ResizeNearestStripsU8VarShapeKernel");
-                continue;
+                int rows  = C == 1 ? kStripRows : 4;
+                int total = buildTiles(kStripsWaveW<true>, rows, flat);
+                if (C == 1 && total < 8 * 256)
+                {
+                    rows  = 4;
+                    total = buildTiles(kStripsWaveW<true>, rows, flat);
+                }
+                if (total >= 2 * 256)
+                {
+                    auto kernel = rows == 4 ? ResizeNearestStripsU8VarShapeKernel<C, 4> : ResizeNearestStripsU8VarShapeKernel<C, C == 1 ? kStripRows : 4>;
+                    hipLaunchKernelGGL(kernel, dim3(total), dim3(256), 0, stream, a, tiles, (int)flat);
+                    CheckLaunch("ResizeNearestStripsU8VarShapeKernel");
+                    continue;
+                }
             }
         }
         if constexpr (INTERP == NVCV_INTERP_CUBIC && std::is_same_v<T, uint8_t> && (C == 3 || C == 4))

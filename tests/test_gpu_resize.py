@@ -789,3 +789,29 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
         assert bool((buf == -7.0).all()), "floats outside the rows written"
     assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
     assert not torch.isnan(results[0]).any()
+
+
+# Rows per wave by the size of the launch: the box filter at scales of 1 to 3 (4 rows to a wave up to 2048 waves of 16, 8 up to 8192, then 16), for nearest
+# neighbour enlarging by 1.5 or more (strips of 4 rows from 1024 strips of 8 on, 1536 with three channels; 8 rows for one channel
+# from 15360 on) and for float bicubic (4 rows, 8, 16; from 128 waves of 4 rows on, 512 with three and four channels)
+@pytest.mark.parametrize("row", [(sw, sh, dw, dh, AREA, n, np.uint8, c)
+                                 for c in (1, 3, 4)
+                                 for (sw, sh, dw, dh, n) in [(97, 23, 61, 9, 1), (64, 40, 65, 39, 2), (130, 30, 64, 15, 3), (190, 50, 63, 17, 4),
+                                                             (70, 18, 64, 16, 2048), (70, 19, 64, 17, 1025), (70, 19, 65, 16, 4096),
+                                                             (70, 18, 64, 16, 8193)]]
+                         + [(sw, sh, dw, dh, NEAREST, n, np.uint8, c)
+                            for c in (1, 3, 4)
+                            for (sw, sh, dw, dh, n) in [(100, 6, 256, 7, 1024), (100, 6, 253, 9, 513), (100, 6, 257, 8, 768), (100, 8, 255, 3, 1535),
+                                                        (100, 8, 256, 8, 1536), (170, 5, 256, 5, 1600)]]
+                         + [(100, 6, 256, 8, NEAREST, 15360, np.uint8, 1), (100, 6, 256, 7, NEAREST, 15360, np.uint8, 1), (100, 6, 253, 8, NEAREST, 15360, np.uint8, 1)]
+                         + [(sw, sh, dw, dh, CUBIC, n, np.float32, c)
+                            for c in (1, 3, 4)
+                            for (sw, sh, dw, dh, n) in [(40, 8, 64, 4, 127), (40, 8, 64, 4, 128), (40, 8, 64, 5, 256), (40, 8, 64, 3, 512),
+                                                        (60, 9, 65, 6, 256), (60, 9, 63, 7, 3840), (60, 9, 63, 7, 4500), (60, 9, 64, 9, 2560),
+                                                        (60, 9, 64, 9, 2305)]],
+                         ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
+def test_tensor_rows_per_wave(cv, orc, gpu, row):
+    if row[4] == AREA:
+        test_area_tensor(cv, orc, gpu, row[:4] + row[5:])
+    else:
+        test_tensor_table(cv, orc, gpu, row)
