@@ -165,13 +165,21 @@ template<class TI, class TO, int C>
 __device__ __forceinline__ void NormRun(const NormArgs &a, const uint8_t *srcRow, uint8_t *dstRow, int W, int x0)
 {
     constexpr int P = kNormRunPixels<TI, TO, C>;
-    // every uniform value is loaded before the first use, so the loads share one round trip
+    // every uniform value is loaded before the first use, so the loads share one round trip, and the pixels are requested
+    // before the scales are finished, which wait for it: one round trip to memory less in a wave that has two or three (f32x3 with
+    // standard deviations, 16 x 224 x 224 6.8 -> 6.0 us, 55 x 299 x 299 23.8 -> 21.2; a wave of 2 or 4 rows gave no more)
     float b[C], m[C];
 #pragma unroll
     for (int c = 0; c < C; ++c)
     {
         b[c] = a.base.ptr[c * a.base.sC];
         m[c] = a.scale.ptr[c * a.scale.sC];
+    }
+    const bool whole = x0 + P <= W;
+    TI         in[P * C];
+    if (whole)
+    {
+        LoadRun<TI, P * C>(srcRow + (int64_t)x0 * C * sizeof(TI), in);
     }
     if (a.stddev)
     {
@@ -182,11 +190,9 @@ __device__ __forceinline__ void NormRun(const NormArgs &a, const uint8_t *srcRow
             m[c]          = 1.0f / sqrtf(t);
         }
     }
-    if (x0 + P <= W)
+    if (whole)
     {
-        TI in[P * C];
         TO out[P * C];
-        LoadRun<TI, P * C>(srcRow + (int64_t)x0 * C * sizeof(TI), in);
         if (a.gscale == 1.f && a.shift == 0.f) // wave-uniform; x * 1 + 0 == x, two operations per element saved
         {
 #pragma unroll
