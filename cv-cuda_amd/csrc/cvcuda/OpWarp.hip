@@ -12,12 +12,12 @@
 // owns no device buffer and launches no separate inversion kernel; several var-shape submissions of
 // one operator handle may therefore be in flight at once. Var-shape batches run on a packed tile grid.
 //
-// Kernel shape. A 256-thread block produces a 64 x 16 pixel tile of the destination; each of its four
-// waves works on its own 32 x 8 part, no barrier.
+// Kernel shape. A 256-thread block produces a 64 x 16 pixel tile of the destination (64 x 8 in small launches); each of its four
+// waves works on its own 32 x 8 (16 x 8) part, no barrier.
 // Gather: the cost of the gather is set by how many distinct cache lines one wave-wide load touches,
 // and under a rotation every source row a wave's footprint crosses is another line; so a wave samples
 // compact 8 x 8 pixel patches (one lane per pixel, ~10 source rows per load where a 64 x 1 strip would
-// cross ~20), four patches side by side per wave, i.e. kPxPerLane = 4 independent samples per lane
+// cross ~20), four patches (two) side by side per wave, i.e. 4 independent samples per lane
 // whose loads are in flight together. Taps that lie inside the source image - nearly all of them -
 // skip the border logic and fetch the horizontally adjacent taps of a row with one load (u8x3: the 6
 // bytes of two pixels from an aligned 12-byte window).
@@ -40,13 +40,18 @@ namespace cvamd {
 
 namespace {
 
-constexpr int kPatch     = 8;  // gather granule: a wave samples kPatch x kPatch pixels per step
-constexpr int kPxPerLane = 4;  // steps per wave
-constexpr int kTileW     = 64; // = 8 patches
-constexpr int kTileH     = 16; // = 2 patches; 16 patches / 4 waves = kPxPerLane
-constexpr int kWaveW     = kPatch * kPxPerLane; // a wave's patches lie side by side
-constexpr int kWavesX    = kTileW / kWaveW;
-constexpr int kThreads   = kTileW * kTileH / kPxPerLane;
+constexpr int kPatch   = 8; // gather granule: a wave samples kPatch x kPatch pixels per step
+constexpr int kThreads = 256;
+// A wave's N patches lie side by side, N = kMostPatches or kFewPatches (see LaunchMap); a block's four waves as two by two or in a row.
+constexpr int kMostPatches = 4, kFewPatches = 2;
+template<int N>
+constexpr int kWaveW = kPatch * N;
+template<int N>
+constexpr int kWavesX = N == kMostPatches ? 2 : 4;
+template<int N>
+constexpr int kTileW = kWaveW<N> * kWavesX<N>;
+template<int N>
+constexpr int kTileH = kThreads / 64 / kWavesX<N> * kPatch;
 
 struct WarpArgs
 {
@@ -258,7 +263,6 @@ __device__ __forceinline__ float ReciprocalInRange(float x)
 template<bool PERSPECTIVE, int N>
 __device__ __forceinline__ void MapCoords(const float (&m)[9], const int (&dx)[N], const int (&dy)[N], float (&sx)[N], float (&sy)[N])
 {
-    static_assert(N == 4);
     if constexpr (PERSPECTIVE)
     {
         float    coeff[N];
@@ -283,7 +287,13 @@ __device__ __forceinline__ void MapCoords(const float (&m)[9], const int (&dx)[N
 #pragma nounroll
             for (int k = 0; k < N; ++k)
             {
-                const float q = 1.0f / (k == 0 ? coeff[0] : k == 1 ? coeff[1] : k == 2 ? coeff[2] : coeff[3]);
+                float c = coeff[0];
+#pragma unroll
+                for (int j = 1; j < N; ++j)
+                {
+                    c = j == k ? coeff[j] : c;
+                }
+                const float q = 1.0f / c;
 #pragma unroll
                 for (int j = 0; j < N; ++j)
                 {
@@ -480,16 +490,15 @@ __device__ __forceinline__ void SampleWithBorder(const Img &im, const WarpArgs &
 // of the float's bit pattern: non-negative floats order like their bits, negative ones and NaNs have
 // patterns above every finite positive limit (-0.0 fails too and takes the generic path, which
 // computes the same result).
-// The test runs on a lane's kPxPerLane samples at once: the largest bit pattern per axis against the limit.
-template<int INTERP>
-__device__ __forceinline__ bool TapsInside(float limX, float limY, const float (&sx)[kPxPerLane],
-                                           const float (&sy)[kPxPerLane])
+// The test runs on a lane's N samples at once: the largest bit pattern per axis against the limit.
+template<int INTERP, int N>
+__device__ __forceinline__ bool TapsInside(float limX, float limY, const float (&sx)[N], const float (&sy)[N])
 {
     // taps span [floor(v) - lo, floor(v) + hi] per axis; NEAREST takes floor(v + .5)
     constexpr float lo = INTERP == NVCV_INTERP_CUBIC ? 1.f : (INTERP == NVCV_INTERP_NEAREST ? -.5f : 0.f);
     uint32_t        ux = 0, uy = 0;
 #pragma unroll
-    for (int k = 0; k < kPxPerLane; ++k)
+    for (int k = 0; k < N; ++k)
     {
         ux = max(ux, __float_as_uint(sx[k] - lo));
         uy = max(uy, __float_as_uint(sy[k] - lo));
@@ -1340,29 +1349,29 @@ __device__ __forceinline__ bool NarrowTapsPay(const float (&m)[9])
     return fabsf(m[3]) > (INTERP == NVCV_INTERP_LINEAR ? 1.f : 1.5f) * fabsf(m[0]);
 }
 
-// One 64 x 16 tile of the destination image `dst` (tile coordinates tx, ty), all 256 threads.
-template<class T, int C, int INTERP, bool PERSP, bool LIST>
+// One tile of kTileW<N> x kTileH<N> pixels of the destination image `dst` (tile coordinates tx, ty), all 256 threads.
+template<class T, int C, int INTERP, bool PERSP, bool LIST, int N>
 __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const float (&m)[9], uint8_t *dst, int dstRow,
                                          int dstW, int dstH, int tx, int ty)
 {
     constexpr int PB = C * sizeof(T), D = (PB + 3) / 4;
 
-    // ---- gather: lane (lx, ly) of wave w samples its pixel in patches 4w .. 4w+3 (side by side: a
-    // wave covers 32 columns x 8 rows)
+    // ---- gather: lane (lx, ly) of wave w samples its pixel in N patches (side by side: a
+    // wave covers 8 N columns x 8 rows)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lx = threadIdx.x & (kPatch - 1),
               ly = (threadIdx.x >> 3) & (kPatch - 1);
-    const int x0 = tx * kTileW + wave % kWavesX * kWaveW, y0 = ty * kTileH + wave / kWavesX * kPatch;
+    const int x0 = tx * kTileW<N> + wave % kWavesX<N> * kWaveW<N>, y0 = ty * kTileH<N> + wave / kWavesX<N> * kPatch;
     // m maps to source coordinates times kCoordScale; so do sx, sy and the limits
     constexpr float kScale = kCoordScale<T, INTERP>;
     const float     limX = InsideLimit<INTERP>(im.w, kTapOverrun<T, C, INTERP>) * kScale, limY = InsideLimit<INTERP>(im.h, 0) * kScale;
-    int         px[kPxPerLane], py[kPxPerLane]; // the lane's destination pixels
-    float       sx[kPxPerLane], sy[kPxPerLane];
-    uint32_t    q[D][kPxPerLane]; // q[d][k]: dword d of this lane's pixel in patch k
+    int         px[N], py[N]; // the lane's destination pixels
+    float       sx[N], sy[N];
+    uint32_t    q[D][N]; // q[d][k]: dword d of this lane's pixel in patch k
     // rows too long or too many for 24-bit offset arithmetic go through the generic path
     // (and, in fixed point, coordinates too large for coordinate * 2^15 in 31 bits)
     const bool fits = (im.row | im.h) < (1 << 23) && (!kFixedPoint<T, INTERP> || (im.w | im.h) < (1 << 16));
 #pragma unroll
-    for (int k = 0; k < kPxPerLane; ++k)
+    for (int k = 0; k < N; ++k)
     {
         // pixels of the tile beyond the image edge repeat the edge pixel's sample; they are never stored
         px[k] = min(x0 + k * kPatch + lx, dstW - 1);
@@ -1370,18 +1379,18 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     }
     MapCoords<PERSP>(m, px, py, sx, sy);
     // the wave's pixels as rows, for the store (kPitch: neighbouring rows on other banks)
-    constexpr int kPitch = kWaveW * D + (D == 1 ? 8 : D == 2 ? 16 : D == 4 ? 24 : 0);
+    constexpr int kPitch = kWaveW<N> * D + (D == 1 ? 8 : D == 2 ? 16 : D == 4 ? 24 : 0);
     __shared__ __align__(16) uint32_t room[kThreads / 64][kPatch][kPitch];
     auto     &rows = room[wave];
     const int lane = threadIdx.x & 63;
 
     auto sampleInside = [&]()
     {
-        uint32_t w[kPxPerLane][D];
+        uint32_t w[N][D];
         auto sample = [&](auto form)
         {
 #pragma unroll
-            for (int k = 0; k < kPxPerLane; ++k)
+            for (int k = 0; k < N; ++k)
             {
                 SampleInsidePacked<T, C, INTERP, decltype(form)::value>(im, sx[k], sy[k], w[k]);
             }
@@ -1399,7 +1408,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             sample(std::integral_constant<int, kOddRows>{});
         }
 #pragma unroll
-        for (int k = 0; k < kPxPerLane; ++k)
+        for (int k = 0; k < N; ++k)
         {
 #pragma unroll
             for (int d = 0; d < D; ++d)
@@ -1425,7 +1434,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         // third are such: 3 x 258 x 271 f32x1 bicubic 16.0 -> 6.7 us, 7 x 318 x 538 f32x4 bilinear 14.6 -> 9.6, 3 x 646 x 752 f32x1 bilinear
         // 9.7 -> 6.2, 40 x 1021 x 1523 of these 169 -> 145; 38 images of 75 .. 801 x 232 .. 359 u8x3 bicubic 36.3 -> 32.0.
         const bool whole  = __builtin_amdgcn_ballot_w64(!fits || !TapsInside<INTERP>(limX, limY, sx, sy)) == 0;
-        __shared__ uint8_t list[kThreads / 64][64 * kPxPerLane];
+        __shared__ uint8_t list[kThreads / 64][64 * N];
         uint32_t inside = 0xf, colour[D] = {}; // inside: bit k: sample k
         int      edges  = 0;
         if (!whole)
@@ -1434,7 +1443,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             BorderDwords<T, C>(a, colour);
             inside = 0;
 #pragma unroll
-            for (int k = 0; k < kPxPerLane; ++k)
+            for (int k = 0; k < N; ++k)
             {
                 const bool in  = fits && TapInside<INTERP>(limX, limY, sx[k], sy[k]);
                 const bool out = constant && TapsOutside<INTERP>(im, sx[k] * (1.f / kScale), sy[k] * (1.f / kScale));
@@ -1476,7 +1485,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         if (whole)
         {
 #pragma unroll
-            for (int k = 0; k < kPxPerLane; ++k)
+            for (int k = 0; k < N; ++k)
             {
                 place(k);
             }
@@ -1484,7 +1493,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         else
         {
 #pragma unroll
-            for (int k = 0; k < kPxPerLane; ++k)
+            for (int k = 0; k < N; ++k)
             {
                 if ((inside >> k) & 1)
                 {
@@ -1548,14 +1557,14 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             const BorderFold foldX = MakeBorderFold(a.border, im.w), foldY = MakeBorderFold(a.border, im.h);
             bool             outside = constant;
 #pragma unroll
-            for (int k = 0; k < kPxPerLane; ++k)
+            for (int k = 0; k < N; ++k)
             {
                 outside &= TapsOutside<INTERP>(im, sx[k] * (1.f / kScale), sy[k] * (1.f / kScale));
             }
             if (outside)
             {
 #pragma unroll
-                for (int k = 0; k < kPxPerLane; ++k)
+                for (int k = 0; k < N; ++k)
                 {
                     if constexpr (kFixedPointCubic<T, INTERP>)
                     {
@@ -1581,10 +1590,15 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                 // one sample at a time (all four at once took 143 registers, which every wave of the launch would have held;
                 // held to the 64 of full occupancy the u8x3 kernel spills and loses 1 to 2 %)
 #pragma nounroll
-                for (int k = 0; k < kPxPerLane; ++k)
+                for (int k = 0; k < N; ++k)
                 {
-                    const float    bx = k == 0 ? sx[0] : (k == 1 ? sx[1] : (k == 2 ? sx[2] : sx[3]));
-                    const float    by = k == 0 ? sy[0] : (k == 1 ? sy[1] : (k == 2 ? sy[2] : sy[3]));
+                    float bx = sx[0], by = sy[0];
+#pragma unroll
+                    for (int j = 1; j < N; ++j)
+                    {
+                        bx = k == j ? sx[j] : bx;
+                        by = k == j ? sy[j] : by;
+                    }
                     // (a copy for each border: in one, the replicating border does the colour's share of the work as well; 32 x 256 x
                     // 256 u8x1 11.9 us in one copy, 10.0 in two, 4 x 1283 x 721 u8x3 27.4 and 25.9)
                     uint32_t v;
@@ -1597,7 +1611,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                         v = SampleClampedCubicQ14<C>(im, false, colour[0], bx, by);
                     }
 #pragma unroll
-                    for (int j = 0; j < kPxPerLane; ++j)
+                    for (int j = 0; j < N; ++j)
                     {
                         q[0][j] = k == j ? v : q[0][j];
                     }
@@ -1606,7 +1620,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             else
             {
 #pragma unroll
-                for (int k = 0; k < kPxPerLane; ++k)
+                for (int k = 0; k < N; ++k)
                 {
                     if constexpr (kFixedPoint<T, INTERP>)
                     {
@@ -1638,7 +1652,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         else
         {
 #pragma nounroll
-            for (int k = 0; k < kPxPerLane; ++k)
+            for (int k = 0; k < N; ++k)
             {
                 // position and coordinates recomputed rather than indexed, results placed by selects: a
                 // run-time index would put the arrays in scratch memory
@@ -1663,7 +1677,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                 {
                     asm("" : "+v"(w[d]));
 #pragma unroll
-                    for (int j = 0; j < kPxPerLane; ++j)
+                    for (int j = 0; j < N; ++j)
                     {
                         q[d][j] = k == j ? w[d] : q[d][j];
                     }
@@ -1671,7 +1685,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             }
         }
 #pragma unroll
-        for (int k = 0; k < kPxPerLane; ++k)
+        for (int k = 0; k < N; ++k)
         {
             place(k);
         }
@@ -1685,14 +1699,14 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     // large; a second form of the store for these cost all others 3 to 5 %).
     if constexpr (PB >= 12)
     {
-        constexpr int kChunks = kWaveW * PB / 16;
-        const int dwords = min(dstW - x0, kWaveW) * D; // of a row
+        constexpr int kChunks = kWaveW<N> * PB / 16;
+        const int dwords = min(dstW - x0, kWaveW<N>) * D; // of a row
         uint8_t  *to = dst + (int64_t)y0 * dstRow + (int64_t)x0 * PB;
 #pragma unroll
-        for (int i = 0; i < D; ++i)
+        for (int i = 0; i < (kPatch * kChunks + 63) / 64; ++i)
         {
             const int row = (lane + 64 * i) / kChunks, at = (lane + 64 * i) % kChunks * 4;
-            if (y0 + row >= dstH || at >= dwords)
+            if (y0 + row >= dstH || at >= dwords || (kPatch * kChunks % 64 != 0 && row >= kPatch))
             {
                 continue;
             }
@@ -1722,6 +1736,11 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     // instructions; moves and selects between lanes took 20 for each dword of a pixel, and left a row's pieces in another
     // order than the lanes'.)
     const int dx0 = x0 + 4 * lx;
+    uint32_t  quad[D][4] = {};
+    if (N < kMostPatches && lx >= kWaveW<N> / 4)
+    {
+        return;
+    }
     if constexpr (PB < 12)
     {
 #pragma unroll
@@ -1730,7 +1749,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
             for (int d = 0; d < D; ++d)
             {
-                q[d][k] = rows[ly][(4 * lx + k) * D + d];
+                quad[d][k] = rows[ly][(4 * lx + k) * D + d];
             }
         }
     }
@@ -1744,7 +1763,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     if (dx0 + 4 <= dstW)
     {
         uint32_t w[PB];
-        PackQuad<PB>(q, w);
+        PackQuad<PB>(quad, w);
         StoreDwordsNT<PB>(to, w); // 4 pixels = PB dwords
     }
     else
@@ -1758,7 +1777,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
 #pragma unroll
                 for (int d = 0; d < D; ++d)
                 {
-                    w[d] = q[d][k];
+                    w[d] = quad[d][k];
                 }
                 Vec<T, C> px;
                 __builtin_memcpy(&px, w, PB);
@@ -1828,7 +1847,7 @@ __device__ __forceinline__ void LoadMatrix(const WarpArgs &a, int image, float s
     }
 }
 
-template<class T, int C, int INTERP, bool PERSP, bool LIST>
+template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES>
 __global__ __launch_bounds__(kThreads) void WarpTensor(const WarpArgs a)
 {
     const int n  = blockIdx.z;
@@ -1839,10 +1858,10 @@ __global__ __launch_bounds__(kThreads) void WarpTensor(const WarpArgs a)
     {
         m[i] = a.m[i];
     }
-    WarpTile<T, C, INTERP, PERSP, LIST>(im, a, m, a.dst + n * a.dstN, a.dstRow, a.dstW, a.dstH, blockIdx.x, blockIdx.y);
+    WarpTile<T, C, INTERP, PERSP, LIST, PATCHES>(im, a, m, a.dst + n * a.dstN, a.dstRow, a.dstW, a.dstH, blockIdx.x, blockIdx.y);
 }
 
-template<class T, int C, int INTERP, bool PERSP, bool LIST>
+template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES>
 __global__ __launch_bounds__(kThreads) void WarpVarShape(const WarpArgs a, const VarTiles tiles)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
@@ -1853,26 +1872,54 @@ __global__ __launch_bounds__(kThreads) void WarpVarShape(const WarpArgs a, const
     float                       m[9];
     LoadMatrix<PERSP>(a, tc.image, kCoordScale<T, INTERP>, m);
     const Img im = {AsGlobal(s.basePtr), s.rowStride, s.width, s.height};
-    WarpTile<T, C, INTERP, PERSP, LIST>(im, a, m, AsGlobal(d.basePtr), d.rowStride, d.width, d.height, tc.tx, tc.ty);
+    WarpTile<T, C, INTERP, PERSP, LIST, PATCHES>(im, a, m, AsGlobal(d.basePtr), d.rowStride, d.width, d.height, tc.tx, tc.ty);
 }
+
+// Two patches per wave instead of four where that leaves a SIMD no more than 3 waves of four: such launches run as long as one
+// wave does, whose four samples a lane follow one another in issue, and half of it is done in little more than half the
+// time. From about 5 waves per SIMD on the waves' own start (matrix, tile search, edge tests) is what counts. Kernel us with four / two
+// patches, under a constant border: u8x3 bicubic 320 x 240 8.8 / 6.0, 640 x 480 8.8 / 6.6, 2 of them (2 400 waves) 8.0 / 7.0, 4 10.6 / 10.0,
+// 8 15.1 / 15.5, 16 24.9 / 27.0; bilinear 4.6 / 3.8, 5.1 / 4.1, 5.3 / 4.6, 6.1 / 6.0, 8.8 / 8.7, 13.4 / 14.4; f32x4 bicubic 7.6 / 5.4, 8.0 / 7.0, 10.0 /
+// 9.3, 14.6 / 13.4; f32x1 bilinear 4.4 / 3.8, 4.6 / 4.4, 4.6 / 4.4, 5.3 / 5.5, 7.2 / 7.8; u8x3 nearest 3.8 / 3.4, 3.8 / 3.3, 4.2 / 3.9, 4.6 / 4.8.
+// (One patch: 320 x 240 u8x3 bicubic 5.2, but 2 x 640 x 480 7.4 and 16 30.5; elements of 16 bits keep four, for the size of the library.)
+constexpr int64_t kFewWaves = 3 * 1024;
+template<class T>
+constexpr bool kFewPatchesForm = std::is_same_v<T, uint8_t> || std::is_same_v<T, float>;
 
 template<class T, int C, int INTERP, bool PERSP, bool LIST>
 void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, hipStream_t stream)
 {
+    constexpr int kMost = kMostPatches, kFew = kFewPatchesForm<T> ? kFewPatches : kMost;
+    const auto    few = [](int64_t tiles) { return kFew != kMost && tiles * (kThreads / 64) <= kFewWaves; };
     if (dstHost == nullptr)
     {
-        dim3 grid(DivUp(a.dstW, kTileW), DivUp(a.dstH, kTileH), N);
-        hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST>), grid, dim3(kThreads), 0, stream, a);
+        const dim3 most(DivUp(a.dstW, kTileW<kMost>), DivUp(a.dstH, kTileH<kMost>), N);
+        if (few((int64_t)most.x * most.y * most.z))
+        {
+            const dim3 grid(DivUp(a.dstW, kTileW<kFew>), DivUp(a.dstH, kTileH<kFew>), N);
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kFew>), grid, dim3(kThreads), 0, stream, a);
+        }
+        else
+        {
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kMost>), most, dim3(kThreads), 0, stream, a);
+        }
         CheckLaunch("WarpTensor");
         return;
     }
     for (int first = 0; first < N; first += kMaxTileImages)
     {
-        VarTiles tiles;
-        int      total = BuildVarTiles(tiles, dstHost, first, std::min(kMaxTileImages, N - first), kTileW, kTileH);
-        if (total > 0)
+        VarTiles  tiles;
+        const int count = std::min(kMaxTileImages, N - first);
+        int       total = BuildVarTiles(tiles, dstHost, first, count, kTileW<kMost>, kTileH<kMost>);
+        if (total > 0 && few(total))
         {
-            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
+            total = BuildVarTiles(tiles, dstHost, first, count, kTileW<kFew>, kTileH<kFew>);
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kFew>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
+            CheckLaunch("WarpVarShape");
+        }
+        else if (total > 0)
+        {
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kMost>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
             CheckLaunch("WarpVarShape");
         }
     }

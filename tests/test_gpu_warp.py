@@ -231,6 +231,54 @@ def test_wide_pixels_at_the_tile_edges(cv, orc, gpu, dw, dh, c):
     assert (res[:4] == -7).all() and (res[-4:] == -7).all()
 
 
+# launches of up to 3072 waves of four patches give each wave two: results about both tiles' edges, in the largest launch of the one
+# form and the smallest of the other, each image of a batch as the oracle has it and nothing written beside them
+@pytest.mark.parametrize("dt,c", [(np.uint8, 1), (np.uint8, 3), (np.uint8, 4), (np.float32, 1), (np.float32, 3), (np.float32, 4)])
+@pytest.mark.parametrize("dw,dh", [(1, 1), (15, 7), (17, 9), (31, 8), (33, 17), (62, 5), (64, 16), (67, 23)])
+def test_patches_per_wave(cv, orc, gpu, dw, dh, dt, c):
+    src = (orc.fill_f32((2, 21, 37, c), 5 + dw) * 255).astype(dt)
+    tiles, size = -(-dw // 64) * -(-dh // 16), np.dtype(dt).itemsize
+    for n in (768 // tiles, 768 // tiles + 1):
+        tin = cv.Tensor.from_numpy(src[np.arange(n) % 2], "NHWC")
+        buf = torch.empty((n * dh * dw * c * size + 32,), dtype=torch.uint8, device="cuda")
+        tout = cv.Tensor.wrap(buf.data_ptr() + 16, [n, dh, dw, c], [dh * dw * c * size, dw * c * size, c * size, size], dt, "NHWC", keep=buf)
+        for interp, border in itertools.product((NEAREST, LINEAR, CUBIC), (0, 1, 4)):
+            m = rotation(37, 21, 12.0 + border, 0.9)
+            buf.fill_(0xA5)
+            cv.WarpAffine(0)(None, tin, tout, m, interp, border, (9, 8, 7, 6))
+            torch.cuda.synchronize()
+            res = buf.cpu().numpy()
+            assert (res[:16] == 0xA5).all() and (res[-16:] == 0xA5).all()
+            got = res[16:-16].view(dt).reshape(n, dh, dw, c)
+            np.testing.assert_array_equal(got, got[np.arange(n) % 2])
+            dev = orc.warp(src, (dh, dw), orc.invert_affine(m), interp, border, (9, 8, 7, 6), variant=device_variant(interp, dt))
+            if dt == np.float32:
+                assert np.abs(got[:2] - dev).max() <= 1e-3, (interp, border)  # (as above)
+            else:
+                np.testing.assert_array_equal(got[:2], dev, err_msg=str((interp, border)))
+
+
+@pytest.mark.parametrize("n", [2, 3])  # of 300 tiles of 64 x 16 each, and what is left over at their edges
+def test_patches_per_wave_of_image_batches(cv, K, orc, gpu, n):
+    bi, bo, hosts, outs, mats = cv.ImageBatchVarShape(n), cv.ImageBatchVarShape(n), [], [], []
+    for i in range(n):
+        w, h = 639 - 17 * i, 475 + i
+        hosts.append(orc.fill_u8((h, w, 3), 70 + i))
+        bi.push_back(cv.Image.from_numpy(hosts[i], K.IMAGE_FORMAT_RGB8))
+        outs.append(cv.Image.alloc((w, h), K.IMAGE_FORMAT_RGB8))
+        bo.push_back(outs[i])
+        mats.append(rotation(w, h, 11.0 - 9 * i, 1.1))
+    mats = np.asarray(mats, np.float32)
+    for interp, border in itertools.product((NEAREST, LINEAR, CUBIC), (0, 1)):
+        cv.WarpAffine(n)(None, bi, bo, cv.Tensor.from_numpy(mats, "NW"), interp, border, (10, 20, 30, 40))
+        torch.cuda.synchronize()
+        for i in range(n):
+            w, h = outs[i].size
+            dev = orc.warp(hosts[i][None], (h, w), orc.invert_affine(mats[i]), interp, border, (10, 20, 30, 40),
+                           variant=device_variant(interp))[0]
+            np.testing.assert_array_equal(outs[i].plane_view(0, np.uint8, 3).cpu().numpy(), dev, err_msg=str((interp, border, i)))
+
+
 # the same for the other interpolations and borders, and for sources and results that are views: rows 4 bytes off a 16-byte
 # boundary in another pitch. A view's result is the dense one's, bit for bit
 @pytest.mark.parametrize("c", [3, 4])
