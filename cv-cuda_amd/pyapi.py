@@ -661,7 +661,7 @@ def _plane_list(buffers, format):
     planes = _native.planes(buffers) if len(buffers) else None
     if planes is None:
         return None
-    kind = (buffers[0].dtype, planes[0])
+    kind = (next(iter(buffers)).dtype, planes[0])
     if kind[0] not in _PLANE_TORCH or (format is None and kind not in _FORMAT_OF_TORCH):
         return None
     return (_FORMAT_OF_TORCH[kind] if format is None else int(format)), planes[1]
@@ -678,12 +678,13 @@ def as_images(buffers, format=None):
     tensors go to the library in one call, and their Image objects are made when somebody asks for them: 61 images one
     by one were 340 us of a 380 us call of an operator whose kernel takes 14."""
     batch = ImageBatchVarShape(len(buffers))
+    buffers = list(buffers)
     planes = _plane_list(buffers, format)
     if planes is None:
         batch.pushback([as_image(b, format) for b in buffers])
     else:
         check(_nv.nvcvxImageBatchVarShapePushBuffers(batch.handle, planes[0], planes[1], len(buffers)))
-        batch._buffers = list(buffers)
+        batch._buffers = buffers
     return batch
 
 

@@ -270,6 +270,15 @@ def test_a_stream_that_follows_the_default_one_waits_for_what_it_reads_alone(api
     assert FakeEvent.made - before == api._FOLLOWED_CALLS < 2000
 
 
+def test_planes_of_buffers_that_have_no_index(api, monkeypatch):
+    import types
+
+    import torch
+    monkeypatch.setattr(api, "_native", types.SimpleNamespace(planes=lambda buffers: (3, b"planes")))
+    frames = {"left": torch.zeros((4, 5, 3), dtype=torch.uint8), "right": torch.zeros((6, 5, 3), dtype=torch.uint8)}
+    assert api._plane_list(frames.values(), None) == (int(api.Format.RGB8), b"planes")
+
+
 def test_images_of_a_batch_asked_for_by_several_threads(api, monkeypatch):
     # a batch made in one call makes its Image objects when they are asked for: every thread gets all of them, the same
     # ones, and a failure loses no buffer (no GPU: the library's call is a stand-in that takes its time)
