@@ -462,7 +462,7 @@ PyObject *Submit(PyObject *, PyObject *const *a, Py_ssize_t n)
     Py_RETURN_NONE;
 }
 
-// default_stream_key(): pyapi._default_stream_key(None).
+// default_stream_key(): pyapi._default_stream_key(None) outside `with stream:`; None inside, where Python looks at the stream.
 PyObject *DefaultKey(PyObject *, PyObject *)
 {
     long key;

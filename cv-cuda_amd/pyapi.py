@@ -470,7 +470,8 @@ def clear_cache():
 def _result(shape, dtype, layout, stream):
     """A tensor for an operator's result. Only a call on the default stream takes one that is handed out again: another
     stream would have to wait for the default stream's last use of it, which one that is being captured cannot."""
-    if (_native.default_stream_key() if stream is None else _default_stream_key(stream)) is None:
+    key = _native.default_stream_key() if stream is None else None
+    if key is None and _default_stream_key(stream) is None:
         return Tensor(tuple(shape), dtype, layout)
     return _outputs.get(shape, dtype, layout)
 

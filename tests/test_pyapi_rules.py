@@ -422,6 +422,19 @@ def test_results_on_other_streams_are_always_new(api, monkeypatch):
     assert api._result([2, 3], np.uint8, "HW", FakeStream(0)) == "kept"
 
 
+def test_results_under_an_entered_default_stream_are_kept_ones(api, monkeypatch):
+    # `with Stream.default:` is the default stream too
+    class FakeStream:
+        cuda_stream, device_index = 0, 0
+
+    monkeypatch.setattr(api, "Tensor", lambda *args: "new")
+    monkeypatch.setattr(api._outputs, "get", lambda *args: "kept")
+    monkeypatch.setattr(api.Stream._tls, "stack", [FakeStream()], raising=False)
+    assert api._result((2, 4), np.float32, "NC", None) == "kept"
+    monkeypatch.setattr(FakeStream, "cuda_stream", 7)
+    assert api._result((2, 4), np.float32, "NC", None) == "new"
+
+
 def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
     # an allocation that finds no memory is tried once more without the kept results, which it would otherwise never reach;
     # clear_cache() gives them and the library's blocks back (no GPU: the library's tensors are stand-ins)
