@@ -22,6 +22,7 @@
 
 #include <climits>
 #include <cstring>
+#include <memory>
 
 namespace {
 
@@ -611,19 +612,21 @@ PyObject *TorchView(PyObject *, PyObject *args)
     }
     try
     {
-        auto drop = [owner](void *)
-        {
-            if (Py_IsInitialized())
-            {
-                const PyGILState_STATE state = PyGILState_Ensure();
-                Py_DECREF(owner);
-                PyGILState_Release(state);
-            }
-        };
+        // torch keeps the owner for as long as it keeps the deleter, which it drops where the tensor cannot be made, uncalled
+        Py_INCREF(owner);
+        std::shared_ptr<PyObject> kept(owner,
+                                       [](PyObject *o)
+                                       {
+                                           if (Py_IsInitialized())
+                                           {
+                                               const PyGILState_STATE state = PyGILState_Ensure();
+                                               Py_DECREF(o);
+                                               PyGILState_Release(state);
+                                           }
+                                       });
         const auto options = at::TensorOptions().dtype(isFloat ? at::kFloat : at::kByte).device(at::kCUDA);
-        Py_INCREF(owner); // (the deleter's, which also runs where the tensor cannot be made)
         at::Tensor t = at::from_blob(data.buffer.strided.basePtr, at::IntArrayRef(data.shape, data.rank), at::IntArrayRef(strides, data.rank),
-                                     drop, options);
+                                     [kept = std::move(kept)](void *) {}, options);
         if (t.device().index() != device)
         {
             Py_RETURN_NONE;

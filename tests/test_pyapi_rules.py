@@ -435,6 +435,20 @@ def test_results_under_an_entered_default_stream_are_kept_ones(api, monkeypatch)
     assert api._result((2, 4), np.float32, "NC", None) == "new"
 
 
+def test_view_that_cannot_be_made_gives_its_owner_back(api, cv):
+    # (memory of the host, which torch does not take for a device's)
+    class Owner:
+        pass
+
+    memory, owner = np.zeros((2, 3), np.uint8), Owner()
+    t = cv.Tensor.wrap(memory.ctypes.data, [2, 3], [3, 1], np.uint8, "HW", keep=memory)
+    before = sys.getrefcount(owner)
+    for _ in range(3):
+        with pytest.raises(RuntimeError):
+            api._native.torch_view(t.handle.value, 0, 0, owner)
+    assert sys.getrefcount(owner) == before
+
+
 def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
     # an allocation that finds no memory is tried once more without the kept results, which it would otherwise never reach;
     # clear_cache() gives them and the library's blocks back (no GPU: the library's tensors are stand-ins)
