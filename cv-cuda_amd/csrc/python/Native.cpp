@@ -27,7 +27,6 @@
 namespace {
 
 // names of pyapi and of the containers
-PyObject *g_api; // pyapi's dictionary (its names are looked up in each call: they can be replaced)
 PyObject *s_submit, *s_Tensor, *s_ImageBatchVarShape, *s_lock, *s_followed, *s_tls, *s_stack, *s_check, *s_t, *s_handle, *s_wrote, *s_read,
     *s_kind, *s_acquire, *s_release, *s_torch, *s_C, *s_getDevice, *s_getStream;
 
@@ -51,16 +50,18 @@ struct Ref
     }
 };
 
-PyObject *Name(PyObject *name) // of pyapi; borrowed
+// `api`: pyapi's dictionary, which bind() makes the `self` of the functions that use it (each copy of the package in a process
+// has its own). Its names are looked up in each call: they can be replaced. Borrowed.
+PyObject *Name(PyObject *api, PyObject *name)
 {
-    return PyDict_GetItem(g_api, name);
+    return PyDict_GetItem(api, name);
 }
 
 // The key of the current device's default stream (0, -1, -2 ...) where that is the current stream: false elsewhere, and where
 // a Python error is set.
-bool DefaultStreamKey(long &key)
+bool DefaultStreamKey(PyObject *api, long &key)
 {
-    PyObject *tls = Name(s_tls);
+    PyObject *tls = Name(api, s_tls);
     PyObject *stack = nullptr;
     if (tls == nullptr || _PyObject_LookupAttr(tls, s_stack, &stack) < 0)
     {
@@ -71,7 +72,7 @@ bool DefaultStreamKey(long &key)
     {
         return false;
     }
-    PyObject *torch = Name(s_torch);
+    PyObject *torch = Name(api, s_torch);
     Ref       c(torch != nullptr ? PyObject_GetAttr(torch, s_C) : nullptr);
     if (!c)
     {
@@ -95,10 +96,10 @@ enum Kind
 };
 
 // The library's handle of a container of pyapi.
-Kind HandleOf(PyObject *obj, void *&handle)
+Kind HandleOf(PyObject *api, PyObject *obj, void *&handle)
 {
-    const bool tensor = Py_TYPE(obj) == reinterpret_cast<PyTypeObject *>(Name(s_Tensor));
-    if (!tensor && Py_TYPE(obj) != reinterpret_cast<PyTypeObject *>(Name(s_ImageBatchVarShape)))
+    const bool tensor = Py_TYPE(obj) == reinterpret_cast<PyTypeObject *>(Name(api, s_Tensor));
+    if (!tensor && Py_TYPE(obj) != reinterpret_cast<PyTypeObject *>(Name(api, s_ImageBatchVarShape)))
     {
         return kNone;
     }
@@ -190,14 +191,14 @@ struct Call
     double             d[4];
     float              m[9], bv[4];
 
-    bool Parse(PyObject *const *a, Py_ssize_t n)
+    bool Parse(PyObject *api, PyObject *const *a, Py_ssize_t n)
     {
         auto handles = [&](std::initializer_list<int> at)
         {
             int k = 0;
             for (int index : at)
             {
-                const Kind got = HandleOf(a[index], h[k]);
+                const Kind got = HandleOf(api, a[index], h[k]);
                 if (k == 0)
                 {
                     batch = got == kBatch;
@@ -226,11 +227,11 @@ struct Call
             return n == 9 && handles({0, 1}) && Pair(a[2], i[0], i[1]) && Int(a[3], i[2]) && Pair(a[4], i[3], i[4]) && Int(a[5], i[5])
                 && Real(a[6], d[0]) && Real(a[7], d[1]) && PyBool_Check(a[8]);
         case 7: // CropFlipNormalizeReformat
-            return n == 12 && handles({0, 1, 2, 5, 6}) && HandleOf(a[7], h4) != kNone && batch && Int(a[3], i[0]) && Real(a[4], d[0])
+            return n == 12 && handles({0, 1, 2, 5, 6}) && HandleOf(api, a[7], h4) != kNone && batch && Int(a[3], i[0]) && Real(a[4], d[0])
                 && Real(a[8], d[1]) && Real(a[9], d[2]) && Real(a[10], d[3]) && Int(a[11], i[1]) && i[1] >= 0;
         case 8: // WarpAffine
         case 9: // WarpPerspective
-            return n == 6 && handles({0, 1}) && (batch ? HandleOf(a[2], h[2]) != kNone : Reals(a[2], m, kind == 8 ? 6 : 9)) && Int(a[3], i[0])
+            return n == 6 && handles({0, 1}) && (batch ? HandleOf(api, a[2], h[2]) != kNone : Reals(a[2], m, kind == 8 ? 6 : 9)) && Int(a[3], i[0])
                 && Int(a[4], i[1]) && Reals(a[5], bv, 4);
         default:
             return false;
@@ -394,29 +395,29 @@ bool Mark(PyObject *reads, PyObject *writes, PyObject *key)
 
 // submit(stream, reads, writes, op, *args): pyapi._submit for calls on the current device's default stream, given as None, that
 // wait for nothing; others are handed on to it.
-PyObject *Submit(PyObject *, PyObject *const *a, Py_ssize_t n)
+PyObject *Submit(PyObject *api, PyObject *const *a, Py_ssize_t n)
 {
     auto handOn = [&]() -> PyObject *
     {
-        PyObject *submit = Name(s_submit);
+        PyObject *submit = Name(api, s_submit);
         return submit != nullptr ? PyObject_Vectorcall(submit, a, (size_t)n, nullptr)
                                  : (PyErr_SetString(PyExc_RuntimeError, "pyapi is gone"), nullptr);
     };
     Call call;
     long key;
-    if (n < 4 || a[0] != Py_None || !PyList_CheckExact(a[1]) || !PyList_CheckExact(a[2]) || !DefaultStreamKey(key))
+    if (n < 4 || a[0] != Py_None || !PyList_CheckExact(a[1]) || !PyList_CheckExact(a[2]) || !DefaultStreamKey(api, key))
     {
         PyErr_Clear();
         return handOn();
     }
     Ref kind(PyObject_GetAttr(a[3], s_kind));
-    if (!kind || !Int(kind.o, call.kind) || !OperatorHandle(a[3], call.op) || !call.Parse(a + 4, n - 4))
+    if (!kind || !Int(kind.o, call.kind) || !OperatorHandle(a[3], call.op) || !call.Parse(api, a + 4, n - 4))
     {
         PyErr_Clear();
         return handOn();
     }
     Ref       keyObject(PyLong_FromLong(key));
-    PyObject *lock = Name(s_lock), *followed = Name(s_followed);
+    PyObject *lock = Name(api, s_lock), *followed = Name(api, s_followed);
     // the marks are read under their lock; where another thread holds it, Python waits for it
     Ref got(lock != nullptr && followed != nullptr && keyObject ? PyObject_CallMethodOneArg(lock, s_acquire, Py_False) : nullptr);
     if (!got || got.o != Py_True)
@@ -438,7 +439,7 @@ PyObject *Submit(PyObject *, PyObject *const *a, Py_ssize_t n)
     Py_END_ALLOW_THREADS
     if (status != NVCV_SUCCESS)
     {
-        PyObject *check = Name(s_check);
+        PyObject *check = Name(api, s_check);
         Ref       value(PyLong_FromLong((long)status));
         Ref       raised(check != nullptr && value ? PyObject_CallOneArg(check, value.o) : nullptr);
         if (!PyErr_Occurred())
@@ -464,10 +465,10 @@ PyObject *Submit(PyObject *, PyObject *const *a, Py_ssize_t n)
 }
 
 // default_stream_key(): pyapi._default_stream_key(None) outside `with stream:`; None inside, where Python looks at the stream.
-PyObject *DefaultKey(PyObject *, PyObject *)
+PyObject *DefaultKey(PyObject *api, PyObject *)
 {
     long key;
-    if (DefaultStreamKey(key))
+    if (DefaultStreamKey(api, key))
     {
         return PyLong_FromLong(key);
     }
@@ -640,24 +641,25 @@ PyObject *TorchView(PyObject *, PyObject *args)
     }
 }
 
-// setup(names of pyapi)
-PyObject *Setup(PyObject *, PyObject *names)
+PyMethodDef kBound[] = {
+    {"submit", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Submit)), METH_FASTCALL, nullptr},
+    {"default_stream_key", DefaultKey, METH_NOARGS, nullptr},
+};
+
+// bind(pyapi's dictionary): (submit, default_stream_key) for it.
+PyObject *Bind(PyObject *, PyObject *names)
 {
     if (!PyDict_Check(names))
     {
-        PyErr_SetString(PyExc_TypeError, "setup(dict)");
+        PyErr_SetString(PyExc_TypeError, "bind(dict)");
         return nullptr;
     }
-    Py_INCREF(names);
-    Py_XDECREF(g_api);
-    g_api = names;
-    Py_RETURN_NONE;
+    Ref submit(PyCFunction_New(&kBound[0], names)), key(PyCFunction_New(&kBound[1], names));
+    return submit && key ? PyTuple_Pack(2, submit.o, key.o) : nullptr;
 }
 
 PyMethodDef kMethods[] = {
-    {"setup", Setup, METH_O, nullptr},
-    {"submit", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Submit)), METH_FASTCALL, nullptr},
-    {"default_stream_key", DefaultKey, METH_NOARGS, nullptr},
+    {"bind", Bind, METH_O, nullptr},
     {"planes", Planes, METH_O, nullptr},
     {"tensor_alloc", TensorAlloc, METH_VARARGS, nullptr},
     {"torch_view", TorchView, METH_VARARGS, nullptr},

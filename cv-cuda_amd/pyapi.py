@@ -470,7 +470,7 @@ def clear_cache():
 def _result(shape, dtype, layout, stream):
     """A tensor for an operator's result. Only a call on the default stream takes one that is handed out again: another
     stream would have to wait for the default stream's last use of it, which one that is being captured cannot."""
-    key = _native.default_stream_key() if stream is None else None
+    key = _native_stream_key() if stream is None else None
     if key is None and _default_stream_key(stream) is None:
         return Tensor(tuple(shape), dtype, layout)
     return _outputs.get(shape, dtype, layout)
@@ -858,8 +858,7 @@ def _same_images(src, fmt=None, sizes=None):
 
 
 # what every operator below goes through: _submit, in native code for calls on the default stream that wait for nothing
-_native.setup(globals())
-_run = _native.submit
+_run, _native_stream_key = _native.bind(globals())
 
 
 def _image_axes(layout):

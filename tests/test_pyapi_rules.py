@@ -449,6 +449,21 @@ def test_view_that_cannot_be_made_gives_its_owner_back(api, cv):
     assert sys.getrefcount(owner) == before
 
 
+def test_two_copies_of_the_package_in_one_process(api, monkeypatch):
+    # what one copy's operators go through are that copy's names
+    package = importlib.import_module(api.__package__)
+    path = os.path.dirname(package.__file__)
+    spec = importlib.util.spec_from_file_location("cvcuda_amd_twice", package.__file__, submodule_search_locations=[path])
+    monkeypatch.setitem(sys.modules, "cvcuda_amd_twice", importlib.util.module_from_spec(spec))
+    spec.loader.exec_module(sys.modules["cvcuda_amd_twice"])
+    other = importlib.import_module("cvcuda_amd_twice.pyapi")
+    for name in [m for m in sys.modules if m.startswith("cvcuda_amd_twice.")]:
+        monkeypatch.setitem(sys.modules, name, sys.modules[name])
+    for one in (api, other):
+        monkeypatch.setattr(one, "_submit", lambda *args, one=one: one)
+    assert api._run(None, [], [], None) is api and other._run(None, [], [], None) is other
+
+
 def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
     # an allocation that finds no memory is tried once more without the kept results, which it would otherwise never reach;
     # clear_cache() gives them and the library's blocks back (no GPU: the library's tensors are stand-ins)
