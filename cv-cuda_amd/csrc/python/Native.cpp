@@ -62,13 +62,22 @@ PyObject *Name(PyObject *api, PyObject *name)
 bool DefaultStreamKey(PyObject *api, long &key)
 {
     PyObject *tls = Name(api, s_tls);
-    PyObject *stack = nullptr;
-    if (tls == nullptr || _PyObject_LookupAttr(tls, s_stack, &stack) < 0)
+    if (tls == nullptr)
     {
         return false;
     }
-    Ref       own(stack);
-    if (stack != nullptr && PyObject_IsTrue(stack) != 0)
+    Ref stack(PyObject_GetAttr(tls, s_stack));
+    if (!stack && PyErr_ExceptionMatches(PyExc_AttributeError))
+    {
+        // a thread's first call: the list that `with stream:` would make, so that the next call finds it
+        PyErr_Clear();
+        stack.o = PyList_New(0);
+        if (stack && PyObject_SetAttr(tls, s_stack, stack.o) < 0)
+        {
+            return false;
+        }
+    }
+    if (!stack || PyObject_IsTrue(stack.o) != 0)
     {
         return false;
     }
@@ -297,11 +306,15 @@ struct Call
     }
 };
 
-// The container's attributes (borrowed: the container holds them).
+// The container's attributes (a new reference), null where it has none.
 PyObject *AttributesOf(PyObject *obj)
 {
-    PyObject **dict = _PyObject_GetDictPtr(obj);
-    return dict != nullptr ? *dict : nullptr;
+    PyObject *dict = PyObject_GenericGetDict(obj, nullptr);
+    if (dict == nullptr)
+    {
+        PyErr_Clear();
+    }
+    return dict;
 }
 
 bool SameKey(PyObject *o, long key)
@@ -344,16 +357,16 @@ bool NothingToWaitFor(PyObject *reads, PyObject *writes, long key)
 {
     for (Py_ssize_t k = 0; k < PyList_GET_SIZE(reads); ++k)
     {
-        PyObject *attributes = AttributesOf(PyList_GET_ITEM(reads, k));
-        if (attributes == nullptr || !WroteBy(attributes, key))
+        Ref attributes(AttributesOf(PyList_GET_ITEM(reads, k)));
+        if (!attributes || !WroteBy(attributes.o, key))
         {
             return false;
         }
     }
     for (Py_ssize_t k = 0; k < PyList_GET_SIZE(writes); ++k)
     {
-        PyObject *attributes = AttributesOf(PyList_GET_ITEM(writes, k));
-        if (attributes == nullptr || !WroteBy(attributes, key) || !ReadBy(attributes, key))
+        Ref attributes(AttributesOf(PyList_GET_ITEM(writes, k)));
+        if (!attributes || !WroteBy(attributes.o, key) || !ReadBy(attributes.o, key))
         {
             return false;
         }
@@ -366,7 +379,8 @@ bool Mark(PyObject *reads, PyObject *writes, PyObject *key)
 {
     for (Py_ssize_t k = 0; k < PyList_GET_SIZE(reads); ++k)
     {
-        PyObject *attributes = AttributesOf(PyList_GET_ITEM(reads, k)), *read = attributes ? PyDict_GetItem(attributes, s_read) : nullptr;
+        Ref       attributes(AttributesOf(PyList_GET_ITEM(reads, k)));
+        PyObject *read = attributes ? PyDict_GetItem(attributes.o, s_read) : nullptr;
         if (read != nullptr)
         {
             if (PyDict_SetItem(read, key, Py_None) < 0)
