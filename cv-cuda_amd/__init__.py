@@ -130,7 +130,7 @@ class Tensor(_Handle):
     @classmethod
     def alloc(cls, shape, dtype, layout, base_align=0, row_align=0):
         """Library-allocated tensor (hipMalloc through the default allocator)."""
-        if len(shape) <= capi.NVCV_TENSOR_MAX_RANK and len(layout) <= capi.NVCV_TENSOR_MAX_RANK:
+        if capi.native is not None and len(shape) <= capi.NVCV_TENSOR_MAX_RANK and len(layout) <= capi.NVCV_TENSOR_MAX_RANK:
             status, handle = capi.native.tensor_alloc(shape, _as_dtype(dtype), layout, base_align, row_align)
             check(status)
             return cls(handle)

@@ -1,7 +1,8 @@
 """ctypes declarations of the C ABI in include/nvcv/*.h and include/cvcuda/*.h.
 
 The two shared libraries are loaded from ./lib next to this file; a missing library is an error
-(there is no fallback path). torch is imported first so that the HIP runtime already in the
+(there is no fallback path). The Python extension beside them is loaded as well; pyapi, which goes through it in
+every call, does not import without it. torch is imported first so that the HIP runtime already in the
 process is the one the libraries bind to.
 """
 import ctypes as C
@@ -28,20 +29,26 @@ nvcv = _load("libnvcv_types.so")
 cvcuda = _load("libcvcuda.so")
 
 
-
 def _load_native():
-    """The Python extension csrc/python/Native.cpp; the libraries it needs are those loaded above."""
-    path = os.path.join(_HERE, "lib", "_cvcuda_native.so")
-    if not os.path.exists(path):
-        raise ImportError(
-            "%s not found: build the native libraries first (python cv-cuda_amd/build.py)" % path)
-    loader = importlib.machinery.ExtensionFileLoader("_cvcuda_native", path)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_cvcuda_native", path, loader=loader))
-    loader.exec_module(module)
-    return module
+    """(the Python extension csrc/python/Native.cpp, None) or (None, why there is none). From the directory of the libraries,
+    or else this package's own: its references are to the libraries loaded above in either case (they are found by name).
+    It is tied to the torch and the Python that it was built with; what is in this file needs the two C libraries alone."""
+    for libdir in (_LIBDIR, os.path.join(_HERE, "lib")):
+        path = os.path.join(libdir, "_cvcuda_native.so")
+        if not os.path.exists(path):
+            continue
+        loader = importlib.machinery.ExtensionFileLoader("_cvcuda_native", path)
+        spec = importlib.util.spec_from_file_location("_cvcuda_native", path, loader=loader)
+        try:
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+        except ImportError as e:
+            return None, "%s was built for another torch or Python, build it again (python cv-cuda_amd/build.py): %s" % (path, e)
+        return module, None
+    return None, "%s not found: build the native libraries first (python cv-cuda_amd/build.py)" % os.path.join(_LIBDIR, "_cvcuda_native.so")
 
 
-native = _load_native()
+native, native_missing = _load_native()
 
 NVCV_TENSOR_MAX_RANK = 15
 NVCV_MAX_PLANE_COUNT = 6

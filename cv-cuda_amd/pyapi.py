@@ -30,8 +30,11 @@ from . import Image as _Image
 from . import ImageBatchVarShape as _ImageBatchVarShape
 from . import Tensor as _Tensor
 from . import _DT2NP, check
-from ._capi import native as _native
+from ._capi import native as _native, native_missing as _native_missing
 from ._capi import nvcv as _nv
+
+if _native is None:
+    raise ImportError(_native_missing)
 
 __all__ = ["Error", "Interp", "Border", "ChannelManip", "NormalizeFlags", "ColorConversion", "Format", "Type", "TensorLayout", "RectI",
            "Stream", "as_stream", "cuda", "Tensor", "Image", "ImageBatchVarShape", "as_tensor", "as_image", "as_images", "reshape"]

@@ -17,7 +17,7 @@ def load_package():
     if "cvcuda_amd" in sys.modules:
         return sys.modules["cvcuda_amd"]
     libdir = os.path.join(PKG, "lib")
-    if not (os.path.exists(os.path.join(libdir, "libcvcuda.so")) and os.path.exists(os.path.join(libdir, "libnvcv_types.so"))):
+    if not all(os.path.exists(os.path.join(libdir, so)) for so in ("libcvcuda.so", "libnvcv_types.so", "_cvcuda_native.so")):
         spec = importlib.util.spec_from_file_location("_cvbuild", os.path.join(PKG, "build.py"))
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)

@@ -4,6 +4,7 @@ the output shapes and formats of cvtcolor (CvtColorUtil.cpp:244-330) and the arg
 make themselves."""
 import importlib
 import os
+import shutil
 import subprocess
 import sys
 
@@ -462,6 +463,25 @@ def test_two_copies_of_the_package_in_one_process(api, monkeypatch):
     for one in (api, other):
         monkeypatch.setattr(one, "_submit", lambda *args, one=one: one)
     assert api._run(None, [], [], None) is api and other._run(None, [], [], None) is other
+
+
+def test_package_over_libraries_kept_elsewhere(api, tmp_path):
+    # CVCUDA_AMD_LIBDIR names all that is needed: with the extension there pyapi as well, with the two C libraries alone the
+    # ctypes layer, whose tensors are then made through it
+    package = os.path.dirname(api.__file__)
+    for whole in (False, True):
+        root, libdir = tmp_path / str(whole), tmp_path / str(whole) / "elsewhere"
+        shutil.copytree(package, root / "pkg", ignore=shutil.ignore_patterns("lib*", "build*", "csrc", "__pycache__"))
+        libdir.mkdir()
+        for so in ("libnvcv_types.so", "libcvcuda.so") + (("_cvcuda_native.so",) if whole else ()):
+            os.symlink(os.path.join(package, "lib", so), libdir / so)
+        code = ("import numpy as np, pkg\nassert (pkg.capi.native is None) != %s\n"
+                "try:\n    pkg.Tensor.alloc([-1], np.uint8, 'N')\nexcept pkg.Error as e:\n    assert e.status == 2\n"
+                "try:\n    import pkg.pyapi\nexcept ImportError as e:\n    assert '_cvcuda_native.so not found' in str(e)\n"
+                "    print('no pyapi')\nelse:\n    print('pyapi')\n" % whole)
+        r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, CVCUDA_AMD_LIBDIR=str(libdir), PYTHONPATH=str(root)),
+                           capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0 and r.stdout.strip() == ("pyapi" if whole else "no pyapi"), r.stdout + r.stderr
 
 
 def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
