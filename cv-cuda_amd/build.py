@@ -78,19 +78,27 @@ def _compile(src, obj, extra, force, newest_header):
 
 
 def _compile_native(src, obj, force, newest_header):
-    """The Python extension, by the host compiler against the headers of Python, torch and the HIP runtime."""
-    if (not force and os.path.exists(obj) and os.path.getmtime(obj) >= os.path.getmtime(src)
-            and os.path.getmtime(obj) >= newest_header):
-        return None
+    """The Python extension, by the host compiler against the headers of Python, torch and the HIP runtime. What it was
+    compiled against is kept beside the object: another torch or Python has other headers, and their files may be older."""
     torch = _torch_dir()
     cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wextra", "-Wno-unused-parameter", "-D__HIP_PLATFORM_AMD__",
            "-DUSE_ROCM", "-I" + INCLUDE]
     for d in (os.path.join(torch, "include"), os.path.join(torch, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
               sysconfig.get_paths()["include"]):
         cmd += ["-isystem", d]
+    with open(os.path.join(torch, "version.py")) as f:
+        against = "\n".join([" ".join(cmd), sys.version, f.read()])
+    stamp = obj + ".against"
+    if (not force and os.path.exists(obj) and os.path.getmtime(obj) >= os.path.getmtime(src) and os.path.getmtime(obj) >= newest_header
+            and os.path.exists(stamp)):
+        with open(stamp) as f:
+            if f.read() == against:
+                return None
     r = subprocess.run(cmd + ["-c", src, "-o", obj], capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("compile failed: %s\n%s" % (" ".join(cmd), r.stdout + r.stderr))
+    with open(stamp, "w") as f:
+        f.write(against)
     return r.stdout + r.stderr
 
 

@@ -484,6 +484,25 @@ def test_package_over_libraries_kept_elsewhere(api, tmp_path):
         assert r.returncode == 0 and r.stdout.strip() == ("pyapi" if whole else "no pyapi"), r.stdout + r.stderr
 
 
+def test_extension_is_compiled_again_for_another_python(api, tmp_path, monkeypatch):
+    spec = importlib.util.spec_from_file_location("_cvbuild_again", os.path.join(os.path.dirname(api.__file__), "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    src, obj, made = tmp_path / "Native.cpp", tmp_path / "Native.o", []
+    src.write_text("")
+
+    def run(cmd, **kw):
+        made.append(cmd)
+        obj.write_text("")
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(build.subprocess, "run", run)
+    for compiled, version in ((1, "one"), (1, "one"), (2, "two"), (2, "two")):
+        monkeypatch.setattr(build.sys, "version", version)
+        build._compile_native(str(src), str(obj), False, 0)
+        assert len(made) == compiled
+
+
 def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
     # an allocation that finds no memory is tried once more without the kept results, which it would otherwise never reach;
     # clear_cache() gives them and the library's blocks back (no GPU: the library's tensors are stand-ins)
