@@ -879,21 +879,14 @@ __device__ __forceinline__ uint32_t SampleNearBorderCubicQ14(const Img &im, cons
     return BlendCubicQ14<C>(r, sx, sy);
 }
 
-// Whether the image has room for the windows of SampleClampedCubicQ14, and they pay where a lane takes its own samples, one
-// after the other, which a launch that fills the chip hides and a small one waits for. One and four channels gain at any
-// size. Three channels, whose windows take the most instructions, gain (under a replicating border; under a constant one waves
-// list their samples at the edge) from 256 blocks on: one 320 x 240, 75 blocks, 6.9 us with SampleNearBorderCubicQ14 and 8.1 with
-// windows; one 640 x 480, 300 blocks, 9.9 and 9.2; 32 x 1280 x 780 202 and 158.
+// Whether the image has room for the windows of SampleClampedCubicQ14. Where it has they pay at every size of launch, us with
+// SampleNearBorderCubicQ14 / with windows, u8x3 under a replicating border: one 64 x 48 4.6 / 4.2, 200 x 150 4.7 / 4.7, 320 x 240 4.3 /
+// 4.3 (in perspective 4.5 / 4.4), 400 x 300 5.7 / 5.1, 640 x 480 6.2 / 5.2, 1280 x 720 11.6 / 9.5; 40 x 16 x 16 4.4 / 4.0, 12 x 224 x 224 9.6 /
+// 7.8; 32 x 1280 x 780 202 / 158.
 template<int C>
 __device__ __forceinline__ bool ClampedCubicFits(const Img &im)
 {
     return im.w >= 4 && __mul24(im.h - 1, im.row) + im.w * C >= 16;
-}
-
-template<int C>
-__device__ __forceinline__ bool ClampedCubicPays(const Img &im)
-{
-    return ClampedCubicFits<C>(im) && (C != 3 || gridDim.x * gridDim.y * gridDim.z >= 256u);
 }
 
 // SampleNearBorderCubicQ14 under a constant or replicating border: 4 loads per sample instead of 16. A row is the window of
@@ -1550,7 +1543,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             // that the edge passes through goes through them alone, no longer through both forms. Kernel us before / after, replicating:
             // u8x4 32 x 256 x 256 18.7 / 15.5, 4 x 640 x 480 11.0 / 9.8, 16 x 1240 x 1754 in perspective 184 / 173; u8x3 32 x 256 x 256 21.3 / 19.3, 4 x 640 x
             // 480 12.0 / 11.2; u8x1 12.7 / 11.7, 7.4 / 7.0. (Listing the samples at the edge, as float images do: u8x3 26.6 and 14.0.)
-            if (a.border <= NVCV_BORDER_REPLICATE && ClampedCubicPays<C>(im)) // uniform
+            if (a.border <= NVCV_BORDER_REPLICATE && ClampedCubicFits<C>(im)) // uniform
             {
                 in = __builtin_amdgcn_ballot_w64(!in) == 0;
             }
@@ -1604,7 +1597,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                     }
                 }
             }
-            else if (INTERP == NVCV_INTERP_CUBIC && a.border <= NVCV_BORDER_REPLICATE && ClampedCubicPays<C>(im)) // uniform
+            else if (INTERP == NVCV_INTERP_CUBIC && a.border <= NVCV_BORDER_REPLICATE && ClampedCubicFits<C>(im)) // uniform
             {
                 // one sample at a time (all four at once took 143 registers, which every wave of the launch would have held;
                 // held to the 64 of full occupancy the u8x3 kernel spills and loses 1 to 2 %)

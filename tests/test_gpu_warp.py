@@ -137,12 +137,13 @@ def test_single_channel_quarter_turns(cv, orc, gpu, size, lead):
                 np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((deg, scale, interp)))
 
 
-# three channels under the replicating border in launches of 256 blocks and more, and under the constant one of 2048, which take the
-# windows next to the edge (smaller ones take tap by tap): the smallest sources that have room for a window, dense rows that start at every byte of a dword
+# the windows next to the edge, three channels, in launches of two patches a wave (one image) and of four: the smallest sources that
+# have room for a window, dense rows that start at every byte of a dword
+@pytest.mark.parametrize("n", [1, 205])
 @pytest.mark.parametrize("lead", [0, 1, 2, 3])
 @pytest.mark.parametrize("size", [(4, 4), (5, 2), (7, 5), (37, 21), (70, 41)], ids=lambda s: "%dx%d" % s)
-def test_bicubic_windows_of_large_launches(cv, orc, gpu, size, lead):
-    (w, h), n, c = size, 205, 3
+def test_bicubic_windows_of_large_launches(cv, orc, gpu, size, lead, n):
+    (w, h), c = size, 3
     dw, dh = 66, 66  # 2 x 5 tiles
     src = orc.fill_u8((n, h, w, c), 0xB1C + w + lead)
     buf = torch.zeros(lead + src.size, dtype=torch.uint8, device="cuda")
