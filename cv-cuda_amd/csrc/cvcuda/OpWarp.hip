@@ -2,7 +2,8 @@
 //
 // Coordinates, sampling and border handling follow the reference in float32 without FMA
 // contraction (the bilinear sum in the association of the reference's golden, tap * (wx * wy),
-// tests/cvcuda/system/TestOpWarpAffine.cpp:159-170, so integer results equal the golden's bit for bit): destination->source map src/cvcuda/priv/legacy/CvCudaLegacy.h:143-183, matrix
+// tests/cvcuda/system/TestOpWarpAffine.cpp:159-170, so integer results equal the golden's bit for bit; bicubic weights and sums
+// of floats and of 8-bit pixels are the exceptions, see CubicWeights and kFixedPointCubic): destination->source map src/cvcuda/priv/legacy/CvCudaLegacy.h:143-183, matrix
 // inversion warp.cu:139-150 (affine) and cuda_tools/math/LinAlg.hpp:1446-1450, 1640-1654 (3x3),
 // samplers cuda_tools/InterpolationWrap.hpp:83-104, 332-339, 429-447, 535-565, border index maps
 // cuda_tools/BorderWrap.hpp:62-121. Validation follows warp.cu:152-232 and warp_var_shape.cu:194-299.
@@ -17,13 +18,12 @@
 // Gather: the cost of the gather is set by how many distinct cache lines one wave-wide load touches,
 // and under a rotation every source row a wave's footprint crosses is another line; so a wave samples
 // compact 8 x 8 pixel patches (one lane per pixel, ~10 source rows per load where a 64 x 1 strip would
-// cross ~20), four patches (two) side by side per wave, i.e. 4 independent samples per lane
+// cross ~20), four patches (two) side by side per wave, i.e. 4 (2) independent samples per lane
 // whose loads are in flight together. Taps that lie inside the source image - nearly all of them -
 // skip the border logic and fetch the horizontally adjacent taps of a row with one load (u8x3: the 6
 // bytes of two pixels from an aligned 12-byte window).
-// Store: "one pixel in each of 4 patches" becomes "4 consecutive pixels of one row", which the lane writes as whole
-// dwords (through LDS, or by a 4x4 transpose inside every group of 4 lanes); single-byte stores scattered over 8 rows
-// are several times slower. Pixels of 12 and 16 bytes leave as whole rows of the wave's part, 16 bytes per lane.
+// Store: "one pixel in each patch" becomes "4 consecutive pixels of one row" through LDS, which the lane writes as whole
+// dwords; single-byte stores scattered over 8 rows are several times slower. Pixels of 12 and 16 bytes leave as whole rows of the wave's part, 16 bytes per lane.
 #include "DeviceUtils.hpp"
 #include "FixedPointBlend.hpp"
 #include "LaneExchange.hpp"
@@ -1294,12 +1294,11 @@ constexpr EdgeLists kEdgeLists = INTERP == NVCV_INTERP_NEAREST        ? kNoLists
                                : INTERP == NVCV_INTERP_CUBIC && C == 3 ? kConstantBorderLists
                                                                       : kNoLists;
 
-// A sample at the image's edge that NearBorderForm lets through, as the dwords of its pixel.
+// A listed sample that NearBorderForm lets through, as the dwords of its pixel.
 template<class T, int C, int INTERP>
 __device__ __forceinline__ void SampleNearEdge(const Img &im, const WarpArgs &a, uint32_t borderPx, float sx, float sy,
                                                uint32_t (&w)[(C * sizeof(T) + 3) / 4])
 {
-    const bool       constant = a.border == NVCV_BORDER_CONSTANT;
     const BorderFold foldX = MakeBorderFold(a.border, im.w), foldY = MakeBorderFold(a.border, im.h);
     if constexpr (!kNearBorderForms<T, C>)
     {
@@ -1312,21 +1311,17 @@ __device__ __forceinline__ void SampleNearEdge(const Img &im, const WarpArgs &a,
         }
         __builtin_memcpy(w, v, C * sizeof(T));
     }
-    else if constexpr (INTERP == NVCV_INTERP_LINEAR)
-    {
-        w[0] = SampleNearBorderQ15<C>(im, foldX, foldY, constant, borderPx, sx, sy);
-    }
-    else if constexpr (INTERP == NVCV_INTERP_NEAREST)
-    {
-        w[0] = SampleNearBorderNearest<C>(im, foldX, foldY, constant, borderPx, sx, sy);
-    }
-    else if (ClampedCubicFits<C>(im)) // uniform; (a constant border: kListEdges)
-    {
-        w[0] = SampleClampedCubicQ14<C>(im, true, borderPx, sx, sy);
-    }
     else
     {
-        w[0] = SampleNearBorderCubicQ14<C>(im, foldX, foldY, true, borderPx, sx, sy);
+        static_assert(INTERP == NVCV_INTERP_CUBIC && kEdgeLists<T, C, INTERP> == kConstantBorderLists);
+        if (ClampedCubicFits<C>(im)) // uniform
+        {
+            w[0] = SampleClampedCubicQ14<C>(im, true, borderPx, sx, sy);
+        }
+        else
+        {
+            w[0] = SampleNearBorderCubicQ14<C>(im, foldX, foldY, true, borderPx, sx, sy);
+        }
     }
 }
 
@@ -1420,6 +1415,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     };
     if constexpr (LIST)
     {
+        static_assert(kEdgeLists<T, C, INTERP> != kNoLists && kScale == 1.f);
         // ---- a wave that the image's edge passes through: its samples at the edge, usually fewer than 64 of the 256, are listed and,
         // when all lanes have sampled as in the other waves (those with taps outside at a place inside), handed out to the
         // lanes again; what is all outside under a constant border takes the colour. Where every lane went through all its four
@@ -1439,17 +1435,13 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
             for (int k = 0; k < N; ++k)
             {
                 const bool in  = fits && TapInside<INTERP>(limX, limY, sx[k], sy[k]);
-                const bool out = constant && TapsOutside<INTERP>(im, sx[k] * (1.f / kScale), sy[k] * (1.f / kScale));
+                const bool out = constant && TapsOutside<INTERP>(im, sx[k], sy[k]);
                 if (out)
                 {
-                    uint32_t w[D]; // (the tap itself, or taps whose weights add up to exactly 1; else their sum)
-                    __builtin_memcpy(w, colour, sizeof(w));
-                    if constexpr (INTERP != NVCV_INTERP_NEAREST && !kFixedPoint<T, INTERP>)
-                    {
-                        T v[C];
-                        SampleAllOutside<T, C, INTERP>(a, sx[k] * (1.f / kScale), sy[k] * (1.f / kScale), v);
-                        __builtin_memcpy(w, v, PB);
-                    }
+                    T        v[C];
+                    uint32_t w[D] = {};
+                    SampleAllOutside<T, C, INTERP>(a, sx[k], sy[k], v);
+                    __builtin_memcpy(w, v, PB);
 #pragma unroll
                     for (int d = 0; d < D; ++d)
                     {
@@ -1516,7 +1508,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                     else
                     {
                         T v[C];
-                        SampleWithBorder<T, C, INTERP>(im, a, bx[0] * (1.f / kScale), by[0] * (1.f / kScale), v);
+                        SampleWithBorder<T, C, INTERP>(im, a, bx[0], by[0], v);
                         __builtin_memcpy(w, v, PB);
                     }
 #pragma unroll
