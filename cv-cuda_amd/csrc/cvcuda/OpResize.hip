@@ -2169,11 +2169,10 @@ constexpr int kPairsTileW = 128, kPairsTileH = 8; // image batches: block = 4 wa
 // The tile (in units of a wave's tile) of this wave in a launch of the tensor kernels below: a block's waves lie side by
 // side (flat) or are stacked. Flat, a block writes few long row pieces instead of many short ones, which the memory
 // likes better when the launch is bound by it (32 x u8x3, the two shapes alternating on one machine: 720p -> 1080p
-// bilinear 67.3 -> 65.1 us, nearest 58.0 -> 55.4 us; 1080p -> 720p box filter 61.5 -> 59.6 us, bicubic 79.0 -> 77.3 us,
-// bilinear 51.4 -> 51.2 us; bicubic enlarging 120.9 -> 125.8 us, which stays stacked). Rows much shorter than a flat
-// block's span leave most of its waves without columns, and on small images the rows of a stacked block share source
-// rows in the L1 (256 x 448 x 448 -> 300 x 300 u8x3 bicubic: 72.6 us stacked, 91.8 us flat), so the host chooses flat
-// blocks for rows of 1024 pixels and more that fill their blocks to 80 % (FlatBlocks).
+// bilinear 67.3 -> 65.1 us, nearest 58.0 -> 55.4 us; 1080p -> 720p box filter 61.5 -> 59.6 us, bilinear 51.4 -> 51.2 us).
+// Rows much shorter than a flat block's span leave most of its waves without columns, and on small images the rows of a
+// stacked block share source rows in the L1, so the host chooses flat blocks for rows of 1024 pixels and more that fill their blocks to 80 %
+// (FlatBlocks). The bicubic walk has a line of its own (LaunchTensor): rows of any length that fill their blocks.
 struct WaveTile
 {
     int x, y;

@@ -394,7 +394,7 @@ class _Outputs:
     def get(self, shape, dtype, layout):
         if type(shape) is not tuple:
             shape = tuple(shape)
-        if type(dtype) is not np.dtype:
+        if not isinstance(dtype, np.dtype):
             dtype = np.dtype(dtype)
         device = torch._C._cuda_getDevice()
         key = (shape, dtype, layout, device)
