@@ -3920,17 +3920,31 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         constexpr int tileW = kCubicWalkW<C>;
         auto          waves = [&](int rows) { return (int64_t)DivUp(a.dstW, tileW) * DivUp(a.dstH, rows) * N; };
         // Fewer waves than 4 to a CU are left to the patches, whose waves are shorter (us as patches / so: 8 x 224 x 224 x 1 -> 256 x
-        // 256 4.0 / 4.0, 100 x 100 x 3 -> 128 x 128 3.5 / 3.6; 640 x 480 x 3 -> 800 x 600 4.9 / 4.4).
-        if (CubicWalks<C>(a.srcW, a.srcH, a.dstW, a.dstH) && waves(4) >= 4 * 256)
+        // 256 4.0 / 4.0, 100 x 100 x 3 -> 128 x 128 3.5 / 3.6; 640 x 480 x 3 -> 800 x 600 4.9 / 4.4). The farther the output rows are
+        // apart, the less of a row's sums serve two of them, and the later it pays, in us as patches / in strips of 4 rows: 4 x 1209 x
+        // 432 x 3 -> 448 x 160, 1120 waves, 4.6 / 5.0, 16 of these 8.0 / 8.0; from 1747 x 624 4.7 / 5.8 and 11.4 / 11.2, in strips of 8 12.2;
+        // 12 x 1728 x 972 x 3 -> 640 x 360, in strips of 8, 15.2 / 14.1. Four channels: 4 x 1747 x 624 -> 448 x 160 4.7 / 5.0, 6 x 2496 x
+        // 1404 -> 640 x 360 16.3 / 15.6. One: 1024 to 1536 waves, at a scale of 2, 3 to 10 % more as strips, from 1536 on 8 % less. Where a quarter of the
+        // lanes have no column it does not pay at these scales (51 x 481 x 723 x 1 -> 257 x 387 14.6 / 17.7; 33 x 405 x 1099 x 3 -> 133 x
+        // 362, in strips of 8, 13.7 / 16.2).
+        const bool    over2 = a.srcH > 2 * (int64_t)a.dstH, reducing = a.srcH > a.dstH;
+        const bool    far   = C == 1 ? 4 * (int64_t)a.srcH > 7 * (int64_t)a.dstH : C == 3 ? over2 : a.srcH > 3 * (int64_t)a.dstH;
+        const int64_t least = !far ? 4 : C == 1 ? 6 : C == 3 ? 32 : 16;
+        const bool    idle  = C != 4 && far && 4 * (int64_t)a.dstW < 3 * (int64_t)DivUp(a.dstW, tileW) * tileW;
+        if (CubicWalks<C>(a.srcW, a.srcH, a.dstW, a.dstH) && waves(4) >= least * 256 && !idle)
         {
             // A wave's first row costs three row sums more than the others, its end leaves the CU to fewer waves. us with 4 / 8 / 16 / 32
-            // rows: 1280 x 720 x 3 -> 1080p 7.6 / 6.8 / 7.4 / 10.8; 64 x 256 x 256 x 3 -> 224 x 224 12.1 / 10.6 / 11.6 / 14.9; 21 x 1119 x
-            // 343 x 3 -> 1140 x 403 27.2 / 21.7 / 20.6 / 23.1; 32 x 1280 x 720 x 3 -> 1080p 139 / 101 / 87 / 79. 32 only where the lines
-            // of memory that output rows end in are not shared with a neighbour that comes to them late (9 x 1515 x 649 x 3 -> 3815 x
+            // rows, enlarging: 1280 x 720 x 3 -> 1080p 7.6 / 6.8 / 7.4 / 10.8; 6 x 576 x 324 x 4 -> 640 x 360 5.7 / 6.1 / 7.2; 21 x 1119 x
+            // 343 x 3 -> 1140 x 403 27.2 / 21.7 / 20.6 / 23.1; 32 x 1280 x 720 x 3 -> 1080p 139 / 101 / 87 / 79. Reducing, where a strip has
+            // more row sums to each output row: 4 x 896 x 503 x 3 -> 640 x 360 5.7 / 6.5 / 8.6, 8 of these 7.5 / 8.1 / 10.0, 24 of these
+            // 16.3 / 14.4 / 15.9; 64 x 256 x 256 x 3 -> 224 x 224 12.1 / 10.6 / 11.6 / 14.9; 64 x 627 x 224 x 3 -> 448 x 160 16.4 / 14.5 / 15.0; by
+            // more than 2 the rows of four channels are what the launch reads, 6 x 1728 x 972 x 4 -> 640 x 360 10.7 / 10.0 / 13.0. One
+            // channel, whose waves are four times as wide: 8 x 2560 x 720 -> 1280 x 360, 3600 waves of 4 rows, 8.3 / 7.7 / 9.7. 32 only where the
+            // lines of memory that output rows end in are not shared with a neighbour that comes to them late (9 x 1515 x 649 x 3 -> 3815 x
             // 1860, 16 / 32: 74 / 90).
             int rows = 4;
-            rows     = waves(8) >= 1536 ? 8 : rows;
-            rows     = waves(16) >= 16 * 256 ? 16 : rows;
+            rows     = waves(8) >= (C == 1 ? 6 : C == 4 && over2 ? 8 : reducing ? 16 : 10) * 256 ? 8 : rows;
+            rows     = waves(16) >= (C == 3 ? 20 : 16) * 256 ? 16 : rows;
             rows     = waves(32) >= 64 * 256 && a.dstH > a.srcH && a.dstRowStride % 64 == 0 ? 32 : rows;
             // Side by side wherever that leaves few waves without columns: rows that end in the middle of a line of memory want
             // their neighbour soon (the same, stacked / side by side: 114 / 74; 8 x 1080p x 4 -> 640 x 360 15.5 / 13.8).

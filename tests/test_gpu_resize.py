@@ -83,7 +83,7 @@ def test_tensor_cubic_reduction(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
 
 
-# 8-bit bicubic at vertical scales up to 4 walks the source rows, 4 to 32 output rows per wave: the benchmark's shape, ragged
+# 8-bit bicubic at vertical scales up to 4 walks the source rows, here 4 and 8 output rows per wave: the benchmark's images, ragged
 # widths and heights, scale 2 exactly (every window advances by 2), 1.25, an enlargement beyond 2, horizontal enlargement with
 # vertical reduction
 STRIPS = [(sw, sh, dw, dh, CUBIC, n, np.uint8, c)
@@ -102,7 +102,8 @@ def test_tensor_cubic_u8_strips(cv, orc, gpu, row):
 
 
 # The same at its limits: outputs one column short of a wave, a wave and one more (the last tile overlaps its neighbour); rows of
-# 16 bytes and of 8; four source rows; vertical scale 4 and a little more; horizontal scales on both sides of 1.3 and 3.9
+# 16 bytes and of 8; four source rows; vertical scale 4 and a little more (three and four channels; one channel, which walks from
+# 128 columns on, and launches that pass every line: the test after this one)
 @pytest.mark.parametrize("c", [1, 3, 4])
 @pytest.mark.parametrize("shape", [(40, 30, 63, 67, 64), (40, 30, 64, 67, 64), (40, 30, 65, 67, 32), (200, 31, 257, 61, 64), (254, 64, 255, 64, 64),
                                    (9, 4, 71, 64, 64), (6, 9, 66, 33, 128), (90, 256, 68, 64, 64), (90, 260, 68, 64, 64), (129, 70, 99, 66, 64),
@@ -116,6 +117,36 @@ def test_tensor_cubic_u8_walks(cv, orc, gpu, shape, c):
     cv.Resize()(None, cv.Tensor.from_torch(torch.from_numpy(src).cuda(), "NHWC"), cv.Tensor.from_torch(out, "NHWC"), CUBIC)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), CUBIC, threads=8))
+
+
+# The same in launches on both sides of each line that decides it: (channels, source, output, images, columns between output rows).
+# Strips of 4, 8, 16 and 32 rows, the last of an image one row or cut off; 32 only under a row pitch of whole lines of 64 bytes;
+# reductions by more than 2 (one channel: 1.75), also with a quarter of the lanes idle. One channel: horizontal scales on both sides of
+# 1.3 (one 8-byte load or two) and of 3.9, rows of 8 bytes, four source rows, vertical scale 4
+WALKS = [(1, 169, 70, 130, 66, 64, 0), (1, 170, 70, 130, 66, 64, 0), (1, 507, 70, 130, 66, 64, 0), (1, 508, 70, 130, 66, 64, 0),
+         (1, 8, 40, 128, 64, 64, 0), (1, 7, 40, 128, 64, 64, 0), (1, 260, 4, 255, 66, 61, 0), (1, 300, 264, 200, 66, 90, 0),
+         (1, 300, 264, 200, 66, 91, 0), (1, 300, 264, 191, 66, 91, 3), (1, 300, 265, 200, 66, 91, 0),
+         (1, 250, 9, 256, 9, 767, 0), (1, 250, 9, 256, 9, 768, 0), (1, 250, 20, 256, 17, 2047, 0), (1, 250, 20, 256, 17, 2048, 0),
+         (1, 200, 25, 256, 33, 8191, 0), (1, 200, 25, 256, 33, 8192, 0), (1, 200, 25, 256, 33, 8192, 1),
+         (3, 40, 20, 64, 9, 1400, 0), (3, 64, 264, 64, 66, 481, 0), (3, 64, 264, 64, 66, 482, 0), (3, 70, 264, 70, 66, 300, 5),
+         (3, 60, 8, 66, 9, 639, 0), (3, 60, 8, 66, 9, 640, 0), (3, 60, 12, 66, 9, 1023, 0), (3, 60, 12, 66, 9, 1024, 2),
+         (3, 50, 20, 64, 17, 2559, 0), (3, 50, 20, 64, 17, 2560, 0), (3, 41, 30, 64, 33, 8191, 0), (3, 41, 30, 64, 33, 8192, 0),
+         (3, 41, 30, 64, 47, 8192, 1), (4, 64, 264, 64, 66, 240, 0), (4, 64, 264, 64, 66, 241, 0), (4, 40, 20, 60, 9, 1023, 0),
+         (4, 40, 20, 60, 9, 1024, 0), (4, 50, 20, 60, 17, 2048, 3), (4, 41, 30, 64, 33, 8192, 0), (4, 41, 30, 64, 33, 8192, 1)]
+
+
+@pytest.mark.parametrize("row", WALKS, ids=lambda r: "x%d-%dx%d-%dx%d-n%d-gap%d" % r)
+def test_tensor_cubic_u8_walks_by_launch(cv, orc, gpu, row):
+    c, sw, sh, dw, dh, n, gap = row
+    some = make_input(orc, (3, sh, sw, c), np.uint8, 0x31 + sw + dw + c)
+    which = torch.arange(n, device="cuda") % 3  # (images next to each other differ)
+    src = torch.from_numpy(some).cuda()[which]
+    out = torch.full((n, dh, dw + gap, c), 7, dtype=torch.uint8, device="cuda")
+    cv.Resize()(None, cv.Tensor.from_torch(src, "NHWC"), cv.Tensor.from_torch(out[:, :, :dw], "NHWC"), CUBIC)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(orc.resize_shipped(some, (dh, dw), CUBIC, threads=8)).cuda()
+    assert torch.equal(out[:, :, :dw], want[which])
+    assert bool((out[:, :, dw:] == 7).all())
 
 
 # 8-bit bilinear in launches of few waves, whose strips are 2 rows (two columns per lane; four, up to 768 strips of 8) and 4 (four
