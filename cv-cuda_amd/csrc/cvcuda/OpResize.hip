@@ -4114,7 +4114,12 @@ void LaunchVarShape(const ResizeArgs &a, const NVCVImageBufferStrided *srcHost, 
         }
         if constexpr (INTERP == NVCV_INTERP_CUBIC && std::is_same_v<T, uint8_t> && (C == 3 || C == 4))
         {
-            // walked where most output pixels belong to images that can be and every CU still gets 8 blocks
+            // walked where most output pixels belong to images that can be and every CU still gets 8 blocks (us as patches / so, images
+            // of sizes up to 10 % about these, three channels: 128 x 256 x 256 -> 224 x 224, 2048 blocks, 28.0 / 26.7, 64 of these 15.9 /
+            // 16.0; 16 x 640 x 480 -> 800 x 600, 2140, 27.9 / 24.1, 4 of these 9.9 / 11.1; 8 x 1080p -> 720p, 2041, 29.1 / 28.7, 4 of these
+            // 17.6 / 19.8; 24 x 1000 x 700 -> 400 x 300, 835, 16.6 / 22.6; four channels 27.4 / 23.2 and 15.8 / 13.7, 30.1 / 23.1 and 10.2 /
+            // 10.4, 31.1 / 27.7 and 18.3 / 17.5, 19.0 / 19.2). 16 rows a wave: with 8 / 16 / 32 16 x 640 x 480 -> 800 x 600 25.0 / 24.1 / 26.2, 32 x
+            // 1080p -> 720p 102 / 94 / 93, 32 x 720p -> 1080p 157 / 137 / 128.
             int64_t walked = 0, all = 0;
             for (int i = first; i < first + count; ++i)
             {
