@@ -3803,18 +3803,21 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         // From a scale of 2 on a row sum serves one output row or two; a few waves leave their CUs idle in both forms, where a wave of one
         // row ends soonest (us as pixels / so, three channels: 224 x 224 -> 256 x 256 3.0 / 3.5, 320 x 240 -> 400 x 300 4.0 / 3.8; one
-        // channel, the same: 3.7 / 3.1, 4.1 / 3.2).
+        // channel, the same: 3.7 / 3.1, 4.1 / 3.2; four channels reducing, 8 x 1050 x 93 -> 579 x 51, 1040 waves, 4.7 / 5.6, 3 x 1815 x 81 ->
+        // 1012 x 43, 528, 3.6 / 4.4, 1 x 1550 x 121 -> 1480 x 115, 696, 3.8 / 4.0).
         auto waves = [&](int rows) { return (int64_t)DivUp(a.dstW, kTileW) * DivUp(a.dstH, rows) * N; };
-        if (a.srcW < 2 * (int64_t)a.dstW && a.srcH < 2 * (int64_t)a.dstH && a.srcW >= 4 && a.srcH >= 4 && waves(4) >= (C == 1 ? 128 : 512))
+        const int64_t least = C == 1 ? 128 : C == 4 && a.srcH > a.dstH ? (2 * (int64_t)a.srcH > 3 * (int64_t)a.dstH ? 2048 : 1024) : 512;
+        if (a.srcW < 2 * (int64_t)a.dstW && a.srcH < 2 * (int64_t)a.dstH && a.srcW >= 4 && a.srcH >= 4 && waves(4) >= least)
         {
             // Rows per wave: a wave begins with four row sums. us with 4 / 8 / 16, three channels: 640 x 480 -> 800 x 600 4.8 / 5.1 / 7.3;
             // 8 x 256 x 256 -> 224 x 224 5.2 / 6.0 / 9.2; 32 of these 11.2 / 11.4 / 12.6; 720p -> 1080p 9.4 / 8.8 / 8.9; 2 x 1080p, as many, 21.2 /
             // 22.2 / 20.3; 4K 30.6 / 27.9 / 26.0; reducing, 4 x 1283 x 721 -> 963 x 541 15.8 / 17.0 / 16.1, four channels 20.3 / 21.5 / 19.4, one
             // 8.3 / 8.4 / 11.3. Enlarged rows that start at no line of memory are the better the sooner their neighbours follow (20 x 515
             // x 313 -> 815 x 460, 8 / 16, one channel 15.0 / 18.0, three 29.3 / 33.4, four 34.3 / 40.5; 12 x 1283 x 721 -> 1931 x 1081 39.8 / 53.0,
-            // 112 / 118, 141 / 141).
+            // 112 / 118, 141 / 141), but not those that are about as many as the source's (four channels, 48 x 1461 x 42 -> 1478 x 42 22.8 / 19.3).
             const bool enlarging = a.srcH <= a.dstH, few = waves(8) <= 18 * 256 && (C == 1 || enlarging);
-            const int  rows      = waves(4) <= 30 * 256 ? 4 : few || (enlarging && a.dstRowStride % 64 != 0) ? 8 : 16;
+            const bool soon      = 5 * (int64_t)a.srcH <= 4 * (int64_t)a.dstH && a.dstRowStride % 64 != 0;
+            const int  rows      = waves(4) <= 30 * 256 ? 4 : few || soon ? 8 : 16;
             hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), dim3(DivUp(a.dstW, kTileW), DivUp(a.dstH, 4 * rows), N), dim3(256), 0, stream, a,
                                rows);
             CheckLaunch("ResizeCubicStripF32Kernel");

@@ -824,7 +824,8 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
 
 # Rows per wave by the size of the launch: the box filter at scales of 1 to 3 (4 rows to a wave up to 2048 waves of 16, 8 up to 8192, then 16), for nearest
 # neighbour enlarging by 1.5 or more (strips of 4 rows from 1024 strips of 8 on, 1536 with three channels; 8 rows for one channel
-# from 15360 on) and for float bicubic (4 rows, 8, 16; from 128 waves of 4 rows on, 512 with three and four channels)
+# from 15360 on, 6144 where a source row is 2.2 output rows and more) and for float bicubic (4 rows, 8, 16; from 128 waves of 4 rows on,
+# 512 with three and four channels, with four reducing 1024, by more than 1.5 2048)
 @pytest.mark.parametrize("row", [(sw, sh, dw, dh, AREA, n, np.uint8, c)
                                  for c in (1, 3, 4)
                                  for (sw, sh, dw, dh, n) in [(97, 23, 61, 9, 1), (64, 40, 65, 39, 2), (130, 30, 64, 15, 3), (190, 50, 63, 17, 4),
@@ -839,7 +840,10 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
                             for c in (1, 3, 4)
                             for (sw, sh, dw, dh, n) in [(40, 8, 64, 4, 127), (40, 8, 64, 4, 128), (40, 8, 64, 5, 256), (40, 8, 64, 3, 512),
                                                         (60, 9, 65, 6, 256), (60, 9, 63, 7, 3840), (60, 9, 63, 7, 4500), (60, 9, 64, 9, 2560),
-                                                        (60, 9, 64, 9, 2305)]],
+                                                        (60, 9, 64, 9, 2305)]]
+                         + [(100, 5, 256, 11, NEAREST, 3071, np.uint8, 1), (100, 5, 256, 11, NEAREST, 3072, np.uint8, 1), (90, 5, 253, 12, NEAREST, 3073, np.uint8, 1),
+                            (60, 9, 61, 7, CUBIC, 511, np.float32, 4), (60, 9, 61, 7, CUBIC, 512, np.float32, 4), (60, 9, 64, 5, CUBIC, 1023, np.float32, 4),
+                            (60, 9, 64, 5, CUBIC, 1024, np.float32, 4), (60, 9, 63, 12, CUBIC, 2600, np.float32, 3), (60, 10, 63, 12, CUBIC, 2600, np.float32, 3)],
                          ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensor_rows_per_wave(cv, orc, gpu, row):
     if row[4] == AREA:
