@@ -3834,9 +3834,11 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         {
             // 4 rows: fewer registers, more waves in flight (8 / 4 rows: 8 x 720p -> 1080p 9.0 / 8.5, 15.3 / 13.6, 17.5 / 15.9; 32 x 224 x 224 ->
             // 448 x 448 6.1 / 5.3, 8.5 / 7.0, 9.4 / 7.2). One channel's largest launches pay more for the column terms (24 x 720p -> 1080p
-            // 16.0 / 17.0, 32 of these 19.8 / 21.8) unless rows end inside lines of memory (100 x 300 x 300 -> 1000 x 500 20.5 / 18.7).
+            // 16.0 / 17.0, 32 of these 19.8 / 21.8) unless rows end inside lines of memory (100 x 300 x 300 -> 1000 x 500 20.5 / 18.7) and a
+            // source row is fewer than three output rows (3 x 1336 x 1189 -> 3870 x 3444 13.4 / 15.5, 23 x 41 x 1275 -> 122 x 3819 9.3 / 10.5).
             const bool flat   = FlatBlocks(a.dstW, kQuadsTileW);
-            const int  rows   = C == 1 && strips >= 60 * 256 && a.dstRowStride % 64 == 0 ? kStripRows : 4;
+            const bool many   = 5 * (int64_t)a.dstH >= 11 * (int64_t)a.srcH ? strips >= 24 * 256 : strips >= 60 * 256 && a.dstRowStride % 64 == 0;
+            const int  rows   = C == 1 && many ? kStripRows : 4;
             auto       kernel = rows == 4 ? ResizeNearestQuadsU8Kernel<C, 4> : ResizeNearestQuadsU8Kernel<C, C == 1 ? kStripRows : 4>;
             hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeNearestQuadsU8Kernel");
