@@ -863,6 +863,41 @@ def test_native_calls_leave_the_rest_to_submit(cvcuda):
         api.resize_into(dst, None, api.Interp.LINEAR)
 
 
+def test_native_calls_of_two_threads_on_one_container(cvcuda, monkeypatch):
+    import threading
+
+    import torch
+    api = cvcuda
+
+    # one source that both read, one result that both write: the marks are whole, and no call waits for the other's for good. (A
+    # thread that finds the marks' lock taken leaves its call to _submit.)
+    handed_on, submit = [], api._submit
+    monkeypatch.setattr(api, "_submit", lambda *a: handed_on.append(0) or submit(*a))
+    src = api.as_tensor((torch.arange(2 * 40 * 50 * 3, device="cuda") % 251).to(torch.uint8).reshape(2, 40, 50, 3), "NHWC")
+    want = api.Tensor((2, 30, 35, 3), np.uint8, "NHWC")
+    api.resize_into(want, src, api.Interp.LINEAR)
+    shared, own, failed, calls = api.Tensor((2, 30, 35, 3), np.uint8, "NHWC"), [None, None], [], 400
+
+    def work(k):
+        try:
+            for _ in range(calls):
+                own[k] = api.resize(src, (2, 30, 35, 3), api.Interp.LINEAR)
+                api.resize_into(shared, src, api.Interp.LINEAR)
+        except Exception as e:  # noqa: BLE001
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not failed and not any(t.is_alive() for t in threads)
+    assert src._read == {0: None} and shared._wrote == (0, None) and shared._read == {} and not api._events_lock.locked()
+    assert len(handed_on) < 2 * calls  # of 4 * calls
+    for t in own + [shared]:
+        np.testing.assert_array_equal(host(t), host(want))
+
+
 def test_native_views_and_planes(cvcuda):
     import torch
     api = cvcuda
