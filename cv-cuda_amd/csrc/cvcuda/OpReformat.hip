@@ -31,25 +31,21 @@ struct ReformatArgs
 template<class T, int C>
 using Vec = Packed<T, C>;
 
-// A block is 64 lanes x 4 rows, or 256 lanes of the one row where there is only one. (arithmetic rather than a branch, so that
-// the other arguments are loaded at once)
-__device__ __forceinline__ void LaneAndRow(const ReformatArgs &a, int &lane, int &y)
+// A block is 64 lanes x 4 rows, or 256 lanes of the one row where there is only one. (a kernel for each: chosen in one kernel,
+// by arithmetic on the image's height, 32 x 1920 x 1080 u8x3 took 68.1 us for 66.5)
+template<bool ONE_ROW>
+__device__ __forceinline__ void LaneAndRow(int &lane, int &y)
 {
-    const int f = a.H == 1;
-    lane        = blockIdx.x * (64 << (2 * f)) + (threadIdx.x & (63 | (192 * f)));
-    y           = blockIdx.y * (4 - 3 * f) + (threadIdx.x >> 6) * (1 - f);
+    lane = blockIdx.x * (ONE_ROW ? 256 : 64) + (threadIdx.x & (ONE_ROW ? 255 : 63));
+    y    = ONE_ROW ? 0 : blockIdx.y * 4 + (threadIdx.x >> 6);
 }
 
-// The grid; where rows follow each other without a gap on both sides and do not fill their tiles, the image becomes one row
-// first: no lanes idle past the ends of rows, and one partial run per image. u8x3 NCHW -> NHWC, 25 x 518 x 542: 13.8 -> 9.7 us
-// (4.5 TB/s), 8 x 222 x 1084 5.6 -> 4.2, 20 x 960 x 540 13.7 -> 12.2. Rows of whole runs that fill nine tenths of their tiles
-// stay rows where the data is more than the memory-side cache's 256 MB: 32 x 1920 x 1080 68.1 and, as one row, 71.4.
+// The grid; where rows follow each other without a gap on both sides the image becomes one row first: no lanes idle past the
+// ends of rows, and one partial run per image. u8x3 NCHW -> NHWC, 25 x 518 x 542: 13.8 -> 9.7 us (4.5 TB/s), 8 x 222 x 1084 5.6 ->
+// 4.2, 20 x 960 x 540 13.7 -> 12.2; of rows that fill their tiles 32 x 1920 x 1080 66.4 -> 65.8.
 dim3 GridOf(ReformatArgs &a, int pixelsPerLane, int N)
 {
-    const int64_t tile = 64 * pixelsPerLane, padded = (a.W + tile - 1) / tile * tile;
-    const bool    keep = a.W % pixelsPerLane == 0
-                   && (padded == a.W || (padded * 9 <= (int64_t)a.W * 10 && N * (a.sN + a.dN) > ((int64_t)256 << 20)));
-    if (!keep && a.sH == a.W * a.sW && a.dH == a.W * a.dW && (int64_t)a.W * a.H <= INT32_MAX - 4 * tile)
+    if (a.sH == a.W * a.sW && a.dH == a.W * a.dW && (int64_t)a.W * a.H <= INT32_MAX - 256 * pixelsPerLane)
     {
         a.W *= a.H;
         a.H = 1;
@@ -60,11 +56,11 @@ dim3 GridOf(ReformatArgs &a, int pixelsPerLane, int N)
 
 // C > 0: channel count known at compile time; SRC_IL / DST_IL: that side has its channels
 // interleaved and packed (stride of C == element size), so the whole pixel moves as one vector.
-template<class T, int C, bool SRC_IL, bool DST_IL>
+template<class T, int C, bool SRC_IL, bool DST_IL, bool ONE_ROW>
 __global__ __launch_bounds__(256) void ReformatKernel(const ReformatArgs a)
 {
     int x, y;
-    LaneAndRow(a, x, y);
+    LaneAndRow<ONE_ROW>(x, y);
     if (x >= a.W || y >= a.H)
     {
         return;
@@ -104,11 +100,11 @@ __global__ __launch_bounds__(256) void ReformatKernel(const ReformatArgs a)
 }
 
 // Runs of 4 pixels per lane; SRC_IL / DST_IL: interleaved packed rows, otherwise planar packed rows.
-template<class T, int C, bool SRC_IL, bool DST_IL>
+template<class T, int C, bool SRC_IL, bool DST_IL, bool ONE_ROW>
 __global__ __launch_bounds__(256) void ReformatRunsKernel(const ReformatArgs a)
 {
     int x0, y;
-    LaneAndRow(a, x0, y);
+    LaneAndRow<ONE_ROW>(x0, y);
     x0 *= kRunPixels;
     if (x0 >= a.W || y >= a.H)
     {
@@ -208,7 +204,7 @@ void LaunchC(ReformatArgs a, int N, bool srcIl, bool dstIl, hipStream_t stream)
             b.sW = b.dW = 4;
             b.sC = b.dC = 1;
             const dim3 grid = GridOf(b, kRunPixels, N), block(256);
-            hipLaunchKernelGGL((ReformatRunsKernel<uint8_t, 4, true, true>), grid, block, 0, stream, b);
+            hipLaunchKernelGGL((b.H == 1 ? ReformatRunsKernel<uint8_t, 4, true, true, true> : ReformatRunsKernel<uint8_t, 4, true, true, false>), grid, block, 0, stream, b);
             CheckLaunch("ReformatRunsKernel");
             return;
         }
@@ -225,19 +221,19 @@ void LaunchC(ReformatArgs a, int N, bool srcIl, bool dstIl, hipStream_t stream)
             const bool sIl = srcIl && !(C == 1), dIl = dstIl && !(C == 1);
             if (sIl && dIl)
             {
-                hipLaunchKernelGGL((ReformatRunsKernel<T, C, true, true>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((a.H == 1 ? ReformatRunsKernel<T, C, true, true, true> : ReformatRunsKernel<T, C, true, true, false>), grid, block, 0, stream, a);
             }
             else if (sIl)
             {
-                hipLaunchKernelGGL((ReformatRunsKernel<T, C, true, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((a.H == 1 ? ReformatRunsKernel<T, C, true, false, true> : ReformatRunsKernel<T, C, true, false, false>), grid, block, 0, stream, a);
             }
             else if (dIl)
             {
-                hipLaunchKernelGGL((ReformatRunsKernel<T, C, false, true>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((a.H == 1 ? ReformatRunsKernel<T, C, false, true, true> : ReformatRunsKernel<T, C, false, true, false>), grid, block, 0, stream, a);
             }
             else
             {
-                hipLaunchKernelGGL((ReformatRunsKernel<T, C, false, false>), grid, block, 0, stream, a);
+                hipLaunchKernelGGL((a.H == 1 ? ReformatRunsKernel<T, C, false, false, true> : ReformatRunsKernel<T, C, false, false, false>), grid, block, 0, stream, a);
             }
             CheckLaunch("ReformatRunsKernel");
             return;
@@ -246,19 +242,19 @@ void LaunchC(ReformatArgs a, int N, bool srcIl, bool dstIl, hipStream_t stream)
     const dim3 grid = GridOf(a, 1, N), block(256);
     if (srcIl && dstIl)
     {
-        hipLaunchKernelGGL((ReformatKernel<T, C, true, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((a.H == 1 ? ReformatKernel<T, C, true, true, true> : ReformatKernel<T, C, true, true, false>), grid, block, 0, stream, a);
     }
     else if (srcIl)
     {
-        hipLaunchKernelGGL((ReformatKernel<T, C, true, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((a.H == 1 ? ReformatKernel<T, C, true, false, true> : ReformatKernel<T, C, true, false, false>), grid, block, 0, stream, a);
     }
     else if (dstIl)
     {
-        hipLaunchKernelGGL((ReformatKernel<T, C, false, true>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((a.H == 1 ? ReformatKernel<T, C, false, true, true> : ReformatKernel<T, C, false, true, false>), grid, block, 0, stream, a);
     }
     else
     {
-        hipLaunchKernelGGL((ReformatKernel<T, C, false, false>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((a.H == 1 ? ReformatKernel<T, C, false, false, true> : ReformatKernel<T, C, false, false, false>), grid, block, 0, stream, a);
     }
     CheckLaunch("ReformatKernel");
 }
@@ -285,7 +281,7 @@ void LaunchT(ReformatArgs a, int N, hipStream_t stream)
     default:
     {
         const dim3 grid = GridOf(a, 1, N);
-        hipLaunchKernelGGL((ReformatKernel<T, 0, false, false>), grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((a.H == 1 ? ReformatKernel<T, 0, false, false, true> : ReformatKernel<T, 0, false, false, false>), grid, dim3(256), 0, stream, a);
         CheckLaunch("ReformatKernel");
     }
     }
