@@ -167,8 +167,11 @@ __device__ __forceinline__ void NormRun(const NormArgs &a, const uint8_t *srcRow
     constexpr int P = kNormRunPixels<TI, TO, C>;
     // every uniform value is loaded before the first use, so the loads share one round trip, and the pixels are requested
     // before the scales are finished, which wait for it: one round trip to memory less in a wave that has two or three (f32x3 with
-    // standard deviations, 16 x 224 x 224 6.8 -> 6.0 us, 55 x 299 x 299 23.8 -> 21.2; a wave of 2 or 4 rows gave no more)
-    float b[C], m[C];
+    // standard deviations, 16 x 224 x 224 6.8 -> 6.0 us, 55 x 299 x 299 23.8 -> 21.2; a wave of 2 or 4 rows gave no more).
+    // Not the one load of f32x1, which goes out no sooner by it: image batches without standard deviations, whose rows
+    // follow one another in a wave, took 7 % more (one 839 x 1713 4.7 us, 5.2 so), and with them the same.
+    constexpr bool kPixelsFirst = C > 1 || sizeof(TI) == 1;
+    float          b[C], m[C];
 #pragma unroll
     for (int c = 0; c < C; ++c)
     {
@@ -177,7 +180,7 @@ __device__ __forceinline__ void NormRun(const NormArgs &a, const uint8_t *srcRow
     }
     const bool whole = x0 + P <= W;
     TI         in[P * C];
-    if (whole)
+    if (kPixelsFirst && whole)
     {
         LoadRun<TI, P * C>(srcRow + (int64_t)x0 * C * sizeof(TI), in);
     }
@@ -192,6 +195,10 @@ __device__ __forceinline__ void NormRun(const NormArgs &a, const uint8_t *srcRow
     }
     if (whole)
     {
+        if constexpr (!kPixelsFirst)
+        {
+            LoadRun<TI, P * C>(srcRow + (int64_t)x0 * C * sizeof(TI), in);
+        }
         TO out[P * C];
         if (a.gscale == 1.f && a.shift == 0.f) // wave-uniform; x * 1 + 0 == x, two operations per element saved
         {
