@@ -110,6 +110,12 @@ __global__ __launch_bounds__(256) void ReformatRunsKernel(const ReformatArgs a)
     {
         return;
     }
+    if constexpr (!DST_IL)
+    {
+        // a row's last run ends where the row does and writes the pixels that it shares with its neighbour a second time, with
+        // the same values
+        x0 = a.W >= kRunPixels ? min(x0, a.W - kRunPixels) : x0;
+    }
     const int      n = blockIdx.z;
     const uint8_t *s = a.src + n * a.sN + y * a.sH + x0 * a.sW;
     uint8_t       *d = a.dst + n * a.dN + y * a.dH + x0 * a.dW;

@@ -63,6 +63,25 @@ def test_reformat_rows_without_gaps(cv, orc, gpu, dt, shape):
     assert (wide[:, :, w:] == 9).all()
 
 
+@pytest.mark.parametrize("dt", [np.uint8, np.int16])
+@pytest.mark.parametrize("w", [1, 2, 3, 4, 5, 6, 7, 255, 257, 259])
+@pytest.mark.parametrize("c", [1, 3])
+def test_reformat_to_planes_row_ends(cv, orc, gpu, dt, w, c):
+    # the last run of a row of 4 pixels or more ends where the row does; what lies between rows stays as it is
+    a = rand(orc, (2, 6, w, c), dt, 11 + w)
+    wide = torch.full((2, 6, w + 5, c), 9, dtype=torch.from_numpy(a).dtype, device="cuda")
+    wide[:, :, :w] = torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    planes = torch.full((2, c, 6, w + 3), 7, dtype=wide.dtype, device="cuda")
+    again = torch.full((2, c, 6, w + 1), 5, dtype=wide.dtype, device="cuda")
+    op = cv.Reformat()
+    op(None, cv.Tensor.from_torch(wide[:, :, :w], "NHWC"), cv.Tensor.from_torch(planes[..., :w], "NCHW"))
+    op(None, cv.Tensor.from_torch(planes[..., :w], "NCHW"), cv.Tensor.from_torch(again[..., :w], "NCHW"))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(planes[..., :w].cpu().numpy(), a.transpose(0, 3, 1, 2))
+    np.testing.assert_array_equal(again[..., :w].cpu().numpy(), a.transpose(0, 3, 1, 2))
+    assert (planes[..., w:] == 7).all() and (again[..., w:] == 5).all()
+
+
 def test_reformat_hwc_chw_copy_and_errors(cv, orc, gpu):
     a = rand(orc, (30, 40, 3), np.float32, 9)
     t_hwc = cv.Tensor.from_numpy(a, "HWC")
