@@ -1887,6 +1887,14 @@ __global__ __launch_bounds__(kThreads) void WarpVarShape(const WarpArgs a, const
 // 9.3, 14.6 / 13.4; f32x1 bilinear 4.4 / 3.8, 4.6 / 4.4, 4.6 / 4.4, 5.3 / 5.5, 7.2 / 7.8; u8x3 nearest 3.8 / 3.4, 3.8 / 3.3, 4.2 / 3.9, 4.6 / 4.8.
 // (One patch: 320 x 240 u8x3 bicubic 5.2, but 2 x 640 x 480 7.4 and 16 30.5; elements of 16 bits keep four, for the size of the library.)
 constexpr int64_t kFewWaves = 3 * 1024;
+// Waves of image batches start with the tile search and the matrix' inversion as well, so the line lies lower where the samples are
+// few instructions. Two patches over four by numbers of waves, means over 700 random launches: nearest neighbour up to 1 536 0.95,
+// to 2 048 0.99, to 2 560 1.01 (in perspective 1.04), to 3 072 1.02 (60 of 48 x 176 u8x4 in perspective 6.1 us with four and 7.05 with
+// two); 8-bit bilinear in perspective to 2 560 0.92, to 3 072 1.02; bilinear of floats to 3 072 0.93, bicubic 0.90.
+template<class T, int INTERP, bool PERSP>
+constexpr int64_t kFewWavesOfBatches = INTERP == NVCV_INTERP_NEAREST                                    ? 1536
+                                     : INTERP == NVCV_INTERP_LINEAR && PERSP && std::is_same_v<T, uint8_t> ? 2560
+                                                                                                        : kFewWaves;
 template<class T>
 constexpr bool kFewPatchesForm = std::is_same_v<T, uint8_t> || std::is_same_v<T, float>;
 
@@ -1894,11 +1902,11 @@ template<class T, int C, int INTERP, bool PERSP, bool LIST>
 void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, hipStream_t stream)
 {
     constexpr int kMost = kMostPatches, kFew = kFewPatchesForm<T> ? kFewPatches : kMost;
-    const auto    few = [](int64_t tiles) { return kFew != kMost && tiles * (kThreads / 64) <= kFewWaves; };
+    const auto    few = [](int64_t tiles, int64_t most) { return kFew != kMost && tiles * (kThreads / 64) <= most; };
     if (dstHost == nullptr)
     {
         const dim3 most(DivUp(a.dstW, kTileW<kMost>), DivUp(a.dstH, kTileH<kMost>), N);
-        if (few((int64_t)most.x * most.y * most.z))
+        if (few((int64_t)most.x * most.y * most.z, kFewWaves))
         {
             const dim3 grid(DivUp(a.dstW, kTileW<kFew>), DivUp(a.dstH, kTileH<kFew>), N);
             hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kFew>), grid, dim3(kThreads), 0, stream, a);
@@ -1915,7 +1923,7 @@ void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, 
         VarTiles  tiles;
         const int count = std::min(kMaxTileImages, N - first);
         int       total = BuildVarTiles(tiles, dstHost, first, count, kTileW<kMost>, kTileH<kMost>);
-        if (total > 0 && few(total))
+        if (total > 0 && few(total, kFewWavesOfBatches<T, INTERP, PERSP>))
         {
             total = BuildVarTiles(tiles, dstHost, first, count, kTileW<kFew>, kTileH<kFew>);
             hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kFew>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
