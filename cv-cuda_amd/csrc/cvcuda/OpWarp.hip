@@ -1486,18 +1486,34 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                 }
             }
             WaveExchangeFence();
-            auto edgeSamples = [&](auto nearby) // the listed samples that NearBorderForm lets through, or the others; whether there are others
+            // The first `count` listed samples, 64 at a time (once for most waves that have any); `nearby`: those that NearBorderForm lets
+            // through, the others move to the list's front. Returns how many these are.
+            auto edgeSamples = [&](auto nearby, int count)
             {
-                bool others = false;
+                int others = 0;
 #pragma nounroll
-                for (int i = lane; i < edges; i += 64) // (once for most waves that have any)
+                for (int first = 0; first < count; first += 64)
                 {
-                    const int id = list[wave][i], at = (id >> 6) * kPatch + (id & (kPatch - 1)), line = (id >> 3) & (kPatch - 1);
-                    float     bx[1], by[1];
+                    const bool listed = first + lane < count;
+                    const int  id = list[wave][listed ? first + lane : first], at = (id >> 6) * kPatch + (id & (kPatch - 1)), line = (id >> 3) & (kPatch - 1);
+                    float      bx[1], by[1];
                     MapCoord<PERSP>(m, x0 + at, y0 + line, bx[0], by[0]);
-                    if ((fits && NearBorderForm<T, C, INTERP>(im, a, bx, by)) != nearby.value)
+                    bool mine = listed;
+                    if constexpr (nearby.value)
                     {
-                        others = true;
+                        mine = listed && fits && NearBorderForm<T, C, INTERP>(im, a, bx, by);
+                        if (const uint64_t mask = __builtin_amdgcn_ballot_w64(listed && !mine))
+                        {
+                            if (listed && !mine) // (to places that have been read)
+                            {
+                                const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+                                list[wave][others + before] = (uint8_t)id;
+                            }
+                            others += __builtin_popcountll(mask);
+                        }
+                    }
+                    if (!mine)
+                    {
                         continue;
                     }
                     uint32_t w[D] = {};
@@ -1517,12 +1533,12 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
                         rows[line][at * D + d] = w[d];
                     }
                 }
-                return __builtin_amdgcn_ballot_w64(others) != 0;
+                return others;
             };
-            if (edgeSamples(std::true_type{})) // (two loops: one with both samplers holds the registers of both)
-            {
-                edgeSamples(std::false_type{});
-            }
+            // (two loops: one with both samplers holds the registers of both)
+            const int others = edgeSamples(std::true_type{}, edges);
+            WaveExchangeFence();
+            edgeSamples(std::false_type{}, others);
         }
     }
     else

@@ -95,6 +95,25 @@ def test_mirroring_and_repeating_borders_near_and_far(cv, orc, gpu, c):
         np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((c, interp, border)))
 
 
+# The same of elements that list their samples at the edge: a wave's list has samples of both kinds, few and more than 64 of each.
+@pytest.mark.parametrize("dt,c", [(np.int16, 3), (np.uint16, 1), (np.float32, 1), (np.float32, 4)])
+@pytest.mark.parametrize("scale", [0.3, 1.0, 2.5])
+def test_listed_samples_near_and_far(cv, orc, gpu, dt, c, scale):
+    sw, sh = 23, 17
+    src = (orc.fill_u8((2, sh, sw, c), 77 + c).astype(np.float64) - (100 if dt == np.int16 else 0)).astype(dt)
+    m = [0.93 * scale, 0.11, -2.3 * sw * scale, -0.07, 1.04 * scale, -1.9 * sh * scale]
+    for interp, border in itertools.product((NEAREST, LINEAR, CUBIC), (2, 3, 4)):
+        tout = cv.Tensor.alloc([2, 5 * sh, 5 * sw, c], dt, "NHWC")
+        cv.WarpAffine(0)(None, cv.Tensor.from_numpy(src, "NHWC"), tout, m, interp | INVERSE_MAP, border, (0, 0, 0, 0))
+        torch.cuda.synchronize()
+        dev = orc.warp(src, (5 * sh, 5 * sw), np.asarray(m, np.float32), interp, border, (0, 0, 0, 0), variant=device_variant(interp, dt))
+        if dt == np.float32:
+            # 16 products of up to 255 * 1.6 each rounded in another order: 16 * 408 * 2^-24 = 3.9e-4
+            assert np.abs(tout.numpy() - dev).max() <= 4e-4, (interp, border)
+        else:
+            np.testing.assert_array_equal(tout.numpy(), dev, err_msg=str((interp, border)))
+
+
 # row windows of dense images whose rows start at every byte of a dword in turn, from every start of the first; widths about
 # the tap blocks' and the windows' own (samples whose window would pass the row's end take the border's forms). The buffer
 # ends with the last image.
