@@ -118,7 +118,7 @@ class Fused:
     KERNELS = {"fused": "FusedBilinear<float,false,false,false,true>",
                "fused-normalize": "FusedBilinear<float,false,false,true,true>",
                "fused-chain": "FusedBilinear<float,false,false,false,false> + NormRunsTensor<float,float,3> + "
-                              "ReformatKernel<unsigned int,3,true,false>",
+                              "ReformatKernel<unsigned int,3,true,false,true>",
                "fused-copy-bound": "FusedCopyBound"}
     TEXT = {"fused": "scale/offset", "fused-normalize": "per-channel mean/std in the same kernel (extension entry point)",
             "fused-chain": "per-channel mean/std as the three-operator chain fused -> Normalize -> Reformat",
@@ -688,7 +688,7 @@ class Streaming:
         "normalize-f32": ("Normalize", 16, ("float32", 3), ("float32", 3, "NHWC"), "NormRunsTensor<float,float,3>",
                           "f32", "Normalize (per-channel base/scale)"),
         "reformat-nhwc-nchw": ("Reformat", 32, ("uint8", 3), ("uint8", 3, "NCHW"),
-                               "ReformatRunsKernel<uint8_t,3,true,false>", "u8", "Reformat NHWC -> NCHW"),
+                               "ReformatRunsKernel<uint8_t,3,true,false,true>", "u8", "Reformat NHWC -> NCHW"),
         "convertto-u8-f32": ("ConvertTo", 32, ("uint8", 3), ("float32", 3, "NHWC"), "ConvertKernel<uint8_t,float>",
                              "f32", "ConvertTo x 1/255"),
         "flip-horizontal": ("Flip", 32, ("uint8", 3), ("uint8", 3, "NHWC"), "PixelMapTensor<uint8_t,3>", "u8",
@@ -708,7 +708,7 @@ class Streaming:
         "cvtcolor-bgr2hsv": ("CvtColor", 32, ("uint8", 3), ("uint8", 3, "NHWC"), "MapTensor<HsvFromBgr<uint8_t,false>>", "f32",
                              "CvtColor BGR2HSV"),
         "cvtcolor-bgr2nv12": ("CvtColor", 32, ("uint8", 3), ("uint8", 1, "NHWC", 1620, 1920),
-                              "PixelTensor<Yuv420FromBgr<3,true>>", "int32", "CvtColor BGR2YUV_NV12"),
+                              "PixelGroupsTensor<Yuv420FromBgr<3,true>>", "int32", "CvtColor BGR2YUV_NV12"),
         "cvtcolor-yuy2-bgr": ("CvtColor", 32, ("uint8", 1, 1080, 3840), ("uint8", 3, "NHWC", 1080, 1920), "PixelTensor<BgrFromYuv422<3>>", "int32",
                               "CvtColor YUV2BGR_YUY2"),
     }
