@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) void Yuv420ToRgbTensor(const YuvArgs a, const 
     __shared__ __attribute__((aligned(16))) uint8_t stage[4][2 * 64 * RB];
 
     const int      lane  = threadIdx.x & 63;
-    const uint32_t first = blockIdx.x * 256 + (threadIdx.x & 192); // of the wave
+    const uint32_t first = blockIdx.x * blockDim.x + (threadIdx.x & 192); // of the wave
     if (first >= blocks)
     {
         return;
@@ -740,7 +740,12 @@ void LaunchYuv(const YuvArgs &a, int N, const NVCVImageBufferStrided *dstHost, h
         {
             const DivBy    perRow(DivUp(a.W, kYuvBlockW));
             const uint32_t blocks = perRow.d * (uint32_t)(a.H / 2);
-            hipLaunchKernelGGL((Yuv420ToRgbTensor<DCN, SEMIPLANAR>), dim3(DivUp((int)blocks, 256), 1, N), dim3(256), 0, stream,
+            // Launches of up to 4 waves per CU in workgroups of one wave, which go to as many CUs: dealt across rows the waves are fewer
+            // than the tiles' were, and four to a CU small launches had become slower (us in tiles / by four waves / by one: 328 x 348 NV12
+            // 2.9 / 3.5 / 3.2, 64 x 1550 4.9 / 3.2 / 2.9; by four and one: 960 x 124 2.9 / 2.8, 808 x 584 3.7 / 3.6; 1160 x 776, 880 waves, 3.9
+            // both; 1856 x 1410, 2556 waves, 5.0 / 5.4; 39 x 1176 x 286 12.5 / 15.0).
+            const int threads = (int64_t)DivUp((int)blocks, 64) * N <= 4 * 256 ? 64 : 256;
+            hipLaunchKernelGGL((Yuv420ToRgbTensor<DCN, SEMIPLANAR>), dim3(DivUp((int)blocks, threads), 1, N), dim3(threads), 0, stream,
                                a, perRow, blocks);
             CheckLaunch("Yuv420ToRgbTensor");
             return;

@@ -49,7 +49,7 @@ def test_yuv420_to_rgb(cv, K, orc, gpu, name, size):
 
 @pytest.mark.parametrize("name", ["YUV2RGB_NV12", "YUV2BGRA_NV21", "YUV2BGR_YV12", "YUV2RGBA_YV12"])
 @pytest.mark.parametrize("size", [(8, 4, 1), (10, 4, 2), (14, 8, 3), (18, 132, 2), (62, 40, 1), (504, 8, 1), (512, 8, 2), (514, 12, 1),
-                                  (1030, 8, 2)])
+                                  (1030, 8, 2), (66, 4, 1024), (66, 4, 1025)])  # (up to 1024 waves: workgroups of one)
 def test_yuv420_rows_that_end_inside_a_wave(cv, K, orc, gpu, name, size):
     # blocks of 8 columns are dealt to lanes across rows; the last one of a row overlaps its neighbour
     w, h, n = size
