@@ -37,7 +37,7 @@ NEAREST, LINEAR, CUBIC, AREA = 0, 1, 2, 3
 # write parts are in the summary files named below. The counters sit between the L2s and the fabric:
 # a batch that fits the memory-side cache (warp-affine-varshape) has part of those reads served there.
 MEASURED_TRAFFIC_BYTES = {"fused": 122963893, "resize-cubic-4k": 1474458644, "resize-nearest": 12249763,
-                          "resize-linear": 23286608, "nv12-to-rgb": 298659855, "warp-affine-varshape": 297249937}
+                          "resize-linear": 23286608, "nv12-to-rgb": 298640033, "warp-affine-varshape": 297249937}
 # The rocprofv3 counter summary each figure above is the "total" line of (a CPU test compares them).
 TRAFFIC_PROFILES = {"fused": "FusedBilinear_batch64_1080p_to_224",
                     "resize-cubic-4k": "ResizeCubicStagedKernel_f32x4_batch16_4k_to_640x360",
@@ -296,7 +296,7 @@ class CubicC5:
 class Nv12C3:
     key, config_id, mover = "nv12-to-rgb", 3, "stream-mix-1-2"
     N, H, W = 32, 1080, 1920
-    kernel = "Yuv420ToRgbTensor<3,true>"
+    kernel = "Yuv420ToRgbTensor<3,true,256>"
     dtype = "int32"
     workload = "CvtColor YUV2RGB_NV12: batch 32 u8 [1620,1920,1] -> [1080,1920,3]"
 

@@ -276,14 +276,14 @@ __device__ __forceinline__ void ConvertLaneBlock(const uint8_t *src, int srcRow,
 //
 // Both output rows of a wave go through its LDS and leave as 16-byte pieces, lane after lane (RunIO.hpp on why). A piece lies
 // in one block or in two next to each other; where the second of these is in another row the piece is two of 8 bytes.
-template<int DCN, bool SEMIPLANAR>
-__global__ __launch_bounds__(256) void Yuv420ToRgbTensor(const YuvArgs a, const DivBy perRow, const uint32_t blocks)
+template<int DCN, bool SEMIPLANAR, int THREADS>
+__global__ __launch_bounds__(THREADS) void Yuv420ToRgbTensor(const YuvArgs a, const DivBy perRow, const uint32_t blocks)
 {
     constexpr int BW = kYuvBlockW, NC = BW / 2, RB = BW * DCN;
-    __shared__ __attribute__((aligned(16))) uint8_t stage[4][2 * 64 * RB];
+    __shared__ __attribute__((aligned(16))) uint8_t stage[THREADS / 64][2 * 64 * RB];
 
     const int      lane  = threadIdx.x & 63;
-    const uint32_t first = blockIdx.x * blockDim.x + (threadIdx.x & 192); // of the wave
+    const uint32_t first = blockIdx.x * THREADS + (threadIdx.x & (THREADS - 64)); // of the wave
     if (first >= blocks)
     {
         return;
@@ -744,9 +744,10 @@ void LaunchYuv(const YuvArgs &a, int N, const NVCVImageBufferStrided *dstHost, h
             // than the tiles' were, and four to a CU small launches had become slower (us in tiles / by four waves / by one: 328 x 348 NV12
             // 2.9 / 3.5 / 3.2, 64 x 1550 4.9 / 3.2 / 2.9; by four and one: 960 x 124 2.9 / 2.8, 808 x 584 3.7 / 3.6; 1160 x 776, 880 waves, 3.9
             // both; 1856 x 1410, 2556 waves, 5.0 / 5.4; 39 x 1176 x 286 12.5 / 15.0).
-            const int threads = (int64_t)DivUp((int)blocks, 64) * N <= 4 * 256 ? 64 : 256;
-            hipLaunchKernelGGL((Yuv420ToRgbTensor<DCN, SEMIPLANAR>), dim3(DivUp((int)blocks, threads), 1, N), dim3(threads), 0, stream,
-                               a, perRow, blocks);
+            const bool few     = (int64_t)DivUp((int)blocks, 64) * N <= 4 * 256;
+            const int  threads = few ? 64 : 256;
+            hipLaunchKernelGGL((few ? Yuv420ToRgbTensor<DCN, SEMIPLANAR, 64> : Yuv420ToRgbTensor<DCN, SEMIPLANAR, 256>),
+                               dim3(DivUp((int)blocks, threads), 1, N), dim3(threads), 0, stream, a, perRow, blocks);
             CheckLaunch("Yuv420ToRgbTensor");
             return;
         }
