@@ -3169,12 +3169,16 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
 {
     using Window = AreaWindow<C, K>;
     const Plane p    = GetPlanes<false>(a, blockIdx.z);
-    const int   lane = threadIdx.x & 63, dx = blockIdx.x * kTileW + lane;
+    const int   lane = threadIdx.x & 63, dx = min((int)blockIdx.x * kTileW + lane, p.dstW - 1);
     const int   dy   = blockIdx.y * kTileH + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (dx >= p.dstW || dy >= p.dstH)
+    if (dy >= p.dstH)
     {
         return;
     }
+    // (Lanes past the last column work on it again. In a launch that leaves most of the chip idle a wave of 1 to 8 active lanes
+    // issues 2 to 3 times slower than one of more: a kernel of such sums alone, 26 blocks, 14.7 us with 9 to 64 lanes and 48 with
+    // 1 to 8, 512 blocks no difference. One 640 x 480 u8x3 -> 66 x 50 15.0 -> 6.5 us, -> 78 x 50 8.4 -> 6.5; 500 x 480 -> 130 x 50 8.9 ->
+    // 4.9; 6 x 584 x 650 u8x4 -> 68 x 67 18.0 -> 8.5; 64 x 640 x 480 -> 66 x 50 22.2 and 22.4.)
     // ResizeValue's terms; the vertical ones are the same in all lanes
     const float fsx1 = dx * p.scaleX, fsx2 = fsx1 + p.scaleX, fsy1 = dy * p.scaleY, fsy2 = fsy1 + p.scaleY;
     const int   xmin = (int)ceilf(fsx1), xmax = (int)floorf(fsx2);
@@ -3316,7 +3320,10 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
     {
         out.v[c] = SaturateCast<uint8_t>(sum[c]);
     }
-    StorePx<uint8_t, C>(p.dst + (int64_t)dy * p.dstRow, dx, out);
+    if ((int)blockIdx.x * kTileW + lane < p.dstW)
+    {
+        StorePx<uint8_t, C>(p.dst + (int64_t)dy * p.dstRow, dx, out);
+    }
 }
 
 // The kernel whose window holds a row of boxes `s` wide.
