@@ -264,6 +264,11 @@ private:
 
 } // namespace
 
+void CheckWrappedImage(const NVCVImageData &d)
+{
+    (void)WrappedImage(d, nullptr, nullptr);
+}
+
 NVCVImageHandle CreateWrappedImage(const NVCVImageData &d)
 {
     return static_cast<NVCVImageHandle>(ImagePool().create(std::make_unique<WrappedImage>(d, nullptr, nullptr)));

@@ -330,6 +330,8 @@ public:
 
 // An image over memory that somebody else keeps (validated as nvcvImageWrapDataConstruct does); one reference.
 NVCVImageHandle CreateWrappedImage(const NVCVImageData &d);
+// Throws what that would throw for such data.
+void CheckWrappedImage(const NVCVImageData &d);
 
 void ValidateWrappedTensor(const NVCVTensorData &d);
 

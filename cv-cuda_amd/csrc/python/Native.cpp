@@ -1,6 +1,7 @@
 // The part of the Python interface that runs for every call: operators submitted on the default stream without a wait, the
-// planes of a list of torch tensors, tensors of the library's own memory and torch's views of them. In Python one call of an
-// operator was 5.3 to 6.2 us of the interpreter beside 2 to 3 us of the library, a batch of 61 images another 43 us.
+// planes of a list of torch tensors and batches of them, tensors of the library's own memory, the results that are handed out
+// again and torch's views of them. In Python one call of an operator was 5.3 to 6.2 us of the interpreter beside 2 to 3 us of the
+// library, a result tensor 2.0 us, a batch of 61 images another 43 us.
 //
 // What is here does what its Python counterpart does or leaves the call to it (pyapi._submit), before anything has happened:
 // other streams, waits, threads at the containers' marks, arguments of other types.
@@ -18,6 +19,7 @@
 #include <cvcuda/OpWarpAffine.h>
 #include <cvcuda/OpWarpPerspective.h>
 #include <nvcv/Tensor.h>
+#include <structmember.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <climits>
@@ -28,7 +30,8 @@ namespace {
 
 // names of pyapi and of the containers
 PyObject *s_submit, *s_Tensor, *s_ImageBatchVarShape, *s_lock, *s_followed, *s_tls, *s_stack, *s_check, *s_t, *s_handle, *s_wrote, *s_read,
-    *s_kind, *s_acquire, *s_release, *s_torch, *s_C, *s_getDevice, *s_getStream;
+    *s_kind, *s_acquire, *s_release, *s_torch, *s_C, *s_getDevice, *s_getStream, *s_value, *s_key, *s_meta, *s_nbytes, *s_np, *s_dtype, *s_made,
+    *s_sizeOf;
 
 // A new reference that goes with the scope.
 struct Ref
@@ -104,6 +107,24 @@ enum Kind
     kBatch
 };
 
+// The pointer that an object's `handle` (a ctypes.c_void_p) holds.
+bool Pointer(PyObject *obj, void *&p)
+{
+    Ref h(PyObject_GetAttr(obj, s_handle)), value(h ? PyObject_GetAttr(h.o, s_value) : nullptr);
+    if (!value || !PyLong_CheckExact(value.o))
+    {
+        PyErr_Clear();
+        return false;
+    }
+    p = PyLong_AsVoidPtr(value.o);
+    if (PyErr_Occurred())
+    {
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
+
 // The library's handle of a container of pyapi.
 Kind HandleOf(PyObject *api, PyObject *obj, void *&handle)
 {
@@ -112,39 +133,13 @@ Kind HandleOf(PyObject *api, PyObject *obj, void *&handle)
     {
         return kNone;
     }
-    Ref       inner(tensor ? PyObject_GetAttr(obj, s_t) : nullptr);
-    Ref       h(!tensor || inner ? PyObject_GetAttr(tensor ? inner.o : obj, s_handle) : nullptr);
-    Py_buffer view;
-    if (!h || h.o == Py_None || PyObject_GetBuffer(h.o, &view, PyBUF_SIMPLE) < 0)
+    Ref inner(tensor ? PyObject_GetAttr(obj, s_t) : nullptr);
+    if (tensor && !inner)
     {
         PyErr_Clear();
         return kNone;
     }
-    const bool pointer = view.len == sizeof(void *);
-    if (pointer)
-    {
-        std::memcpy(&handle, view.buf, sizeof(handle));
-    }
-    PyBuffer_Release(&view);
-    return pointer && handle != nullptr ? (tensor ? kTensor : kBatch) : kNone;
-}
-
-bool OperatorHandle(PyObject *op, NVCVOperatorHandle &handle)
-{
-    Ref       h(PyObject_GetAttr(op, s_handle));
-    Py_buffer view;
-    if (!h || PyObject_GetBuffer(h.o, &view, PyBUF_SIMPLE) < 0)
-    {
-        PyErr_Clear();
-        return false;
-    }
-    const bool pointer = view.len == sizeof(handle);
-    if (pointer)
-    {
-        std::memcpy(&handle, view.buf, sizeof(handle));
-    }
-    PyBuffer_Release(&view);
-    return pointer;
+    return Pointer(tensor ? inner.o : obj, handle) && handle != nullptr ? (tensor ? kTensor : kBatch) : kNone;
 }
 
 bool Int(PyObject *o, int &v)
@@ -383,7 +378,7 @@ bool Mark(PyObject *reads, PyObject *writes, PyObject *key)
         PyObject *read = attributes ? PyDict_GetItem(attributes.o, s_read) : nullptr;
         if (read != nullptr)
         {
-            if (PyDict_SetItem(read, key, Py_None) < 0)
+            if (PyDict_GetItem(read, key) != Py_None && PyDict_SetItem(read, key, Py_None) < 0)
             {
                 return false;
             }
@@ -398,10 +393,26 @@ bool Mark(PyObject *reads, PyObject *writes, PyObject *key)
     for (Py_ssize_t k = 0; k < PyList_GET_SIZE(writes); ++k)
     {
         PyObject *obj = PyList_GET_ITEM(writes, k);
-        Ref       wrote(PyTuple_Pack(2, key, Py_None)), none(PyDict_New());
-        if (!wrote || !none || PyObject_SetAttr(obj, s_wrote, wrote.o) < 0 || PyObject_SetAttr(obj, s_read, none.o) < 0)
+        Ref       attributes(AttributesOf(obj));
+        PyObject *was = attributes ? PyDict_GetItem(attributes.o, s_wrote) : nullptr, *read = attributes ? PyDict_GetItem(attributes.o, s_read) : nullptr;
+        // (marks that stand already stay; another thread may have set others meanwhile)
+        const bool stands = was != nullptr && PyTuple_CheckExact(was) && PyTuple_GET_SIZE(was) == 2 && PyTuple_GET_ITEM(was, 1) == Py_None
+                         && PyObject_RichCompareBool(PyTuple_GET_ITEM(was, 0), key, Py_EQ) == 1;
+        if (!stands)
         {
-            return false;
+            Ref wrote(PyTuple_Pack(2, key, Py_None));
+            if (!wrote || PyObject_SetAttr(obj, s_wrote, wrote.o) < 0)
+            {
+                return false;
+            }
+        }
+        if (read == nullptr || !PyDict_CheckExact(read) || PyDict_GET_SIZE(read) != 0)
+        {
+            Ref none(PyDict_New());
+            if (!none || PyObject_SetAttr(obj, s_read, none.o) < 0)
+            {
+                return false;
+            }
         }
     }
     return true;
@@ -424,12 +435,14 @@ PyObject *Submit(PyObject *api, PyObject *const *a, Py_ssize_t n)
         PyErr_Clear();
         return handOn();
     }
-    Ref kind(PyObject_GetAttr(a[3], s_kind));
-    if (!kind || !Int(kind.o, call.kind) || !OperatorHandle(a[3], call.op) || !call.Parse(api, a + 4, n - 4))
+    Ref   kind(PyObject_GetAttr(a[3], s_kind));
+    void *op = nullptr;
+    if (!kind || !Int(kind.o, call.kind) || !Pointer(a[3], op) || !call.Parse(api, a + 4, n - 4))
     {
         PyErr_Clear();
         return handOn();
     }
+    call.op = reinterpret_cast<NVCVOperatorHandle>(op);
     Ref       keyObject(PyLong_FromLong(key));
     PyObject *lock = Name(api, s_lock), *followed = Name(api, s_followed);
     // the marks are read under their lock; where another thread holds it, Python waits for it
@@ -655,6 +668,315 @@ PyObject *TorchView(PyObject *, PyObject *args)
     }
 }
 
+// batch_alloc(capacity): (status, handle) of an image batch.
+PyObject *BatchAlloc(PyObject *, PyObject *capacity)
+{
+    int n;
+    if (!Int(capacity, n))
+    {
+        PyErr_SetString(PyExc_TypeError, "capacity: a 32-bit number");
+        return nullptr;
+    }
+    NVCVImageBatchVarShapeRequirements needs;
+    NVCVImageBatchHandle               handle = nullptr;
+    NVCVStatus                         status;
+    Py_BEGIN_ALLOW_THREADS
+    status = nvcvImageBatchVarShapeCalcRequirements(n, &needs);
+    if (status == NVCV_SUCCESS)
+    {
+        status = nvcvImageBatchVarShapeConstruct(&needs, nullptr, &handle);
+    }
+    Py_END_ALLOW_THREADS
+    return Py_BuildValue("iK", (int)status, (unsigned long long)reinterpret_cast<uintptr_t>(handle));
+}
+
+// push_planes(batch's handle, format, planes' array as planes() gives it): status.
+PyObject *PushPlanes(PyObject *, PyObject *args)
+{
+    unsigned long long handle, format;
+    const char        *planes;
+    Py_ssize_t         bytes;
+    if (!PyArg_ParseTuple(args, "KKy#", &handle, &format, &planes, &bytes))
+    {
+        return nullptr;
+    }
+    NVCVStatus status;
+    Py_BEGIN_ALLOW_THREADS
+    status = nvcvxImageBatchVarShapePushBuffers(reinterpret_cast<NVCVImageBatchHandle>((uintptr_t)handle), format,
+                                                reinterpret_cast<const NVCVImagePlaneStrided *>(planes),
+                                                (int32_t)(bytes / (Py_ssize_t)sizeof(NVCVImagePlaneStrided)));
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong((long)status);
+}
+
+// batch_state(batch's handle): (status, number of images, the format that all of them have, 0 without one).
+PyObject *BatchState(PyObject *, PyObject *handle)
+{
+    auto *h = reinterpret_cast<NVCVImageBatchHandle>(PyLong_AsVoidPtr(handle));
+    if (PyErr_Occurred())
+    {
+        return nullptr;
+    }
+    int32_t         n      = 0;
+    NVCVImageFormat format = NVCV_IMAGE_FORMAT_NONE;
+    NVCVStatus      status = nvcvImageBatchGetNumImages(h, &n);
+    if (status == NVCV_SUCCESS)
+    {
+        status = nvcvImageBatchVarShapeGetUniqueFormat(h, &format);
+    }
+    return Py_BuildValue("iiK", (int)status, (int)n, (unsigned long long)format);
+}
+
+// tensor_release(handle), batch_release(handle): gives a reference back.
+template<class Handle, NVCVStatus (*DecRef)(Handle, int *)>
+PyObject *Release(PyObject *, PyObject *handle)
+{
+    auto *h = reinterpret_cast<Handle>(PyLong_AsVoidPtr(handle));
+    if (PyErr_Occurred())
+    {
+        return nullptr;
+    }
+    Py_BEGIN_ALLOW_THREADS
+    (void)DecRef(h, nullptr);
+    Py_END_ALLOW_THREADS
+    Py_RETURN_NONE;
+}
+
+// ---- operators' results that are handed out again: see pyapi._Outputs, which is this type by another name. Its tables are
+// touched under the interpreter's lock alone, and no object is given up between a table and the numbers that go with it.
+struct Outputs
+{
+    PyObject_HEAD
+    PyObject *api;  // pyapi's dictionary
+    PyObject *free; // (shape, element type, layout, device) -> list of the library's tensors
+    long long bytes, count, mostBytes, mostTensors;
+};
+
+int OutputsInit(PyObject *self, PyObject *args, PyObject *)
+{
+    auto     *o = reinterpret_cast<Outputs *>(self);
+    PyObject *api;
+    if (!PyArg_ParseTuple(args, "O!", &PyDict_Type, &api))
+    {
+        return -1;
+    }
+    Py_INCREF(api);
+    Py_XSETREF(o->api, api);
+    Py_XSETREF(o->free, PyDict_New());
+    o->bytes = o->count = 0;
+    o->mostBytes        = 256 << 20;
+    o->mostTensors      = 64;
+    return o->free != nullptr ? 0 : -1;
+}
+
+void OutputsDealloc(PyObject *self)
+{
+    auto         *o    = reinterpret_cast<Outputs *>(self);
+    PyTypeObject *type = Py_TYPE(self);
+    Py_CLEAR(o->free);
+    Py_CLEAR(o->api);
+    type->tp_free(self);
+    Py_DECREF(type);
+}
+
+// The tables as they were, with empty ones in their place (a new reference).
+PyObject *OutputsTakeAll(Outputs *o)
+{
+    PyObject *empty = PyDict_New();
+    if (empty == nullptr)
+    {
+        return nullptr;
+    }
+    PyObject *all = o->free;
+    o->free       = empty;
+    o->bytes = o->count = 0;
+    return all;
+}
+
+// clear(): gives everything held back to the allocator; False if there was nothing.
+PyObject *OutputsClear(PyObject *self, PyObject *)
+{
+    auto      *o    = reinterpret_cast<Outputs *>(self);
+    const bool held = o->count != 0;
+    Ref        all(OutputsTakeAll(o));
+    return all ? PyBool_FromLong(held) : nullptr;
+}
+
+// get(shape, dtype, layout): a tensor for a result.
+PyObject *OutputsGet(PyObject *self, PyObject *const *a, Py_ssize_t n)
+{
+    auto *o = reinterpret_cast<Outputs *>(self);
+    if (n != 3)
+    {
+        PyErr_SetString(PyExc_TypeError, "get(shape, dtype, layout)");
+        return nullptr;
+    }
+    Ref       shape(PySequence_Tuple(a[0])); // (a tuple itself)
+    PyObject *np = Name(o->api, s_np), *torch = Name(o->api, s_torch);
+    Ref       dtypes(shape && np != nullptr ? PyObject_GetAttr(np, s_dtype) : nullptr);
+    if (!dtypes || !PyType_Check(dtypes.o))
+    {
+        return nullptr;
+    }
+    Ref dtype(nullptr);
+    if (PyObject_TypeCheck(a[1], reinterpret_cast<PyTypeObject *>(dtypes.o)))
+    {
+        Py_INCREF(a[1]);
+        dtype.o = a[1];
+    }
+    else
+    {
+        dtype.o = PyObject_CallOneArg(dtypes.o, a[1]);
+    }
+    Ref c(dtype && torch != nullptr ? PyObject_GetAttr(torch, s_C) : nullptr);
+    Ref device(c ? PyObject_CallMethodNoArgs(c.o, s_getDevice) : nullptr);
+    Ref key(device ? PyTuple_Pack(4, shape.o, dtype.o, a[2], device.o) : nullptr);
+    if (!key)
+    {
+        return nullptr;
+    }
+    Ref       raw(nullptr);
+    PyObject *kept = PyDict_GetItemWithError(o->free, key.o);
+    if (kept == nullptr && PyErr_Occurred())
+    {
+        return nullptr;
+    }
+    const bool again = kept != nullptr && PyList_GET_SIZE(kept) > 0;
+    if (again)
+    {
+        const Py_ssize_t last = PyList_GET_SIZE(kept) - 1;
+        raw.o                 = PyList_GET_ITEM(kept, last);
+        Py_INCREF(raw.o);
+        if (PyList_SetSlice(kept, last, last + 1, nullptr) < 0)
+        {
+            return nullptr;
+        }
+        --o->count;
+        Ref size(PyObject_GetAttr(raw.o, s_nbytes));
+        o->bytes -= size ? PyLong_AsLongLong(size.o) : 0;
+        if (PyErr_Occurred())
+        {
+            return nullptr;
+        }
+    }
+    else
+    {
+        PyObject *make = Name(o->api, s_made);
+        raw.o = make != nullptr ? PyObject_CallFunctionObjArgs(make, shape.o, dtype.o, a[2], nullptr) : nullptr;
+        if (!raw)
+        {
+            return nullptr;
+        }
+    }
+    PyObject *type = Name(o->api, s_Tensor);
+    if (type == nullptr || !PyType_Check(type))
+    {
+        PyErr_SetString(PyExc_TypeError, "Tensor is no type");
+        return nullptr;
+    }
+    Ref none(PyTuple_New(0));
+    Ref out(none ? reinterpret_cast<PyTypeObject *>(type)->tp_new(reinterpret_cast<PyTypeObject *>(type), none.o, nullptr) : nullptr);
+    Ref attributes(out ? PyObject_GenericGetDict(out.o, nullptr) : nullptr);
+    Ref meta(attributes ? PyTuple_Pack(3, shape.o, dtype.o, PyObject_IsTrue(a[2]) == 1 ? a[2] : Py_None) : nullptr);
+    if (!meta || PyDict_SetItem(attributes.o, s_t, raw.o) < 0 || PyDict_SetItem(attributes.o, s_meta, meta.o) < 0)
+    {
+        return nullptr;
+    }
+    if (again) // another stream's first use of it waits for the default stream's last
+    {
+        Ref by(PyNumber_Negative(device.o)), wrote(by ? PyTuple_Pack(2, by.o, Py_None) : nullptr);
+        if (!wrote || PyDict_SetItem(attributes.o, s_wrote, wrote.o) < 0)
+        {
+            return nullptr;
+        }
+    }
+    if (PyDict_SetItem(attributes.o, s_key, key.o) < 0) // (the last: from here on it comes back)
+    {
+        return nullptr;
+    }
+    Py_INCREF(out.o);
+    return out.o;
+}
+
+// put(tensor): keeps the library's tensor of one whose owner is gone, if every use of it was on its device's default stream.
+PyObject *OutputsPut(PyObject *self, PyObject *tensor)
+{
+    auto *o = reinterpret_cast<Outputs *>(self);
+    Ref   attributes(AttributesOf(tensor));
+    // (where the interpreter is ending, names and attributes may be gone: then it is not kept)
+    PyObject *key = attributes ? PyDict_GetItem(attributes.o, s_key) : nullptr, *raw = attributes ? PyDict_GetItem(attributes.o, s_t) : nullptr;
+    if (key == nullptr || raw == nullptr || !PyTuple_CheckExact(key) || PyTuple_GET_SIZE(key) != 4 || o->free == nullptr)
+    {
+        Py_RETURN_NONE;
+    }
+    const long by = -PyLong_AsLong(PyTuple_GET_ITEM(key, 3));
+    if (PyErr_Occurred() || !WroteBy(attributes.o, by) || !ReadBy(attributes.o, by))
+    {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    Ref held(raw);
+    Py_INCREF(raw);
+    Ref size(PyObject_GetAttr(raw, s_nbytes));
+    if (!size)
+    {
+        PyErr_Clear();
+        PyObject *sizeOf = Name(o->api, s_sizeOf);
+        size.o           = sizeOf != nullptr && sizeOf != Py_None ? PyObject_CallOneArg(sizeOf, raw) : nullptr;
+        if (!size || PyObject_SetAttr(raw, s_nbytes, size.o) < 0)
+        {
+            PyErr_Clear();
+            Py_RETURN_NONE;
+        }
+    }
+    const long long bytes = PyLong_AsLongLong(size.o);
+    if (PyErr_Occurred())
+    {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    Ref drop(nullptr);
+    if (o->count >= o->mostTensors || o->bytes + bytes > o->mostBytes)
+    {
+        drop.o = OutputsTakeAll(o);
+    }
+    if (bytes <= o->mostBytes / 4)
+    {
+        Ref       fresh(PyDict_GetItem(o->free, key) == nullptr ? PyList_New(0) : nullptr);
+        PyObject *kept = fresh ? PyDict_SetDefault(o->free, key, fresh.o) : PyDict_GetItem(o->free, key);
+        if (kept != nullptr && PyList_Append(kept, raw) == 0)
+        {
+            o->bytes += bytes;
+            ++o->count;
+        }
+        PyErr_Clear();
+    }
+    Py_RETURN_NONE;
+}
+
+PyMethodDef kOutputsMethods[] = {
+    {"get", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(OutputsGet)), METH_FASTCALL, nullptr},
+    {"put", OutputsPut, METH_O, nullptr},
+    {"clear", OutputsClear, METH_NOARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyMemberDef kOutputsMembers[] = {
+    {"most_bytes", T_LONGLONG, offsetof(Outputs, mostBytes), 0, nullptr},
+    {"most_tensors", T_LONGLONG, offsetof(Outputs, mostTensors), 0, nullptr},
+    {"_bytes", T_LONGLONG, offsetof(Outputs, bytes), READONLY, nullptr},
+    {"_count", T_LONGLONG, offsetof(Outputs, count), READONLY, nullptr},
+    {nullptr, 0, 0, 0, nullptr},
+};
+
+PyType_Slot kOutputsSlots[] = {
+    {Py_tp_init, reinterpret_cast<void *>(OutputsInit)}, {Py_tp_dealloc, reinterpret_cast<void *>(OutputsDealloc)},
+    {Py_tp_new, reinterpret_cast<void *>(PyType_GenericNew)}, {Py_tp_methods, kOutputsMethods},
+    {Py_tp_members, kOutputsMembers}, {0, nullptr},
+};
+
+PyType_Spec kOutputsSpec = {"_cvcuda_native.Outputs", sizeof(Outputs), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE, kOutputsSlots};
+
 PyMethodDef kBound[] = {
     {"submit", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Submit)), METH_FASTCALL, nullptr},
     {"default_stream_key", DefaultKey, METH_NOARGS, nullptr},
@@ -677,6 +999,11 @@ PyMethodDef kMethods[] = {
     {"planes", Planes, METH_O, nullptr},
     {"tensor_alloc", TensorAlloc, METH_VARARGS, nullptr},
     {"torch_view", TorchView, METH_VARARGS, nullptr},
+    {"tensor_release", Release<NVCVTensorHandle, nvcvTensorDecRef>, METH_O, nullptr},
+    {"batch_alloc", BatchAlloc, METH_O, nullptr},
+    {"push_planes", PushPlanes, METH_VARARGS, nullptr},
+    {"batch_state", BatchState, METH_O, nullptr},
+    {"batch_release", Release<NVCVImageBatchHandle, nvcvImageBatchDecRef>, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 
@@ -698,6 +1025,9 @@ PyMODINIT_FUNC PyInit__cvcuda_native(void)
         {&s_kind, "_native"},     {&s_acquire, "acquire"}, {&s_release, "release"},
         {&s_torch, "torch"},      {&s_C, "_C"},            {&s_getDevice, "_cuda_getDevice"},
         {&s_getStream, "_cuda_getCurrentRawStream"},
+        {&s_value, "value"},      {&s_key, "_key"},        {&s_meta, "_meta"},
+        {&s_nbytes, "_nbytes"},   {&s_np, "np"},           {&s_dtype, "dtype"},
+        {&s_made, "_new_result"}, {&s_sizeOf, "_bytes_of"},
     };
     for (const auto &n : names)
     {
@@ -706,5 +1036,11 @@ PyMODINIT_FUNC PyInit__cvcuda_native(void)
             return nullptr;
         }
     }
-    return PyModule_Create(&kModule);
+    Ref module(PyModule_Create(&kModule)), outputs(PyType_FromSpec(&kOutputsSpec));
+    if (!module || !outputs || PyModule_AddObjectRef(module.o, "Outputs", outputs.o) < 0)
+    {
+        return nullptr;
+    }
+    Py_INCREF(module.o);
+    return module.o;
 }

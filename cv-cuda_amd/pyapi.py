@@ -17,6 +17,7 @@ raised as the same types here.
 """
 import ctypes as C
 import enum
+import functools
 import re
 import threading
 
@@ -265,7 +266,7 @@ def _torch_stream(stream):
 # ---- containers --------------------------------------------------------------------------------------------------
 def _np_dtype(dtype):
     """numpy dtype of a numpy type, a torch dtype or a member of Type."""
-    if isinstance(dtype, (int, enum.IntEnum)) and not isinstance(dtype, bool):
+    if isinstance(dtype, int) and not isinstance(dtype, bool):
         if int(dtype) not in _DT2NP:
             raise ValueError("data type 0x%x has no array element type" % int(dtype))
         return _DT2NP[int(dtype)]
@@ -377,75 +378,27 @@ _CoreTensor = _Tensor
 _DIRECT_VIEW = {np.dtype(np.uint8): 0, np.dtype(np.float32): 1}
 
 
-class _Outputs:
+class _Outputs(_native.Outputs):
     """Tensors that operators made for their results and whose owners are gone, for results of the same shape, type and
     layout: the intermediate results of a chain of operators. (The reference's bindings keep such objects too, in their
     object cache.) A tensor comes back here only if every use of it was a call of this module on the default stream,
     where the next user's work is ordered behind the last one's; one whose memory, handle or views were given out goes
-    back to the library's allocator, which knows when the device is done with it. Bounded: beyond `most_bytes` or
-    `most_tensors` everything held goes back to the allocator, as it does when the device is out of memory and in
-    `clear_cache()`."""
-    most_bytes, most_tensors = 256 << 20, 64
+    back to the library's allocator, which knows when the device is done with it. Bounded: beyond `most_bytes` (256 MiB)
+    or `most_tensors` (64) everything held goes back to the allocator, as it does when the device is out of memory and in
+    `clear_cache()`. get(shape, dtype, layout), put(tensor) and clear() (False if there was nothing) are native: in Python a
+    result was 2.0 us of a call of 6."""
 
     def __init__(self):
-        self._lock = threading.Lock()
-        self._free, self._bytes, self._count = {}, 0, 0
+        super().__init__(globals())
 
-    def get(self, shape, dtype, layout):
-        if type(shape) is not tuple:
-            shape = tuple(shape)
-        if not isinstance(dtype, np.dtype):
-            dtype = np.dtype(dtype)
-        device = torch._C._cuda_getDevice()
-        key = (shape, dtype, layout, device)
-        out = Tensor.__new__(Tensor)
-        with self._lock:
-            stack = self._free.get(key)
-            raw = stack.pop() if stack else None
-            if raw is not None:
-                self._bytes -= raw._nbytes
-                self._count -= 1
-        if raw is not None:
-            out._t, out._wrote = raw, (-device, None)  # another stream's first use of it waits for the default stream's last
-        else:
-            out._t = raw = _allocated(_Tensor.alloc, list(shape), dtype, layout or "")
-            d = raw.export()
-            raw._nbytes = d.buffer.strides[0] * d.shape[0] if d.rank else 0
-        out._key, out._meta = key, (shape, dtype, layout or None)
-        return out
 
-    def put(self, tensor):
-        try:
-            seen, key = tensor.__dict__, tensor._key
-            by = -key[3]
-            if seen.get("_wrote", (by, None))[0] != by:
-                return
-            for k in seen.get("_read", _NO_READS):
-                if k != by:
-                    return
-            # (not waited for: the collector may have stepped in while this thread holds the lock)
-            if not self._lock.acquire(False):
-                return
-            drop = None
-            try:
-                raw = tensor._t
-                if self._count >= self.most_tensors or self._bytes + raw._nbytes > self.most_bytes:
-                    drop, self._free, self._bytes, self._count = self._free, {}, 0, 0
-                if raw._nbytes <= self.most_bytes // 4:
-                    self._free.setdefault(key, []).append(raw)
-                    self._bytes += raw._nbytes
-                    self._count += 1
-            finally:
-                self._lock.release()
-            del drop
-        except (AttributeError, TypeError):
-            pass  # the interpreter is ending: the module's names are gone
+def _new_result(shape, dtype, layout):
+    return _allocated(_Tensor.alloc, list(shape), dtype, layout or "")
 
-    def clear(self):
-        """Gives everything held back to the allocator; False if there was nothing."""
-        with self._lock:
-            drop, self._free, self._bytes, self._count = self._free, {}, 0, 0
-        return any(drop.values())
+
+def _bytes_of(raw):
+    d = raw.export()
+    return d.buffer.strides[0] * d.shape[0] if d.rank else 0
 
 
 _NO_READS = {}
@@ -477,6 +430,12 @@ def _result(shape, dtype, layout, stream):
     if key is None and _default_stream_key(stream) is None:
         return Tensor(tuple(shape), dtype, layout)
     return _outputs.get(shape, dtype, layout)
+
+
+def _like(src, stream):
+    """A tensor for a result of `src`'s shape, type and layout."""
+    shape, dtype, layout = src._properties()
+    return _result(shape, dtype or src.dtype, layout, stream)
 
 
 def reshape(tensor, shape, layout=None):
@@ -687,7 +646,9 @@ def as_images(buffers, format=None):
     if planes is None:
         batch.pushback([as_image(b, format) for b in buffers])
     else:
-        check(_nv.nvcvxImageBatchVarShapePushBuffers(batch.handle, planes[0], planes[1], len(buffers)))
+        status = _native.push_planes(batch.handle.value, planes[0], planes[1])
+        if status:
+            check(status)
         batch._buffers = buffers
     return batch
 
@@ -752,7 +713,7 @@ _ops_lock = threading.Lock()
 
 
 def _op(cls, *args):
-    key = (cls,) + args
+    key = (cls,) + args if args else cls
     op = _ops.get(key)
     if op is None:
         with _ops_lock:
@@ -963,7 +924,7 @@ def normalize_into(dst, src, base, scale, flags=None, *, globalscale=1.0, global
 
 
 def normalize(src, base, scale, flags=None, *, globalscale=1.0, globalshift=0.0, epsilon=0.0, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _like(src, stream)
     return normalize_into(dst, src, base, scale, flags, globalscale=globalscale, globalshift=globalshift,
                           epsilon=epsilon, stream=stream)
 
@@ -976,10 +937,17 @@ def reformat_into(dst, src, *, stream=None):
 def reformat(src, layout, *, stream=None):
     """The output has the input's dimensions in the order of `layout` (OpReformat.cpp:48-55)."""
     have = src.layout or ""
-    if sorted(have) != sorted(layout):
+    order = _order(have, layout)
+    if order is None:
         raise ValueError("layout %r is not a permutation of %r" % (layout, have))
-    shape = tuple(src.shape[have.index(c)] for c in layout)
-    return reformat_into(_result(shape, src.dtype, layout, stream), src, stream=stream)
+    shape = src.shape
+    return reformat_into(_result(tuple([shape[k] for k in order]), src.dtype, layout, stream), src, stream=stream)
+
+
+@functools.lru_cache(64)
+def _order(have, layout):
+    """Places in `have` of the letters of `layout`; None where it is no permutation."""
+    return tuple(have.index(c) for c in layout) if sorted(have) == sorted(layout) else None
 
 
 def convertto_into(dst, src, scale=1, offset=0, *, stream=None):
@@ -1032,7 +1000,7 @@ def flip_into(dst, src, flipCode, *, stream=None):
 
 
 def flip(src, flipCode, *, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _like(src, stream)
     return flip_into(dst, src, flipCode, stream=stream)
 
 
@@ -1069,7 +1037,7 @@ def warp_affine_into(dst, src, xform, flags, *, border_mode=Border.CONSTANT, bor
 
 
 def warp_affine(src, xform, flags, *, border_mode=Border.CONSTANT, border_value=0, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _like(src, stream)
     return warp_affine_into(dst, src, xform, flags, border_mode=border_mode, border_value=border_value, stream=stream)
 
 
@@ -1079,7 +1047,7 @@ def warp_perspective_into(dst, src, xform, flags, *, border_mode, border_value, 
 
 
 def warp_perspective(src, xform, flags, *, border_mode, border_value, stream=None):
-    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _result(src.shape, src.dtype, src.layout, stream)
+    dst = _same_images(src) if isinstance(src, _ImageBatchVarShape) else _like(src, stream)
     return warp_perspective_into(dst, src, xform, flags, border_mode=border_mode, border_value=border_value,
                                  stream=stream)
 
@@ -1096,26 +1064,30 @@ def resize_crop_convert_reformat(src, resize_dim, interp, crop_rect, *, layout="
     """Output: the input's batch and channels, the crop's height and width, in `layout` (default: the input's) with
     elements of `data_type` (0: the input's). An image batch gives an N-image tensor, `layout` NHWC or NCHW
     (OpResizeCropConvertReformat.cpp:60-103, 132-180)."""
-    rect = RectI(*crop_rect)
+    rect = crop_rect if type(crop_rect) is RectI else RectI(*crop_rect)
+    height, width = int(rect.height), int(rect.width)
     if isinstance(src, _ImageBatchVarShape):
-        fmt = src.uniqueformat
-        if fmt is None or int(fmt) not in _PLANE_NP:
+        status, count, fmt = _native.batch_state(src.handle.value)
+        if status:
+            check(status)
+        if fmt not in _PLANE_NP:
             raise Error(7, "All images in input must have the same single-plane format")
-        npdt, ch = _PLANE_NP[int(fmt)]
-        src_layout, nhwc = "NHWC", (len(src), rect.height, rect.width, ch)
+        npdt, ch = _PLANE_NP[fmt]
+        src_layout, nhwc = "NHWC", (count, height, width, ch)
         src_dtype = np.dtype(npdt)
     else:
         src_layout, src_dtype = src.layout, src.dtype
         if src_layout not in ("HWC", "NHWC"):
             raise Error(7, "Input tensor must have layout 'HWC' or 'NHWC'.")
         shp = (1,) * (4 - src.ndim) + tuple(src.shape)
-        nhwc = (shp[0], rect.height, rect.width, shp[3])
+        nhwc = (shp[0], height, width, shp[3])
     out_layout = layout or src_layout
     if len(out_layout) != len(src_layout):
         raise Error(7, "Output tensor rank must match input tensor rank.")
     if out_layout not in ("HWC", "NHWC", "CHW", "NCHW"):
         raise Error(7, "Output tensor must have layout 'HWC', 'NHWC', 'CHW', or 'NCHW'.")
-    shape = tuple(nhwc["NHWC".index(c)] for c in out_layout)
+    n, h, w, c = nhwc
+    shape = (n, c, h, w) if out_layout == "NCHW" else nhwc if out_layout == "NHWC" else (h, w, c) if out_layout == "HWC" else (c, h, w)
     dst = _result(shape, _np_dtype(data_type) if data_type else src_dtype, out_layout, stream)
     return resize_crop_convert_reformat_into(dst, src, resize_dim, interp, (rect.x, rect.y), manip=manip, scale=scale,
                                              offset=offset, srcCast=srcCast, stream=stream)

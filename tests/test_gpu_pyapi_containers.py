@@ -336,6 +336,43 @@ def test_as_images_of_torch_tensors_in_one_call(nvcv):
     assert mixed._buffers is None and mixed.uniqueformat is None
 
 
+def test_images_of_buffers_are_made_once(nvcv):
+    # a batch made of buffers makes its image objects when the library is asked for them, once for all threads; a plane that
+    # is refused leaves the batch as it was
+    import ctypes as C
+    import threading
+
+    import torch
+    tensors = [torch.zeros((4 + i, 6, 3), dtype=torch.uint8, device="cuda") for i in range(40)]
+    batch, n, got = nvcv.as_images(tensors), len(tensors), []
+
+    def ask():
+        handles = (C.c_void_p * n)()
+        nvcv.check(nvcv._nv.nvcvImageBatchVarShapeGetImages(batch.handle, 0, handles, n))
+        got.append(list(handles))
+
+    threads = [threading.Thread(target=ask) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(set(got[0])) == n and all(g == got[0] for g in got) and nvcv.Image(_handle=C.c_void_p(got[0][3])).refcount() == 9
+    for handles in got[1:] + [[h for k, h in enumerate(got[0]) if k != 3]]:
+        for h in handles:
+            nvcv.check(nvcv._nv.nvcvImageDecRef(C.c_void_p(h), None))
+    assert batch[3].size == (6, 7)
+    short = nvcv.ImageBatchVarShape(3)
+    fmt, planes = nvcv._plane_list(tensors[:2], None)
+    assert nvcv._native.push_planes(short.handle.value, fmt, planes) == 0
+    bad = bytearray(planes)
+    bad[len(planes) // 2:len(planes) // 2 + 4] = bytes(4)  # the second one's width
+    for wrong in (bytes(bad)[len(planes) // 2:], planes, bytes(bad)):  # no width; one image too many; both
+        with pytest.raises(nvcv.Error):
+            nvcv.check(nvcv._native.push_planes(short.handle.value, fmt, wrong))
+        assert len(short) == 2 and short.maxsize == (6, 5) and short.uniqueformat == nvcv.Format.RGB8
+    assert [i.size for i in nvcv.as_images(tensors[:2])] == [(6, 4), (6, 5)]
+
+
 def test_kept_memory_is_given_back(nvcv):
     # results that were dropped and blocks of freed tensors stay with the process until clear_cache()
     import torch
