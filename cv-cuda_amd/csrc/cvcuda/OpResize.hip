@@ -1929,8 +1929,8 @@ __device__ __forceinline__ void ResizeLinearQuadStripU8(const Plane &p, int x0, 
     }
 }
 
-// Nearest neighbour when enlarging by 1.5 or more (3 * srcW <= 2 * dstW), in the shape of the four-column strips:
-// the source pixels of four neighbouring output columns lie within 3 source pixels, so a lane owns 4 columns x R
+// Nearest neighbour when enlarging, in the shape of the four-column strips:
+// the source pixels of four neighbouring output columns lie within 4 source pixels, so a lane owns 4 columns x R
 // rows, takes them from one window per source row and stores every output row that maps to that source row from
 // the same registers. The wave patches spend one 3-byte load per output pixel there (8 x 720p -> 1080p u8x3: 19.0 us,
 // the bilinear strips 22.9; as strips 13.6). Indices are those of Axis<NEAREST>; waves that reach the image's last row,
@@ -2009,6 +2009,118 @@ __device__ __forceinline__ void ResizeNearestQuadStripU8(const Plane &p, int x0,
                 ++r;
             }
         }
+    }
+}
+
+// Nearest neighbour of 1 and 3 channels where the output rows' source rows are not consecutive: a lane owns 4 columns as in
+// the strips, but each of its R rows comes from a window of its own, DWORDS dwords from the one of the lane's first source
+// pixel on. Bound by the writes: the wave patches' rows of 64 pixels (64 bytes of one channel, mostly not at a sector's start) end in
+// partly written sectors twice for each, these rows of 256 once for four, and four pixels are one load instead of four. One
+// channel, 40 MB each: by 1.3 20.7 -> 11.9 us, by 2 14.8 -> 10.8, by 3 13.6 -> 10.9; 200 x 258 x 752 -> 244 x 711 37.5 -> 19.0. Three channels enlarged
+// across alone (117 x 453 x 113 -> 455 x 84) 10.2 -> 7.7.
+constexpr int kNearestRows = 4;
+
+template<int C, int DWORDS>
+__device__ __forceinline__ void ResizeNearestRowsU8(const Plane &p, int x0, int y0)
+{
+    static_assert(C == 1 ? DWORDS == 2 || DWORDS == 4 : C == 3 && DWORDS == 4);
+    constexpr int R = kNearestRows;
+    if (x0 >= p.dstW || y0 >= p.dstH)
+    {
+        return;
+    }
+    const int lane = threadIdx.x & 63, dx0 = x0 + 4 * lane;
+    int       s[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        s[j] = Axis<NVCV_INTERP_NEAREST>(p.scaleX, min(dx0 + j, p.dstW - 1), p.srcW).s;
+    }
+    // lane r holds the source row of output row y0 + r
+    const int  rowLane = Axis<NVCV_INTERP_NEAREST>(p.scaleY, min(y0 + (lane & (R - 1)), p.dstH - 1), p.srcH).s;
+    const bool fits    = (s[3] - s[0] + 1) * C <= 4 * DWORDS - 3; // wherever in a dword the first byte is
+    // (a window may run past its row, so the image's last row is left to the patches)
+    if (__builtin_amdgcn_readlane(rowLane, R - 1) >= p.srcH - 1 || __builtin_amdgcn_ballot_w64(!fits) != 0) // wave-uniform
+    {
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i)
+        {
+            ResizeWavePatch<uint8_t, C, NVCV_INTERP_NEAREST, false>(p, x0 + 64 * i, y0);
+        }
+        return;
+    }
+    struct alignas(4) Window
+    {
+        uint32_t d[DWORDS];
+    };
+    Window   w[R];
+    uint32_t at[R]; // of the first byte, from a dword in front of it on (the low two bits: in its dword)
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+    {
+        const uint8_t *row = p.src + (int64_t)__builtin_amdgcn_readlane(rowLane, r) * p.srcRow;
+        const uint32_t odd = (uint32_t)reinterpret_cast<uintptr_t>(row) & 3u;
+        at[r]              = odd + (uint32_t)(s[0] * C);
+        w[r]               = *reinterpret_cast<const Window *>(row - odd + (at[r] & ~3u));
+    }
+    __builtin_amdgcn_sched_barrier(0); // (every load before the first use)
+    // Selectors of v_perm_b32 that make the lane's C dwords of a row from the window's bytes, counted from the first one on: of
+    // the last dword, which may need bytes behind the eighth, two halves, whose missing bytes are zeros (selector 0x0c).
+    constexpr bool kHalves = DWORDS > 2;
+    uint32_t       low[C] = {}, high = 0;
+#pragma unroll
+    for (int b = 0; b < 4 * C; ++b)
+    {
+        const uint32_t k    = (uint32_t)((s[b / C] - s[0]) * C + b % C);
+        const bool     last = kHalves && b / 4 == C - 1;
+        low[b / 4] |= (last && k >= 8 ? 0x0cu : k) << (8 * (b % 4));
+        high |= last ? (k >= 8 ? k - 8 : 0x0cu) << (8 * (b % 4)) : 0u;
+    }
+    uint8_t  *to    = p.dst + (int64_t)y0 * p.dstRow + (int64_t)dx0 * C;
+    const int nRows = min(R, p.dstH - y0);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+    {
+        if (r >= nRows) // uniform
+        {
+            break;
+        }
+        uint32_t out[C];
+        if constexpr (!kHalves)
+        {
+            out[0] = __builtin_amdgcn_perm(w[r].d[1], w[r].d[0], low[0] + (at[r] & 3u) * 0x01010101u);
+        }
+        else
+        {
+            uint32_t t[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                t[i] = __builtin_amdgcn_alignbyte(i < 3 ? w[r].d[i + 1] : 0u, w[r].d[i], at[r]);
+            }
+#pragma unroll
+            for (int i = 0; i < C; ++i)
+            {
+                out[i] = __builtin_amdgcn_perm(t[1], t[0], low[i]);
+            }
+            out[C - 1] |= __builtin_amdgcn_perm(t[3], t[2], high);
+        }
+        if (dx0 + 4 <= p.dstW)
+        {
+            StoreDwordsNT<C>(to, out);
+        }
+        else
+        {
+#pragma unroll
+            for (int i = 0; i < 3 * C; ++i)
+            {
+                if (dx0 + i / C < p.dstW)
+                {
+                    to[i] = (uint8_t)(out[i >> 2] >> (8 * (i & 3)));
+                }
+            }
+        }
+        to += p.dstRow;
     }
 }
 
@@ -2225,6 +2337,14 @@ __global__ __launch_bounds__(256) void ResizeNearestQuadsU8Kernel(const ResizeAr
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     const WaveTile t = WaveTileOf(flat);
     ResizeNearestQuadStripU8<C, R>(p, t.x * kQuadsTileW, t.y * R);
+}
+
+template<int C, int DWORDS>
+__global__ __launch_bounds__(256) void ResizeNearestRowsU8Kernel(const ResizeArgs a, const int flat)
+{
+    const Plane p = GetPlanes<false>(a, blockIdx.z);
+    const WaveTile t = WaveTileOf(flat);
+    ResizeNearestRowsU8<C, DWORDS>(p, t.x * kQuadsTileW, t.y * kNearestRows);
 }
 
 // Image batches: the same 128 x 8 tile per block for every image; an image whose horizontal scale is
@@ -3837,19 +3957,38 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     if constexpr (std::is_same_v<T, uint8_t> && INTERP == NVCV_INTERP_NEAREST && (C == 1 || C == 3 || C == 4))
     {
         const int64_t strips = (int64_t)DivUp(a.dstW, kQuadsTileW) * DivUp(a.dstH, kStripRows) * N;
-        if (NearestStripScale<C>(a.srcW, a.srcH, a.dstW, a.dstH) && strips >= (C == 3 ? 6 : 4) * 256)
+        const bool    flat   = FlatBlocks(a.dstW, kQuadsTileW);
+        // Enlarged by less than 1.5 the patches, whose waves are a quarter as wide, are the faster form until the chip is full (us as
+        // patches / so: 18 x 2140 x 137 x 1 -> 1089 x 98 4.2 / 5.0, 30 x 1219 x 75 x 1 -> 1201 x 78 4.4 / 5.0, 105 x 465 x 40 x 3 -> 576 x 50 5.3 / 6.9) and where most of a wave's 256 columns do not
+        // exist (159 x 146 x 685 x 3 -> 53 x 361 9.7 / 13.8, 65 x 50 x 951 x 3 -> 64 x 1214 6.3 / 9.5; half of them, 18 x 514 x 1146 x 3 -> 558 x 1426, 22.0 / 17.4). 9 x 2475 x
+        // 1391 x 1 -> 2801 x 1564 25.6 / 15.7; 39 x 830 x 212 x 3 -> 1054 x 366 22.7 / 16.4.
+        const bool wide = C != 4 && a.srcW >= 24 && strips >= 10 * 256 && 5 * (int64_t)a.dstW >= 2 * (int64_t)DivUp(a.dstW, kQuadsTileW) * kQuadsTileW;
+        if ((NearestStripScale<C>(a.srcW, a.srcH, a.dstW, a.dstH) && strips >= (C == 3 ? 6 : 4) * 256)
+            || (wide && a.srcW <= a.dstW && a.srcH <= a.dstH))
         {
             // 4 rows: fewer registers, more waves in flight (8 / 4 rows: 8 x 720p -> 1080p 9.0 / 8.5, 15.3 / 13.6, 17.5 / 15.9; 32 x 224 x 224 ->
             // 448 x 448 6.1 / 5.3, 8.5 / 7.0, 9.4 / 7.2). One channel's largest launches pay more for the column terms (24 x 720p -> 1080p
             // 16.0 / 17.0, 32 of these 19.8 / 21.8) unless rows end inside lines of memory (100 x 300 x 300 -> 1000 x 500 20.5 / 18.7) and a
             // source row is fewer than three output rows (3 x 1336 x 1189 -> 3870 x 3444 13.4 / 15.5, 23 x 41 x 1275 -> 122 x 3819 9.3 / 10.5).
-            const bool flat   = FlatBlocks(a.dstW, kQuadsTileW);
             const bool many   = 5 * (int64_t)a.dstH >= 11 * (int64_t)a.srcH ? strips >= 24 * 256 : strips >= 60 * 256 && a.dstRowStride % 64 == 0;
             const int  rows   = C == 1 && many ? kStripRows : 4;
             auto       kernel = rows == 4 ? ResizeNearestQuadsU8Kernel<C, 4> : ResizeNearestQuadsU8Kernel<C, C == 1 ? kStripRows : 4>;
             hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
             CheckLaunch("ResizeNearestQuadsU8Kernel");
             return;
+        }
+        if constexpr (C != 4)
+        {
+            if (wide && (C == 3 ? a.srcW <= a.dstW : a.srcW <= 4 * (int64_t)a.dstW))
+            {
+                // (a lane's 4 columns lie within 4 pixels of one channel more than the first one up to a scale of 4 / 3, 12 up to 4; within 3 of
+                // three channels up to 1. Three channels reduced across, each pixel a load of its own: 143 launches from 0.83 to 1.27 of the patches' time)
+                auto kernel = C == 1 && 3 * (int64_t)a.srcW <= 4 * (int64_t)a.dstW ? ResizeNearestRowsU8Kernel<C, C == 1 ? 2 : 4>
+                                                                                   : ResizeNearestRowsU8Kernel<C, 4>;
+                hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, kNearestRows, flat), dim3(256), 0, stream, a, (int)flat);
+                CheckLaunch("ResizeNearestRowsU8Kernel");
+                return;
+            }
         }
     }
     if constexpr (kPairsForm<T, C, INTERP>)

@@ -183,6 +183,25 @@ def test_tensor_nearest_u8_strips(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
 
 
+# Nearest neighbour of 1 and 3 channels in rows of 256: at their limits (one channel's windows of 2 dwords up to a scale of 4 / 3, of
+# 4 up to 4; three channels up to 1; 2560 strips of 8 rows, 2 of 5 of the last tile's columns, 24 source columns), each side of
+# them, over packed rows of odd widths and pitched ones, where the image's last row is used and where it is not
+@pytest.mark.parametrize("c", [1, 3])
+@pytest.mark.parametrize("row_align", [0, 1])
+@pytest.mark.parametrize("size", [(300, 9, 256, 9, 1280), (341, 13, 256, 9, 1280), (342, 13, 256, 9, 1280), (1024, 20, 256, 9, 1280),
+                                  (1025, 20, 256, 9, 1280), (399, 40, 397, 17, 427), (24, 30, 103, 9, 1280), (23, 30, 103, 9, 1280),
+                                  (99, 30, 102, 9, 1280), (255, 12, 256, 9, 1280), (255, 9, 256, 11, 1280), (257, 9, 257, 9, 640),
+                                  (513, 33, 514, 7, 853), (511, 36, 509, 12, 640), (100, 9, 1021, 6, 640), (100, 9, 1021, 6, 639)])
+def test_tensor_nearest_u8_rows(cv, orc, gpu, size, row_align, c):
+    sw, sh, dw, dh, n = size
+    src = orc.fill_u8((n, sh, sw, c), 77 + sw)
+    tin  = cv.Tensor.from_numpy(src, "NHWC", row_align=row_align)
+    tout = cv.Tensor.alloc([n, dh, dw, c], np.uint8, "NHWC", row_align=row_align)
+    tout.torch_view().fill_(7)
+    cv.Resize()(None, tin, tout, NEAREST)
+    np.testing.assert_array_equal(tout.numpy(), orc.resize(src, (dh, dw), NEAREST, variant=0))
+
+
 # the strip kernels on views that start at an odd byte and have an odd row pitch (their window loads take the aligned
 # dwords around a pixel: nothing may be assumed of where a row starts), output bytes outside the rows untouched
 @pytest.mark.parametrize("c", [3, 1, 4])
