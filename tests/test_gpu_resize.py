@@ -841,6 +841,17 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
     assert not torch.isnan(results[0]).any()
 
 
+# Float bicubic reductions by 4 and more down, whose waves are counted along the rows: tiles of 64 columns that do not fill blocks of
+# four or rows, one wave in the last block, and each side of the scale of 4
+@pytest.mark.parametrize("row", [(sw, sh, dw, dh, CUBIC, n, np.float32, c)
+                                 for c in (3, 4)
+                                 for (sw, sh, dw, dh, n) in [(200, 33, 63, 8, 2), (200, 32, 64, 8, 1), (261, 31, 65, 8, 2), (700, 21, 130, 5, 3),
+                                                             (1300, 9, 257, 1, 2), (517, 40, 129, 3, 1), (640, 101, 320, 25, 2)]],
+                         ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
+def test_tensor_cubic_waves_along_rows(cv, orc, gpu, row):
+    test_tensor_table(cv, orc, gpu, row)
+
+
 # Rows per wave by the size of the launch: the box filter at scales of 1 to 3 (4 rows to a wave up to 2048 waves of 16, 8 up to 8192, then 16), for nearest
 # neighbour enlarging by 1.5 or more (strips of 4 rows from 1024 strips of 8 on, 1536 with three channels; 8 rows for one channel
 # from 15360 on, 6144 where a source row is 2.2 output rows and more) and for float bicubic (4 rows, 8, 16; from 128 waves of 4 rows on,
