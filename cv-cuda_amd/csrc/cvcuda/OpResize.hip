@@ -3796,13 +3796,14 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
 // size). Bound by the output's writes. Rows of such outputs rarely start at a multiple of 64 bytes (a dense row of 1917
 // floats), and then every store instruction of a wave ends in two partly written 64-byte sectors that its neighbours
 // complete in stores of their own: 3.78 M write requests where the output has 3.10 M sectors (24 x 513 x 289 ->
-// 1917 x 1079). So a block produces kRowsPerGroup whole rows (`groups` times, where one group does not give every wave a
-// piece of 256 columns), collects them in LDS at the place they have relative to a 64-byte boundary and writes them
+// 1917 x 1079). Writing alone, 199 MB in pieces of 30 KB to a block, takes 43.3 us where a wave's 1024 bytes start anywhere, 36.5 at
+// 64-byte boundaries and 34.7 at 128-byte ones. So a block produces kRowsPerGroup whole rows (`groups` times, where one group does not give every wave a
+// piece of 256 columns), collects them in LDS at the place they have relative to a 128-byte boundary and writes them
 // out 16 bytes per lane on 16-byte boundaries: a dense output's rows as one run, whose two ends alone are partial. A
 // lane's columns are 64 apart (LDS writes without bank conflicts); the tap pairs of all source rows that 4 output
 // rows can need are requested before the first is used: 3, 4 or 5 by the scale. Against wave patches: 68.8 -> 44.1 us, 4.8 TB/s
 // (24 x 513 x 289 -> 1917 x 1079), 22.8 -> 15.4 us (16 x 320 x 180 -> 1280 x 720), 13.9 -> 12.1 us (3 x 1901 x 900 -> 1300 x
-// 1920). The first case by other forms, each 3 to 4 us longer for an event behind every launch: this one 48.2 us, with 8 rows
+// 1920). At 128-byte boundaries instead of 64-byte ones 41.3 -> 40.5 us (27 x 497 x 113 -> 2373 x 540 36.3 -> 35.0). The first case by other forms, each 3 to 4 us longer for an event behind every launch: this one 48.2 us, with 8 rows
 // per group 61.6 us (61 KB of LDS leave two blocks per CU), streaming stores from the lanes that formed the values
 // 53.5 us, cached stores, which the L2 merges to 3.13 M requests, 79 us (they evict the source rows).
 constexpr int kRowsPerGroup = 4;
@@ -3825,13 +3826,13 @@ __global__ __launch_bounds__(256) void ResizeLinearRowsKernel(const ResizeArgs a
     const int   lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int R  = kRowsPerGroup;
     const int   yBlock = blockIdx.x * groups * R, rowsBlock = min(groups * R, p.dstH - yBlock);
-    // Row i of the block is staged from float i * pitch + lead(i) on, where lead is the row's distance from the 64-byte
+    // Row i of the block is staged from float i * pitch + lead(i) on, where lead is the row's distance from the 128-byte
     // boundary in front of it; dense rows follow one another in LDS as they do in memory (and keep the block's lead).
     const bool  dense = p.dstRow == 4 * p.dstW;
-    const int   pitch = dense ? p.dstW : ((p.dstW + 15) & ~15) + 16;
+    const int   pitch = dense ? p.dstW : ((p.dstW + 31) & ~31) + 32;
     auto        lead  = [&](int i)
     {
-        return (int)(reinterpret_cast<uintptr_t>(p.dst + (int64_t)(yBlock + (dense ? 0 : i)) * p.dstRow) & 63) / 4;
+        return (int)(reinterpret_cast<uintptr_t>(p.dst + (int64_t)(yBlock + (dense ? 0 : i)) * p.dstRow) & 127) / 4;
     };
     for (int t = wave; t < chunks * groups; t += 4)
     {
@@ -4125,7 +4126,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         const int sources = LinearRowsSources(a), chunks = DivUp(a.dstW, 256);
         const int groups = chunks >= 3 ? 1 : chunks == 2 ? 2 : 4;
-        const int lds = (groups * kRowsPerGroup * (((a.dstW + 15) & ~15) + 16) + 16) * 4;
+        const int lds = (groups * kRowsPerGroup * (((a.dstW + 31) & ~31) + 32) + 32) * 4;
         const dim3 rgrid(DivUp(a.dstH, groups * kRowsPerGroup), N);
         const int64_t blocks = (int64_t)rgrid.x * N;
         // us as patches / as rows:
