@@ -41,17 +41,27 @@ namespace cvamd {
 namespace {
 
 constexpr int kPatch   = 8; // gather granule: a wave samples kPatch x kPatch pixels per step
-constexpr int kThreads = 256;
-// A wave's N patches lie side by side, N = kMostPatches or kFewPatches (see LaunchMap); a block's four waves as two by two or in a row.
+// A wave's N patches lie side by side, N = kMostPatches or kFewPatches (see LaunchMap); a block's waves as two by two, four in a
+// row or one alone.
 constexpr int kMostPatches = 4, kFewPatches = 2;
 template<int N>
 constexpr int kWaveW = kPatch * N;
-template<int N>
-constexpr int kWavesX = N == kMostPatches ? 2 : 4;
-template<int N>
-constexpr int kTileW = kWaveW<N> * kWavesX<N>;
-template<int N>
-constexpr int kTileH = kThreads / 64 / kWavesX<N> * kPatch;
+
+// A block of 64 x WAVES threads. Waves of 8-bit bicubic with three channels are the longest and their lengths differ most (the
+// image's edge), so a block of four holds its places until the last one ends: they go alone. us with four waves / one: 24 images
+// of 697 .. 1194 x 187 .. 545 39.0 / 36.2, 9 x 1241 x 955 in perspective 48.1 / 46.8, 16 x 1240 x 1754 175.6 / 172.2. Others gain nothing by it (u8x4 34.6 /
+// 35.0, u8x1 41.0 / 41.1) or are held up by the launch of so many blocks, 4.6 a ns at most (nearest neighbour u8x1 27.2 / 36.2, u8x3 85.9 /
+// 102.5, bilinear u8x3 48.1 / 53.4).
+template<int N, int WAVES>
+struct Block
+{
+    static constexpr int kWaves = WAVES, kThreads = 64 * WAVES;
+    static constexpr int kAcross = WAVES == 1 ? 1 : N == kMostPatches ? 2 : 4;
+    static constexpr int kTileW = kWaveW<N> * kAcross, kTileH = WAVES / kAcross * kPatch;
+};
+
+template<class T, int C, int INTERP, int N>
+using BlockOf = Block<N, std::is_same_v<T, uint8_t> && C == 3 && INTERP == NVCV_INTERP_CUBIC && N == kMostPatches ? 1 : 4>;
 
 struct WarpArgs
 {
@@ -1337,18 +1347,19 @@ __device__ __forceinline__ bool NarrowTapsPay(const float (&m)[9])
     return fabsf(m[3]) > (INTERP == NVCV_INTERP_LINEAR ? 1.f : 1.5f) * fabsf(m[0]);
 }
 
-// One tile of kTileW<N> x kTileH<N> pixels of the destination image `dst` (tile coordinates tx, ty), all 256 threads.
+// One block's tile of the destination image `dst` (tile coordinates tx, ty), all its threads.
 template<class T, int C, int INTERP, bool PERSP, bool LIST, int N>
 __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const float (&m)[9], uint8_t *dst, int dstRow,
                                          int dstW, int dstH, int tx, int ty)
 {
     constexpr int PB = C * sizeof(T), D = (PB + 3) / 4;
+    using B          = BlockOf<T, C, INTERP, N>;
 
     // ---- gather: lane (lx, ly) of wave w samples its pixel in N patches (side by side: a
     // wave covers 8 N columns x 8 rows)
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lx = threadIdx.x & (kPatch - 1),
+    const int wave = B::kWaves == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lx = threadIdx.x & (kPatch - 1),
               ly = (threadIdx.x >> 3) & (kPatch - 1);
-    const int x0 = tx * kTileW<N> + wave % kWavesX<N> * kWaveW<N>, y0 = ty * kTileH<N> + wave / kWavesX<N> * kPatch;
+    const int x0 = tx * B::kTileW + wave % B::kAcross * kWaveW<N>, y0 = ty * B::kTileH + wave / B::kAcross * kPatch;
     // m maps to source coordinates times kCoordScale; so do sx, sy and the limits
     constexpr float kScale = kCoordScale<T, INTERP>;
     const float     limX = InsideLimit<INTERP>(im.w, kTapOverrun<T, C, INTERP>) * kScale, limY = InsideLimit<INTERP>(im.h, 0) * kScale;
@@ -1368,7 +1379,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     MapCoords<PERSP>(m, px, py, sx, sy);
     // the wave's pixels as rows, for the store (kPitch: neighbouring rows on other banks)
     constexpr int kPitch = kWaveW<N> * D + (D == 1 ? 8 : D == 2 ? 16 : D == 4 ? 24 : 0);
-    __shared__ __align__(16) uint32_t room[kThreads / 64][kPatch][kPitch];
+    __shared__ __align__(16) uint32_t room[B::kWaves][kPatch][kPitch];
     auto     &rows = room[wave];
     const int lane = threadIdx.x & 63;
 
@@ -1423,7 +1434,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
         // third are such: 3 x 258 x 271 f32x1 bicubic 16.0 -> 6.7 us, 7 x 318 x 538 f32x4 bilinear 14.6 -> 9.6, 3 x 646 x 752 f32x1 bilinear
         // 9.7 -> 6.2, 40 x 1021 x 1523 of these 169 -> 145; 38 images of 75 .. 801 x 232 .. 359 u8x3 bicubic 36.3 -> 32.0.
         const bool whole  = __builtin_amdgcn_ballot_w64(!fits || !TapsInside<INTERP>(limX, limY, sx, sy)) == 0;
-        __shared__ uint8_t list[kThreads / 64][64 * N];
+        __shared__ uint8_t list[B::kWaves][64 * N];
         uint32_t inside = 0xf, colour[D] = {}; // inside: bit k: sample k
         int      edges  = 0;
         if (!whole)
@@ -1868,7 +1879,7 @@ __device__ __forceinline__ void LoadMatrix(const WarpArgs &a, int image, float s
 }
 
 template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES>
-__global__ __launch_bounds__(kThreads) void WarpTensor(const WarpArgs a)
+__global__ __launch_bounds__((BlockOf<T, C, INTERP, PATCHES>::kThreads)) void WarpTensor(const WarpArgs a)
 {
     const int n  = blockIdx.z;
     const Img im = {a.src + n * a.srcN, a.srcRow, a.srcW, a.srcH};
@@ -1882,7 +1893,7 @@ __global__ __launch_bounds__(kThreads) void WarpTensor(const WarpArgs a)
 }
 
 template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES>
-__global__ __launch_bounds__(kThreads) void WarpVarShape(const WarpArgs a, const VarTiles tiles)
+__global__ __launch_bounds__((BlockOf<T, C, INTERP, PATCHES>::kThreads)) void WarpVarShape(const WarpArgs a, const VarTiles tiles)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
     // descriptors and matrix depend on the image index only: read by value here, ahead of the matrix
@@ -1918,18 +1929,22 @@ template<class T, int C, int INTERP, bool PERSP, bool LIST>
 void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, hipStream_t stream)
 {
     constexpr int kMost = kMostPatches, kFew = kFewPatchesForm<T> ? kFewPatches : kMost;
-    const auto    few = [](int64_t tiles, int64_t most) { return kFew != kMost && tiles * (kThreads / 64) <= most; };
+    using Most          = BlockOf<T, C, INTERP, kMost>;
+    using Few           = BlockOf<T, C, INTERP, kFew>;
+    // (counted in tiles of four waves, whatever a block has)
+    using Four     = Block<kMost, 4>;
+    const auto few = [](int64_t tiles, int64_t most) { return kFew != kMost && tiles * Four::kWaves <= most; };
     if (dstHost == nullptr)
     {
-        const dim3 most(DivUp(a.dstW, kTileW<kMost>), DivUp(a.dstH, kTileH<kMost>), N);
-        if (few((int64_t)most.x * most.y * most.z, kFewWaves))
+        if (few((int64_t)DivUp(a.dstW, Four::kTileW) * DivUp(a.dstH, Four::kTileH) * N, kFewWaves))
         {
-            const dim3 grid(DivUp(a.dstW, kTileW<kFew>), DivUp(a.dstH, kTileH<kFew>), N);
-            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kFew>), grid, dim3(kThreads), 0, stream, a);
+            const dim3 grid(DivUp(a.dstW, Few::kTileW), DivUp(a.dstH, Few::kTileH), N);
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kFew>), grid, dim3(Few::kThreads), 0, stream, a);
         }
         else
         {
-            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kMost>), most, dim3(kThreads), 0, stream, a);
+            const dim3 grid(DivUp(a.dstW, Most::kTileW), DivUp(a.dstH, Most::kTileH), N);
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kMost>), grid, dim3(Most::kThreads), 0, stream, a);
         }
         CheckLaunch("WarpTensor");
         return;
@@ -1938,16 +1953,20 @@ void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, 
     {
         VarTiles  tiles;
         const int count = std::min(kMaxTileImages, N - first);
-        int       total = BuildVarTiles(tiles, dstHost, first, count, kTileW<kMost>, kTileH<kMost>);
+        int       total = BuildVarTiles(tiles, dstHost, first, count, Four::kTileW, Four::kTileH);
         if (total > 0 && few(total, kFewWavesOfBatches<T, INTERP, PERSP>))
         {
-            total = BuildVarTiles(tiles, dstHost, first, count, kTileW<kFew>, kTileH<kFew>);
-            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kFew>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
+            total = BuildVarTiles(tiles, dstHost, first, count, Few::kTileW, Few::kTileH);
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kFew>), dim3(total), dim3(Few::kThreads), 0, stream, a, tiles);
             CheckLaunch("WarpVarShape");
         }
         else if (total > 0)
         {
-            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kMost>), dim3(total), dim3(kThreads), 0, stream, a, tiles);
+            if (Most::kWaves != Four::kWaves)
+            {
+                total = BuildVarTiles(tiles, dstHost, first, count, Most::kTileW, Most::kTileH);
+            }
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kMost>), dim3(total), dim3(Most::kThreads), 0, stream, a, tiles);
             CheckLaunch("WarpVarShape");
         }
     }

@@ -299,6 +299,15 @@ def test_patches_per_wave_of_image_batches(cv, K, orc, gpu, n):
             np.testing.assert_array_equal(outs[i].plane_view(0, np.uint8, 3).cpu().numpy(), dev, err_msg=str((interp, border, i)))
 
 
+# 75 000 rows of tiles of the form whose blocks are one wave; at whole places a bicubic sum is the pixel itself
+def test_bicubic_of_a_tall_image(cv, orc, gpu):
+    src = orc.fill_u8((1, 600000, 16, 3), 91)
+    tin, tout = cv.Tensor.from_numpy(src, "NHWC"), cv.Tensor.alloc([1, 600000, 16, 3], np.uint8, "NHWC")
+    cv.WarpAffine(0)(None, tin, tout, [1.0, 0.0, 0.0, 0.0, 1.0, 0.0], CUBIC, 1, (0, 0, 0, 0))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(tout.numpy(), src)
+
+
 # the same for the other interpolations and borders, and for sources and results that are views: rows 4 bytes off a 16-byte
 # boundary in another pitch. A view's result is the dense one's, bit for bit
 @pytest.mark.parametrize("c", [3, 4])
