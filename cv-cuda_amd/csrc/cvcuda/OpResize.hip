@@ -2278,27 +2278,47 @@ __host__ __device__ __forceinline__ bool PairsFormScale(int srcW, int dstW)
 
 constexpr int kPairsTileW = 128, kPairsTileH = 8; // image batches: block = 4 waves of 128 columns x 2 rows, stacked
 
-// The tile (in units of a wave's tile) of this wave in a launch of the tensor kernels below: a block's waves lie side by
-// side (flat) or are stacked. Flat, a block writes few long row pieces instead of many short ones, which the memory
-// likes better when the launch is bound by it (32 x u8x3, the two shapes alternating on one machine: 720p -> 1080p
-// bilinear 67.3 -> 65.1 us, nearest 58.0 -> 55.4 us; 1080p -> 720p box filter 61.5 -> 59.6 us, bilinear 51.4 -> 51.2 us).
-// Rows much shorter than a flat block's span leave most of its waves without columns, and on small images the rows of a
-// stacked block share source rows in the L1, so the host chooses flat blocks for rows of 1024 pixels and more that fill their blocks to 80 %
-// (FlatBlocks). The bicubic walk has a line of its own (LaunchTensor): rows of any length that fill their blocks.
+// The tile (in units of a wave's tile) of this wave in a launch of the tensor kernels below. Counted along the rows of tiles, a block
+// writes and reads few long row pieces instead of many short ones, which the memory likes better, and no wave of a block stands
+// outside the image, as where a block's four waves stood side by side (rows of 1024 pixels and more) or below one another. us
+// as they stood / counted along the rows: bicubic u8x3 182 x 219 x 77 -> 593 x 209 41.6 / 28.7, 101 x 241 x 274 -> 572 x 655 56.3 / 42.9, 40 x 300 x 300 -> 600 x
+// 600 24.6 / 21.8, 32 x 720p -> 1080p 90.1 / 86.4; u8x4 40 x 300 x 300 -> 600 x 600 22.7 / 20.5; nearest neighbour u8x4 200 x 86 x 80 -> 307 x 287 22.5 / 18.3,
+// u8x3 50 x 209 x 770 -> 362 x 1335 25.2 / 19.5; box filter u8x3 4 x 3146 x 1185 -> 1646 x 620 25.5 / 20.6, u8x1 171 x 1723 x 388 -> 609 x 137 65.7 / 57.3; wave
+// patches, bilinear u8x3 193 x 171 x 925 -> 68 x 367 30.9 / 26.9, u8x4 12 x 702 x 2707 -> 466 x 1447 26.5 / 22.7. The bilinear strips of 8-bit pixels
+// alone lose by it where rows are short (u8x3 80 x 650 x 104 -> 1274 x 195 24.0 / 29.5, u8x4 190 x 307 x 16 -> 942 x 50 14.9 / 16.7): they count along rows of
+// 1024 pixels and more that fill blocks to 80 % (FlatBlocks) and stand below one another otherwise.
 struct WaveTile
 {
     int x, y;
 };
 
-__device__ __forceinline__ WaveTile WaveTileOf(int flat)
+// How the waves of a launch are counted: along the rows of tiles, `across` of them in a row, wherever a block ends; across = 0:
+// a block's waves stand below one another.
+struct WaveOrder
 {
-    // (arithmetic, not a branch: behind a branch on `flat` the compiler loads the kernel's other arguments only after
+    uint32_t across, magic; // magic: 2^32 / across and a little more (0: across is 1), exact up to 2^32 / across waves
+};
+
+__device__ __forceinline__ WaveTile WaveTileOf(const WaveOrder &order)
+{
+    // (arithmetic, not a branch: behind a branch the compiler loads the kernel's other arguments only after
     // that test, one more round trip to memory before a wave's first pixel load, 0.3 us on the 4 - 6 us launches of small
     // batches)
     // (the wave's number as a scalar: tile origins, row terms and loop counters then stay on the scalar unit)
-    const int waves = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), f = flat != 0;
-    const int across = f * (waves - 1) + 1, down = waves + 1 - across; // flat: waves, 1; stacked: 1, waves
-    return WaveTile{(int)blockIdx.x * across + wave * f, (int)blockIdx.y * down + wave * (1 - f)};
+    const uint32_t waves = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t along = blockIdx.x * waves + wave, row = order.magic == 0 ? along : __umulhi(along, order.magic);
+    const bool     stacked = order.across == 0;
+    return WaveTile{(int)(stacked ? blockIdx.x : along - row * order.across), (int)(stacked ? blockIdx.y * waves + wave : row)};
+}
+
+static inline WaveOrder AlongRows(int dstW, int dstH, int waveW, int waveH)
+{
+    const int64_t across = DivUp(dstW, waveW), down = DivUp(dstH, waveH);
+    if (across * across * down >= (int64_t)1 << 32)
+    {
+        return {0, 0};
+    }
+    return {(uint32_t)across, across == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)across + 1)};
 }
 
 static inline bool FlatBlocks(int dstW, int waveW)
@@ -2308,42 +2328,43 @@ static inline bool FlatBlocks(int dstW, int waveW)
 }
 
 // Grid of a launch of four-wave blocks whose waves own tiles of waveW x waveH.
-static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH, bool flat, int waves = 4)
+static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH, const WaveOrder &order, int waves = 4)
 {
-    return flat ? dim3(DivUp(dstW, waves * waveW), DivUp(dstH, waveH), N) : dim3(DivUp(dstW, waveW), DivUp(dstH, waves * waveH), N);
+    return order.across != 0 ? dim3((unsigned)(((int64_t)order.across * DivUp(dstH, waveH) + waves - 1) / waves), 1, N)
+                             : dim3(DivUp(dstW, waveW), DivUp(dstH, waves * waveH), N);
 }
 
 template<int C, int R>
-__global__ __launch_bounds__(256) void ResizeLinearPairsU8Kernel(const ResizeArgs a, const int flat)
+__global__ __launch_bounds__(256) void ResizeLinearPairsU8Kernel(const ResizeArgs a, const WaveOrder order)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeLinearPairStripU8<C, R>(p, t.x * kPairsTileW, t.y * R);
 }
 
 constexpr int kQuadsTileW = 256; // a wave's columns; tensors: block = 4 waves side by side (1024 columns x a strip's rows)
 
 template<int C, int R>
-__global__ __launch_bounds__(256) void ResizeLinearQuadsU8Kernel(const ResizeArgs a, const int flat)
+__global__ __launch_bounds__(256) void ResizeLinearQuadsU8Kernel(const ResizeArgs a, const WaveOrder order)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeLinearQuadStripU8<C, R>(p, t.x * kQuadsTileW, t.y * R);
 }
 
 template<int C, int R>
-__global__ __launch_bounds__(256) void ResizeNearestQuadsU8Kernel(const ResizeArgs a, const int flat)
+__global__ __launch_bounds__(256) void ResizeNearestQuadsU8Kernel(const ResizeArgs a, const WaveOrder order)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeNearestQuadStripU8<C, R>(p, t.x * kQuadsTileW, t.y * R);
 }
 
 template<int C, int DWORDS>
-__global__ __launch_bounds__(256) void ResizeNearestRowsU8Kernel(const ResizeArgs a, const int flat)
+__global__ __launch_bounds__(256) void ResizeNearestRowsU8Kernel(const ResizeArgs a, const WaveOrder order)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeNearestRowsU8<C, DWORDS>(p, t.x * kQuadsTileW, t.y * kNearestRows);
 }
 
@@ -2467,11 +2488,11 @@ __global__ __launch_bounds__(256) void ResizeNearestStripsU8VarShapeKernel(const
 constexpr int kPatchTileW = 64, kPatchTileH = 16; // block = 4 waves stacked vertically
 
 template<class T, int C, int INTERP, bool ODD>
-__global__ __launch_bounds__(256) void ResizePatchTensorKernel(const ResizeArgs a, const int flat)
+__global__ __launch_bounds__(256) void ResizePatchTensorKernel(const ResizeArgs a, const WaveOrder order)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
     // blocks are 4 waves, or single waves when the whole launch is small
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeWavePatch<T, C, INTERP, false, ODD>(p, t.x * kPatchTileW, t.y * 4);
 }
 
@@ -2782,10 +2803,10 @@ __device__ __forceinline__ void ResizeCubicWalkU8(const Plane &p, int x0, int y0
 }
 
 template<int C, int LOADS, bool ODD>
-__global__ __launch_bounds__(256) void ResizeCubicWalkU8Kernel(const ResizeArgs a, const int rows, const int flat)
+__global__ __launch_bounds__(256) void ResizeCubicWalkU8Kernel(const ResizeArgs a, const int rows, const WaveOrder order)
 {
     const Plane    p = GetPlanes<false>(a, blockIdx.z);
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeCubicWalkU8<C, LOADS, ODD>(p, t.x * kCubicWalkW<C>, t.y * rows, rows);
 }
 
@@ -3147,10 +3168,10 @@ __device__ __forceinline__ void ResizeAreaPlainWaveTile(const Plane &p, int x0, 
 }
 
 template<int C, bool ODD>
-__global__ __launch_bounds__(256) void ResizeAreaFixedTensorKernel(const ResizeArgs a, const int rows, const int flat)
+__global__ __launch_bounds__(256) void ResizeAreaFixedTensorKernel(const ResizeArgs a, const int rows, const WaveOrder order)
 {
     const Plane p = GetPlanes<false>(a, blockIdx.z);
-    const WaveTile t = WaveTileOf(flat);
+    const WaveTile t = WaveTileOf(order);
     ResizeAreaFixedWaveTile<C, ODD>(p, t.x * kAreaTileW, t.y * rows, rows);
 }
 
@@ -4046,7 +4067,6 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     if constexpr (std::is_same_v<T, uint8_t> && INTERP == NVCV_INTERP_NEAREST && (C == 1 || C == 3 || C == 4))
     {
         const int64_t strips = (int64_t)DivUp(a.dstW, kQuadsTileW) * DivUp(a.dstH, kStripRows) * N;
-        const bool    flat   = FlatBlocks(a.dstW, kQuadsTileW);
         // Enlarged by less than 1.5 the patches, whose waves are a quarter as wide, are the faster form until the chip is full (us as
         // patches / so: 18 x 2140 x 137 x 1 -> 1089 x 98 4.2 / 5.0, 30 x 1219 x 75 x 1 -> 1201 x 78 4.4 / 5.0, 105 x 465 x 40 x 3 -> 576 x 50 5.3 / 6.9) and where most of a wave's 256 columns do not
         // exist (159 x 146 x 685 x 3 -> 53 x 361 9.7 / 13.8, 65 x 50 x 951 x 3 -> 64 x 1214 6.3 / 9.5; half of them, 18 x 514 x 1146 x 3 -> 558 x 1426, 22.0 / 17.4). 9 x 2475 x
@@ -4061,8 +4081,9 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             // source row is fewer than three output rows (3 x 1336 x 1189 -> 3870 x 3444 13.4 / 15.5, 23 x 41 x 1275 -> 122 x 3819 9.3 / 10.5).
             const bool many   = 5 * (int64_t)a.dstH >= 11 * (int64_t)a.srcH ? strips >= 24 * 256 : strips >= 60 * 256 && a.dstRowStride % 64 == 0;
             const int  rows   = C == 1 && many ? kStripRows : 4;
+            const auto order  = AlongRows(a.dstW, a.dstH, kQuadsTileW, rows);
             auto       kernel = rows == 4 ? ResizeNearestQuadsU8Kernel<C, 4> : ResizeNearestQuadsU8Kernel<C, C == 1 ? kStripRows : 4>;
-            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, order), dim3(256), 0, stream, a, order);
             CheckLaunch("ResizeNearestQuadsU8Kernel");
             return;
         }
@@ -4072,9 +4093,10 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             {
                 // (a lane's 4 columns lie within 4 pixels of one channel more than the first one up to a scale of 4 / 3, 12 up to 4; within 3 of
                 // three channels up to 1. Three channels reduced across, each pixel a load of its own: 143 launches from 0.83 to 1.27 of the patches' time)
+                const auto order = AlongRows(a.dstW, a.dstH, kQuadsTileW, kNearestRows);
                 auto kernel = C == 1 && 3 * (int64_t)a.srcW <= 4 * (int64_t)a.dstW ? ResizeNearestRowsU8Kernel<C, C == 1 ? 2 : 4>
                                                                                    : ResizeNearestRowsU8Kernel<C, 4>;
-                hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, kNearestRows, flat), dim3(256), 0, stream, a, (int)flat);
+                hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, kNearestRows, order), dim3(256), 0, stream, a, order);
                 CheckLaunch("ResizeNearestRowsU8Kernel");
                 return;
             }
@@ -4089,13 +4111,13 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             // 448 8.2 / 6.6 / 5.2; 720p -> 1080p 8.8 / 6.9 / 7.2; 16 x 320 x 240 -> 640 x 480 11.4 / 11.2 / 11.2), from there on the
             // source rows that strips share and their column terms count (32 x 224 x 224 -> 448 x 448 12.2 / 13.0 / 13.2; one channel,
             // 8 x 720p -> 1080p 12.6 / 13.5 / 15.5).
-            const bool    flat   = FlatBlocks(a.dstW, kQuadsTileW);
             const int64_t strips = (int64_t)DivUp(a.dstW, kQuadsTileW) * DivUp(a.dstH, kStripRows) * N;
             const int     rows   = strips <= 3 * 256 ? 2 : strips <= 12 * 256 ? 4 : kStripRows;
+            const auto    order  = FlatBlocks(a.dstW, kQuadsTileW) ? AlongRows(a.dstW, a.dstH, kQuadsTileW, rows) : WaveOrder{};
             auto          kernel = rows == 2   ? ResizeLinearQuadsU8Kernel<C, 2>
                                    : rows == 4 ? ResizeLinearQuadsU8Kernel<C, 4>
                                                : ResizeLinearQuadsU8Kernel<C, kStripRows>;
-            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kQuadsTileW, rows, order), dim3(256), 0, stream, a, order);
             CheckLaunch("ResizeLinearQuadsU8Kernel");
             return;
         }
@@ -4104,11 +4126,11 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             // Shorter strips while waves are few, as above (us with 4 / 2 rows, three channels: 720p -> 640 x 360 4.0 / 3.3; 15 x
             // 1136 x 166 -> 680 x 99 6.3 / 5.3; 32 x 256 x 256 -> 224 x 224 6.5 / 6.2, 64 of these 9.0 / 9.4; one channel, 4 x 720p ->
             // 960 x 540 5.0 / 5.0, 16 of these 11.2 / 12.5).
-            const bool    flat   = FlatBlocks(a.dstW, kPairsTileW);
             const int64_t strips = (int64_t)DivUp(a.dstW, kPairsTileW) * DivUp(a.dstH, kPairStripRows) * N;
             const int     rows   = strips <= 16 * 256 ? 2 : kPairStripRows;
+            const auto    order  = FlatBlocks(a.dstW, kPairsTileW) ? AlongRows(a.dstW, a.dstH, kPairsTileW, rows) : WaveOrder{};
             auto          kernel = rows == 2 ? ResizeLinearPairsU8Kernel<C, 2> : ResizeLinearPairsU8Kernel<C, kPairStripRows>;
-            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPairsTileW, rows, flat), dim3(256), 0, stream, a, (int)flat);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPairsTileW, rows, order), dim3(256), 0, stream, a, order);
             CheckLaunch("ResizeLinearPairsU8Kernel");
             return;
         }
@@ -4117,10 +4139,10 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         if (AreaFixedDomain(a.scaleX, a.scaleY, a.srcW * C, a.srcH))
         {
-            const bool flat = FlatBlocks(a.dstW, kAreaTileW);
             auto kernel = RowsAreOdd<C>(a) ? ResizeAreaFixedTensorKernel<C, C != 4> : ResizeAreaFixedTensorKernel<C, false>;
             const int rows = AreaRowsPerWave((int64_t)DivUp(a.dstW, kAreaTileW) * DivUp(a.dstH, kAreaRowsMost) * N);
-            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, rows, flat), dim3(256), 0, stream, a, rows, (int)flat);
+            const auto order = AlongRows(a.dstW, a.dstH, kAreaTileW, rows);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kAreaTileW, rows, order), dim3(256), 0, stream, a, rows, order);
             CheckLaunch("ResizeAreaFixedTensorKernel");
             return;
         }
@@ -4186,13 +4208,11 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             rows     = waves(8) >= (C == 1 ? 6 : C == 4 && over2 ? 8 : reducing ? 16 : 10) * 256 ? 8 : rows;
             rows     = waves(16) >= (C == 3 ? 20 : 16) * 256 ? 16 : rows;
             rows     = waves(32) >= 64 * 256 && a.dstH > a.srcH && a.dstRowStride % 64 == 0 ? 32 : rows;
-            // Side by side wherever that leaves few waves without columns: rows that end in the middle of a line of memory want
-            // their neighbour soon (the same, stacked / side by side: 114 / 74; 8 x 1080p x 4 -> 640 x 360 15.5 / 13.8).
-            const bool    flat = DivUp(a.dstW, 4 * tileW) * (int64_t)(4 * tileW) * 4 <= (int64_t)a.dstW * 5;
+            const auto    order = AlongRows(a.dstW, a.dstH, tileW, rows);
             constexpr int kTwo = C == 1 ? 2 : 1;
             auto kernel = C == 1 ? (10 * (int64_t)a.srcW <= 13 * (int64_t)a.dstW ? ResizeCubicWalkU8Kernel<C, 1, false> : ResizeCubicWalkU8Kernel<C, kTwo, false>)
                                  : (RowsAreOdd<C>(a) ? ResizeCubicWalkU8Kernel<C, 1, C == 3> : ResizeCubicWalkU8Kernel<C, 1, false>);
-            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, tileW, rows, flat), dim3(256), 0, stream, a, rows, (int)flat);
+            hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, tileW, rows, order), dim3(256), 0, stream, a, rows, order);
             CheckLaunch("ResizeCubicWalkU8Kernel");
             return;
         }
@@ -4229,11 +4249,11 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         // and finishes sooner the more CUs take part
         const int64_t blocks = (int64_t)DivUp(a.dstW, kPatchTileW) * DivUp(a.dstH, kPatchTileH) * N;
         const int     waves  = blocks < 8 * 256 ? 1 : 4;
-        const bool    flat   = waves == 4 && FlatBlocks(a.dstW, kPatchTileW);
+        const auto    order  = AlongRows(a.dstW, a.dstH, kPatchTileW, 4);
         constexpr bool kOdd   = INTERP == NVCV_INTERP_CUBIC && kFixedCubic<T> && C != 4;
         auto           kernel = kOdd && RowsAreOdd<C>(a) ? ResizePatchTensorKernel<T, C, INTERP, kOdd> : ResizePatchTensorKernel<T, C, INTERP, false>;
-        hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, 4, flat, waves),
-                           dim3(64 * waves), 0, stream, a, (int)flat);
+        hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, 4, order, waves),
+                           dim3(64 * waves), 0, stream, a, order);
         CheckLaunch("ResizePatchTensorKernel");
         return;
     }
