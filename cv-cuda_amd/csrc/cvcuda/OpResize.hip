@@ -835,12 +835,67 @@ __device__ __forceinline__ void ResizePixel(const Plane &p, int dx, int dy)
     StorePx<T, C>(p.dst + (int64_t)dy * p.dstRow, dx, ResizeValue<T, C, INTERP, VARSHAPE>(p, dx, dy));
 }
 
-template<class T, int C, int INTERP>
-__global__ __launch_bounds__(256) void ResizeTensorKernel(const ResizeArgs a, const int flat)
+// The tile (in units of a wave's tile) of this wave in a launch of the tensor kernels below. Counted along the rows of tiles, a block
+// writes and reads few long row pieces instead of many short ones, which the memory likes better, and no wave of a block stands
+// outside the image, as where a block's four waves stood side by side (rows of 1024 pixels and more) or below one another. us
+// as they stood / counted along the rows: bicubic u8x3 182 x 219 x 77 -> 593 x 209 41.6 / 28.7, 101 x 241 x 274 -> 572 x 655 56.3 / 42.9, 40 x 300 x 300 -> 600 x
+// 600 24.6 / 21.8, 32 x 720p -> 1080p 90.1 / 86.4; u8x4 40 x 300 x 300 -> 600 x 600 22.7 / 20.5; nearest neighbour u8x4 200 x 86 x 80 -> 307 x 287 22.5 / 18.3,
+// u8x3 50 x 209 x 770 -> 362 x 1335 25.2 / 19.5; box filter u8x3 4 x 3146 x 1185 -> 1646 x 620 25.5 / 20.6, u8x1 171 x 1723 x 388 -> 609 x 137 65.7 / 57.3; wave
+// patches, bilinear u8x3 193 x 171 x 925 -> 68 x 367 30.9 / 26.9, u8x4 12 x 702 x 2707 -> 466 x 1447 26.5 / 22.7. The bilinear strips of 8-bit pixels
+// alone lose by it where rows are short (u8x3 80 x 650 x 104 -> 1274 x 195 24.0 / 29.5, u8x4 190 x 307 x 16 -> 942 x 50 14.9 / 16.7): they count along rows of
+// 1024 pixels and more that fill blocks to 80 % (FlatBlocks) and stand below one another otherwise.
+struct WaveTile
 {
-    // a block is 64 columns x 4 rows, or (flat) its four waves side by side on one row
-    const int dx = flat ? blockIdx.x * (kTileW * kTileH) + threadIdx.x : blockIdx.x * kTileW + (threadIdx.x & 63);
-    const int dy = flat ? blockIdx.y : blockIdx.y * kTileH + (threadIdx.x >> 6);
+    int x, y;
+};
+
+// How the waves of a launch are counted: along the rows of tiles, `across` of them in a row, wherever a block ends; across = 0:
+// a block's waves stand below one another.
+struct WaveOrder
+{
+    uint32_t across, magic; // magic: 2^32 / across and a little more (0: across is 1), exact up to 2^32 / across waves
+};
+
+__device__ __forceinline__ WaveTile WaveTileOf(const WaveOrder &order)
+{
+    // (arithmetic, not a branch: behind a branch the compiler loads the kernel's other arguments only after
+    // that test, one more round trip to memory before a wave's first pixel load, 0.3 us on the 4 - 6 us launches of small
+    // batches)
+    // (the wave's number as a scalar: tile origins, row terms and loop counters then stay on the scalar unit)
+    const uint32_t waves = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t along = blockIdx.x * waves + wave, row = order.magic == 0 ? along : __umulhi(along, order.magic);
+    const bool     stacked = order.across == 0;
+    return WaveTile{(int)(stacked ? blockIdx.x : along - row * order.across), (int)(stacked ? blockIdx.y * waves + wave : row)};
+}
+
+static inline WaveOrder AlongRows(int dstW, int dstH, int waveW, int waveH)
+{
+    const int64_t across = DivUp(dstW, waveW), down = DivUp(dstH, waveH);
+    if (across * across * down >= (int64_t)1 << 32)
+    {
+        return {0, 0};
+    }
+    return {(uint32_t)across, across == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)across + 1)};
+}
+
+static inline bool FlatBlocks(int dstW, int waveW)
+{
+    const int64_t span = 4 * (int64_t)waveW;
+    return dstW >= 1024 && DivUp(dstW, (int)span) * span * 4 <= (int64_t)dstW * 5;
+}
+
+// Grid of a launch of four-wave blocks whose waves own tiles of waveW x waveH.
+static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH, const WaveOrder &order, int waves = 4)
+{
+    return order.across != 0 ? dim3((unsigned)(((int64_t)order.across * DivUp(dstH, waveH) + waves - 1) / waves), 1, N)
+                             : dim3(DivUp(dstW, waveW), DivUp(dstH, waves * waveH), N);
+}
+
+template<class T, int C, int INTERP>
+__global__ __launch_bounds__(256) void ResizeTensorKernel(const ResizeArgs a, const WaveOrder order)
+{
+    const WaveTile t  = WaveTileOf(order);
+    const int      dx = t.x * kTileW + (threadIdx.x & 63), dy = t.y;
     if (dx >= a.dstW || dy >= a.dstH)
     {
         return;
@@ -2277,62 +2332,6 @@ __host__ __device__ __forceinline__ bool PairsFormScale(int srcW, int dstW)
 }
 
 constexpr int kPairsTileW = 128, kPairsTileH = 8; // image batches: block = 4 waves of 128 columns x 2 rows, stacked
-
-// The tile (in units of a wave's tile) of this wave in a launch of the tensor kernels below. Counted along the rows of tiles, a block
-// writes and reads few long row pieces instead of many short ones, which the memory likes better, and no wave of a block stands
-// outside the image, as where a block's four waves stood side by side (rows of 1024 pixels and more) or below one another. us
-// as they stood / counted along the rows: bicubic u8x3 182 x 219 x 77 -> 593 x 209 41.6 / 28.7, 101 x 241 x 274 -> 572 x 655 56.3 / 42.9, 40 x 300 x 300 -> 600 x
-// 600 24.6 / 21.8, 32 x 720p -> 1080p 90.1 / 86.4; u8x4 40 x 300 x 300 -> 600 x 600 22.7 / 20.5; nearest neighbour u8x4 200 x 86 x 80 -> 307 x 287 22.5 / 18.3,
-// u8x3 50 x 209 x 770 -> 362 x 1335 25.2 / 19.5; box filter u8x3 4 x 3146 x 1185 -> 1646 x 620 25.5 / 20.6, u8x1 171 x 1723 x 388 -> 609 x 137 65.7 / 57.3; wave
-// patches, bilinear u8x3 193 x 171 x 925 -> 68 x 367 30.9 / 26.9, u8x4 12 x 702 x 2707 -> 466 x 1447 26.5 / 22.7. The bilinear strips of 8-bit pixels
-// alone lose by it where rows are short (u8x3 80 x 650 x 104 -> 1274 x 195 24.0 / 29.5, u8x4 190 x 307 x 16 -> 942 x 50 14.9 / 16.7): they count along rows of
-// 1024 pixels and more that fill blocks to 80 % (FlatBlocks) and stand below one another otherwise.
-struct WaveTile
-{
-    int x, y;
-};
-
-// How the waves of a launch are counted: along the rows of tiles, `across` of them in a row, wherever a block ends; across = 0:
-// a block's waves stand below one another.
-struct WaveOrder
-{
-    uint32_t across, magic; // magic: 2^32 / across and a little more (0: across is 1), exact up to 2^32 / across waves
-};
-
-__device__ __forceinline__ WaveTile WaveTileOf(const WaveOrder &order)
-{
-    // (arithmetic, not a branch: behind a branch the compiler loads the kernel's other arguments only after
-    // that test, one more round trip to memory before a wave's first pixel load, 0.3 us on the 4 - 6 us launches of small
-    // batches)
-    // (the wave's number as a scalar: tile origins, row terms and loop counters then stay on the scalar unit)
-    const uint32_t waves = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t along = blockIdx.x * waves + wave, row = order.magic == 0 ? along : __umulhi(along, order.magic);
-    const bool     stacked = order.across == 0;
-    return WaveTile{(int)(stacked ? blockIdx.x : along - row * order.across), (int)(stacked ? blockIdx.y * waves + wave : row)};
-}
-
-static inline WaveOrder AlongRows(int dstW, int dstH, int waveW, int waveH)
-{
-    const int64_t across = DivUp(dstW, waveW), down = DivUp(dstH, waveH);
-    if (across * across * down >= (int64_t)1 << 32)
-    {
-        return {0, 0};
-    }
-    return {(uint32_t)across, across == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)across + 1)};
-}
-
-static inline bool FlatBlocks(int dstW, int waveW)
-{
-    const int64_t span = 4 * (int64_t)waveW;
-    return dstW >= 1024 && DivUp(dstW, (int)span) * span * 4 <= (int64_t)dstW * 5;
-}
-
-// Grid of a launch of four-wave blocks whose waves own tiles of waveW x waveH.
-static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH, const WaveOrder &order, int waves = 4)
-{
-    return order.across != 0 ? dim3((unsigned)(((int64_t)order.across * DivUp(dstH, waveH) + waves - 1) / waves), 1, N)
-                             : dim3(DivUp(dstW, waveW), DivUp(dstH, waves * waveH), N);
-}
 
 template<int C, int R>
 __global__ __launch_bounds__(256) void ResizeLinearPairsU8Kernel(const ResizeArgs a, const WaveOrder order)
@@ -3782,15 +3781,15 @@ AreaFloatKernelPtr AreaFloatKernel(int pieces)
 // f32x3 -> 1931 x 1081 64.9 -> 36.5 us (4.6 TB/s), -> 1200 x 700 27.3 -> 17.5, -> 963 x 541 19.6 -> 15.9; 2 x f32x4 -> 1280 x
 // 960 21.6 -> 14.4; 12 x f32x1 -> 1931 x 1081 67.3 -> 51.7 (its writes: rows that start at no sector).
 template<int C>
-__global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArgs a, const int rows)
+__global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArgs a, const int rows, const WaveOrder order)
 {
     struct Taps
     {
         Pixel<float, C> px[4];
     };
     const Plane p    = GetPlanes<false>(a, blockIdx.z);
-    const int   lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int   dx = blockIdx.x * kTileW + lane, y0 = (blockIdx.y * 4 + wave) * rows;
+    const WaveTile tile = WaveTileOf(order);
+    const int   lane = threadIdx.x & 63, dx = tile.x * kTileW + lane, y0 = tile.y * rows;
     if (y0 >= p.dstH)
     {
         return;
@@ -4055,8 +4054,12 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             const bool enlarging = a.srcH <= a.dstH, few = waves(8) <= 18 * 256 && (C == 1 || enlarging);
             const bool soon      = 5 * (int64_t)a.srcH <= 4 * (int64_t)a.dstH && a.dstRowStride % 64 != 0;
             const int  rows      = waves(4) <= 30 * 256 ? 4 : few || soon ? 8 : 16;
-            hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), dim3(DivUp(a.dstW, kTileW), DivUp(a.dstH, 4 * rows), N), dim3(256), 0, stream, a,
-                               rows);
+            // (along the rows where the chip is full, below one another, where rows share sources in the L1, before: one channel, 44 x 237 x 1008 -> 182 x
+            // 962 30.2 -> 21.6, 65 x 569 x 51 -> 1915 x 128 26.4 -> 20.3; three, 11 x 793 x 146 -> 2918 x 454 54.8 -> 46.5, but 1 x 392 x 1105 -> 556 x 1567, 3528
+            // waves of 4 rows, 6.4 and 7.3; four 44 x 286 x 59 -> 1071 x 223 48.6 and 42.5, but 128 x 104 x 88 -> 106 x 90 9.7 and 11.5)
+            const auto order     = C != 4 && rows > 4 ? AlongRows(a.dstW, a.dstH, kTileW, rows) : WaveOrder{};
+            hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kTileW, rows, order), dim3(256), 0, stream, a,
+                               rows, order);
             CheckLaunch("ResizeCubicStripF32Kernel");
             return;
         }
@@ -4261,9 +4264,17 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     // f32x3 bilinear 56.4 -> 45.5 us, f32x4 68.1 -> 56.3 us); reducing, it is the reads, and the four rows of the
     // 64 x 4 block share source rows (1080p -> 720p f32x3 bilinear 41.1 us against 49.3 us flat).
     // (bicubic keeps the 64 x 4 block: its time is the arithmetic's and did not change with the block)
-    const int flat = INTERP != NVCV_INTERP_CUBIC && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);
-    hipLaunchKernelGGL((ResizeTensorKernel<T, C, INTERP>), flat ? dim3(DivUp(a.dstW, kTileW * kTileH), a.dstH, N) : grid, dim3(256), 0, stream,
-                       a, flat);
+    // (nearest neighbour shares no source rows but with itself: 76 x 107 x 227 f32x3 -> 66 x 140 6.9 -> 5.6 us, 65 x 80 x 82 -> 307 x 314 18.5 -> 15.4, 104 x
+    // 46 x 743 f32x4 -> 65 x 1048 36.8 -> 31.1. Bilinear rows share theirs with the next one below a vertical scale of 2: 20 x 722 x 418 f32x3 -> 836 x
+    // 484 33.9 us in the 64 x 4 block and 40.7 along the rows, 12 x 399 x 367 f32x4 -> 534 x 492 14.9 and 19.2; at 2.8, 121 x 194 x 594 f32x3 -> 69 x 211,
+    // 31.2 and 25.4)
+    // Enlarged rows of 1024 pixels and more start with a block: 1 x 1716 x 858 f32x4 -> 1852 x 926 10.3 us so and 11.7 along the rows.
+    const bool along = INTERP == NVCV_INTERP_NEAREST || (INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH);
+    const bool flat  = INTERP != NVCV_INTERP_CUBIC && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);
+    const auto order = along ? AlongRows(a.dstW, a.dstH, kTileW, 1)
+                     : flat  ? AlongRows(DivUp(a.dstW, 4 * kTileW) * 4 * kTileW, a.dstH, kTileW, 1)
+                             : WaveOrder{};
+    hipLaunchKernelGGL((ResizeTensorKernel<T, C, INTERP>), WaveTileGrid(a.dstW, a.dstH, N, kTileW, 1, order), dim3(256), 0, stream, a, order);
     CheckLaunch("ResizeTensorKernel");
 }
 
