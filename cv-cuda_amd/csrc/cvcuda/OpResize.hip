@@ -2341,7 +2341,7 @@ __global__ __launch_bounds__(256) void ResizeLinearPairsU8Kernel(const ResizeArg
     ResizeLinearPairStripU8<C, R>(p, t.x * kPairsTileW, t.y * R);
 }
 
-constexpr int kQuadsTileW = 256; // a wave's columns; tensors: block = 4 waves side by side (1024 columns x a strip's rows)
+constexpr int kQuadsTileW = 256; // a wave's columns; where a block's waves stand: WaveTileOf
 
 template<int C, int R>
 __global__ __launch_bounds__(256) void ResizeLinearQuadsU8Kernel(const ResizeArgs a, const WaveOrder order)
@@ -2859,7 +2859,7 @@ template<class T, int C, int INTERP>
 constexpr bool kAreaFixed = std::is_same_v<T, uint8_t> && INTERP == NVCV_INTERP_AREA && (C == 1 || C == 3 || C == 4);
 
 constexpr int kAreaRowsMost = 16; // output rows per wave: 4, 8 or 16
-constexpr int kAreaTileW = 64;    // image batches: block = 4 waves stacked vertically; tensors: side by side
+constexpr int kAreaTileW = 64;    // image batches: block = 4 waves stacked vertically; tensors: along the rows (WaveTileOf)
 
 // Rows per wave, given the launch's waves of 16. A wave's steps of 4 rows follow one another, so a launch that does not fill
 // the chip takes as long as one wave: fewer steps each until there are enough of them. us with 16 / 8 / 4 rows, three
