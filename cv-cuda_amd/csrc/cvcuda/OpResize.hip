@@ -37,6 +37,7 @@
 #include "OpCommon.hpp"
 #include "RunIO.hpp"
 #include "VarShapeTiles.hpp"
+#include "WaveOrder.hpp"
 
 #include <cvcuda/OpResize.h>
 
@@ -844,38 +845,10 @@ __device__ __forceinline__ void ResizePixel(const Plane &p, int dx, int dy)
 // patches, bilinear u8x3 193 x 171 x 925 -> 68 x 367 30.9 / 26.9, u8x4 12 x 702 x 2707 -> 466 x 1447 26.5 / 22.7. The bilinear strips of 8-bit pixels
 // alone lose by it where rows are short (u8x3 80 x 650 x 104 -> 1274 x 195 24.0 / 29.5, u8x4 190 x 307 x 16 -> 942 x 50 14.9 / 16.7): they count along rows of
 // 1024 pixels and more that fill blocks to 80 % (FlatBlocks) and stand below one another otherwise.
-struct WaveTile
-{
-    int x, y;
-};
-
-// How the waves of a launch are counted: along the rows of tiles, `across` of them in a row, wherever a block ends; across = 0:
-// a block's waves stand below one another.
-struct WaveOrder
-{
-    uint32_t across, magic; // magic: 2^32 / across and a little more (0: across is 1), exact up to 2^32 / across waves
-};
-
 __device__ __forceinline__ WaveTile WaveTileOf(const WaveOrder &order)
 {
-    // (arithmetic, not a branch: behind a branch the compiler loads the kernel's other arguments only after
-    // that test, one more round trip to memory before a wave's first pixel load, 0.3 us on the 4 - 6 us launches of small
-    // batches)
     // (the wave's number as a scalar: tile origins, row terms and loop counters then stay on the scalar unit)
-    const uint32_t waves = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t along = blockIdx.x * waves + wave, row = order.magic == 0 ? along : __umulhi(along, order.magic);
-    const bool     stacked = order.across == 0;
-    return WaveTile{(int)(stacked ? blockIdx.x : along - row * order.across), (int)(stacked ? blockIdx.y * waves + wave : row)};
-}
-
-static inline WaveOrder AlongRows(int dstW, int dstH, int waveW, int waveH)
-{
-    const int64_t across = DivUp(dstW, waveW), down = DivUp(dstH, waveH);
-    if (across * across * down >= (int64_t)1 << 32)
-    {
-        return {0, 0};
-    }
-    return {(uint32_t)across, across == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)across + 1)};
+    return TileOfWave(order, blockIdx.x, blockIdx.y, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockDim.x >> 6);
 }
 
 static inline bool FlatBlocks(int dstW, int waveW)
@@ -884,11 +857,11 @@ static inline bool FlatBlocks(int dstW, int waveW)
     return dstW >= 1024 && DivUp(dstW, (int)span) * span * 4 <= (int64_t)dstW * 5;
 }
 
-// Grid of a launch of four-wave blocks whose waves own tiles of waveW x waveH.
+// Grid of a launch whose waves own tiles of waveW x waveH.
 static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH, const WaveOrder &order, int waves = 4)
 {
-    return order.across != 0 ? dim3((unsigned)(((int64_t)order.across * DivUp(dstH, waveH) + waves - 1) / waves), 1, N)
-                             : dim3(DivUp(dstW, waveW), DivUp(dstH, waves * waveH), N);
+    const WaveBlocks blocks = BlocksOfWaves(dstW, dstH, waveW, waveH, order, waves);
+    return dim3(blocks.x, blocks.y, N);
 }
 
 template<class T, int C, int INTERP>

@@ -1,0 +1,68 @@
+// Which tile of a tensor each wave of a launch works on. Plain arithmetic, the same on the host and the device.
+#ifndef CVCUDA_AMD_WAVEORDER_HPP
+#define CVCUDA_AMD_WAVEORDER_HPP
+
+#include <cstdint>
+
+namespace cvamd {
+
+struct WaveTile // in units of a wave's tile
+{
+    int x, y;
+};
+
+// How the waves of a launch are counted: along the rows of tiles, `across` of them in a row, wherever a block ends; across = 0:
+// a block's waves stand below one another.
+struct WaveOrder
+{
+    uint32_t across, magic; // magic: 2^32 / across and a little more (0: across is 1), exact up to 2^32 / across waves
+};
+
+constexpr int64_t TilesIn(int64_t size, int64_t tile)
+{
+    return (size + tile - 1) / tile;
+}
+
+// Whether `waves` waves, in blocks of up to four, fit the one dimension of a launch, which has less than 2^32 threads. (Of rows of one or
+// a few tiles there may be more: one column of 67.2 million 12-byte pixels.)
+constexpr bool WavesFitARow(int64_t waves)
+{
+    return (waves + 3) / 4 * 256 < (int64_t)1 << 32;
+}
+
+constexpr WaveOrder AlongRows(int dstW, int dstH, int waveW, int waveH)
+{
+    const int64_t across = TilesIn(dstW, waveW), down = TilesIn(dstH, waveH);
+    if (across * across * down >= (int64_t)1 << 32 || !WavesFitARow(across * down))
+    {
+        return WaveOrder{0, 0};
+    }
+    return WaveOrder{(uint32_t)across, across == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)across + 1)};
+}
+
+// The tile of wave `wave` of the `waves` in block (blockX, blockY).
+constexpr WaveTile TileOfWave(const WaveOrder &order, uint32_t blockX, uint32_t blockY, uint32_t wave, uint32_t waves)
+{
+    // (arithmetic, not a branch: behind a branch the compiler loads the kernel's other arguments only after
+    // that test, one more round trip to memory before a wave's first pixel load, 0.3 us on the 4 - 6 us launches of small
+    // batches)
+    const uint32_t along = blockX * waves + wave, row = order.magic == 0 ? along : (uint32_t)(((uint64_t)along * order.magic) >> 32);
+    const bool     stacked = order.across == 0;
+    return WaveTile{(int)(stacked ? blockX : along - row * order.across), (int)(stacked ? blockY * waves + wave : row)};
+}
+
+// The blocks of a launch whose waves own tiles of waveW x waveH, `waves` of them to a block.
+struct WaveBlocks
+{
+    uint32_t x, y;
+};
+
+constexpr WaveBlocks BlocksOfWaves(int dstW, int dstH, int waveW, int waveH, const WaveOrder &order, int waves)
+{
+    return order.across != 0 ? WaveBlocks{(uint32_t)TilesIn(order.across * TilesIn(dstH, waveH), waves), 1}
+                             : WaveBlocks{(uint32_t)TilesIn(dstW, waveW), (uint32_t)TilesIn(dstH, (int64_t)waves * waveH)};
+}
+
+} // namespace cvamd
+
+#endif // CVCUDA_AMD_WAVEORDER_HPP

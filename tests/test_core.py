@@ -584,6 +584,15 @@ def test_block_pool_of_the_default_allocator(tmp_path):
     assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "ok"
 
 
+def test_tiles_of_a_launchs_waves(tmp_path):
+    here = os.path.dirname(os.path.abspath(__file__))
+    exe = str(tmp_path / "wave_order_cases")
+    csrc = os.path.join(os.path.dirname(here), "cv-cuda_amd", "csrc", "cvcuda")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I" + csrc, os.path.join(here, "golden", "wave_order_cases.cpp"),
+                    "-o", exe], check=True)
+    assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "ok"
+
+
 def test_what_an_image_batch_uploads(tmp_path):
     # the device's lists follow the host's, and the room of a batch that is not full is not copied: the library's sources
     # over a stand-in for the HIP runtime

@@ -841,6 +841,16 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
     assert not torch.isnan(results[0]).any()
 
 
+# One column of more rows than one dimension of a launch has waves for
+def test_nearest_of_a_tall_image(cv, orc, gpu):
+    h   = 2 ** 26
+    src = np.ascontiguousarray(orc.fill_u8((1, 997, 1, 3), 17), np.float32)
+    tin, tout = cv.Tensor.from_numpy(src, "NHWC", row_align=1), cv.Tensor.alloc([1, h, 1, 3], np.float32, "NHWC", row_align=1)
+    cv.Resize()(None, tin, tout, NEAREST)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(tout.numpy(), orc.resize(src, (h, 1), NEAREST, variant=0))
+
+
 # Float bicubic reductions by 4 and more down, whose waves are counted along the rows: tiles of 64 columns that do not fill blocks of
 # four or rows, one wave in the last block, and each side of the scale of 4
 @pytest.mark.parametrize("row", [(sw, sh, dw, dh, CUBIC, n, np.float32, c)
