@@ -769,14 +769,43 @@ int OutputsInit(PyObject *self, PyObject *args, PyObject *)
     return o->free != nullptr ? 0 : -1;
 }
 
-void OutputsDealloc(PyObject *self)
+// (pyapi's dictionary holds the object that holds it: a copy of the package that nobody has any more goes by the collector)
+int OutputsTraverse(PyObject *self, visitproc visit, void *arg)
 {
-    auto         *o    = reinterpret_cast<Outputs *>(self);
-    PyTypeObject *type = Py_TYPE(self);
+    auto *o = reinterpret_cast<Outputs *>(self);
+    Py_VISIT(Py_TYPE(self));
+    Py_VISIT(o->api);
+    Py_VISIT(o->free);
+    return 0;
+}
+
+int OutputsCollect(PyObject *self)
+{
+    auto *o  = reinterpret_cast<Outputs *>(self);
+    o->bytes = o->count = 0;
     Py_CLEAR(o->free);
     Py_CLEAR(o->api);
+    return 0;
+}
+
+void OutputsDealloc(PyObject *self)
+{
+    PyTypeObject *type = Py_TYPE(self);
+    PyObject_GC_UnTrack(self);
+    (void)OutputsCollect(self);
     type->tp_free(self);
     Py_DECREF(type);
+}
+
+// Whether it has its tables: not before __init__, nor once the collector has taken them (an error is set).
+bool OutputsLive(const Outputs *o)
+{
+    if (o->api != nullptr && o->free != nullptr)
+    {
+        return true;
+    }
+    PyErr_SetString(PyExc_RuntimeError, "no tables of results");
+    return false;
 }
 
 // The tables as they were, with empty ones in their place (a new reference).
@@ -796,7 +825,11 @@ PyObject *OutputsTakeAll(Outputs *o)
 // clear(): gives everything held back to the allocator; False if there was nothing.
 PyObject *OutputsClear(PyObject *self, PyObject *)
 {
-    auto      *o    = reinterpret_cast<Outputs *>(self);
+    auto *o = reinterpret_cast<Outputs *>(self);
+    if (!OutputsLive(o))
+    {
+        return nullptr;
+    }
     const bool held = o->count != 0;
     Ref        all(OutputsTakeAll(o));
     return all ? PyBool_FromLong(held) : nullptr;
@@ -809,6 +842,10 @@ PyObject *OutputsGet(PyObject *self, PyObject *const *a, Py_ssize_t n)
     if (n != 3)
     {
         PyErr_SetString(PyExc_TypeError, "get(shape, dtype, layout)");
+        return nullptr;
+    }
+    if (!OutputsLive(o))
+    {
         return nullptr;
     }
     Ref       shape(PySequence_Tuple(a[0])); // (a tuple itself)
@@ -971,11 +1008,13 @@ PyMemberDef kOutputsMembers[] = {
 
 PyType_Slot kOutputsSlots[] = {
     {Py_tp_init, reinterpret_cast<void *>(OutputsInit)}, {Py_tp_dealloc, reinterpret_cast<void *>(OutputsDealloc)},
+    {Py_tp_traverse, reinterpret_cast<void *>(OutputsTraverse)}, {Py_tp_clear, reinterpret_cast<void *>(OutputsCollect)},
     {Py_tp_new, reinterpret_cast<void *>(PyType_GenericNew)}, {Py_tp_methods, kOutputsMethods},
     {Py_tp_members, kOutputsMembers}, {0, nullptr},
 };
 
-PyType_Spec kOutputsSpec = {"_cvcuda_native.Outputs", sizeof(Outputs), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE, kOutputsSlots};
+PyType_Spec kOutputsSpec = {"_cvcuda_native.Outputs", sizeof(Outputs), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC,
+                                  kOutputsSlots};
 
 PyMethodDef kBound[] = {
     {"submit", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Submit)), METH_FASTCALL, nullptr},

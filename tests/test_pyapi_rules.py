@@ -575,6 +575,39 @@ def test_kept_results_make_room_where_there_is_no_memory(api, monkeypatch):
     assert Raw.alive == outputs._count == outputs._bytes == 0
 
 
+def test_a_copy_of_the_package_that_nobody_has_is_collected(api):
+    # with the results that it kept, which belong to a table that holds the copy's names
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    program = """
+import gc, importlib, importlib.util, sys, weakref
+package = %r
+spec = importlib.util.spec_from_file_location("pkg", package + "/__init__.py", submodule_search_locations=[package])
+module = sys.modules["pkg"] = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(module)
+api = importlib.import_module("pkg.pyapi")
+class Raw:
+    _nbytes = 1
+    api = api
+result = api.Tensor(_wrap=Raw())
+result._key, result._wrote = ((1,), "u1", "N", 0), (0, None)
+result = None
+assert api._outputs._count == 1
+gone = [weakref.ref(o) for o in (module, api, api._outputs, api.Tensor, Raw)]
+for name in [n for n in sys.modules if n.split(".")[0] == "pkg"]:
+    del sys.modules[name]
+del spec, module, api, Raw
+gc.collect()
+assert [g() for g in gone] == [None] * 5, gone
+""" % os.path.join(root, "cv-cuda_amd")
+    r = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and not r.stderr, r.stderr
+    empty = api._native.Outputs.__new__(api._native.Outputs)  # without tables: not a crash
+    for call in (empty.clear, lambda: empty.get((1,), np.uint8, "N")):
+        with pytest.raises(RuntimeError):
+            call()
+    empty.put(api.Tensor(_wrap=object()))
+
+
 def test_results_alive_at_the_end_of_the_program_say_nothing():
     # a module's result tensors that outlive this package's module globals: nothing on stderr
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
