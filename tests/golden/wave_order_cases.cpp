@@ -21,6 +21,7 @@ static void EveryTileOnce(int w, int h, int tileW, int tileH, int waves, const W
 {
     const WaveBlocks blocks = BlocksOfWaves(w, h, tileW, tileH, order, waves);
     const int        across = (w + tileW - 1) / tileW, down = (h + tileH - 1) / tileH;
+    Check(order.across == 0 || blocks.x % 16 != 0, "blocks", w, h, tileW, tileH, waves);
     std::vector<int> seen((size_t)across * down);
     for (uint32_t y = 0; y < blocks.y; ++y)
     {
@@ -49,6 +50,7 @@ static void Ends(int w, int h, int tileW, int tileH, int waves, bool counted)
     const WaveOrder  order  = AlongRows(w, h, tileW, tileH);
     const WaveBlocks blocks = BlocksOfWaves(w, h, tileW, tileH, order, waves);
     Check((order.across != 0) == counted, "order", w, h, tileW, tileH, waves);
+    Check(order.across == 0 || blocks.x % 16 != 0, "blocks", w, h, tileW, tileH, waves);
     Check((uint64_t)blocks.x * 64 * (uint64_t)waves < (uint64_t)1 << 32, "threads", w, h, tileW, tileH, waves);
     if (order.across == 0)
     {
@@ -79,7 +81,7 @@ int main()
             {
                 for (int w : {1, 63, 64, 65, 129, 257, 1025, 1917, 4097})
                 {
-                    for (int h : {1, 3, 4, 5, 16, 17, 255})
+                    for (int h : {1, 3, 4, 5, 16, 17, 64, 255})
                     {
                         const WaveOrder order = AlongRows(w, h, tileW, tileH);
                         Check(order.across != 0, "order", w, h, tileW, tileH, waves);
@@ -89,8 +91,8 @@ int main()
                 }
             }
         }
-        // at the limits and one tile past them: 2^26 waves of at most 64 x 4 threads, and products of 2^32 beyond which the division is not exact
-        const int most = (1 << 26) - 4;
+        // at the limits and one tile past them: 2^26 waves with a block to spare, and products of 2^32 beyond which the division is not exact
+        const int most = (1 << 26) - 8;
         Ends(1, most, 64, 1, waves, true);
         Ends(1, most + 1, 64, 1, waves, false);
         Ends(64, 4 * most, 64, 4, waves, true);

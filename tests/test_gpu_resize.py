@@ -841,6 +841,17 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
     assert not torch.isnan(results[0]).any()
 
 
+# Images whose waves, counted along the rows, fill a multiple of 16 blocks, which get one more: in the forms that are counted so
+@pytest.mark.parametrize("row", [(300, 20, 1021, 64, NEAREST, 48, np.uint8, 3), (300, 20, 1021, 64, NEAREST, 48, np.uint8, 1),
+                                 (1100, 80, 1021, 64, NEAREST, 80, np.uint8, 1), (200, 50, 256, 64, CUBIC, 16, np.uint8, 3),
+                                 (200, 50, 256, 64, CUBIC, 16, np.uint8, 4), (600, 160, 256, 64, AREA, 3, np.uint8, 3),
+                                 (900, 200, 256, 64, LINEAR, 3, np.uint8, 1), (200, 12, 256, 16, NEAREST, 3, np.float32, 3),
+                                 (200, 100, 256, 128, CUBIC, 64, np.float32, 1), (700, 40, 256, 16, LINEAR, 3, np.float32, 4)],
+                         ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
+def test_tensors_of_16_blocks(cv, orc, gpu, row):
+    test_tensor_table(cv, orc, gpu, row)
+
+
 # One column of more rows than one dimension of a launch has waves for
 def test_nearest_of_a_tall_image(cv, orc, gpu):
     h   = 2 ** 26
