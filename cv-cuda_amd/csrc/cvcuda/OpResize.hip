@@ -4237,13 +4237,20 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     // f32x3 bilinear 56.4 -> 45.5 us, f32x4 68.1 -> 56.3 us); reducing, it is the reads, and the four rows of the
     // 64 x 4 block share source rows (1080p -> 720p f32x3 bilinear 41.1 us against 49.3 us flat).
     // (bicubic keeps the 64 x 4 block: its time is the arithmetic's and did not change with the block)
-    // (nearest neighbour shares no source rows but with itself: 76 x 107 x 227 f32x3 -> 66 x 140 6.9 -> 5.6 us, 65 x 80 x 82 -> 307 x 314 18.5 -> 15.4, 104 x
-    // 46 x 743 f32x4 -> 65 x 1048 36.8 -> 31.1. Bilinear rows share theirs with the next one below a vertical scale of 2: 20 x 722 x 418 f32x3 -> 836 x
+    // (Nearest neighbour shares no source rows but with itself: 76 x 107 x 227 f32x3 -> 66 x 140 6.9 -> 5.6 us, 65 x 80 x 82 -> 307 x 314 18.5 -> 15.4, 104 x
+    // 46 x 743 f32x4 -> 65 x 1048 36.8 -> 31.1. Enlarged down by 4/3 and more it shares enough to keep the 64 x 4 block where output rows end with a sector of
+    // memory and fill the waves to 80 % (block / along the rows: 107 x 140 x 35 x 4 -> 436 x 152 20.3 / 24.5, 38 x 146 x 90 x 4 -> 556 x 383 21.5 / 25.1; 172
+    // launches of f32x4 and 47 of f32x3, 2 to 9 % and 2 to 6 % in the mean of their classes). Where they do not, along the rows is the faster one, by up to 10 %.
+    // Bilinear rows share theirs with the next one below a vertical scale of 2: 20 x 722 x 418 f32x3 -> 836 x
     // 484 33.9 us in the 64 x 4 block and 40.7 along the rows, 12 x 399 x 367 f32x4 -> 534 x 492 14.9 and 19.2; at 2.8, 121 x 194 x 594 f32x3 -> 69 x 211,
-    // 31.2 and 25.4)
-    // Enlarged rows of 1024 pixels and more start with a block: 1 x 1716 x 858 f32x4 -> 1852 x 926 10.3 us so and 11.7 along the rows.
-    const bool along = INTERP == NVCV_INTERP_NEAREST || (INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH);
-    const bool flat  = INTERP != NVCV_INTERP_CUBIC && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);
+    // 31.2 and 25.4.)
+    // Enlarged rows of 1024 pixels and more start with a block, where they are not counted along the rows: 4 x 720p -> 1080p f32x3 nearest neighbour 22.7 so, 23.7
+    // along the rows, 24.6 in the 64 x 4 block; but 16 bytes to a pixel keep that block, 39 launches at 0.90 to 0.95 of the time in the mean.
+    const bool shared = 4 * (int64_t)a.srcH <= 3 * (int64_t)a.dstH && a.dstRowStride % 64 == 0
+                     && 4 * (int64_t)DivUp(a.dstW, kTileW) * kTileW <= 5 * (int64_t)a.dstW;
+    const bool along = INTERP == NVCV_INTERP_NEAREST ? !shared : INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH;
+    const bool flat  = INTERP != NVCV_INTERP_CUBIC && (INTERP != NVCV_INTERP_NEAREST || sizeof(Pixel<T, C>) < 16)
+                    && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);
     const auto order = along ? AlongRows(a.dstW, a.dstH, kTileW, 1)
                      : flat  ? AlongRows(DivUp(a.dstW, 4 * kTileW) * 4 * kTileW, a.dstH, kTileW, 1)
                              : WaveOrder{};

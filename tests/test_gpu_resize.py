@@ -852,6 +852,22 @@ def test_tensors_of_16_blocks(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
 
 
+# Nearest neighbour of larger pixels on both sides of what keeps the block of 64 x 4: enlarged down by 4/3, rows that end with a sector
+# (pitches of their own and packed), waves filled to 80 %
+@pytest.mark.parametrize("c", [3, 4])
+@pytest.mark.parametrize("row_align", [0, 1])
+@pytest.mark.parametrize("size", [(50, 30, 208, 40), (50, 31, 208, 41), (50, 30, 205, 40), (50, 30, 204, 43), (33, 9, 103, 45), (33, 9, 102, 45), (7, 3, 64, 5),
+                                  (300, 20, 1280, 37), (300, 20, 1281, 37)])
+def test_tensor_nearest_of_larger_pixels(cv, orc, gpu, size, row_align, c):
+    sw, sh, dw, dh = size
+    src = np.ascontiguousarray(orc.fill_u8((3, sh, sw, c), 5 + dw), np.float32)
+    tin = cv.Tensor.from_numpy(src, "NHWC", row_align=row_align)
+    tout = cv.Tensor.alloc([3, dh, dw, c], np.float32, "NHWC", row_align=row_align)
+    tout.torch_view().fill_(-7)
+    cv.Resize()(None, tin, tout, NEAREST)
+    np.testing.assert_array_equal(tout.numpy(), orc.resize(src, (dh, dw), NEAREST, variant=0))
+
+
 # One column of more rows than one dimension of a launch has waves for
 def test_nearest_of_a_tall_image(cv, orc, gpu):
     h   = 2 ** 26
