@@ -34,6 +34,7 @@
 #include "DeviceUtils.hpp"
 #include "FixedPointBlend.hpp"
 #include "LaneExchange.hpp"
+#include "LinearRows.hpp"
 #include "OpCommon.hpp"
 #include "RunIO.hpp"
 #include "VarShapeTiles.hpp"
@@ -3876,8 +3877,6 @@ __global__ __launch_bounds__(256) void ResizeCubicStripF32Kernel(const ResizeArg
 // 53.5 us, cached stores, which the L2 merges to 3.13 M requests, 79 us (they evict the source rows).
 constexpr int kRowsPerGroup = 4;
 
-constexpr int kLdsBytes = 163840; // of a CU
-
 // Source rows from the first on that kRowsPerGroup output rows span, 3 to 5; 0: more than 5 (rows reduced). A place is
 // a rounded product and a rounded difference, each off by at most 2^-11 below 8192: two of them by less than the margin.
 static inline int LinearRowsSources(const ResizeArgs &a)
@@ -3897,7 +3896,7 @@ __global__ __launch_bounds__(256) void ResizeLinearRowsKernel(const ResizeArgs a
     // Row i of the block is staged from float i * pitch + lead(i) on, where lead is the row's distance from the 128-byte
     // boundary in front of it; dense rows follow one another in LDS as they do in memory (and keep the block's lead).
     const bool  dense = p.dstRow == 4 * p.dstW;
-    const int   pitch = dense ? p.dstW : ((p.dstW + 31) & ~31) + 32;
+    const int   pitch = LinearRowsPitch(p.dstW, dense);
     auto        lead  = [&](int i)
     {
         return (int)(reinterpret_cast<uintptr_t>(p.dst + (int64_t)(yBlock + (dense ? 0 : i)) * p.dstRow) & 127) / 4;
@@ -4197,7 +4196,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         const int sources = LinearRowsSources(a), chunks = DivUp(a.dstW, 256);
         const int groups = chunks >= 3 ? 1 : chunks == 2 ? 2 : 4;
-        const int lds = (groups * kRowsPerGroup * (((a.dstW + 31) & ~31) + 32) + 32) * 4;
+        const int lds = LinearRowsLds(a.dstW, a.dstRowStride == 4 * (int64_t)a.dstW, groups * kRowsPerGroup);
         const dim3 rgrid(DivUp(a.dstH, groups * kRowsPerGroup), N);
         const int64_t blocks = (int64_t)rgrid.x * N;
         // us as patches / as rows:
@@ -4205,11 +4204,12 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         //   blocks: 5.3 / 6.3; 3 x 1281 x 721, 543: 7.0 / 7.9; 4 x 1026 x 578, 580: 5.9 / 6.5; 4 x 1281 x 721, 724: 8.8 / 8.2).
         // - Rows that fill a wave's 256 columns well: 2929 x 64 x 64 18.0 / 29.7; 244 x 128 x 128 7.7 / 8.3, from 64 x 64 7.2 / 7.1,
         //   732 of these 17.5 / 14.9; 156 x 160 x 160 8.4 / 7.8.
-        // - Three blocks per CU and more in the LDS (one 1080p -> 4K, two per CU: 13.2 / 19.7, 4 of these 45.6 / 49.3), and with
+        // - Three blocks per CU and more in the LDS (one 1080p -> 4K, two per CU: 13.2 / 19.7, 4 of these 45.6 / 49.3; 4 maps of 3100 rows of
+        //   3352 floats, the last of three: 51.5 / 47.7, of 3355 floats: 54.0 / 62.3), and with
         //   three no second round of blocks that is nearly empty (2 x 2560 x 1440, 720 blocks for 768 places: 12.3 / 10.6; 2 x
-        //   2816 x 1584, 792: 14.9 / 17.2; 4 of these 26.6 / 26.0).
+        //   2816 x 1584, 792: 14.9 / 17.2; 4 of these 26.6 / 26.0). 3 maps of 2000 rows of 2513 floats, four per CU: 22.2 / 19.7.
         const bool wide   = a.dstW >= 144 || (a.dstW >= 96 && a.dstW >= 2 * a.srcW && (int64_t)a.dstW * a.dstH * N >= 4000000);
-        const int  perCu  = kLdsBytes / lds;
+        const int  perCu  = BlocksPerCu(lds);
         const bool rounds = perCu >= 4 || (perCu == 3 && (blocks <= 3 * 256 || blocks >= 6 * 256));
         if (sources != 0 && a.srcW >= 2 && a.srcH >= 2 && blocks >= 704 && wide && rounds)
         {

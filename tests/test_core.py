@@ -584,13 +584,16 @@ def test_block_pool_of_the_default_allocator(tmp_path):
     assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "ok"
 
 
-def test_tiles_of_a_launchs_waves(tmp_path):
+@pytest.mark.parametrize("name", ["wave_order_cases", "linear_rows_cases"])
+def test_arithmetic_of_launches(tmp_path, name):
+    # tests/golden/<name>.cpp over a header that the kernels share with the host
     here = os.path.dirname(os.path.abspath(__file__))
-    exe = str(tmp_path / "wave_order_cases")
+    exe = str(tmp_path / name)
     csrc = os.path.join(os.path.dirname(here), "cv-cuda_amd", "csrc", "cvcuda")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I" + csrc, os.path.join(here, "golden", "wave_order_cases.cpp"),
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-I" + csrc, os.path.join(here, "golden", name + ".cpp"),
                     "-o", exe], check=True)
-    assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "ok"
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.stdout.strip() == "ok", r.stdout
 
 
 def test_what_an_image_batch_uploads(tmp_path):

@@ -619,6 +619,13 @@ def test_linear_float_maps_by_whole_rows(cv, orc, gpu, n, sw, sh, dw, dh, kind):
         assert bool((spare == -7.0).all()), "floats outside the rows written"
 
 
+# the same at the widths that leave room for one block less in a CU's LDS, each with all it may have of it
+@pytest.mark.parametrize("dw", [2528, 2529, 2552, 2553, 3325, 3328, 3329, 3352, 3353])
+@pytest.mark.parametrize("kind", ["dense", "padded", "view"])
+def test_linear_float_maps_by_whole_rows_at_the_lds_limits(cv, orc, gpu, dw, kind):
+    test_linear_float_maps_by_whole_rows(cv, orc, gpu, 512, 40, 4, dw, 9, kind)
+
+
 # seeded random cases: 8-bit pixels of 1, 3 and 4 channels, every interpolation, scales of 0.42 to 2.4 per axis (now
 # and then equal, or exactly 1/2, 2/3, 1, 1.5, 2), small and 1080p-sized images, batches below and above the sizes
 # at which the strip kernels take over, as packed tensors, as views with odd leads and pitches (bytes outside the
