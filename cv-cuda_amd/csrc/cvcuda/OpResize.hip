@@ -4000,7 +4000,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     {
         if (a.srcW >= 2 * a.dstW)
         {
-            const int  across = a.srcH >= 4 * (int64_t)a.dstH ? DivUp(a.dstW, kTileW) : 0;
+            const int  across = a.srcH >= 4 * (int64_t)a.dstH ? TilesAlongRows(a.dstW, a.dstH, kTileW) : 0;
             const dim3 sgrid  = across == 0 ? grid : dim3((unsigned)(((int64_t)across * a.dstH + 3) / 4), 1, N);
             hipLaunchKernelGGL((ResizeCubicStagedKernel<T, C>), sgrid, dim3(256), 0, stream, a, across);
             CheckLaunch("ResizeCubicStagedKernel");

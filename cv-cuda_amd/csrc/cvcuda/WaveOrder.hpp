@@ -40,6 +40,13 @@ constexpr WaveOrder AlongRows(int dstW, int dstH, int waveW, int waveH)
     return WaveOrder{(uint32_t)across, across == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)across + 1)};
 }
 
+// The tiles of a row where a launch's waves, of one row each, are counted along the rows and divided by them; 0: more waves than fit.
+constexpr int TilesAlongRows(int dstW, int dstH, int waveW)
+{
+    const int64_t across = TilesIn(dstW, waveW);
+    return WavesFitARow(across * dstH) ? (int)across : 0;
+}
+
 // The tile of wave `wave` of the `waves` in block (blockX, blockY).
 constexpr WaveTile TileOfWave(const WaveOrder &order, uint32_t blockX, uint32_t blockY, uint32_t wave, uint32_t waves)
 {

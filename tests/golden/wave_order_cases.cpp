@@ -106,6 +106,14 @@ int main()
         Ends(65535 * 64, 1, 64, 1, waves, true);
         Ends(65536 * 64, 1, 64, 1, waves, false);
     }
+    // without an order of their own: 4 waves to a block
+    for (int tiles : {1, 3, 64})
+    {
+        const int most = ((1 << 26) - 8) / tiles;
+        Check(TilesAlongRows(tiles * 64 - 63, most, 64) == tiles, "fits", tiles * 64 - 63, most, 64, 1, 4);
+        Check(TilesIn(tiles * (int64_t)most, 4) * 256 < (int64_t)1 << 32, "threads", tiles * 64 - 63, most, 64, 1, 4);
+        Check(TilesAlongRows(tiles * 64, most + 1, 64) == 0, "too many", tiles * 64, most + 1, 64, 1, 4);
+    }
     std::puts(s_bad == 0 ? "ok" : "bad");
     return s_bad != 0;
 }
