@@ -858,6 +858,14 @@ static inline bool FlatBlocks(int dstW, int waveW)
     return dstW >= 1024 && DivUp(dstW, (int)span) * span * 4 <= (int64_t)dstW * 5;
 }
 
+// Whether the source pixels that the output rows of a stacked block need not fetch again, because the row above has, are `of` / `in` of the
+// pixels written or more, and the rows fill their waves to 80 %. Such launches lose along the rows.
+static inline bool SharedRowsPay(const ResizeArgs &a, int waveW, int in, int of)
+{
+    return in * (int64_t)(a.dstH - a.srcH) * a.srcW >= of * (int64_t)a.dstW * a.dstH
+        && 4 * (int64_t)DivUp(a.dstW, waveW) * waveW <= 5 * (int64_t)a.dstW;
+}
+
 // Grid of a launch whose waves own tiles of waveW x waveH.
 static inline dim3 WaveTileGrid(int dstW, int dstH, int N, int waveW, int waveH, const WaveOrder &order, int waves = 4)
 {
@@ -4028,8 +4036,11 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             const int  rows      = waves(4) <= 30 * 256 ? 4 : few || soon ? 8 : 16;
             // (along the rows where the chip is full, below one another, where rows share sources in the L1, before: one channel, 44 x 237 x 1008 -> 182 x
             // 962 30.2 -> 21.6, 65 x 569 x 51 -> 1915 x 128 26.4 -> 20.3; three, 11 x 793 x 146 -> 2918 x 454 54.8 -> 46.5, but 1 x 392 x 1105 -> 556 x 1567, 3528
-            // waves of 4 rows, 6.4 and 7.3; four 44 x 286 x 59 -> 1071 x 223 48.6 and 42.5, but 128 x 104 x 88 -> 106 x 90 9.7 and 11.5)
-            const auto order     = C != 4 && rows > 4 ? AlongRows(a.dstW, a.dstH, kTileW, rows) : WaveOrder{};
+            // waves of 4 rows, 6.4 and 7.3; four 44 x 286 x 59 -> 1071 x 223 48.6 and 42.5, but 128 x 104 x 88 -> 106 x 90 9.7 and 11.5. Not
+            // three channels that share 4/5 of what is written: 189 x 424 x 66 -> 276 x 139 30.7 and 35.9, 1 x 955 x 1954 -> 521 x 4096 10.3 and 13.5, 33 launches up
+            // to 4/3 1.04 times slower along the rows in the mean, from 1/4 to 2/3 0.97 to 0.98; one channel there 1.00.)
+            const bool along     = C != 4 && rows > 4 && !(C == 3 && SharedRowsPay(a, kTileW, 5, 4));
+            const auto order     = along ? AlongRows(a.dstW, a.dstH, kTileW, rows) : WaveOrder{};
             hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kTileW, rows, order), dim3(256), 0, stream, a,
                                rows, order);
             CheckLaunch("ResizeCubicStripF32Kernel");
@@ -4225,7 +4236,14 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         // and finishes sooner the more CUs take part
         const int64_t blocks = (int64_t)DivUp(a.dstW, kPatchTileW) * DivUp(a.dstH, kPatchTileH) * N;
         const int     waves  = blocks < 8 * 256 ? 1 : 4;
-        const auto    order  = AlongRows(a.dstW, a.dstH, kPatchTileW, 4);
+        // (Below one another where rows share much more than they write. Bicubic f32x1 from 4/3 on: 105 x 1100 x 213 -> 336 x 461 61.0 and along the rows 74.1, 9 x
+        // 797 x 345 -> 296 x 923 9.8 and 12.5, 42 launches 1.05 to 1.29 times slower so, 1.02 to 1.17 with inputs out of the memory's cache; less shared 0.96 to 1.01.
+        // u8x4 from 5/3 on: 4 x 1223 x 1985 -> 447 x 3990 15.5 and 17.2, 105 x 1100 x 213 -> 336 x 461 31.6 and 35.6, 22 launches 1.05, out of the cache 1.00; less 0.96
+        // to 1.00. Smaller pixels and bilinear f32x1: 0.98 to 1.00.)
+        constexpr bool kCubicF = std::is_same_v<T, float> && C == 1 && INTERP == NVCV_INTERP_CUBIC,
+                       kLinear4 = std::is_same_v<T, uint8_t> && C == 4 && INTERP == NVCV_INTERP_LINEAR;
+        const bool shared = waves == 4 && ((kCubicF && SharedRowsPay(a, kPatchTileW, 3, 4)) || (kLinear4 && SharedRowsPay(a, kPatchTileW, 3, 5)));
+        const auto order = shared ? WaveOrder{} : AlongRows(a.dstW, a.dstH, kPatchTileW, 4);
         constexpr bool kOdd   = INTERP == NVCV_INTERP_CUBIC && kFixedCubic<T> && C != 4;
         auto           kernel = kOdd && RowsAreOdd<C>(a) ? ResizePatchTensorKernel<T, C, INTERP, kOdd> : ResizePatchTensorKernel<T, C, INTERP, false>;
         hipLaunchKernelGGL(kernel, WaveTileGrid(a.dstW, a.dstH, N, kPatchTileW, 4, order, waves),
@@ -4240,14 +4258,18 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     // (Nearest neighbour shares no source rows but with itself: 76 x 107 x 227 f32x3 -> 66 x 140 6.9 -> 5.6 us, 65 x 80 x 82 -> 307 x 314 18.5 -> 15.4, 104 x
     // 46 x 743 f32x4 -> 65 x 1048 36.8 -> 31.1. Enlarged down by 4/3 and more it shares enough to keep the 64 x 4 block where output rows end with a sector of
     // memory and fill the waves to 80 % (block / along the rows: 107 x 140 x 35 x 4 -> 436 x 152 20.3 / 24.5, 38 x 146 x 90 x 4 -> 556 x 383 21.5 / 25.1; 172
-    // launches of f32x4 and 47 of f32x3, 2 to 9 % and 2 to 6 % in the mean of their classes). Where they do not, along the rows is the faster one, by up to 10 %.
+    // launches of f32x4 and 47 of f32x3, 2 to 9 % and 2 to 6 % in the mean of their classes). Where they do not, along the rows is the faster one, by up to 10 %, unless what
+    // is shared is half of what is written or more: 168 x 1115 x 34 x 3 -> 375 x 130 36.0 / 54.1, 6 x 1176 x 470 x 3 -> 475 x 1211 14.8 / 22.3, 44 x 321 x 59 x 4 -> 142 x
+    // 193 5.8 / 9.6; 86 launches of f32x3 1.17 times slower along the rows in the mean, 1.08 with inputs that are not in the memory's cache, 79 of f32x4 1.12 and 1.07;
+    // from 1/4 to 1/2 0.98 to 1.00.
     // Bilinear rows share theirs with the next one below a vertical scale of 2: 20 x 722 x 418 f32x3 -> 836 x
     // 484 33.9 us in the 64 x 4 block and 40.7 along the rows, 12 x 399 x 367 f32x4 -> 534 x 492 14.9 and 19.2; at 2.8, 121 x 194 x 594 f32x3 -> 69 x 211,
     // 31.2 and 25.4.)
     // Enlarged rows of 1024 pixels and more start with a block, where they are not counted along the rows: 4 x 720p -> 1080p f32x3 nearest neighbour 22.7 so, 23.7
     // along the rows, 24.6 in the 64 x 4 block; but 16 bytes to a pixel keep that block, 39 launches at 0.90 to 0.95 of the time in the mean.
-    const bool shared = 4 * (int64_t)a.srcH <= 3 * (int64_t)a.dstH && a.dstRowStride % 64 == 0
-                     && 4 * (int64_t)DivUp(a.dstW, kTileW) * kTileW <= 5 * (int64_t)a.dstW;
+    const bool shared = (4 * (int64_t)a.srcH <= 3 * (int64_t)a.dstH && a.dstRowStride % 64 == 0
+                         && 4 * (int64_t)DivUp(a.dstW, kTileW) * kTileW <= 5 * (int64_t)a.dstW)
+                     || SharedRowsPay(a, kTileW, 2, 1);
     const bool along = INTERP == NVCV_INTERP_NEAREST ? !shared : INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH;
     const bool flat  = INTERP != NVCV_INTERP_CUBIC && (INTERP != NVCV_INTERP_NEAREST || sizeof(Pixel<T, C>) < 16)
                     && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);
