@@ -1795,16 +1795,7 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     {
         uint32_t w[PB];
         PackQuad<PB>(quad, w);
-        if constexpr (PB == 1 && INTERP != NVCV_INTERP_CUBIC)
-        {
-            // The 32 bytes of a row that a wave has are parts of sectors, which the L2 puts together if it may keep them (20 x 1333 x 951 nearest
-            // neighbour 26.0 -> 24.0 us, bilinear 36.8 -> 34.4; bicubic 49.6 and 50.0, larger pixels 3 to 33 % slower).
-            __builtin_memcpy(to, w, 4);
-        }
-        else
-        {
-            StoreDwordsNT<PB>(to, w); // 4 pixels = PB dwords
-        }
+        StoreDwordsNT<PB>(to, w); // 4 pixels = PB dwords
     }
     else
     {
