@@ -47,11 +47,7 @@ constexpr int kMostPatches = 4, kFewPatches = 2;
 template<int N>
 constexpr int kWaveW = kPatch * N;
 
-// A block of 64 x WAVES threads. Waves of 8-bit bicubic with three channels are the longest and their lengths differ most (the
-// image's edge), so a block of four holds its places until the last one ends: they go alone. us with four waves / one: 24 images
-// of 697 .. 1194 x 187 .. 545 39.0 / 36.2, 9 x 1241 x 955 in perspective 48.1 / 46.8, 16 x 1240 x 1754 175.6 / 172.2. Others gain nothing by it (u8x4 34.6 /
-// 35.0, u8x1 41.0 / 41.1) or are held up by the launch of so many blocks, 4.6 a ns at most (nearest neighbour u8x1 27.2 / 36.2, u8x3 85.9 /
-// 102.5, bilinear u8x3 48.1 / 53.4).
+// A block of 64 x WAVES threads.
 template<int N, int WAVES>
 struct Block
 {
@@ -60,8 +56,21 @@ struct Block
     static constexpr int kTileW = kWaveW<N> * kAcross, kTileH = WAVES / kAcross * kPatch;
 };
 
+// Waves of 8-bit bicubic with three channels are the longest and their lengths differ most (the image's edge), so a block of four holds its
+// places until the last one ends: in large launches, and where blocks of four have waves outside the images, they go alone. us with four
+// waves / one: 24 images of 697 .. 1194 x 187 .. 545 39.0 / 36.2, 9 x 1241 x 955 in perspective 48.1 / 46.8. Others gain nothing by it (u8x4 34.6 /
+// 35.0, u8x1 41.0 / 41.1) or are held up by the launch of so many blocks, 4.6 a ns at most (nearest neighbour u8x1 27.2 / 36.2, u8x3 85.9 /
+// 102.5, bilinear u8x3 48.1 / 53.4).
 template<class T, int C, int INTERP, int N>
-using BlockOf = Block<N, std::is_same_v<T, uint8_t> && C == 3 && INTERP == NVCV_INTERP_CUBIC && N == kMostPatches ? 1 : 4>;
+constexpr bool kSingleWaves = std::is_same_v<T, uint8_t> && C == 3 && INTERP == NVCV_INTERP_CUBIC && N == kMostPatches;
+
+// The waves of a launch in blocks of one and, with those that stand outside the images, of four. Time of one over four in 400 random launches, inputs
+// and outputs out of the memory's cache: none outside and up to 32 768 waves 1.01 to 1.03 (160 x 196 x 29 11.0 us / 13.6), beyond 0.99 and
+// 0.94; 2 % to 10 % outside and up to 8192 waves 1.00 to 1.05, beyond 0.89 to 0.99; 10 % to 20 % 0.97 to 1.00 and 0.87 to 0.91; more 0.63 to 0.97.
+constexpr bool SingleWavesPay(int64_t ones, int64_t fours)
+{
+    return ones > 32768 || 10 * fours >= 11 * ones || (ones > 8192 && 50 * fours >= 51 * ones);
+}
 
 struct WarpArgs
 {
@@ -1348,12 +1357,12 @@ __device__ __forceinline__ bool NarrowTapsPay(const float (&m)[9])
 }
 
 // One block's tile of the destination image `dst` (tile coordinates tx, ty), all its threads.
-template<class T, int C, int INTERP, bool PERSP, bool LIST, int N>
+template<class T, int C, int INTERP, bool PERSP, bool LIST, int N, int WAVES>
 __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const float (&m)[9], uint8_t *dst, int dstRow,
                                          int dstW, int dstH, int tx, int ty)
 {
     constexpr int PB = C * sizeof(T), D = (PB + 3) / 4;
-    using B          = BlockOf<T, C, INTERP, N>;
+    using B          = Block<N, WAVES>;
 
     // ---- gather: lane (lx, ly) of wave w samples its pixel in N patches (side by side: a
     // wave covers 8 N columns x 8 rows)
@@ -1878,8 +1887,8 @@ __device__ __forceinline__ void LoadMatrix(const WarpArgs &a, int image, float s
     }
 }
 
-template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES>
-__global__ __launch_bounds__((BlockOf<T, C, INTERP, PATCHES>::kThreads)) void WarpTensor(const WarpArgs a)
+template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES, int WAVES>
+__global__ __launch_bounds__((64 * WAVES)) void WarpTensor(const WarpArgs a)
 {
     const int n  = blockIdx.z;
     const Img im = {a.src + n * a.srcN, a.srcRow, a.srcW, a.srcH};
@@ -1889,11 +1898,11 @@ __global__ __launch_bounds__((BlockOf<T, C, INTERP, PATCHES>::kThreads)) void Wa
     {
         m[i] = a.m[i];
     }
-    WarpTile<T, C, INTERP, PERSP, LIST, PATCHES>(im, a, m, a.dst + n * a.dstN, a.dstRow, a.dstW, a.dstH, blockIdx.x, blockIdx.y);
+    WarpTile<T, C, INTERP, PERSP, LIST, PATCHES, WAVES>(im, a, m, a.dst + n * a.dstN, a.dstRow, a.dstW, a.dstH, blockIdx.x, blockIdx.y);
 }
 
-template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES>
-__global__ __launch_bounds__((BlockOf<T, C, INTERP, PATCHES>::kThreads)) void WarpVarShape(const WarpArgs a, const VarTiles tiles)
+template<class T, int C, int INTERP, bool PERSP, bool LIST, int PATCHES, int WAVES>
+__global__ __launch_bounds__((64 * WAVES)) void WarpVarShape(const WarpArgs a, const VarTiles tiles)
 {
     const TileCoord tc = LocateTile(tiles, blockIdx.x);
     // descriptors and matrix depend on the image index only: read by value here, ahead of the matrix
@@ -1903,7 +1912,7 @@ __global__ __launch_bounds__((BlockOf<T, C, INTERP, PATCHES>::kThreads)) void Wa
     float                       m[9];
     LoadMatrix<PERSP>(a, tc.image, kCoordScale<T, INTERP>, m);
     const Img im = {AsGlobal(s.basePtr), s.rowStride, s.width, s.height};
-    WarpTile<T, C, INTERP, PERSP, LIST, PATCHES>(im, a, m, AsGlobal(d.basePtr), d.rowStride, d.width, d.height, tc.tx, tc.ty);
+    WarpTile<T, C, INTERP, PERSP, LIST, PATCHES, WAVES>(im, a, m, AsGlobal(d.basePtr), d.rowStride, d.width, d.height, tc.tx, tc.ty);
 }
 
 // Two patches per wave instead of four where that leaves a SIMD no more than 3 waves of four: such launches run as long as one
@@ -1929,46 +1938,67 @@ template<class T, int C, int INTERP, bool PERSP, bool LIST>
 void LaunchMap(const WarpArgs &a, int N, const NVCVImageBufferStrided *dstHost, hipStream_t stream)
 {
     constexpr int kMost = kMostPatches, kFew = kFewPatchesForm<T> ? kFewPatches : kMost;
-    using Most          = BlockOf<T, C, INTERP, kMost>;
-    using Few           = BlockOf<T, C, INTERP, kFew>;
-    // (counted in tiles of four waves, whatever a block has)
-    using Four     = Block<kMost, 4>;
-    const auto few = [](int64_t tiles, int64_t most) { return kFew != kMost && tiles * Four::kWaves <= most; };
+    using Four          = Block<kMost, 4>;
+    using Few           = Block<kFew, 4>;
+    using One           = Block<kMost, kSingleWaves<T, C, INTERP, kMost> ? 1 : 4>;
+    const auto few  = [](int64_t tiles, int64_t most) { return kFew != kMost && tiles * Four::kWaves <= most; };
+    const auto ones = [](int64_t one, int64_t four) { return One::kWaves == 1 && SingleWavesPay(one, four * Four::kWaves); };
     if (dstHost == nullptr)
     {
-        if (few((int64_t)DivUp(a.dstW, Four::kTileW) * DivUp(a.dstH, Four::kTileH) * N, kFewWaves))
+        const auto    gridOf = [&](int w, int h) { return dim3(DivUp(a.dstW, w), DivUp(a.dstH, h), N); };
+        const auto    count  = [&](int w, int h) { return (int64_t)DivUp(a.dstW, w) * DivUp(a.dstH, h) * N; };
+        const int64_t four   = count(Four::kTileW, Four::kTileH);
+        if (few(four, kFewWaves))
         {
-            const dim3 grid(DivUp(a.dstW, Few::kTileW), DivUp(a.dstH, Few::kTileH), N);
-            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kFew>), grid, dim3(Few::kThreads), 0, stream, a);
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kFew, 4>), gridOf(Few::kTileW, Few::kTileH), dim3(Few::kThreads), 0, stream, a);
+        }
+        else if (ones(count(One::kTileW, One::kTileH), four))
+        {
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kMost, One::kWaves>), gridOf(One::kTileW, One::kTileH), dim3(One::kThreads), 0,
+                               stream, a);
         }
         else
         {
-            const dim3 grid(DivUp(a.dstW, Most::kTileW), DivUp(a.dstH, Most::kTileH), N);
-            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kMost>), grid, dim3(Most::kThreads), 0, stream, a);
+            hipLaunchKernelGGL((WarpTensor<T, C, INTERP, PERSP, LIST, kMost, 4>), gridOf(Four::kTileW, Four::kTileH), dim3(Four::kThreads), 0, stream, a);
         }
         CheckLaunch("WarpTensor");
         return;
     }
     for (int first = 0; first < N; first += kMaxTileImages)
     {
-        VarTiles  tiles;
-        const int count = std::min(kMaxTileImages, N - first);
-        int       total = BuildVarTiles(tiles, dstHost, first, count, Four::kTileW, Four::kTileH);
-        if (total > 0 && few(total, kFewWavesOfBatches<T, INTERP, PERSP>))
+        VarTiles   tiles;
+        const int  count   = std::min(kMaxTileImages, N - first);
+        const auto totalOf = [&](int w, int h) { return BuildVarTiles(tiles, dstHost, first, count, w, h); };
+        const auto tilesOf = [&](int w, int h)
         {
-            total = BuildVarTiles(tiles, dstHost, first, count, Few::kTileW, Few::kTileH);
-            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kFew>), dim3(total), dim3(Few::kThreads), 0, stream, a, tiles);
-            CheckLaunch("WarpVarShape");
-        }
-        else if (total > 0)
-        {
-            if (Most::kWaves != Four::kWaves)
+            int64_t sum = 0;
+            for (int i = first; i < first + count; ++i)
             {
-                total = BuildVarTiles(tiles, dstHost, first, count, Most::kTileW, Most::kTileH);
+                sum += (int64_t)DivUp(dstHost[i].planes[0].width, w) * DivUp(dstHost[i].planes[0].height, h);
             }
-            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kMost>), dim3(total), dim3(Most::kThreads), 0, stream, a, tiles);
-            CheckLaunch("WarpVarShape");
+            return sum;
+        };
+        const int64_t four = tilesOf(Four::kTileW, Four::kTileH);
+        if (four <= 0)
+        {
+            continue;
         }
+        if (few(four, kFewWavesOfBatches<T, INTERP, PERSP>))
+        {
+            const int total = totalOf(Few::kTileW, Few::kTileH);
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kFew, 4>), dim3(total), dim3(Few::kThreads), 0, stream, a, tiles);
+        }
+        else if (One::kWaves == 1 && ones(tilesOf(One::kTileW, One::kTileH), four))
+        {
+            const int total = totalOf(One::kTileW, One::kTileH);
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kMost, One::kWaves>), dim3(total), dim3(One::kThreads), 0, stream, a, tiles);
+        }
+        else
+        {
+            const int total = totalOf(Four::kTileW, Four::kTileH);
+            hipLaunchKernelGGL((WarpVarShape<T, C, INTERP, PERSP, LIST, kMost, 4>), dim3(total), dim3(Four::kThreads), 0, stream, a, tiles);
+        }
+        CheckLaunch("WarpVarShape");
     }
 }
 

@@ -299,6 +299,34 @@ def test_patches_per_wave_of_image_batches(cv, K, orc, gpu, n):
             np.testing.assert_array_equal(outs[i].plane_view(0, np.uint8, 3).cpu().numpy(), dev, err_msg=str((interp, border, i)))
 
 
+# Bicubic of three 8-bit channels on both sides of what its waves stand alone for: blocks of four with no wave outside the images, up to and
+# past 32 768 waves; a tenth, a fiftieth outside
+@pytest.mark.parametrize("size", [(161, 192, 32), (148, 172, 68), (148, 173, 73), (342, 192, 128), (341, 190, 125), (205, 223, 41), (93, 641, 41), (21, 97, 480)])
+@pytest.mark.parametrize("batch", [False, True])
+def test_bicubic_waves_in_blocks(cv, K, orc, gpu, size, batch):
+    n, w, h = size
+    src, m = orc.fill_u8((2, h, w, 3), 80 + w), rotation(w, h, 7.0, 1.05)
+    dev = orc.warp(src, (h, w), orc.invert_affine(m), CUBIC, 1, (0, 0, 0, 0), variant=device_variant(CUBIC))
+    if not batch:
+        tin = cv.Tensor.from_numpy(src[np.arange(n) % 2], "NHWC")
+        tout = cv.Tensor.alloc([n, h, w, 3], np.uint8, "NHWC")
+        cv.WarpAffine(0)(None, tin, tout, m, CUBIC, 1, (0, 0, 0, 0))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(tout.numpy(), dev[np.arange(n) % 2])
+        return
+    two = [cv.Image.from_numpy(s, K.IMAGE_FORMAT_RGB8) for s in src]
+    bi, bo = cv.ImageBatchVarShape(n), cv.ImageBatchVarShape(n)
+    outs = [cv.Image.alloc((w, h), K.IMAGE_FORMAT_RGB8) for _ in range(n)]
+    for i in range(n):
+        bi.push_back(two[i % 2])
+        bo.push_back(outs[i])
+    mats = cv.Tensor.from_numpy(np.asarray([m] * n, np.float32), "NW")
+    cv.WarpAffine(n)(None, bi, bo, mats, CUBIC, 1, (0, 0, 0, 0))
+    torch.cuda.synchronize()
+    for i in range(n):
+        np.testing.assert_array_equal(outs[i].plane_view(0, np.uint8, 3).cpu().numpy(), dev[i % 2], err_msg=str(i))
+
+
 # 75 000 rows of tiles of the form whose blocks are one wave; at whole places a bicubic sum is the pixel itself
 def test_bicubic_of_a_tall_image(cv, orc, gpu):
     src = orc.fill_u8((1, 600000, 16, 3), 91)
