@@ -1804,6 +1804,8 @@ __device__ __forceinline__ void WarpTile(const Img &im, const WarpArgs &a, const
     {
         uint32_t w[PB];
         PackQuad<PB>(quad, w);
+        // (one channel too, whose 32 bytes of a row are mostly parts of sectors: by ordinary stores, which the L2 puts together, 400 launches take 0.97 of
+        // the time for nearest neighbour and 1.00 for bilinear while inputs and outputs stay in the memory's cache, but 1.04 and 1.03, up to 1.28, where they do not)
         StoreDwordsNT<PB>(to, w); // 4 pixels = PB dwords
     }
     else
