@@ -859,11 +859,11 @@ static inline bool FlatBlocks(int dstW, int waveW)
 }
 
 // Whether the source pixels that the output rows of a stacked block need not fetch again, because the row above has, are `of` / `in` of the
-// pixels written or more, and the rows fill their waves to 80 %. Such launches lose along the rows.
-static inline bool SharedRowsPay(const ResizeArgs &a, int waveW, int in, int of)
+// pixels written or more, and the rows fill their waves to `full` per cent. Such launches lose along the rows.
+static inline bool SharedRowsPay(const ResizeArgs &a, int waveW, int in, int of, int full = 80)
 {
     return in * (int64_t)(a.dstH - a.srcH) * a.srcW >= of * (int64_t)a.dstW * a.dstH
-        && 4 * (int64_t)DivUp(a.dstW, waveW) * waveW <= 5 * (int64_t)a.dstW;
+        && full * (int64_t)DivUp(a.dstW, waveW) * waveW <= 100 * (int64_t)a.dstW;
 }
 
 // Grid of a launch whose waves own tiles of waveW x waveH.
@@ -4259,17 +4259,17 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     // 46 x 743 f32x4 -> 65 x 1048 36.8 -> 31.1. Enlarged down by 4/3 and more it shares enough to keep the 64 x 4 block where output rows end with a sector of
     // memory and fill the waves to 80 % (block / along the rows: 107 x 140 x 35 x 4 -> 436 x 152 20.3 / 24.5, 38 x 146 x 90 x 4 -> 556 x 383 21.5 / 25.1; 172
     // launches of f32x4 and 47 of f32x3, 2 to 9 % and 2 to 6 % in the mean of their classes). Where they do not, along the rows is the faster one, by up to 10 %, unless what
-    // is shared is half of what is written or more: 168 x 1115 x 34 x 3 -> 375 x 130 36.0 / 54.1, 6 x 1176 x 470 x 3 -> 475 x 1211 14.8 / 22.3, 44 x 321 x 59 x 4 -> 142 x
-    // 193 5.8 / 9.6; 86 launches of f32x3 1.17 times slower along the rows in the mean, 1.08 with inputs that are not in the memory's cache, 79 of f32x4 1.12 and 1.07;
-    // from 1/4 to 1/2 0.98 to 1.00.
-    // Bilinear rows share theirs with the next one below a vertical scale of 2: 20 x 722 x 418 f32x3 -> 836 x
+    // is shared is half of what is written or more: 168 x 1115 x 34 x 3 -> 375 x 130 36.0 / 54.1, 6 x 1176 x 470 x 3 -> 475 x 1211 14.8 / 22.3, 10 x 530 x 137 x 4 -> 204 x
+    // 496 5.7 / 9.0; 86 launches of f32x3 1.17 times slower along the rows in the mean, 1.08 with inputs that are not in the memory's cache, 79 of f32x4 1.12 and 1.07;
+    // 96 whose waves are filled to 70 .. 80 % 1.11 and 1.07, to 60 .. 70 % 1.02 and 1.01, less 0.89 and 0.95; less shared, from 1/4 to 1/2, 0.98 to 1.00.)
+    // (Bilinear rows share theirs with the next one below a vertical scale of 2: 20 x 722 x 418 f32x3 -> 836 x
     // 484 33.9 us in the 64 x 4 block and 40.7 along the rows, 12 x 399 x 367 f32x4 -> 534 x 492 14.9 and 19.2; at 2.8, 121 x 194 x 594 f32x3 -> 69 x 211,
     // 31.2 and 25.4.)
     // Enlarged rows of 1024 pixels and more start with a block, where they are not counted along the rows: 4 x 720p -> 1080p f32x3 nearest neighbour 22.7 so, 23.7
     // along the rows, 24.6 in the 64 x 4 block; but 16 bytes to a pixel keep that block, 39 launches at 0.90 to 0.95 of the time in the mean.
     const bool shared = (4 * (int64_t)a.srcH <= 3 * (int64_t)a.dstH && a.dstRowStride % 64 == 0
                          && 4 * (int64_t)DivUp(a.dstW, kTileW) * kTileW <= 5 * (int64_t)a.dstW)
-                     || SharedRowsPay(a, kTileW, 2, 1);
+                     || SharedRowsPay(a, kTileW, 2, 1, 70);
     const bool along = INTERP == NVCV_INTERP_NEAREST ? !shared : INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH;
     const bool flat  = INTERP != NVCV_INTERP_CUBIC && (INTERP != NVCV_INTERP_NEAREST || sizeof(Pixel<T, C>) < 16)
                     && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);

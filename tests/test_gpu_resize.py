@@ -880,7 +880,7 @@ def test_tensor_nearest_of_larger_pixels(cv, orc, gpu, size, row_align, c):
                                  for (interp, n, dtype, c, widths) in [(NEAREST, 2, np.float32, 3, (127, 128)), (NEAREST, 2, np.float32, 4, (127, 128)),
                                                                        (CUBIC, 256, np.float32, 1, (341, 342)), (CUBIC, 241, np.float32, 3, (204, 205)),
                                                                        (LINEAR, 256, np.uint8, 4, (426, 427))]
-                                 for (sw, dw) in [(widths[0], 128), (widths[1], 128), (widths[1], 130)]],
+                                 for (sw, dw) in [(widths[0], 128), (widths[1], 128), (widths[1], 130), (2 * widths[1], 135), (2 * widths[1], 134)]],
                          ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensors_whose_rows_share_sources(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
