@@ -3374,21 +3374,23 @@ __device__ __forceinline__ void LoadAreaWindowGuarded(const uint8_t *row, uint32
     }
 }
 
-template<int C, int K, bool PARTIAL, bool REST>
+template<int C, int K, bool PARTIAL, bool REST, int LANES>
 __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a)
 {
     using Window = AreaWindow<C, K>;
     const Plane p    = GetPlanes<false>(a, blockIdx.z);
     const int   lane = threadIdx.x & 63, dx = min((int)blockIdx.x * kTileW + lane, p.dstW - 1);
     const int   dy   = blockIdx.y * kTileH + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (dy >= p.dstH)
+    if (dy >= p.dstH || (lane >= LANES && (int)blockIdx.x * kTileW + lane >= p.dstW))
     {
         return;
     }
-    // (Lanes past the last column work on it again. In a launch that leaves most of the chip idle a wave of 1 to 8 active lanes
-    // issues 2 to 3 times slower than one of more: a kernel of such sums alone, 26 blocks, 14.7 us with 9 to 64 lanes and 48 with
-    // 1 to 8, 512 blocks no difference. One 640 x 480 u8x3 -> 66 x 50 15.0 -> 6.5 us, -> 78 x 50 8.4 -> 6.5; 500 x 480 -> 130 x 50 8.9 ->
-    // 4.9; 6 x 584 x 650 u8x4 -> 68 x 67 18.0 -> 8.5; 64 x 640 x 480 -> 66 x 50 22.2 and 22.4.)
+    // (Of a tile with fewer columns LANES lanes work, those past the last column on it again. In a launch that leaves most of the chip idle a wave of 1 to 8
+    // active lanes issues 2 to 3 times slower than one of more: a kernel of such sums alone, 26 blocks, 14.7 us with 9 to 64 lanes and 48 with
+    // 1 to 8, 512 blocks no difference. One 640 x 480 u8x3 -> 66 x 50 15.1 -> 6.7 us, 500 x 480 -> 130 x 50 9.1 -> 5.1; 6 x 584 x 650 u8x4 -> 68 x 67
+    // 18.1 -> 7.7. Time with 16 / 64 over that with the columns alone, 1200 launches: tiles of 1 to 8 columns, up to 64 blocks 0.73 / 0.69, 1024 0.94 / 0.94, more
+    // 0.98 / 0.98; of 9 to 16, up to 64 0.98 / 0.91, more 1.00 / 0.99; of 17 to 63 0.99 / 0.99 up to 1024 blocks, in large launches 1.00 / 1.03. As an argument that a wave
+    // waits for LANES costs 2 to 5 %.)
     // ResizeValue's terms; the vertical ones are the same in all lanes
     const float fsx1 = dx * p.scaleX, fsx2 = fsx1 + p.scaleX, fsy1 = dy * p.scaleY, fsy2 = fsy1 + p.scaleY;
     const int   xmin = (int)ceilf(fsx1), xmax = (int)floorf(fsx2);
@@ -3539,15 +3541,15 @@ __global__ __launch_bounds__(256) void ResizeAreaWindowKernel(const ResizeArgs a
 // The kernel whose window holds a row of boxes `s` wide.
 using AreaKernelPtr = void (*)(const ResizeArgs);
 
-template<int C, bool PARTIAL, bool REST>
+template<int C, bool PARTIAL, bool REST, int LANES>
 AreaKernelPtr AreaWindowKernel(float s)
 {
-    return s <= 4.f   ? ResizeAreaWindowKernel<C, 4, PARTIAL, REST>
-         : s <= 5.f   ? ResizeAreaWindowKernel<C, 5, PARTIAL, REST>
-         : s <= 6.f   ? ResizeAreaWindowKernel<C, 6, PARTIAL, REST>
-         : s <= 8.f   ? ResizeAreaWindowKernel<C, 8, PARTIAL, REST>
-         : s <= 10.f  ? ResizeAreaWindowKernel<C, 10, PARTIAL, REST>
-                      : ResizeAreaWindowKernel<C, 12, PARTIAL, REST>;
+    return s <= 4.f   ? ResizeAreaWindowKernel<C, 4, PARTIAL, REST, LANES>
+         : s <= 5.f   ? ResizeAreaWindowKernel<C, 5, PARTIAL, REST, LANES>
+         : s <= 6.f   ? ResizeAreaWindowKernel<C, 6, PARTIAL, REST, LANES>
+         : s <= 8.f   ? ResizeAreaWindowKernel<C, 8, PARTIAL, REST, LANES>
+         : s <= 10.f  ? ResizeAreaWindowKernel<C, 10, PARTIAL, REST, LANES>
+                      : ResizeAreaWindowKernel<C, 12, PARTIAL, REST, LANES>;
 }
 
 // Whether rows of the sources start at other places than dwords of memory, where a kernel has a form for that
@@ -4148,8 +4150,13 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             const bool partial = std::ceil(a.scaleX) != a.scaleX;
             const bool wholeY  = std::ceil(a.scaleY) == a.scaleY, batches = wholeY && std::fmod(a.scaleY, (float)kAreaBatch) == 0.f;
             const bool rest    = C == 1 ? !batches : wholeY && !batches && (C == 3 || a.scaleX > 3.f);
-            auto       kernel  = partial ? (rest ? AreaWindowKernel<C, true, true>(a.scaleX) : AreaWindowKernel<C, true, false>(a.scaleX))
-                                         : (rest ? AreaWindowKernel<C, false, true>(a.scaleX) : AreaWindowKernel<C, false, false>(a.scaleX));
+            const auto kernelOf = [&](auto lanes)
+            {
+                constexpr int L = decltype(lanes)::value;
+                return partial ? (rest ? AreaWindowKernel<C, true, true, L>(a.scaleX) : AreaWindowKernel<C, true, false, L>(a.scaleX))
+                               : (rest ? AreaWindowKernel<C, false, true, L>(a.scaleX) : AreaWindowKernel<C, false, false, L>(a.scaleX));
+            };
+            auto kernel = (int64_t)grid.x * grid.y * N <= 4 * 256 ? kernelOf(std::integral_constant<int, 64>{}) : kernelOf(std::integral_constant<int, 16>{});
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
             CheckLaunch("ResizeAreaWindowKernel");
             return;

@@ -498,6 +498,14 @@ def test_area_window_widths(cv, orc, gpu, sw, dw, c):
     np.testing.assert_array_equal(tout.numpy(), orc.resize_shipped(src, (11, dw), AREA, threads=8))
 
 
+# the last tile's lanes without columns: all of them work up to 1024 blocks, beyond that those below 16
+@pytest.mark.parametrize("c", [1, 3, 4])
+@pytest.mark.parametrize("dw", [8, 15, 16, 17, 65, 79, 80, 127])
+@pytest.mark.parametrize("blocks", [1024, 1032])
+def test_area_window_idle_lanes(cv, orc, gpu, blocks, dw, c):
+    test_tensor_table(cv, orc, gpu, (dw * 5 // 2 + 60 // c, 83, dw, 32, AREA, blocks // 8 // -(-dw // 64), np.uint8, c))
+
+
 # boxes of 4 to 11 rows: whole batches of the window form's rows, and one and two rows behind them, with partial rows and not
 @pytest.mark.parametrize("sh", [44, 55, 66, 77, 88, 99, 110, 121, 43, 56, 87, 100])
 @pytest.mark.parametrize("c,dw", [(1, 45), (3, 45), (3, 62), (4, 45), (4, 78)])
