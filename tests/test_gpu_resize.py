@@ -856,6 +856,23 @@ def test_floats_in_views(cv, orc, gpu, n, sw, sh, dw, dh, interp, c):
     assert not torch.isnan(results[0]).any()
 
 
+# Bicubic strips of 4, 8 and 16 rows of three and four channels whose furthest request, the fourth row behind an output row's upper middle one, is the
+# row before the image's last or that row itself: on both sides of what takes the loop without a test for the last row
+@pytest.mark.parametrize("c", [3, 4])
+@pytest.mark.parametrize("rows,n", [(4, 16), (8, 80), (16, 320)])
+@pytest.mark.parametrize("sh", [20, 21, 27, 28, 33, 34, 41, 50, 63])
+def test_cubic_strips_at_the_last_row(cv, orc, gpu, sh, rows, n, c):
+    dw, dh, sw = 256, 64, 201
+    places = np.floor((np.arange(dh, dtype=np.float32) + np.float32(.5)) * (np.float32(sh) / np.float32(dh)) - np.float32(.5))
+    behind = np.clip(places, 1, sh - 3)[rows - 1::rows] + 4 - (sh - 1)  # of each strip; below 0: clear of the last row
+    assert behind.min() < 0 <= behind.max()
+    src = orc.fill_u8((2, sh, sw, c), 40 + sh)
+    out = torch.full((n, dh, dw, c), 7, dtype=torch.uint8, device="cuda")
+    cv.Resize()(None, cv.Tensor.from_torch(torch.from_numpy(src[np.arange(n) % 2]).cuda(), "NHWC"), cv.Tensor.from_torch(out, "NHWC"), CUBIC)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy(), orc.resize_shipped(src, (dh, dw), CUBIC, threads=8)[np.arange(n) % 2])
+
+
 # Images whose waves, counted along the rows, fill a multiple of 16 blocks, which get one more: in the forms that are counted so
 @pytest.mark.parametrize("row", [(300, 20, 1021, 64, NEAREST, 48, np.uint8, 3), (300, 20, 1021, 64, NEAREST, 48, np.uint8, 1),
                                  (1100, 80, 1021, 64, NEAREST, 80, np.uint8, 1), (200, 50, 256, 64, CUBIC, 16, np.uint8, 3),
