@@ -21,7 +21,8 @@ static void EveryTileOnce(int w, int h, int tileW, int tileH, int waves, const W
 {
     const WaveBlocks blocks = BlocksOfWaves(w, h, tileW, tileH, order, waves);
     const int        across = (w + tileW - 1) / tileW, down = (h + tileH - 1) / tileH;
-    Check(order.across == 0 || blocks.x % 16 != 0, "blocks", w, h, tileW, tileH, waves);
+    Check(order.across == 0 || waves == 1 || blocks.x % 16 != 0, "blocks", w, h, tileW, tileH, waves);
+    Check(waves > 1 || (int64_t)blocks.x * blocks.y == (int64_t)across * down, "single waves", w, h, tileW, tileH, waves);
     std::vector<int> seen((size_t)across * down);
     for (uint32_t y = 0; y < blocks.y; ++y)
     {
@@ -50,7 +51,7 @@ static void Ends(int w, int h, int tileW, int tileH, int waves, bool counted)
     const WaveOrder  order  = AlongRows(w, h, tileW, tileH);
     const WaveBlocks blocks = BlocksOfWaves(w, h, tileW, tileH, order, waves);
     Check((order.across != 0) == counted, "order", w, h, tileW, tileH, waves);
-    Check(order.across == 0 || blocks.x % 16 != 0, "blocks", w, h, tileW, tileH, waves);
+    Check(order.across == 0 || waves == 1 || blocks.x % 16 != 0, "blocks", w, h, tileW, tileH, waves);
     Check((uint64_t)blocks.x * 64 * (uint64_t)waves < (uint64_t)1 << 32, "threads", w, h, tileW, tileH, waves);
     if (order.across == 0)
     {
