@@ -838,14 +838,18 @@ __device__ __forceinline__ void ResizePixel(const Plane &p, int dx, int dy)
 }
 
 // The tile (in units of a wave's tile) of this wave in a launch of the tensor kernels below. Counted along the rows of tiles, a block
-// writes and reads few long row pieces instead of many short ones, which the memory likes better, and no wave of a block stands
-// outside the image, as where a block's four waves stood side by side (rows of 1024 pixels and more) or below one another. us
+// writes and reads few long row pieces instead of many short ones, which the memory likes better, and only an image's last block has waves
+// outside it, where many had as a block's four stood side by side (rows of 1024 pixels and more) or below one another. us
 // as they stood / counted along the rows: bicubic u8x3 182 x 219 x 77 -> 593 x 209 41.6 / 28.7, 101 x 241 x 274 -> 572 x 655 56.3 / 42.9, 40 x 300 x 300 -> 600 x
 // 600 24.6 / 21.8, 32 x 720p -> 1080p 90.1 / 86.4; u8x4 40 x 300 x 300 -> 600 x 600 22.7 / 20.5; nearest neighbour u8x4 200 x 86 x 80 -> 307 x 287 22.5 / 18.3,
 // u8x3 50 x 209 x 770 -> 362 x 1335 25.2 / 19.5; box filter u8x3 4 x 3146 x 1185 -> 1646 x 620 25.5 / 20.6, u8x1 171 x 1723 x 388 -> 609 x 137 65.7 / 57.3; wave
-// patches, bilinear u8x3 193 x 171 x 925 -> 68 x 367 30.9 / 26.9, u8x4 12 x 702 x 2707 -> 466 x 1447 26.5 / 22.7. The bilinear strips of 8-bit pixels
-// alone lose by it where rows are short (u8x3 80 x 650 x 104 -> 1274 x 195 24.0 / 29.5, u8x4 190 x 307 x 16 -> 942 x 50 14.9 / 16.7): they count along rows of
-// 1024 pixels and more that fill blocks to 80 % (FlatBlocks) and stand below one another otherwise.
+// patches, bilinear u8x3 193 x 171 x 925 -> 68 x 367 30.9 / 26.9, u8x4 12 x 702 x 2707 -> 466 x 1447 26.5 / 22.7. Means over 280 to 490 random launches each, inputs in and out of
+// the memory's cache: nearest neighbour u8x4 0.92 and 0.94, f32x1 0.91 and 0.93, bicubic u8x1 and u8x4 0.96 and 0.97, f32x1 0.94 and 0.95, box filter 0.97 to 0.99.
+// Single launches lose in all of these, u8x4 nearest neighbour among them that starts rows with a block no more: 37 x 572 x 202 -> 1707 x 622 39.7 / 43.0, 39 x 899 x 224 -> 1983 x 447
+// 34.3 / 37.4, but 72 x 1402 x 50 -> 3280 x 117 26.1 / 21.3, 15 x 1101 x 195 -> 3632 x 646 28.5 / 26.0, 65 of these 0.99 in the mean. Not counted so: the bilinear strips of
+// 8-bit pixels whose rows are short (u8x3 80 x 650 x 104 -> 1274 x 195 24.0 / 29.5, u8x4 190 x 307 x 16 -> 942 x 50 14.9 / 16.7; those of
+// 1024 pixels and more that fill blocks to 80 % are: FlatBlocks), rows that share what they read (SharedRowsPay), the bicubic strips of four floats and of
+// few waves, one-pixel waves of bilinear and bicubic and the staged bicubic below vertical scales of 2 and 4: beside their launches.
 __device__ __forceinline__ WaveTile WaveTileOf(const WaveOrder &order)
 {
     // (the wave's number as a scalar: tile origins, row terms and loop counters then stay on the scalar unit)
@@ -2055,8 +2059,8 @@ __device__ __forceinline__ void ResizeNearestQuadStripU8(const Plane &p, int x0,
 // the strips, but each of its R rows comes from a window of its own, DWORDS dwords from the one of the lane's first source
 // pixel on. Bound by the writes: the wave patches' rows of 64 pixels (64 bytes of one channel, mostly not at a sector's start) end in
 // partly written sectors twice for each, these rows of 256 once for four, and four pixels are one load instead of four. One
-// channel, 40 MB each: by 1.3 20.7 -> 11.9 us, by 2 14.8 -> 10.8, by 3 13.6 -> 10.9; 200 x 258 x 752 -> 244 x 711 37.5 -> 19.0. Three channels enlarged
-// across alone (117 x 453 x 113 -> 455 x 84) 10.2 -> 7.7.
+// channel, with inputs out of the memory's cache: 24 x 1300 x 1300 -> 1000 x 1000 26.9 -> 14.1 us, 12 x 1800 x 1800 -> 900 x 900 14.1 -> 10.2, 4 x 3000 x 3000 -> 1000 x 1000 7.9 ->
+// 7.3 (in it 22.5 -> 9.8, 11.3 -> 6.3, 5.4 -> 4.8); 200 x 258 x 752 -> 244 x 711 36.7 -> 19.0. Three channels enlarged across alone (117 x 453 x 113 -> 455 x 84) 12.0 -> 10.3.
 constexpr int kNearestRows = 4;
 
 template<int C, int DWORDS>
@@ -2371,8 +2375,8 @@ __global__ __launch_bounds__(256) void ResizeLinearPairsU8VarShapeKernel(const R
 }
 
 // Large image-batch launches resize each image in the tensor kernels' strips; a wave owns a tile of 256 x 8 (WIDE: most of
-// the launch is enlarged by 1.5 or more) or 128 x 4 output pixels, a block four of them, side by side or stacked as
-// in the tensor kernels (WaveTileOf; the host chooses by the images' widths). WIDE: four columns per lane where the
+// the launch is enlarged by 1.5 or more) or 128 x 4 output pixels, a block four of them, side by side or stacked
+// (VarWaveTileOf; the host chooses by the images' widths). WIDE: four columns per lane where the
 // image is enlarged so, else two columns per lane at horizontal scales up to 2 (4 strips of 128 x 4), else 8 wave
 // patches. Otherwise a two-column strip, or two wave patches.
 template<bool WIDE>
