@@ -1067,7 +1067,7 @@ def resize_crop_convert_reformat(src, resize_dim, interp, crop_rect, *, layout="
     rect = crop_rect if type(crop_rect) is RectI else RectI(*crop_rect)
     height, width = int(rect.height), int(rect.width)
     if isinstance(src, _ImageBatchVarShape):
-        status, count, fmt = _native.batch_state(src.handle.value)
+        status, count, fmt = _native.batch_state(src.handle.value if src.handle else 0)  # (0 once it is closed: an error)
         if status:
             check(status)
         if fmt not in _PLANE_NP:

@@ -2,6 +2,7 @@
 first name of the reference's headers, as its table of output formats does, python/mod_cvcuda/CvtColorUtil.cpp:30-42),
 the output shapes and formats of cvtcolor (CvtColorUtil.cpp:244-330) and the argument checks the reference's bindings
 make themselves."""
+import ctypes as C
 import importlib
 import os
 import shutil
@@ -606,6 +607,16 @@ assert [g() for g in gone] == [None] * 5, gone
         with pytest.raises(RuntimeError):
             call()
     empty.put(api.Tensor(_wrap=object()))
+
+
+@pytest.mark.parametrize("handle", [None, C.c_void_p()])
+def test_a_closed_image_batch_is_an_invalid_argument(api, handle):
+    batch = api.ImageBatchVarShape.__new__(api.ImageBatchVarShape)
+    batch.handle, batch._keep = handle, []
+    for use in (lambda: len(batch), lambda: batch.uniqueformat,
+                lambda: api.resize_crop_convert_reformat(batch, (4, 4), api.Interp.LINEAR, api.RectI(0, 0, 4, 4))):
+        with pytest.raises(api.Error, match="NVCV_ERROR_INVALID_ARGUMENT"):
+            use()
 
 
 def test_results_alive_at_the_end_of_the_program_say_nothing():
