@@ -501,9 +501,9 @@ def test_area_window_widths(cv, orc, gpu, sw, dw, c):
 # the last tile's lanes without columns: all of them work up to 1024 blocks, beyond that those below 16
 @pytest.mark.parametrize("c", [1, 3, 4])
 @pytest.mark.parametrize("dw", [8, 15, 16, 17, 65, 79, 80, 127])
-@pytest.mark.parametrize("blocks", [1024, 1032])
+@pytest.mark.parametrize("blocks", [1024, 1040])
 def test_area_window_idle_lanes(cv, orc, gpu, blocks, dw, c):
-    test_tensor_table(cv, orc, gpu, (dw * 5 // 2 + 60 // c, 83, dw, 32, AREA, blocks // 8 // -(-dw // 64), np.uint8, c))
+    test_tensor_table(cv, orc, gpu, (dw * 7 // 2 + 60 // c, 83, dw, 32, AREA, blocks // 8 // -(-dw // 64), np.uint8, c))
 
 
 # boxes of 4 to 11 rows: whole batches of the window form's rows, and one and two rows behind them, with partial rows and not
@@ -877,7 +877,7 @@ def test_cubic_strips_at_the_last_row(cv, orc, gpu, sh, rows, n, c):
 @pytest.mark.parametrize("row", [(300, 20, 1021, 64, NEAREST, 48, np.uint8, 3), (300, 20, 1021, 64, NEAREST, 48, np.uint8, 1),
                                  (1100, 80, 1021, 64, NEAREST, 80, np.uint8, 1), (200, 50, 256, 64, CUBIC, 16, np.uint8, 3),
                                  (200, 50, 256, 64, CUBIC, 16, np.uint8, 4), (600, 160, 256, 64, AREA, 3, np.uint8, 3),
-                                 (900, 200, 256, 64, LINEAR, 3, np.uint8, 1), (200, 12, 256, 16, NEAREST, 3, np.float32, 3),
+                                 (900, 200, 256, 64, LINEAR, 128, np.uint8, 1), (200, 20, 256, 16, NEAREST, 3, np.float32, 3),
                                  (200, 100, 256, 128, CUBIC, 64, np.float32, 1), (700, 40, 256, 16, LINEAR, 3, np.float32, 4)],
                          ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensors_of_16_blocks(cv, orc, gpu, row):
@@ -900,12 +900,13 @@ def test_tensor_nearest_of_larger_pixels(cv, orc, gpu, size, row_align, c):
     np.testing.assert_array_equal(tout.numpy(), orc.resize(src, (dh, dw), NEAREST, variant=0))
 
 
-# Rows that share what they read, on both sides of what keeps a block's waves below one another
-@pytest.mark.parametrize("row", [(sw, 32, dw, 64, interp, n, dtype, c)
-                                 for (interp, n, dtype, c, widths) in [(NEAREST, 2, np.float32, 3, (127, 128)), (NEAREST, 2, np.float32, 4, (127, 128)),
-                                                                       (CUBIC, 256, np.float32, 1, (341, 342)), (CUBIC, 241, np.float32, 3, (204, 205)),
-                                                                       (LINEAR, 256, np.uint8, 4, (426, 427))]
-                                 for (sw, dw) in [(widths[0], 128), (widths[1], 128), (widths[1], 130), (2 * widths[1], 135), (2 * widths[1], 134)]],
+# Rows that share what they read, on both sides of what keeps a block's waves below one another: as much as they write of it, and waves filled to
+# 70 or 80 %
+@pytest.mark.parametrize("row", [(sw, 32, dw, 64, interp, 2 * n // -(-dw // 64), dtype, c)
+                                 for (interp, n, dtype, c, least, w, full) in [(NEAREST, 3, np.float32, 3, 140, 140, 135), (NEAREST, 3, np.float32, 4, 140, 140, 135),
+                                                                               (CUBIC, 384, np.float32, 1, 342, 128, 154), (CUBIC, 243, np.float32, 3, 205, 128, 154),
+                                                                               (LINEAR, 384, np.uint8, 4, 427, 128, 154)]
+                                 for (sw, dw) in [(least - 1, w), (least, w), (least, 130), (least * full // w + 2, full), (least * full // w + 2, full - 1)]],
                          ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensors_whose_rows_share_sources(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
