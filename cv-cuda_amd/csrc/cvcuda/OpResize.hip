@@ -881,8 +881,11 @@ template<class T, int C, int INTERP>
 __global__ __launch_bounds__(256) void ResizeTensorKernel(const ResizeArgs a, const WaveOrder order)
 {
     // (the wave's number as a vector here, where a wave is one pixel per lane: with scalar places the store's address waits for the scalar unit. Nearest
-    // neighbour f32x3 19 x 1750 x 278 -> 826 x 706 47.5 us, so 44.2, 2 x 1636 x 1610 -> 1433 x 4096 48.5 and 44.1, others 0.98 to 1.00)
-    const WaveTile t  = TileOfWave(order, blockIdx.x, blockIdx.y, threadIdx.x >> 6, 4);
+    // neighbour f32x3 19 x 1750 x 278 -> 826 x 706 47.5 us, so 44.2, 2 x 1636 x 1610 -> 1433 x 4096 48.5 and 44.1, others 0.98 to 1.00. Not for box sums, whose
+    // loops over rows the scalar unit counts: u8x1 1.07 times slower in the mean of 134 launches as a vector, 3 x 2106 x 1884 -> 12 x 27 418 and 492, u8x3 1.03, f32x1
+    // 1.04; of three and four floats 0.99, u8x4 1.00)
+    constexpr bool kScalar = INTERP == NVCV_INTERP_AREA && sizeof(Pixel<T, C>) <= 4;
+    const WaveTile t  = kScalar ? WaveTileOf(order) : TileOfWave(order, blockIdx.x, blockIdx.y, threadIdx.x >> 6, 4);
     const int      dx = t.x * kTileW + (threadIdx.x & 63), dy = t.y;
     if (dx >= a.dstW || dy >= a.dstH)
     {
