@@ -863,11 +863,18 @@ static inline bool FlatBlocks(int dstW, int waveW)
 }
 
 // Whether the source pixels that the output rows of a stacked block need not fetch again, because the row above has, are `of` / `in` of the
-// pixels written or more, and the rows fill their waves to `full` per cent. Such launches lose along the rows.
-static inline bool SharedRowsPay(const ResizeArgs &a, int waveW, int in, int of, int full = 80)
+// pixels written or more, the rows fill their waves of waveW x waveH to `full` per cent and the columns their blocks of four to 3/4 (6909 x 211 x 2 f32x1 bicubic ->
+// 107 x 17, one row in a second block of 16: 46.8 us along the rows, 68.7 below one another). Such launches lose along the rows, where blocks on all XCDs fetch a source row for
+// the output rows that it serves: as many of them as rows, up to 8. So they do not where the source has less than 1 / `times` of the pixels written,
+// which 8 caches take little time to fetch (the more output rows to a source row, the wider the sources that still lose). Time over that along the rows, 1000 to 1900
+// random launches of each form enlarged 1.3 to 90 times, inputs in the memory's cache, with sources and columns of any size / so: nearest neighbour 0.84 / 0.79, bilinear u8x4
+// 0.94 / 0.93, bicubic f32x3 1.02 / 0.99, f32x1 0.85 / 0.86, the slowest of it 1.47 / 1.26. Just outside `times` nearest neighbour takes 1.03 to 1.14 below one another, u8x4 1.04 to
+// 1.09, f32x3 1.03, f32x1 1.02 to 1.07.
+static inline bool SharedRowsPay(const ResizeArgs &a, int waveW, int waveH, int in, int of, int times, int full = 80)
 {
     return in * (int64_t)(a.dstH - a.srcH) * a.srcW >= of * (int64_t)a.dstW * a.dstH
-        && full * (int64_t)DivUp(a.dstW, waveW) * waveW <= 100 * (int64_t)a.dstW;
+        && times * (int64_t)a.srcW * a.srcH >= (int64_t)a.dstW * a.dstH
+        && full * (int64_t)DivUp(a.dstW, waveW) * waveW <= 100 * (int64_t)a.dstW && 3 * (int64_t)DivUp(a.dstH, 4 * waveH) * 4 * waveH <= 4 * (int64_t)a.dstH;
 }
 
 // Grid of a launch whose waves own tiles of waveW x waveH.
@@ -4050,7 +4057,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
             // waves of 4 rows, 6.4 and 7.3; four 44 x 286 x 59 -> 1071 x 223 48.6 and 42.5, but 128 x 104 x 88 -> 106 x 90 9.7 and 11.5. Not
             // three channels that share 4/5 of what is written: 189 x 424 x 66 -> 276 x 139 30.7 and 35.9, 1 x 955 x 1954 -> 521 x 4096 10.3 and 13.5, 33 launches up
             // to 4/3 1.04 times slower along the rows in the mean, from 1/4 to 2/3 0.97 to 0.98; one channel there 1.00.)
-            const bool along     = C != 4 && rows > 4 && !(C == 3 && SharedRowsPay(a, kTileW, 5, 4));
+            const bool along     = C != 4 && rows > 4 && !(C == 3 && SharedRowsPay(a, kTileW, rows, 5, 4, 4));
             const auto order     = along ? AlongRows(a.dstW, a.dstH, kTileW, rows) : WaveOrder{};
             hipLaunchKernelGGL((ResizeCubicStripF32Kernel<C>), WaveTileGrid(a.dstW, a.dstH, N, kTileW, rows, order), dim3(256), 0, stream, a,
                                rows, order);
@@ -4258,7 +4265,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
         // to 1.00. Smaller pixels and bilinear f32x1: 0.98 to 1.00.)
         constexpr bool kCubicF = std::is_same_v<T, float> && C == 1 && INTERP == NVCV_INTERP_CUBIC,
                        kLinear4 = std::is_same_v<T, uint8_t> && C == 4 && INTERP == NVCV_INTERP_LINEAR;
-        const bool shared = waves == 4 && ((kCubicF && SharedRowsPay(a, kPatchTileW, 3, 4)) || (kLinear4 && SharedRowsPay(a, kPatchTileW, 3, 5)));
+        const bool shared = waves == 4 && ((kCubicF && SharedRowsPay(a, kPatchTileW, 4, 3, 4, 8)) || (kLinear4 && SharedRowsPay(a, kPatchTileW, 4, 3, 5, 4)));
         const auto order = shared ? WaveOrder{} : AlongRows(a.dstW, a.dstH, kPatchTileW, 4);
         constexpr bool kOdd   = INTERP == NVCV_INTERP_CUBIC && kFixedCubic<T> && C != 4;
         auto           kernel = kOdd && RowsAreOdd<C>(a) ? ResizePatchTensorKernel<T, C, INTERP, kOdd> : ResizePatchTensorKernel<T, C, INTERP, false>;
@@ -4285,7 +4292,7 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     // along the rows, 24.6 in the 64 x 4 block; but 16 bytes to a pixel keep that block, 39 launches at 0.90 to 0.95 of the time in the mean.
     const bool shared = (4 * (int64_t)a.srcH <= 3 * (int64_t)a.dstH && a.dstRowStride % 64 == 0
                          && 4 * (int64_t)DivUp(a.dstW, kTileW) * kTileW <= 5 * (int64_t)a.dstW)
-                     || SharedRowsPay(a, kTileW, 2, 1, 70);
+                     || SharedRowsPay(a, kTileW, 1, 2, 1, 10, 70);
     const bool along = INTERP == NVCV_INTERP_NEAREST ? !shared : INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH;
     const bool flat  = INTERP != NVCV_INTERP_CUBIC && (INTERP != NVCV_INTERP_NEAREST || sizeof(Pixel<T, C>) < 16)
                     && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);

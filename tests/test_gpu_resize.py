@@ -900,13 +900,18 @@ def test_tensor_nearest_of_larger_pixels(cv, orc, gpu, size, row_align, c):
     np.testing.assert_array_equal(tout.numpy(), orc.resize(src, (dh, dw), NEAREST, variant=0))
 
 
-# Rows that share what they read, on both sides of what keeps a block's waves below one another: as much as they write of it, and waves filled to
-# 70 or 80 %
-@pytest.mark.parametrize("row", [(sw, 32, dw, 64, interp, 2 * n // -(-dw // 64), dtype, c)
-                                 for (interp, n, dtype, c, least, w, full) in [(NEAREST, 3, np.float32, 3, 140, 140, 135), (NEAREST, 3, np.float32, 4, 140, 140, 135),
-                                                                               (CUBIC, 384, np.float32, 1, 342, 128, 154), (CUBIC, 243, np.float32, 3, 205, 128, 154),
-                                                                               (LINEAR, 384, np.uint8, 4, 427, 128, 154)]
-                                 for (sw, dw) in [(least - 1, w), (least, w), (least, 130), (least * full // w + 2, full), (least * full // w + 2, full - 1)]],
+# Rows that share what they read, on both sides of what keeps a block's waves below one another: as much as they write of it, waves filled to
+# 70 or 80 %, blocks to 3/4, and sources of no less than a tenth, an eighth or a fourth of what is written
+@pytest.mark.parametrize("row", [(sw, sh, dw, 64, interp, 2 * n // -(-dw // 64), dtype, c)
+                                 for (interp, n, dtype, c, least, w, full, small) in [(NEAREST, 3, np.float32, 3, 140, 140, 135, (224, 4)), (NEAREST, 3, np.float32, 4, 140, 140, 135, (224, 4)),
+                                                                                      (CUBIC, 384, np.float32, 1, 342, 128, 154, (256, 4)),
+                                                                                      (CUBIC, 243, np.float32, 3, 205, 128, 154, (205, 10)),
+                                                                                      (LINEAR, 384, np.uint8, 4, 427, 128, 154, (256, 8))]
+                                 for (sw, sh, dw) in [(least - 1, 32, w), (least, 32, w), (least, 32, 130), (least * full // w + 2, 32, full),
+                                                      (least * full // w + 2, 32, full - 1), (small[0] - 1, small[1], w), (small[0], small[1], w)]]
+                                + [(sw, 8, 128, dh, interp, 512, dtype, c) for (sw, interp, dtype, c) in [(300, CUBIC, np.float32, 1), (400, LINEAR, np.uint8, 4)]
+                                   for dh in (23, 24)]
+                                + [(300, 2, 140, dh, NEAREST, 3, np.float32, c) for c in (3, 4) for dh in (5, 6)],
                          ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensors_whose_rows_share_sources(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
