@@ -4289,12 +4289,14 @@ void LaunchTensor(const ResizeArgs &a, int N, hipStream_t stream)
     // 484 33.9 us in the 64 x 4 block and 40.7 along the rows, 12 x 399 x 367 f32x4 -> 534 x 492 14.9 and 19.2; at 2.8, 121 x 194 x 594 f32x3 -> 69 x 211,
     // 31.2 and 25.4.)
     // Enlarged rows of 1024 pixels and more start with a block, where they are not counted along the rows: 4 x 720p -> 1080p f32x3 nearest neighbour 22.7 so, 23.7
-    // along the rows, 24.6 in the 64 x 4 block; but 16 bytes to a pixel keep that block, 39 launches at 0.90 to 0.95 of the time in the mean.
+    // along the rows, 24.6 in the 64 x 4 block; but 16 bytes to a pixel keep that block, 39 launches at 0.90 to 0.95 of the time in the mean, and so do nearest
+    // neighbour's 12 unless a row has a multiple of 8 blocks, which puts a column's rows on one XCD (there 0.79 of the time along the rows, 0.93 in the 64 x 4
+    // block, 73 launches; others 0.73 to 1.27 and 0.68 to 0.82 in their means, 4 x 6565 x 24 -> 2113 x 153 5.5 along the rows, 10.7 so).
     const bool shared = (4 * (int64_t)a.srcH <= 3 * (int64_t)a.dstH && a.dstRowStride % 64 == 0
                          && 4 * (int64_t)DivUp(a.dstW, kTileW) * kTileW <= 5 * (int64_t)a.dstW)
                      || SharedRowsPay(a, kTileW, 1, 2, 1, 10, 70);
     const bool along = INTERP == NVCV_INTERP_NEAREST ? !shared : INTERP == NVCV_INTERP_LINEAR && a.srcH >= 2 * (int64_t)a.dstH;
-    const bool flat  = INTERP != NVCV_INTERP_CUBIC && (INTERP != NVCV_INTERP_NEAREST || sizeof(Pixel<T, C>) < 16)
+    const bool flat  = INTERP != NVCV_INTERP_CUBIC && (INTERP != NVCV_INTERP_NEAREST || (sizeof(Pixel<T, C>) < 16 && DivUp(a.dstW, 4 * kTileW) % 8 == 0))
                     && (int64_t)a.dstW * a.dstH > (int64_t)a.srcW * a.srcH && FlatBlocks(a.dstW, kTileW);
     const auto order = along ? AlongRows(a.dstW, a.dstH, kTileW, 1)
                      : flat  ? AlongRows(DivUp(a.dstW, 4 * kTileW) * 4 * kTileW, a.dstH, kTileW, 1)

@@ -901,7 +901,8 @@ def test_tensor_nearest_of_larger_pixels(cv, orc, gpu, size, row_align, c):
 
 
 # Rows that share what they read, on both sides of what keeps a block's waves below one another: as much as they write of it, waves filled to
-# 70 or 80 %, blocks to 3/4, and sources of no less than a tenth, an eighth or a fourth of what is written
+# 70 or 80 %, blocks to 3/4, and sources of no less than a tenth, an eighth or a fourth of what is written; and rows of 8 blocks and
+# of others
 @pytest.mark.parametrize("row", [(sw, sh, dw, 64, interp, 2 * n // -(-dw // 64), dtype, c)
                                  for (interp, n, dtype, c, least, w, full, small) in [(NEAREST, 3, np.float32, 3, 140, 140, 135, (224, 4)), (NEAREST, 3, np.float32, 4, 140, 140, 135, (224, 4)),
                                                                                       (CUBIC, 384, np.float32, 1, 342, 128, 154, (256, 4)),
@@ -911,7 +912,8 @@ def test_tensor_nearest_of_larger_pixels(cv, orc, gpu, size, row_align, c):
                                                       (least * full // w + 2, 32, full - 1), (small[0] - 1, small[1], w), (small[0], small[1], w)]]
                                 + [(sw, 8, 128, dh, interp, 512, dtype, c) for (sw, interp, dtype, c) in [(300, CUBIC, np.float32, 1), (400, LINEAR, np.uint8, 4)]
                                    for dh in (23, 24)]
-                                + [(300, 2, 140, dh, NEAREST, 3, np.float32, c) for c in (3, 4) for dh in (5, 6)],
+                                + [(300, 2, 140, dh, NEAREST, 3, np.float32, c) for c in (3, 4) for dh in (5, 6)]
+                                + [(sw, 4, dw, 9, NEAREST, 2, np.float32, 3) for (sw, dw) in [(2000, 1800), (2000, 1793), (2000, 1791), (2400, 2100)]],
                          ids=lambda r: "%dx%d-%dx%d-i%d-n%d-%s-c%d" % (r[:6] + (np.dtype(r[6]).name, r[7])))
 def test_tensors_whose_rows_share_sources(cv, orc, gpu, row):
     test_tensor_table(cv, orc, gpu, row)
